@@ -68,6 +68,7 @@ struct DevPool {
         blocks.erase(blocks.begin() + best);
         return p;
     }
+    bool fits(size_t bytes) const { return ((bytes + 255) & ~size_t(255)) <= arena_size - arena_used; }
     void give(void *p, size_t cap) {
         std::lock_guard<std::mutex> lk(mu);
         if (arena) return;

@@ -293,6 +293,8 @@ ag_status ag_plan_destroy(ag_plan *plan);
  * path uses with the one the reference's FP64 distance gives.
  *   far_pairs            pairs handled by the far-field kernel (r > 8 A)
  *   far_bin_flips        of those, pairs whose FP32 bin differs from FP64
+ *                        (the e map takes a bin only for atoms near the point's
+ *                        patch; the others' terms are interpolated)
  *   near_unguarded_flips near pairs whose FP32 bin differs from FP64 outside
  *                        the FP64 recompute band (0 unless the band is too
  *                        narrow)
