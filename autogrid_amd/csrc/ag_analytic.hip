@@ -16,10 +16,10 @@
 // desolvation, d map) is the reference's.
 //
 // Kernels (FP32):
-//   k_an_near   one lane per grid point over the atoms within 8 A (host-built
-//               cell list): affinity, covalent and d maps, plus the tape the
-//               adjoint needs (closest H, the atoms that gave each point's
-//               H-bond min and max);
+//   k_an_near   one workgroup per cube of 4x4x4 points, its four waves sharing
+//               the atoms within 8 A (host-built cell list): affinity, covalent
+//               and d maps, plus the tape the adjoint needs (closest H, the
+//               atoms that gave each point's H-bond min and max);
 //   k_an_e      runs of 13 or 16 points along x per lane over one chunk of
 //               atoms, and k_an_esum the chunks' sums per point: the e map;
 //   k_an_vh     one lane per grid point: the cotangent of the closest H's
@@ -88,6 +88,16 @@ struct APair {            // one (map, receptor type) pair potential
     int a, b, expl;
 };
 
+struct __align__(16) ANear {   // E = c1 (R/s)^a - c2 (R/s)^b, capped (R = 1 for nbp_coeffs pairs)
+    float R, c1, c2, rstar;
+};
+struct __align__(16) ANearType {   // of one receptor type: the forward's form of its pairs
+    ANear pair[kAMaxAff];
+    int form;                      // 2 bits per map: exponents 12-6 (0), 12-10 (1), others (2)
+    int pad[3];
+    int a[kAMaxAff], b[kAMaxAff];
+};
+
 struct AParams {
     int n1[3], ne[3];
     float h;                          // spacing
@@ -108,6 +118,8 @@ struct AParams {
     double cov_pos[3], cov_hw, cov_barrier;
     int d_slot;
     const APair *pairs;               // [naff][T]
+    const ANearType *near_pairs;      // [T]
+    int case_word[7];                 // per atom class, 2 bits per map: its CASE_*
     int T;
     float w_smooth;                   // half window (A)
     float w_desolv, qasp;
@@ -291,52 +303,26 @@ __device__ __forceinline__ void cell_range(const AParams &p, const float c[3], i
     }
 }
 
-// Closest donor H within 8 A of c (lowest index on ties), or -1.
-__device__ __forceinline__ int closest_h(const AParams &p, const float c[3]) {
-    int lo[3], hi[3];
-    cell_range(p, c, lo, hi);
-    float best = 1e30f;
-    int bidx = -1;
-    for (int gz = lo[2]; gz <= hi[2]; gz++)
-        for (int gy = lo[1]; gy <= hi[1]; gy++) {
-            const int row = p.nc[0] * (gy + p.nc[1] * gz);
-            const int s0 = p.cell_start[row + lo[0]], s1 = p.cell_start[row + hi[0] + 1];
-            for (int s = s0; s < s1; s++) {
-                const AAtom &a = p.atoms[s];
-                const int hb = (a.meta >> 8) & 0xff;
-                if (hb != AG_HB_DS && hb != AG_HB_D1) continue;
-                const float dx = a.x - c[0], dy = a.y - c[1], dz = a.z - c[2];
-                const float r2 = dx * dx + dy * dy + dz * dz;
-                if (r2 < best || (r2 == best && a.index < bidx)) {
-                    best = r2;
-                    bidx = a.index;
-                }
-            }
-        }
-    return best < kCut2 ? bidx : -1;
-}
-
 // Per-pair directional factors (forward).
 struct Dir {
     float racc, rdon, Hramp;
 };
-__device__ __forceinline__ Dir dir_of(const AAtom &a, int hb, const float dn[3], int closest, const float *rvH) {
+__device__ __forceinline__ Dir dir_of(const float rv[3], const float rv2[3], int rexp, int index, int hb,
+                                      const float dn[3], int closest, const float *rvH) {
     Dir o{1.f, 1.f, 1.f};
+    const float c = -(dn[0] * rv[0] + dn[1] * rv[1] + dn[2] * rv[2]);
     if (hb == AG_HB_D1) {
-        const float c = -(dn[0] * a.rv[0] + dn[1] * a.rv[1] + dn[2] * a.rv[2]);
         float dc;
-        o.racc = racc_of(c, (a.meta >> 16) & 0xff, dc);
-        if (c > 0.f && a.index != closest && closest >= 0) {
-            const float ct = rvH[0] * a.rv[0] + rvH[1] * a.rv[1] + rvH[2] * a.rv[2];
-            float dct;
-            o.Hramp = hramp_of(ct, dct);
+        o.racc = racc_of(c, rexp, dc);
+        if (c > 0.f && index != closest && closest >= 0) {
+            const float ct = rvH[0] * rv[0] + rvH[1] * rv[1] + rvH[2] * rv[2];
+            o.Hramp = hramp_value(fminf(fmaxf(ct, -1.f), 1.f));
         }
     } else if (hb == AG_HB_A1) {
-        const float c = -(dn[0] * a.rv[0] + dn[1] * a.rv[1] + dn[2] * a.rv[2]);
         o.rdon = c > 0.f ? c * c : 0.f;
     } else if (hb == AG_HB_A2) {
         float g3[3] = {0, 0, 0};
-        o.rdon = a2_rdon<false>(dn, a.rv, a.rv2, 0.f, g3, g3, g3);
+        o.rdon = a2_rdon<false>(dn, rv, rv2, 0.f, g3, g3, g3);
     }
     return o;
 }
@@ -345,94 +331,364 @@ __device__ __forceinline__ Dir dir_of(const AAtom &a, int hb, const float dn[3],
 // forward
 // ---------------------------------------------------------------------------
 
+constexpr int kCube = 4;                 // edge of a workgroup's cube of points
+constexpr int kCubeCap = 1024;           // atoms in the workgroup's list
+constexpr int kCubeHCap = 256;           // donor H in its list
+
+#define AN_CONST __attribute__((address_space(4)))
+
+// A workgroup's cube of points: its corner, this lane's point and the cells
+// around its box (points past the grid's end are clamped onto the last one).
+struct Cube {
+    int ix, iy, iz;          // this lane's point
+    bool inside;
+    float c[3];              // its position
+    float lo[3], hi[3];      // the cube's box
+    int clo[3], chi[3];      // cells overlapping the box grown by 8 A
+};
+__device__ __forceinline__ Cube cube_of(const AParams &p, int block) {
+    Cube q;
+    const int nx = (p.n1[0] + kCube - 1) / kCube, ny = (p.n1[1] + kCube - 1) / kCube;
+    const int b[3] = {block % nx, (block / nx) % ny, block / (nx * ny)};
+    const int lane = threadIdx.x & 63;
+    const int i[3] = {kCube * b[0] + (lane & 3), kCube * b[1] + ((lane >> 2) & 3), kCube * b[2] + (lane >> 4)};
+    q.inside = true;
+    int j[3];
+    for (int d = 0; d < 3; d++) {
+        q.inside = q.inside && i[d] < p.n1[d];
+        j[d] = min(i[d], p.n1[d] - 1);
+        q.c[d] = (float)(j[d] - p.ne[d]) * p.h;
+        q.lo[d] = (float)(kCube * b[d] - p.ne[d]) * p.h;
+        q.hi[d] = (float)(min(kCube * b[d] + kCube, p.n1[d]) - 1 - p.ne[d]) * p.h;
+        // the margin keeps FP32 rounding of an atom's cell from losing it
+        q.clo[d] = max(0, __builtin_amdgcn_readfirstlane((int)floorf((q.lo[d] - 8.01f - p.corg[d]) / kCellA)));
+        q.chi[d] = min(p.nc[d] - 1, __builtin_amdgcn_readfirstlane((int)floorf((q.hi[d] + 8.01f - p.corg[d]) / kCellA)));
+    }
+    q.ix = j[0];
+    q.iy = j[1];
+    q.iz = j[2];
+    return q;
+}
+
+// LDS of the staging below.
+struct CubeStage {
+    int off[kAT + 1];        // first flat index of each cell row
+    int first[kAT];          // its first slot
+    int wave_tot[kAT / 64];
+};
+
+// Walks the atoms of the cube's cells (rows of cells along x are contiguous
+// in the atom array) a tile of kAT at a time, in cell order: fn(slot, near)
+// is called by every lane, near false where the lane has no atom or its atom
+// is past 8 A of the cube's box.  fn may synchronise the workgroup.
+template <typename F>
+__device__ __forceinline__ void cube_atoms(const AParams &p, const Cube &q, CubeStage &st, F &&fn) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int ny = q.chi[1] - q.clo[1] + 1, nz = q.chi[2] - q.clo[2] + 1;
+    const int nrows = (q.chi[0] >= q.clo[0] && ny > 0 && nz > 0) ? ny * nz : 0;
+    for (int r0 = 0; r0 < nrows; r0 += kAT) {
+        int s0 = 0, n = 0;
+        if (r0 + tid < nrows) {
+            const int row = p.nc[0] * (q.clo[1] + (r0 + tid) % ny + p.nc[1] * (q.clo[2] + (r0 + tid) / ny));
+            s0 = p.cell_start[row + q.clo[0]];
+            n = p.cell_start[row + q.chi[0] + 1] - s0;
+        }
+        int x = n;   // inclusive scan: within the wave, then across waves
+        for (int o = 1; o < 64; o <<= 1) {
+            const int y = __shfl_up(x, o);
+            if (lane >= o) x += y;
+        }
+        __syncthreads();   // the last tile's readers are done
+        if (lane == 63) st.wave_tot[wave] = x;
+        __syncthreads();
+        int before = 0, total = 0;
+        for (int w = 0; w < kAT / 64; w++) {
+            before += w < wave ? st.wave_tot[w] : 0;
+            total += st.wave_tot[w];
+        }
+        total = __builtin_amdgcn_readfirstlane(total);
+        st.off[tid] = before + x - n;
+        st.first[tid] = s0;
+        if (tid == 0) st.off[kAT] = total;
+        __syncthreads();
+        for (int j0 = 0; j0 < total; j0 += kAT) {
+            const int j = j0 + tid;
+            int slot = 0;
+            bool near = false;
+            if (j < total) {
+                int lo = 0, hi = kAT;   // the last row with off <= j
+                while (hi - lo > 1) {
+                    const int mid = (lo + hi) >> 1;
+                    if (st.off[mid] <= j) lo = mid;
+                    else hi = mid;
+                }
+                slot = st.first[lo] + j - st.off[lo];
+                const AAtom &a = p.atoms[slot];
+                const float ex = fmaxf(fmaxf(q.lo[0] - a.x, a.x - q.hi[0]), 0.f),
+                            ey = fmaxf(fmaxf(q.lo[1] - a.y, a.y - q.hi[1]), 0.f),
+                            ez = fmaxf(fmaxf(q.lo[2] - a.z, a.z - q.hi[2]), 0.f);
+                near = ex * ex + ey * ey + ez * ez < kCut2 * 1.0001f;
+            }
+            fn(slot, near);
+        }
+    }
+}
+
+// Appends the slots of the flagged lanes to list, in lane order; the count in
+// n, the same in every lane, goes up by theirs.  wave_tot holds one int per
+// wave.  The caller keeps kAT free places.
+__device__ __forceinline__ void append(bool flag, int slot, int *list, int &n, int *wave_tot) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const unsigned long long m = __ballot(flag);
+    __syncthreads();
+    if (lane == 0) wave_tot[wave] = __popcll(m);
+    __syncthreads();
+    int at = n + __popcll(m & ((1ull << lane) - 1));
+    for (int w = 0; w < kAT / 64; w++) {
+        at += w < wave ? wave_tot[w] : 0;
+        n += wave_tot[w];
+    }
+    n = __builtin_amdgcn_readfirstlane(n);
+    if (flag) list[at] = slot;
+}
+
+// Each point's closest donor H within 8 A (the lowest index of equals), or
+// -1: the four waves take every fourth H of the cube's list, and the winners
+// meet in LDS.  is_h picks the atoms; every wave returns the point's answer.
+__device__ __forceinline__ int cube_closest_h(const AParams &p, const Cube &q, CubeStage &st, int *hlist,
+                                              float (*hr2)[64], int (*hix)[64]) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    float best = 1e30f;
+    int bidx = 0x7fffffff, n = 0;
+    const auto scan = [&] {
+        __syncthreads();
+        for (int j = wave; j < n; j += kAT / 64) {
+            const int slot = __builtin_amdgcn_readfirstlane(hlist[j]);
+            const AN_CONST AAtom &a = ((const AN_CONST AAtom *)p.atoms)[slot];
+            const float dx = a.x - q.c[0], dy = a.y - q.c[1], dz = a.z - q.c[2];
+            const float r2 = dx * dx + dy * dy + dz * dz;
+            const int i = a.index;
+            if (r2 < best || (r2 == best && i < bidx)) {
+                best = r2;
+                bidx = i;
+            }
+        }
+        n = 0;
+    };
+    cube_atoms(p, q, st, [&](int slot, bool near) {
+        if (n > kCubeHCap - kAT) scan();   // uniform
+        const int hb = near ? (p.atoms[slot].meta >> 8) & 0xff : 0;
+        append(hb == AG_HB_DS || hb == AG_HB_D1, slot, hlist, n, st.wave_tot);
+    });
+    scan();
+    hr2[wave][lane] = best;
+    hix[wave][lane] = bidx;
+    __syncthreads();
+    for (int w = 0; w < kAT / 64; w++) {
+        const float r2 = hr2[w][lane];
+        const int i = hix[w][lane];
+        if (r2 < best || (r2 == best && i < bidx)) {
+            best = r2;
+            bidx = i;
+        }
+    }
+    return best < kCut2 ? bidx : -1;
+}
+
+__device__ __forceinline__ AAtom load_atom(const AN_CONST AAtom *atoms, int slot) {
+    const AN_CONST AAtom &s = atoms[slot];
+    AAtom a;
+    a.x = s.x;
+    a.y = s.y;
+    a.z = s.z;
+    a.q = s.q;
+    a.vol = s.vol;
+    a.solpar = s.solpar;
+    a.meta = s.meta;
+    a.index = s.index;
+    for (int k = 0; k < 3; k++) {
+        a.rv[k] = s.rv[k];
+        a.rv2[k] = s.rv2[k];
+    }
+    return a;
+}
+
+// One workgroup per cube of 4 x 4 x 4 points; a lane holds one point, the same
+// one in each of the four waves, and the waves take every fourth atom of the
+// cube's list (up to kCubeCap at a time), then add up through LDS in wave
+// order.  An atom is the same for a whole wave, so its record, its pair
+// parameters and its H-bond case come through scalar loads and its branches
+// are scalar.  Bound by the vector unit: about 130 operations per (atom, point)
+// with five maps, of which the pair potentials take 16 each.  One lane per
+// point walking its own cells, with each lane's records and parameters in vector
+// registers, measured 3.42 ms (5,000 atoms at protein density, 65^3 points, 5
+// affinity maps), now 0.35 ms.
+template <int NA>
 __global__ void __launch_bounds__(kAT) k_an_near(AParams p) {
-    const long long pt = (long long)blockIdx.x * kAT + threadIdx.x;
-    if (pt >= p.P) return;
-    int ix, iy, iz;
-    float c[3];
-    point_of(p, pt, ix, iy, iz, c);
-    float hmin[kAMaxAff], hmax[kAMaxAff];
-    int amin[kAMaxAff], amax[kAMaxAff];
-    for (int k = 0; k < kAMaxAff; k++) {
+    __shared__ CubeStage st;
+    __shared__ int list[kCubeCap], hlist[kCubeHCap];
+    __shared__ float hr2[kAT / 64][64];
+    __shared__ int hix[kAT / 64][64];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const Cube q = cube_of(p, blockIdx.x);
+    const int ch = cube_closest_h(p, q, st, hlist, hr2, hix);
+    float rvH[3] = {0.f, 0.f, 0.f};
+    if (ch >= 0)
+        for (int k = 0; k < 3; k++) rvH[k] = p.rv_by_index[3 * ch + k];
+    float acc[NA], hmin[NA], hmax[NA];
+    int amin[NA], amax[NA];
+#pragma unroll
+    for (int k = 0; k < NA; k++) {
+        acc[k] = 0.f;
         hmin[k] = 999999.f;
         hmax[k] = -999999.f;
         amin[k] = amax[k] = -1;
     }
-    // slot-indexed accumulators live in the output maps; per affinity map the
-    // E term goes to aff_slot and the desolvation to des_slot
-    float accE[kAMaxAff], accD[kAMaxAff];
-    for (int k = 0; k < kAMaxAff; k++) accE[k] = accD[k] = 0.f;
-    float dacc = 0.f;
-    const int ch = closest_h(p, c);
-    float rvH[3] = {0.f, 0.f, 0.f};
-    if (ch >= 0)
-        for (int k = 0; k < 3; k++) rvH[k] = p.rv_by_index[3 * ch + k];
-    int lo[3], hi[3];
-    cell_range(p, c, lo, hi);
-    for (int gz = lo[2]; gz <= hi[2]; gz++)
-        for (int gy = lo[1]; gy <= hi[1]; gy++) {
-            const int row = p.nc[0] * (gy + p.nc[1] * gz);
-            const int s0 = p.cell_start[row + lo[0]], s1 = p.cell_start[row + hi[0] + 1];
-            for (int s = s0; s < s1; s++) {
-                const AAtom a = p.atoms[s];
-                const float d[3] = {a.x - c[0], a.y - c[1], a.z - c[2]};
-                const float r2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
+    // the classes' case words, lane = class; read by readlane at the top of an
+    // atom, where every lane is active
+    const int case_word = p.case_word[min(lane, 6)];
+    // desolvation: map k gains sp[k] sum(vol G) + volp[k] sum(solq G)
+    float dv = 0.f, dq = 0.f;
+    int n = 0;
+    const auto process = [&] {
+        __syncthreads();
+        const AN_CONST AAtom *atoms = (const AN_CONST AAtom *)p.atoms;
+        for (int j0 = wave; j0 < n; j0 += kAT) {
+            // 64 of the wave's atoms at a time: their slots in one register,
+            // picked by readlane; each record is loaded one atom ahead
+            const int mine = list[min(j0 + lane * (kAT / 64), n - 1)];
+            const int count = min(64, (n - j0 + kAT / 64 - 1) / (kAT / 64));
+            AAtom a = load_atom(atoms, __builtin_amdgcn_readlane(mine, 0));
+            for (int jj = 0; jj < count; jj++) {
+                const AAtom at = a;
+                int next = __builtin_amdgcn_readlane(mine, min(jj + 1, count - 1));
+                // the next record's loads issue once this one's have arrived
+                asm volatile("" : "+s"(next) : "s"(at.meta), "s"(at.x), "s"(at.index));
+                a = load_atom(atoms, next);
+                const int type = at.meta & 0xff, hb = (at.meta >> 8) & 0xff;
+                const unsigned cases = (unsigned)__builtin_amdgcn_readlane(case_word, hb);
+                const float d[3] = {at.x - q.c[0], at.y - q.c[1], at.z - q.c[2]};
+                const float r2 = __builtin_fmaf(d[0], d[0], __builtin_fmaf(d[1], d[1], d[2] * d[2]));
                 if (!(r2 < kCut2)) continue;
-                // hardware rsq and exp2, about 1 ulp
+                const AN_CONST ANearType &nt = ((const AN_CONST ANearType *)p.near_pairs)[type];
                 const float r2c = fmaxf(r2, 1.0e-12f);
-                const float ir = __builtin_amdgcn_rsqf(r2c);
+                const float ir = __builtin_amdgcn_rsqf(r2c);   // hardware rsq, exp2 and rcp, about 1 ulp
                 const float r = r2c * ir;
-                const float dn[3] = {d[0] * ir, d[1] * ir, d[2] * ir};
-                const int type = a.meta & 0xff, hb = (a.meta >> 8) & 0xff;
                 float dS;
                 const float S = switch_s(r, dS);
                 const float G = p.w_desolv * __builtin_amdgcn_exp2f(r2 * (-kInv2Sig2 * 1.44269504088896341f)) * S;
-                const Dir dr = dir_of(a, hb, dn, ch, rvH);
-                const float solq = a.solpar + p.qasp * fabsf(a.q);
-#pragma unroll
-                for (int k = 0; k < kAMaxAff; k++) {
-                    if (k >= p.naff) continue;
-                    const LJ lj = lj_eval(p.pairs[k * p.T + type], r, p.w_smooth);
-                    const float E = lj.E * S;
-                    const float rsph = fminf(fmaxf(E * 0.01f, 0.f), 1.f);
-                    const int cs = p.cases[k][hb];
-                    if (cs == CASE_PLAIN) {
-                        accE[k] += E;
-                    } else if (cs == CASE_ACC) {
-                        accE[k] += E * dr.Hramp * (dr.racc + (1.f - dr.racc) * rsph);
-                    } else {
-                        const float f = cs == CASE_MM_RACC ? dr.racc : dr.rdon;
-                        const float v = E * (f + (1.f - f) * rsph);
-                        if (v < hmin[k]) { hmin[k] = v; amin[k] = a.index; }
-                        if (v > hmax[k]) { hmax[k] = v; amax[k] = a.index; }
-                    }
-                    accD[k] += (p.sp[k] * a.vol + solq * p.volp[k]) * G;
+                dv = __builtin_fmaf(at.vol, G, dv);
+                dq = __builtin_fmaf(at.solpar + p.qasp * fabsf(at.q), G, dq);
+                Dir dr{1.f, 1.f, 1.f};
+                if (hb == AG_HB_D1 || hb == AG_HB_A1 || hb == AG_HB_A2) {
+                    const float dn[3] = {d[0] * ir, d[1] * ir, d[2] * ir};
+                    dr = dir_of(at.rv, at.rv2, (at.meta >> 16) & 0xff, at.index, hb, dn, ch, rvH);
                 }
-                dacc += p.qasp * a.vol * G;
+                const unsigned form = (unsigned)nt.form;
+#pragma clang loop unroll(full)
+                for (int k = 0; k < NA; k++) {
+                    if (k >= p.naff) continue;
+                    // s = r + w left of the well, r* within w of it, r - w right of it
+                    const float w = __builtin_amdgcn_fmed3f(r - nt.pair[k].rstar, -p.w_smooth, p.w_smooth);
+                    const float rho = nt.pair[k].R * __builtin_amdgcn_rcpf(r - w);
+                    const float rho2 = rho * rho, rho4 = rho2 * rho2;
+                    float pa = rho4 * rho4 * rho4, pb;
+                    const unsigned f2 = (form >> (2 * k)) & 3;
+                    if (f2 == 0) {
+                        pb = rho4 * rho2;
+                    } else if (f2 == 1) {
+                        pb = rho4 * rho4 * rho2;
+                    } else {
+                        pa = pb = 1.f;
+                        const int ea = nt.a[k], eb = nt.b[k];
+#pragma clang loop unroll(disable)
+                        for (int i = 0; i < max(ea, eb); i++) {
+                            pa *= i < ea ? rho : 1.f;
+                            pb *= i < eb ? rho : 1.f;
+                        }
+                    }
+                    const float E = fminf(__builtin_fmaf(nt.pair[k].c1, pa, -(nt.pair[k].c2 * pb)), kClamp) * S;
+                    const unsigned cs = (cases >> (2 * k)) & 3;
+                    if (cs == CASE_PLAIN) {
+                        acc[k] += E;
+                    } else {
+                        const float rsph = __builtin_amdgcn_fmed3f(E * 0.01f, 0.f, 1.f);
+                        const float f = cs == CASE_MM_RDON ? dr.rdon : dr.racc;
+                        const float v = E * __builtin_fmaf(1.f - f, rsph, f);
+                        if (cs == CASE_ACC) {
+                            acc[k] = __builtin_fmaf(v, dr.Hramp, acc[k]);
+                        } else {
+                            if (v < hmin[k]) { hmin[k] = v; amin[k] = at.index; }
+                            if (v > hmax[k]) { hmax[k] = v; amax[k] = at.index; }
+                        }
+                    }
+                }
             }
         }
+        n = 0;
+        __syncthreads();
+    };
+    cube_atoms(p, q, st, [&](int slot, bool near) {
+        if (n > kCubeCap - kAT) process();   // uniform
+        append(near, slot, list, n, st.wave_tot);
+    });
+    process();
+    // waves 1 to 3 hand over one after the other, so that ties between equal
+    // terms go to the earlier wave
+    __shared__ float fx[3 * NA + 2][64];
+    __shared__ int ix[2 * NA][64];
+    for (int w = 1; w < kAT / 64; w++) {
+        if (wave == w) {
+#pragma unroll
+            for (int k = 0; k < NA; k++) {
+                fx[3 * k][lane] = acc[k];
+                fx[3 * k + 1][lane] = hmin[k];
+                fx[3 * k + 2][lane] = hmax[k];
+                ix[2 * k][lane] = amin[k];
+                ix[2 * k + 1][lane] = amax[k];
+            }
+            fx[3 * NA][lane] = dv;
+            fx[3 * NA + 1][lane] = dq;
+        }
+        __syncthreads();
+        if (wave == 0) {
+#pragma unroll
+            for (int k = 0; k < NA; k++) {
+                acc[k] += fx[3 * k][lane];
+                if (fx[3 * k + 1][lane] < hmin[k]) { hmin[k] = fx[3 * k + 1][lane]; amin[k] = ix[2 * k][lane]; }
+                if (fx[3 * k + 2][lane] > hmax[k]) { hmax[k] = fx[3 * k + 2][lane]; amax[k] = ix[2 * k + 1][lane]; }
+            }
+            dv += fx[3 * NA][lane];
+            dq += fx[3 * NA + 1][lane];
+        }
+        __syncthreads();
+    }
+    if (wave != 0 || !q.inside) return;
+    const long long pt = (long long)q.ix + (long long)p.n1[0] * ((long long)q.iy + (long long)p.n1[1] * q.iz);
     // assemble: a desolvation-only map belongs to exactly one affinity map
     // (separate_desolvation_maps), so slot writes do not collide
 #pragma unroll
-    for (int k = 0; k < kAMaxAff; k++) {
+    for (int k = 0; k < NA; k++) {
         if (k >= p.naff) continue;
-        float v = accE[k];
+        float v = acc[k];
         if (amin[k] >= 0) v += hmin[k] + fmaxf(hmax[k], 0.f);
+        const float des = __builtin_fmaf(p.sp[k], dv, p.volp[k] * dq);
         if (p.des_slot[k] == p.aff_slot[k]) {
-            p.maps[(long long)p.aff_slot[k] * p.P + pt] = v + accD[k];
+            p.maps[(long long)p.aff_slot[k] * p.P + pt] = v + des;
         } else {
             p.maps[(long long)p.aff_slot[k] * p.P + pt] = v;
-            p.maps[(long long)p.des_slot[k] * p.P + pt] = accD[k];
+            p.maps[(long long)p.des_slot[k] * p.P + pt] = des;
         }
         p.amin[(long long)k * p.P + pt] = amin[k];
         p.amax[(long long)k * p.P + pt] = (amin[k] >= 0 && hmax[k] > 0.f) ? amax[k] : -1;
     }
-    if (p.d_slot >= 0) p.maps[(long long)p.d_slot * p.P + pt] = dacc;
+    if (p.d_slot >= 0) p.maps[(long long)p.d_slot * p.P + pt] = p.qasp * dv;
     p.closest_h[pt] = ch;
     for (int k = 0; k < p.n_cov; k++) {
-        const double dx = p.cov_pos[0] - (double)(ix - p.ne[0]) * (double)p.h;
-        const double dy = p.cov_pos[1] - (double)(iy - p.ne[1]) * (double)p.h;
-        const double dz = p.cov_pos[2] - (double)(iz - p.ne[2]) * (double)p.h;
+        const double dx = p.cov_pos[0] - (double)(q.ix - p.ne[0]) * (double)p.h;
+        const double dy = p.cov_pos[1] - (double)(q.iy - p.ne[1]) * (double)p.h;
+        const double dz = p.cov_pos[2] - (double)(q.iz - p.ne[2]) * (double)p.h;
         double rc = sqrt(dx * dx + dy * dy + dz * dz) / p.cov_hw;
         if (rc < 1.0e-6) rc = 1.0e-6;
         p.maps[(long long)p.cov_slot[k] * p.P + pt] = (float)(p.cov_barrier * (1. - exp(-0.69314718055994530942 * rc * rc)));
@@ -1071,7 +1327,7 @@ struct ag_analytic {
     std::vector<ag::BondRecipe> recipes;
     std::vector<int> h_atoms, atom_list;
     // device
-    DevBuf d_atoms, d_by_index, d_rv, d_cells, d_pairs, d_eatoms, d_closest, d_amin, d_amax, d_vh, d_hout,
+    DevBuf d_atoms, d_by_index, d_rv, d_cells, d_pairs, d_near_pairs, d_eatoms, d_closest, d_amin, d_amax, d_vh, d_hout,
         d_hatoms, d_alist, d_aout, d_partial, d_eout, d_fatoms, d_epart, d_gcount, d_gpack, d_vcount, d_vpack,
         d_gmask;
     int eK = 16;                       // run length of the forward e kernel
@@ -1269,6 +1525,22 @@ static void analytic_upload(ag_analytic *a) {
                 pp.expl = 1;
             }
         }
+    std::vector<ANearType> near_pairs((size_t)std::max(T, 1));
+    memset(near_pairs.data(), 0, sizeof(ANearType) * near_pairs.size());
+    for (int k = 0; k < a->naff; k++)
+        for (int t = 0; t < T; t++) {
+            const APair &pp = pairs[(size_t)k * T + t];
+            ANearType &nt = near_pairs[t];
+            ANear &q = nt.pair[k];
+            const double ke = (double)pp.eps / (pp.a - pp.b);
+            q.R = pp.expl ? 1.f : pp.R;
+            q.c1 = pp.expl ? pp.cA : (float)(ke * pp.b);
+            q.c2 = pp.expl ? pp.cB : (float)(ke * pp.a);
+            q.rstar = pp.rstar;
+            nt.a[k] = pp.a;
+            nt.b[k] = pp.b;
+            nt.form |= (pp.a == 12 && pp.b == 6 ? 0 : pp.a == 12 && pp.b == 10 ? 1 : 2) << (2 * k);
+        }
     std::vector<float4> eat(std::max(N, 1));
     for (int i = 0; i < N; i++)
         eat[i] = make_float4((float)a->coord[3 * i], (float)a->coord[3 * i + 1], (float)a->coord[3 * i + 2],
@@ -1330,6 +1602,9 @@ static void analytic_upload(ag_analytic *a) {
     p.cov_barrier = a->cov_barrier;
     p.d_slot = a->dsolv;
     p.pairs = (const APair *)up(a->d_pairs, pairs.data(), sizeof(APair) * pairs.size());
+    p.near_pairs = (const ANearType *)up(a->d_near_pairs, near_pairs.data(), sizeof(ANearType) * near_pairs.size());
+    for (int h = 0; h < 7; h++)
+        for (int k = 0; k < a->naff; k++) p.case_word[h] |= a->cases[k][h] << (2 * k);
     p.T = T;
     p.w_smooth = (float)(std::floor(a->r_smooth * AG_A_DIV / 2.) / AG_A_DIV);
     p.w_desolv = (float)a->w[3];
@@ -1374,9 +1649,12 @@ void analytic_forward(ag_analytic *a, float *d_maps) {
     hipStream_t st = c->stream;
     AParams p = a->ap;
     p.maps = d_maps;
-    const unsigned grid = (unsigned)((a->P + kAT - 1) / kAT);
+    long long cubes = 1;
+    for (int d = 0; d < 3; d++) cubes *= (a->grid.n1[d] + kCube - 1) / kCube;
     HIP_CHECK(hipEventRecord(c->ev[0], st));
-    k_an_near<<<grid, kAT, 0, st>>>(p);
+    if (a->naff <= 4) k_an_near<4><<<(unsigned)cubes, kAT, 0, st>>>(p);
+    else if (a->naff <= 6) k_an_near<6><<<(unsigned)cubes, kAT, 0, st>>>(p);
+    else k_an_near<8><<<(unsigned)cubes, kAT, 0, st>>>(p);
     HIP_CHECK(hipGetLastError());
     HIP_CHECK(hipEventRecord(c->ev[1], st));
     if (a->elec >= 0) {

@@ -155,6 +155,24 @@ struct HostStage {
     }
 };
 
+// Hramp of a D1 atom against the closest H (main.cpp:3118-3131):
+// 0.5 - 0.5 cos(4/3 acos(ct)), ct in [-1, 1].  With h = sqrt((1 + ct) / 2), the
+// cosine of the half angle, it is 0.5 - 0.5 cos(8/3 acos h) = (1 - h) Q(h), Q
+// analytic on [0, 1]: a degree-7 Chebyshev fit, 9e-8 off at most; in FP32 2.6e-7
+// at most, where acosf and cosf leave 2.9e-7, in 11 operations for their 60.
+__device__ __forceinline__ float hramp_value(float ct) {
+    const float h = __builtin_amdgcn_sqrtf(fmaxf(__builtin_fmaf(0.5f, ct, 0.5f), 0.f));
+    float q = -0.00196754577f;
+    q = __builtin_fmaf(q, h, 0.0109145399f);
+    q = __builtin_fmaf(q, h, -0.030576898f);
+    q = __builtin_fmaf(q, h, 0.0661250228f);
+    q = __builtin_fmaf(q, h, -0.159349768f);
+    q = __builtin_fmaf(q, h, 1.0157047f);
+    q = __builtin_fmaf(q, h, 1.90470516f);
+    q = __builtin_fmaf(q, h, 0.749999964f);
+    return (1.f - h) * q;
+}
+
 struct ag_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
