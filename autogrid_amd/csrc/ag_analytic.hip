@@ -201,17 +201,25 @@ __device__ __forceinline__ float racc_of(float c, int rexp, float &dc) {
     return c;
 }
 
-// Hramp of a D1 atom against the closest H: 0.5 - 0.5 cos(4/3 acos(ct)).
+// Hramp of a D1 atom against the closest H, 0.5 - 0.5 cos(4/3 acos(ct)), and
+// its derivative -(2/3) sin(4/3 t) / sin t, t = acos(ct).  With h = cos(t / 2),
+// the derivative times h is analytic on [0, 1]: a degree-8 Chebyshev fit,
+// 1.7e-8 off at most.  Past |ct| = 1 (clamped) it is 0; where sin t < 1e-4
+// beside t = pi (h < 5e-5) it is taken as its value at t = 0.
 __device__ __forceinline__ float hramp_of(float ct_raw, float &dct) {
-    if (ct_raw >= 1.f || ct_raw <= -1.f) {
-        dct = 0.f;
-        const float ct = fminf(fmaxf(ct_raw, -1.f), 1.f);
-        return 0.5f - 0.5f * cosf(acosf(ct) * (4.f / 3.f));
-    }
-    const float th = acosf(ct_raw);
-    const float st = sinf(th);
-    dct = st > 1.0e-4f ? -(2.f / 3.f) * sinf(th * (4.f / 3.f)) / st : -8.f / 9.f;
-    return 0.5f - 0.5f * cosf(th * (4.f / 3.f));
+    const float ct = fminf(fmaxf(ct_raw, -1.f), 1.f);
+    const float h = __builtin_amdgcn_sqrtf(fmaxf(__builtin_fmaf(0.5f, ct, 0.5f), 0.f));
+    float g = -0.00302975586f;
+    g = __builtin_fmaf(g, h, 0.0172578153f);
+    g = __builtin_fmaf(g, h, -0.0467509426f);
+    g = __builtin_fmaf(g, h, 0.0856716455f);
+    g = __builtin_fmaf(g, h, -0.13386068f);
+    g = __builtin_fmaf(g, h, 0.229579017f);
+    g = __builtin_fmaf(g, h, -0.881983904f);
+    g = __builtin_fmaf(g, h, -0.444447247f);
+    g = __builtin_fmaf(g, h, 0.288675151f);
+    dct = ct_raw >= 1.f || ct_raw <= -1.f ? 0.f : h > 5.0e-5f ? g * __builtin_amdgcn_rcpf(h) : -8.f / 9.f;
+    return hramp_value(ct);
 }
 
 // Ordered A2 lone-pair rdon (main.cpp:3185-3246) with the identities
@@ -495,6 +503,31 @@ __device__ __forceinline__ int cube_closest_h(const AParams &p, const Cube &q, C
     return best < kCut2 ? bidx : -1;
 }
 
+// The capped energy of map k's pair with an atom of a type, the type (nt, its
+// form word) uniform.
+__device__ __forceinline__ float pair_energy(const AN_CONST ANearType &nt, int k, unsigned form, float r, float w) {
+    // s = r + w left of the well, r* within w of it, r - w right of it
+    const float off = __builtin_amdgcn_fmed3f(r - nt.pair[k].rstar, -w, w);
+    const float rho = nt.pair[k].R * __builtin_amdgcn_rcpf(r - off);
+    const float rho2 = rho * rho, rho4 = rho2 * rho2;
+    float pa = rho4 * rho4 * rho4, pb;
+    const unsigned f2 = (form >> (2 * k)) & 3;
+    if (f2 == 0) {
+        pb = rho4 * rho2;
+    } else if (f2 == 1) {
+        pb = rho4 * rho4 * rho2;
+    } else {
+        pa = pb = 1.f;
+        const int ea = nt.a[k], eb = nt.b[k];
+#pragma clang loop unroll(disable)
+        for (int i = 0; i < max(ea, eb); i++) {
+            pa *= i < ea ? rho : 1.f;
+            pb *= i < eb ? rho : 1.f;
+        }
+    }
+    return fminf(__builtin_fmaf(nt.pair[k].c1, pa, -(nt.pair[k].c2 * pb)), kClamp);
+}
+
 __device__ __forceinline__ AAtom load_atom(const AN_CONST AAtom *atoms, int slot) {
     const AN_CONST AAtom &s = atoms[slot];
     AAtom a;
@@ -589,26 +622,7 @@ __global__ void __launch_bounds__(kAT) k_an_near(AParams p) {
 #pragma clang loop unroll(full)
                 for (int k = 0; k < NA; k++) {
                     if (k >= p.naff) continue;
-                    // s = r + w left of the well, r* within w of it, r - w right of it
-                    const float w = __builtin_amdgcn_fmed3f(r - nt.pair[k].rstar, -p.w_smooth, p.w_smooth);
-                    const float rho = nt.pair[k].R * __builtin_amdgcn_rcpf(r - w);
-                    const float rho2 = rho * rho, rho4 = rho2 * rho2;
-                    float pa = rho4 * rho4 * rho4, pb;
-                    const unsigned f2 = (form >> (2 * k)) & 3;
-                    if (f2 == 0) {
-                        pb = rho4 * rho2;
-                    } else if (f2 == 1) {
-                        pb = rho4 * rho4 * rho2;
-                    } else {
-                        pa = pb = 1.f;
-                        const int ea = nt.a[k], eb = nt.b[k];
-#pragma clang loop unroll(disable)
-                        for (int i = 0; i < max(ea, eb); i++) {
-                            pa *= i < ea ? rho : 1.f;
-                            pb *= i < eb ? rho : 1.f;
-                        }
-                    }
-                    const float E = fminf(__builtin_fmaf(nt.pair[k].c1, pa, -(nt.pair[k].c2 * pb)), kClamp) * S;
+                    const float E = pair_energy(nt, k, form, r, p.w_smooth) * S;
                     const unsigned cs = (cases >> (2 * k)) & 3;
                     if (cs == CASE_PLAIN) {
                         acc[k] += E;
@@ -808,67 +822,76 @@ __global__ void k_an_esum(const float *epart, int nchunk, long long P, float *em
 // ---------------------------------------------------------------------------
 
 // Per point: the cotangent of the closest H's bond vector through the Hramp
-// factor of every other D1 atom within 8 A.
+// factor of every other D1 atom within 8 A.  Cubes and waves as in k_an_near; a
+// cube without a point to do leaves zeros.  (One lane per point with its own
+// cells: 288 us, now 31 us at the shape above; 235 and 14 us on 41^3 points.)
 __global__ void __launch_bounds__(kAT) k_an_vh(AParams p) {
-    const long long pt = (long long)blockIdx.x * kAT + threadIdx.x;
-    if (pt >= p.P) return;
-    int ix, iy, iz;
-    float c[3];
-    point_of(p, pt, ix, iy, iz, c);
+    __shared__ CubeStage st;
+    __shared__ int list[2 * kAT];
+    __shared__ float fx[kAT / 64][3][64];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const Cube q = cube_of(p, blockIdx.x);
+    const long long pt = (long long)q.ix + (long long)p.n1[0] * ((long long)q.iy + (long long)p.n1[1] * q.iz);
     const int ch = p.closest_h[pt];
-    float v[3] = {0.f, 0.f, 0.f};
-    if (ch >= 0) {
-        float rvH[3];
-        for (int k = 0; k < 3; k++) rvH[k] = p.rv_by_index[3 * ch + k];
-        float g[kAMaxAff];
-        bool any = false;
+    const unsigned cases = (unsigned)p.case_word[AG_HB_D1];
+    float g[kAMaxAff];
+    bool any = false;
 #pragma unroll
-        for (int k = 0; k < kAMaxAff; k++) {
-            g[k] = k < p.naff ? p.dmaps[(long long)p.aff_slot[k] * p.P + pt] : 0.f;
-            any = any || (g[k] != 0.f && p.cases[k][AG_HB_D1] == CASE_ACC);
-        }
-        if (any) {
-            int lo[3], hi[3];
-            cell_range(p, c, lo, hi);
-            for (int gz = lo[2]; gz <= hi[2]; gz++)
-                for (int gy = lo[1]; gy <= hi[1]; gy++) {
-                    const int row = p.nc[0] * (gy + p.nc[1] * gz);
-                    const int s0 = p.cell_start[row + lo[0]], s1 = p.cell_start[row + hi[0] + 1];
-                    for (int s = s0; s < s1; s++) {
-                        const AAtom a = p.atoms[s];
-                        const int hb = (a.meta >> 8) & 0xff;
-                        if (hb != AG_HB_D1 || a.index == ch) continue;
-                        const float d[3] = {a.x - c[0], a.y - c[1], a.z - c[2]};
-                        const float r2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
-                        if (!(r2 < kCut2)) continue;
-                        const float r = fmaxf(sqrtf(r2), 1.0e-6f);
-                        const float ir = 1.f / r;
-                        const float dn[3] = {d[0] * ir, d[1] * ir, d[2] * ir};
-                        const float cth = -(dn[0] * a.rv[0] + dn[1] * a.rv[1] + dn[2] * a.rv[2]);
-                        if (!(cth > 0.f)) continue;
-                        float dc;
-                        const float racc = racc_of(cth, (a.meta >> 16) & 0xff, dc);
-                        const float ct = rvH[0] * a.rv[0] + rvH[1] * a.rv[1] + rvH[2] * a.rv[2];
-                        float dct;
-                        hramp_of(ct, dct);
-                        if (dct == 0.f) continue;
-                        float dS;
-                        const float S = switch_s(r, dS);
-                        const int type = a.meta & 0xff;
-                        float gH = 0.f;
-#pragma unroll
-                        for (int k = 0; k < kAMaxAff; k++) {
-                            if (k >= p.naff || p.cases[k][AG_HB_D1] != CASE_ACC || g[k] == 0.f) continue;
-                            const float E = lj_eval(p.pairs[k * p.T + type], r, p.w_smooth).E * S;
-                            const float rsph = fminf(fmaxf(E * 0.01f, 0.f), 1.f);
-                            gH += g[k] * E * (racc + (1.f - racc) * rsph);
-                        }
-                        for (int k = 0; k < 3; k++) v[k] += gH * dct * a.rv[k];
-                    }
-                }
-        }
+    for (int k = 0; k < kAMaxAff; k++) {
+        g[k] = k < p.naff && ((cases >> (2 * k)) & 3) == CASE_ACC ? p.dmaps[(long long)p.aff_slot[k] * p.P + pt] : 0.f;
+        any = any || g[k] != 0.f;
     }
-    for (int k = 0; k < 3; k++) p.vh[3 * pt + k] = v[k];
+    any = any && ch >= 0 && q.inside;
+    float v[3] = {0.f, 0.f, 0.f};
+    if (__ballot(any)) {   // the same in every wave
+        float rvH[3] = {0.f, 0.f, 0.f};
+        if (ch >= 0)
+            for (int k = 0; k < 3; k++) rvH[k] = p.rv_by_index[3 * ch + k];
+        int n = 0;
+        const auto process = [&] {
+            __syncthreads();
+            for (int j = wave; j < n; j += kAT / 64) {
+                const AAtom a = load_atom((const AN_CONST AAtom *)p.atoms, __builtin_amdgcn_readfirstlane(list[j]));
+                if (!any || a.index == ch) continue;
+                const float d[3] = {a.x - q.c[0], a.y - q.c[1], a.z - q.c[2]};
+                const float r2 = __builtin_fmaf(d[0], d[0], __builtin_fmaf(d[1], d[1], d[2] * d[2]));
+                if (!(r2 < kCut2)) continue;
+                const float r2c = fmaxf(r2, 1.0e-12f);
+                const float ir = __builtin_amdgcn_rsqf(r2c), r = r2c * ir;
+                const float cth = -(d[0] * a.rv[0] + d[1] * a.rv[1] + d[2] * a.rv[2]) * ir;
+                if (!(cth > 0.f)) continue;
+                float dc, dct, dS;
+                const float racc = racc_of(cth, (a.meta >> 16) & 0xff, dc);
+                hramp_of(rvH[0] * a.rv[0] + rvH[1] * a.rv[1] + rvH[2] * a.rv[2], dct);
+                if (dct == 0.f) continue;
+                const float S = switch_s(r, dS);
+                const AN_CONST ANearType &nt = ((const AN_CONST ANearType *)p.near_pairs)[a.meta & 0xff];
+                const unsigned form = (unsigned)nt.form;
+                float gH = 0.f;
+#pragma clang loop unroll(full)
+                for (int k = 0; k < kAMaxAff; k++) {
+                    if (k >= p.naff || ((cases >> (2 * k)) & 3) != CASE_ACC) continue;
+                    const float E = pair_energy(nt, k, form, r, p.w_smooth) * S;
+                    const float rsph = fminf(fmaxf(E * 0.01f, 0.f), 1.f);
+                    gH += g[k] != 0.f ? g[k] * E * (racc + (1.f - racc) * rsph) : 0.f;
+                }
+                for (int k = 0; k < 3; k++) v[k] += gH * dct * a.rv[k];
+            }
+            n = 0;
+            __syncthreads();
+        };
+        cube_atoms(p, q, st, [&](int slot, bool near) {
+            if (n > kAT) process();   // uniform
+            append(near && ((p.atoms[slot].meta >> 8) & 0xff) == AG_HB_D1, slot, list, n, st.wave_tot);
+        });
+        process();
+        for (int k = 0; k < 3; k++) fx[wave][k][lane] = v[k];
+        __syncthreads();
+        for (int k = 0; k < 3; k++) v[k] = ((fx[0][k][lane] + fx[1][k][lane]) + fx[2][k][lane]) + fx[3][k][lane];
+    }
+    if (wave == 0 && q.inside)
+        for (int k = 0; k < 3; k++) p.vh[3 * pt + k] = v[k];
 }
 
 // Block reduction of n floats per lane (fixed order): lane 0 of the block
@@ -1642,6 +1665,12 @@ static void analytic_upload(ag_analytic *a) {
     a->uploaded = true;
 }
 
+static unsigned cube_count(const ag_grid &g) {
+    unsigned n = 1;
+    for (int d = 0; d < 3; d++) n *= (unsigned)((g.n1[d] + kCube - 1) / kCube);
+    return n;
+}
+
 void analytic_forward(ag_analytic *a, float *d_maps) {
     ag_ctx *c = a->ctx;
     HIP_CHECK(hipSetDevice(c->device));
@@ -1649,12 +1678,11 @@ void analytic_forward(ag_analytic *a, float *d_maps) {
     hipStream_t st = c->stream;
     AParams p = a->ap;
     p.maps = d_maps;
-    long long cubes = 1;
-    for (int d = 0; d < 3; d++) cubes *= (a->grid.n1[d] + kCube - 1) / kCube;
+    const unsigned cubes = cube_count(a->grid);
     HIP_CHECK(hipEventRecord(c->ev[0], st));
-    if (a->naff <= 4) k_an_near<4><<<(unsigned)cubes, kAT, 0, st>>>(p);
-    else if (a->naff <= 6) k_an_near<6><<<(unsigned)cubes, kAT, 0, st>>>(p);
-    else k_an_near<8><<<(unsigned)cubes, kAT, 0, st>>>(p);
+    if (a->naff <= 4) k_an_near<4><<<cubes, kAT, 0, st>>>(p);
+    else if (a->naff <= 6) k_an_near<6><<<cubes, kAT, 0, st>>>(p);
+    else k_an_near<8><<<cubes, kAT, 0, st>>>(p);
     HIP_CHECK(hipGetLastError());
     HIP_CHECK(hipEventRecord(c->ev[1], st));
     if (a->elec >= 0) {
@@ -1700,7 +1728,7 @@ void analytic_adjoint(ag_analytic *a, const float *d_dmaps, double *g_coord, dou
     float *d_aout = (float *)a->d_aout.get(sizeof(float) * kAtomOut * (size_t)std::max(nl, 1));
     double *d_eout = (double *)a->d_eout.get(sizeof(double) * 4 * (size_t)std::max(N, 1));
     if (nh > 0) {
-        k_an_vh<<<grid, kAT, 0, st>>>(p);
+        k_an_vh<<<cube_count(a->grid), kAT, 0, st>>>(p);
         const int nblk = (int)((a->P + kGPack - 1) / kGPack);
         int *counts = (int *)a->d_vcount.get(sizeof(int) * (2 * (size_t)nblk + 1));
         int *vlist = (int *)a->d_vpack.get(sizeof(int) * (size_t)a->P);
