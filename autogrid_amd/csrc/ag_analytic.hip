@@ -55,6 +55,8 @@
 
 namespace {
 
+#define AN_CONST __attribute__((address_space(4)))   // read-only tables, through scalar loads
+
 constexpr int kAT = 256;                 // threads per workgroup
 constexpr int kAMaxAff = 8;              // affinity maps per analytic set (registers, unrolled)
 constexpr float kSwOn = 7.5f, kSwInvLen = 2.0f;  // switch from 7.5 A, over 0.5 A
@@ -152,6 +154,19 @@ __device__ __forceinline__ float powi(float x, int n) {
             return r;
         }
     }
+}
+
+__device__ __forceinline__ APair load_pair(const AN_CONST APair *p) {
+    APair o;
+    o.R = p->R;
+    o.eps = p->eps;
+    o.cA = p->cA;
+    o.cB = p->cB;
+    o.rstar = p->rstar;
+    o.a = p->a;
+    o.b = p->b;
+    o.expl = p->expl;
+    return o;
 }
 
 // Smoothed, capped pair energy and its derivatives (FP32).
@@ -342,8 +357,6 @@ __device__ __forceinline__ Dir dir_of(const float rv[3], const float rv2[3], int
 constexpr int kCube = 4;                 // edge of a workgroup's cube of points
 constexpr int kCubeCap = 1024;           // atoms in the workgroup's list
 constexpr int kCubeHCap = 256;           // donor H in its list
-
-#define AN_CONST __attribute__((address_space(4)))
 
 // A workgroup's cube of points: its corner, this lane's point and the cells
 // around its box (points past the grid's end are clamped onto the last one).
@@ -894,6 +907,12 @@ __global__ void __launch_bounds__(kAT) k_an_vh(AParams p) {
         for (int k = 0; k < 3; k++) p.vh[3 * pt + k] = v[k];
 }
 
+// Orders a wave's own LDS accesses: its lanes see what the others wrote before.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // Block reduction of n floats per lane (fixed order): lane 0 of the block
 // gets the sums.
 template <int NV>
@@ -941,86 +960,76 @@ __global__ void __launch_bounds__(kAT) k_an_hsum(HsumParams p) {
 // per affinity map.
 constexpr int kAtomOut = 11 + 2 * kAMaxAff;
 
-// Per point: 1 if any cotangent the atom gather reads there (affinity,
-// desolvation and d slots) is nonzero.  Where all are zero a point adds
-// exactly nothing to any atom's gradient, so k_an_atom skips it.
-__global__ void __launch_bounds__(kAT) k_an_gmask(AParams p, unsigned char *mask) {
-    const long long pt = (long long)blockIdx.x * kAT + threadIdx.x;
-    if (pt >= p.P) return;
-    bool any = p.d_slot >= 0 && p.dmaps[(long long)p.d_slot * p.P + pt] != 0.f;
-    for (int k = 0; k < p.naff; k++)
-        any = any || p.dmaps[(long long)p.aff_slot[k] * p.P + pt] != 0.f ||
-              p.dmaps[(long long)p.des_slot[k] * p.P + pt] != 0.f;
-    mask[pt] = any;
+// Bit rows: for each grid row along x, words of 64 points, a bit set where any
+// cotangent the atom gather reads (affinity, desolvation and d slots) is
+// nonzero.  Where all are zero a point adds exactly nothing to any atom's
+// gradient, so k_an_atom skips it.  One wave per word.
+__global__ void __launch_bounds__(kAT) k_an_gmask(AParams p, int words, unsigned long long *bits) {
+    const long long w = (long long)blockIdx.x * (kAT / 64) + (threadIdx.x >> 6);
+    const long long row = w / words;
+    const int ix = (int)(w - row * words) * 64 + (threadIdx.x & 63);
+    bool any = false;
+    if (row < (long long)p.n1[1] * p.n1[2] && ix < p.n1[0]) {
+        const long long pt = row * p.n1[0] + ix;
+        any = p.d_slot >= 0 && p.dmaps[(long long)p.d_slot * p.P + pt] != 0.f;
+        for (int k = 0; k < p.naff; k++)
+            any = any || p.dmaps[(long long)p.aff_slot[k] * p.P + pt] != 0.f ||
+                  p.dmaps[(long long)p.des_slot[k] * p.P + pt] != 0.f;
+    }
+    const unsigned long long m = __ballot(any);
+    if ((threadIdx.x & 63) == 0 && row < (long long)p.n1[1] * p.n1[2]) bits[w] = m;
 }
 
 struct AtomAdjParams {
     AParams a;
     const AAtom *by_index;   // atoms by index
     const int *atom_list;    // atoms whose 8 A sphere meets the box, one per workgroup
-    float *out;
-    const unsigned char *mask;   // k_an_gmask              // [n_list][kAtomOut]
+    float *out;              // [n_list][kAtomOut]
+    const unsigned long long *bits;   // k_an_gmask
+    int words;               // 64-point words per grid row
 };
 
+// One workgroup per atom.  The rows of the box through its 8 A sphere are
+// dealt to the lanes a word of 64 points at a time; a lane keeps the bits
+// (k_an_gmask) of its word that lie within the sphere's chord.  Each wave packs
+// its lanes' points into its own LDS list in lane order and works through it
+// 64 at a time, every lane busy; no barrier until the waves' sums meet.
+// The chord is a little wide: a point past 8 A has S = 0 and adds nothing.
+// Testing the sphere's cube point by point, with the workgroup's barriers,
+// took most of the launch: 865 us (5,000 atoms, 65^3 points, 256 poses), now
+// 450 us.
+template <int NA>
 __global__ void __launch_bounds__(kAT) k_an_atom(AtomAdjParams q) {
+    constexpr int kList = 512;   // a wave's list; one lane appends at most 64
     __shared__ float red[4 * kAtomOut];
+    __shared__ int2 lists[kAT / 64][kList];
     const AParams &p = q.a;
-    const int idx = q.atom_list[blockIdx.x];
-    const AAtom a = q.by_index[idx];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int2 *const list = lists[wave];
+    const int idx = __builtin_amdgcn_readfirstlane(q.atom_list[blockIdx.x]);
+    const AAtom a = load_atom((const AN_CONST AAtom *)q.by_index, idx);
     const int type = a.meta & 0xff, hb = (a.meta >> 8) & 0xff, rexp = (a.meta >> 16) & 0xff;
-    // points of the box within the 8 A cube around the atom
+    const AN_CONST APair *pairs = (const AN_CONST APair *)p.pairs + type;
+    const unsigned cases = (unsigned)p.case_word[hb];
+    // rows and words of the box around the atom
     int lo[3], hi[3];
     const float ac[3] = {a.x, a.y, a.z};
     for (int d = 0; d < 3; d++) {
-        lo[d] = max(0, (int)ceilf((ac[d] - 8.f) / p.h) + p.ne[d]);
-        hi[d] = min(p.n1[d] - 1, (int)floorf((ac[d] + 8.f) / p.h) + p.ne[d]);
+        lo[d] = max(0, __builtin_amdgcn_readfirstlane((int)ceilf((ac[d] - 8.f) / p.h)) + p.ne[d]);
+        hi[d] = min(p.n1[d] - 1, __builtin_amdgcn_readfirstlane((int)floorf((ac[d] + 8.f) / p.h)) + p.ne[d]);
     }
-    const int nx = hi[0] - lo[0] + 1, ny = hi[1] - lo[1] + 1, nz = hi[2] - lo[2] + 1;
-    const long long npt = (nx > 0 && ny > 0 && nz > 0) ? (long long)nx * ny * nz : 0;
+    const int w0 = lo[0] / 64, nw = hi[0] / 64 - w0 + 1, ny = hi[1] - lo[1] + 1, nz = hi[2] - lo[2] + 1;
+    const int nitem = (hi[0] >= lo[0] && ny > 0 && nz > 0) ? nw * ny * nz : 0;
     float acc[kAtomOut];
 #pragma unroll
     for (int k = 0; k < kAtomOut; k++) acc[k] = 0.f;
     const float solq = a.solpar + p.qasp * fabsf(a.q);
     const float sgnq = a.q > 0.f ? 1.f : (a.q < 0.f ? -1.f : 0.f);
-    // The points of the cube within 8 A whose cotangents are not all zero
-    // (k_an_gmask) are appended to an LDS list in cube order, a tile of kAT
-    // cube points at a time; each full kAT of the list is then processed
-    // with every lane busy.  The rest add exactly nothing.
-    __shared__ int list[2 * kAT];
-    __shared__ int wcount[kAT / 64];
-    int nlist = 0;
-    for (long long t0 = 0; t0 < npt || nlist > 0; t0 += kAT) {
-        if (t0 < npt) {
-            const long long j = t0 + threadIdx.x;
-            bool keep = false;
-            int cell = 0;
-            if (j < npt) {
-                const int ix = lo[0] + (int)(j % nx), iy = lo[1] + (int)((j / nx) % ny),
-                          iz = lo[2] + (int)(j / ((long long)nx * ny));
-                const long long pt = (long long)ix + (long long)p.n1[0] * ((long long)iy + (long long)p.n1[1] * iz);
-                const float dx = a.x - (float)(ix - p.ne[0]) * p.h, dy = a.y - (float)(iy - p.ne[1]) * p.h,
-                            dz = a.z - (float)(iz - p.ne[2]) * p.h;
-                keep = dx * dx + dy * dy + dz * dz < kCut2 && q.mask[pt];
-                cell = (int)j;
-            }
-            const unsigned long long m = __ballot(keep);
-            if ((threadIdx.x & 63) == 0) wcount[threadIdx.x >> 6] = __popcll(m);
-            __syncthreads();
-            int before = nlist;
-            for (int w = 0; w < (int)(threadIdx.x >> 6); w++) before += wcount[w];
-            if (keep) list[before + __popcll(m & ((1ull << (threadIdx.x & 63)) - 1))] = cell;
-            int added = 0;
-            for (int w = 0; w < kAT / 64; w++) added += wcount[w];
-            nlist += added;
-            __syncthreads();
-            if (nlist < kAT && t0 + kAT < npt) continue;   // gather a full tile first
-        }
-        // process the first min(nlist, kAT) entries, then move the rest down
-        const int take = min(nlist, kAT);
-        if ((int)threadIdx.x < take) {
-        const long long j = list[threadIdx.x];
-        const int ix = lo[0] + (int)(j % nx), iy = lo[1] + (int)((j / nx) % ny), iz = lo[2] + (int)(j / ((long long)nx * ny));
-        const long long pt = (long long)ix + (long long)p.n1[0] * ((long long)iy + (long long)p.n1[1] * iz);
+    const auto point = [&](int2 e) {   // point index, iy | iz << 16
+        const long long pt = e.x;
+        const int iy = e.y & 0xffff, iz = e.y >> 16;
+        const int ix = e.x - p.n1[0] * (iy + p.n1[1] * iz);
         const float c[3] = {(float)(ix - p.ne[0]) * p.h, (float)(iy - p.ne[1]) * p.h, (float)(iz - p.ne[2]) * p.h};
         const float d[3] = {a.x - c[0], a.y - c[1], a.z - c[2]};
         const float r2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
@@ -1054,16 +1063,16 @@ __global__ void __launch_bounds__(kAT) k_an_atom(AtomAdjParams q) {
             rdon = a2_rdon<false>(dn, a.rv, a.rv2, 0.f, g3, g3, g3);
         }
         float g_r = 0.f, g_racc = 0.f, g_rdon = 0.f, g_H = 0.f;
-#pragma unroll
-        for (int k = 0; k < kAMaxAff; k++) {
+#pragma clang loop unroll(full)
+        for (int k = 0; k < NA; k++) {
             if (k >= p.naff) continue;
             const float gE_up = p.dmaps[(long long)p.aff_slot[k] * p.P + pt];
-            const float gD_up = p.dmaps[(long long)p.des_slot[k] * p.P + pt];
-            const LJ lj = lj_eval(p.pairs[k * p.T + type], r, p.w_smooth);
+            const float gD_up = p.des_slot[k] == p.aff_slot[k] ? gE_up : p.dmaps[(long long)p.des_slot[k] * p.P + pt];
+            const LJ lj = lj_eval(load_pair(pairs + k * p.T), r, p.w_smooth);
             const float E = lj.E * S;
             const float rsph = fminf(fmaxf(E * 0.01f, 0.f), 1.f);
             const float drsph = (E > 0.f && E < 100.f) ? 0.01f : 0.f;
-            const int cs = p.cases[k][hb];
+            const unsigned cs = (cases >> (2 * k)) & 3;
             float gE = 0.f;   // dL/dE of this map's pair term
             if (cs == CASE_PLAIN) {
                 gE = gE_up;
@@ -1125,15 +1134,64 @@ __global__ void __launch_bounds__(kAT) k_an_atom(AtomAdjParams q) {
         // dn = d / r, r = |d|, d = x - c
         const float dot = gdn[0] * dn[0] + gdn[1] * dn[1] + gdn[2] * dn[2];
         for (int k = 0; k < 3; k++) acc[k] += (gdn[k] - dot * dn[k]) * ir + g_r * dn[k];
+    };
+    int n = 0;   // entries in the wave's list (uniform)
+    for (int i0 = 64 * wave; i0 < nitem; i0 += kAT) {
+        unsigned long long m = 0;
+        int first = 0, yz = 0;   // the word's first point
+        if (i0 + lane < nitem) {
+            const int i = i0 + lane, r = i / nw, w = w0 + i - r * nw;
+            const int iy = lo[1] + r % ny, iz = lo[2] + r / ny;
+            const float dy = a.y - (float)(iy - p.ne[1]) * p.h, dz = a.z - (float)(iz - p.ne[2]) * p.h;
+            const float rest = kCut2 - dy * dy - dz * dz;
+            if (rest > 0.f) {
+                const float half = __builtin_amdgcn_sqrtf(rest) * 1.0001f + 1.0e-4f;
+                const int x0 = max(lo[0], (int)ceilf((a.x - half) / p.h) + p.ne[0]) - 64 * w;
+                const int x1 = min(hi[0], (int)floorf((a.x + half) / p.h) + p.ne[0]) - 64 * w;
+                if (x1 >= 0 && x0 < 64 && x0 <= x1) {
+                    const long long row = (long long)iy + (long long)p.n1[1] * iz;
+                    m = q.bits[row * q.words + w];
+                    m &= ~0ull << max(x0, 0);
+                    m &= ~0ull >> (63 - min(x1, 63));
+                    first = (int)(row * p.n1[0]) + 64 * w;
+                    yz = iy | iz << 16;
+                }
+            }
         }
-        __syncthreads();
-        const int rest = nlist - take;
-        const int moved = (int)threadIdx.x < rest ? list[take + threadIdx.x] : 0;
-        __syncthreads();
-        if ((int)threadIdx.x < rest) list[threadIdx.x] = moved;
-        nlist = rest;
-        __syncthreads();
-        if (t0 >= npt && nlist == 0) break;
+        // append the lanes' points in lane order, as many lanes at a time as
+        // fit, and work the list off sixty-four at a time
+        bool more = true;
+        while (more) {
+            const int c = __popcll(m);
+            int x = c;   // inclusive scan over the wave
+            for (int o = 1; o < 64; o <<= 1) {
+                const int y = __shfl_up(x, o);
+                if (lane >= o) x += y;
+            }
+            const bool fits = n + x <= kList;   // a prefix of the lanes
+            int at = n + x - c;
+            const int last = __popcll(__ballot(fits));
+            n += last > 0 ? __builtin_amdgcn_readlane(x, last - 1) : 0;
+            if (fits) {
+                while (m) {
+                    list[at++] = make_int2(first + __builtin_ctzll(m), yz);
+                    m &= m - 1;
+                }
+            }
+            wave_sync();
+            more = last < 64;
+            const bool end = !more && i0 + kAT >= nitem;   // the wave's last points
+            if (more || end || n > kList - 64) {
+                const int todo = end ? n : n & ~63;
+                for (int t = 0; t < todo; t += 64)
+                    if (t + lane < n) point(list[t + lane]);
+                const int2 moved = todo + lane < n ? list[todo + lane] : make_int2(0, 0);
+                wave_sync();
+                if (todo + lane < n) list[lane] = moved;
+                n = end ? 0 : n - todo;
+                wave_sync();
+            }
+        }
     }
     block_sum<kAtomOut>(acc, red);
     if (threadIdx.x == 0)
@@ -1742,10 +1800,14 @@ void analytic_adjoint(ag_analytic *a, const float *d_dmaps, double *g_coord, dou
         q.by_index = (const AAtom *)a->d_by_index.ptr;
         q.atom_list = (const int *)a->d_alist.ptr;
         q.out = d_aout;
-        unsigned char *mask = (unsigned char *)a->d_gmask.get((size_t)a->P);
-        k_an_gmask<<<grid, kAT, 0, st>>>(p, mask);
-        q.mask = mask;
-        k_an_atom<<<nl, kAT, 0, st>>>(q);
+        q.words = (a->grid.n1[0] + 63) / 64;
+        const long long words = (long long)q.words * a->grid.n1[1] * a->grid.n1[2];
+        unsigned long long *bits = (unsigned long long *)a->d_gmask.get(sizeof(unsigned long long) * (size_t)words);
+        k_an_gmask<<<(unsigned)((words + kAT / 64 - 1) / (kAT / 64)), kAT, 0, st>>>(p, q.words, bits);
+        q.bits = bits;
+        if (a->naff <= 4) k_an_atom<4><<<nl, kAT, 0, st>>>(q);
+        else if (a->naff <= 6) k_an_atom<6><<<nl, kAT, 0, st>>>(q);
+        else k_an_atom<8><<<nl, kAT, 0, st>>>(q);
     }
     HIP_CHECK(hipGetLastError());
     const bool want_e = a->elec >= 0 && N > 0;
