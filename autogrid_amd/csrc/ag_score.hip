@@ -14,16 +14,18 @@
 //   k_score      one workgroup per pose, lanes over its atoms: per-atom
 //                energy and gradient dE/dx, the pose's sum reduced in FP64
 //                in a fixed order;
-//   k_score_adj  dL/dmaps = S^T dL/dscores for the scores' sparse matrix S,
-//                one lane per touched map entry over a host-built,
-//                index-sorted list of its contributions: a fixed-order sum,
-//                no atomics.
+//   k_score_place, k_sort_count / _scan / _scatter
+//                new positions: each atom's place on the grid, and its eight
+//                corners sorted by grid point and by (map, grid point), a
+//                stable radix sort, so equal keys stay in atom order;
+//   k_score_adj  dL/dmaps = S^T dL/dscores for the scores' sparse matrix S:
+//                the first entry of each run of equal keys sums its run: a
+//                fixed-order sum, no atomics.
 
 #include <hip/hip_runtime.h>
 #include <algorithm>
 #include <cmath>
 #include <cstring>
-#include <numeric>
 #include <string>
 #include <vector>
 
@@ -107,15 +109,227 @@ __global__ void k_score_zero(float *out, long long n) {
         out[i] = 0.f;
 }
 
-// row r: dmaps[target[r]] = sum over k in [row_start[r], row_start[r+1]) of
-// val[k] * dscore[pose[k]], k in the order the host listed them
-__global__ void k_score_adj(int n_rows, const int *row_start, const long long *target, const int *pose,
-                            const float *val, const float *dscore, float *dmaps) {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= n_rows) return;
-    double s = 0.0;
-    for (int k = row_start[r]; k < row_start[r + 1]; k++) s += (double)val[k] * (double)dscore[pose[k]];
-    dmaps[target[r]] = (float)s;
+struct PlaceParams {
+    const double *xyz;          // [n][3]
+    const float *charge;
+    const int *map, *pose;
+    int n;
+    int n1[3];
+    double shift[3], spacing;   // ne * spacing
+    unsigned P;                 // grid points; the key of an atom off the grid
+    ScoreAtom *atoms;
+    unsigned *key;              // [8 n] corner's grid point
+    int *entry;                 // [8 n] atom * 8 + corner
+};
+
+__global__ void __launch_bounds__(kST) k_score_place(PlaceParams p) {
+    const int a = blockIdx.x * kST + threadIdx.x;
+    if (a >= p.n) return;
+    double g[3];
+    bool inside = true;
+    for (int d = 0; d < 3; d++) {
+        g[d] = (p.xyz[3 * (size_t)a + d] + p.shift[d]) / p.spacing;
+        // the 8 corners must lie on the grid: 0 <= g < n1 - 1
+        inside = inside && g[d] >= 0.0 && g[d] < (double)(p.n1[d] - 1);
+    }
+    ScoreAtom at;
+    at.gx = (float)g[0];
+    at.gy = (float)g[1];
+    at.gz = (float)g[2];
+    // FP32 rounding may carry g onto n1 - 1: keep such atoms outside
+    inside = inside && at.gx < (float)(p.n1[0] - 1) && at.gy < (float)(p.n1[1] - 1) && at.gz < (float)(p.n1[2] - 1);
+    at.q = p.charge[a];
+    at.map = p.map[a];
+    at.pose = p.pose[a];
+    at.inside = inside ? 1 : 0;
+    at.pad = 0;
+    p.atoms[a] = at;
+    const int i0 = (int)floorf(at.gx), j0 = (int)floorf(at.gy), k0 = (int)floorf(at.gz);
+    for (int c = 0; c < 8; c++) {
+        const unsigned pt = inside ? (unsigned)(i0 + (c & 1)) +
+                                         (unsigned)p.n1[0] * ((unsigned)(j0 + ((c >> 1) & 1)) +
+                                                              (unsigned)p.n1[1] * (unsigned)(k0 + (c >> 2)))
+                                   : p.P;
+        p.key[8 * (size_t)a + c] = pt;
+        p.entry[8 * (size_t)a + c] = 8 * a + c;
+    }
+}
+
+// One pass of a stable radix sort of (key, entry) pairs by eight bits: the
+// blocks' digit counts, their places in the output (a digit's blocks follow
+// each other), and the scatter.  A digit comes from the key, or from the entry's
+// atom's map (map + 1, so that atoms without one go first).  10,000 atoms, 80,000
+// pairs: about 11 us a pass, launches and their latency; the host's sort of the
+// 250,000 contributions and their upload took 5.4 ms.
+constexpr int kSortTile = 2048;   // pairs per block
+constexpr int kSortPer = kSortTile / kST;
+
+struct SortPass {
+    const unsigned *key;
+    const int *entry;
+    unsigned *key_out;
+    int *entry_out;
+    int n, shift;
+    const ScoreAtom *by_map;    // null: the digit is (key >> shift) & 255
+    int *count;                 // [blocks][256], then the first place of each
+};
+__device__ __forceinline__ int sort_digit(const SortPass &p, unsigned key, int entry) {
+    return p.by_map ? p.by_map[entry >> 3].map + 1 : (int)((key >> p.shift) & 255u);
+}
+
+__global__ void __launch_bounds__(kST) k_sort_count(SortPass p) {
+    __shared__ int bin[256];
+    bin[threadIdx.x] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kSortPer; r++) {
+        const int i = blockIdx.x * kSortTile + r * kST + threadIdx.x;
+        if (i < p.n) atomicAdd(&bin[sort_digit(p, p.key[i], p.entry[i])], 1);
+    }
+    __syncthreads();
+    p.count[blockIdx.x * 256 + threadIdx.x] = bin[threadIdx.x];
+}
+
+// count[b][d] -> pairs of smaller digits plus digit d's of earlier blocks.  One
+// workgroup: a thread walks a quarter of the blocks for one digit.
+__global__ void __launch_bounds__(1024) k_sort_scan(int *count, int blocks) {
+    __shared__ int part[4][256], wave_sum[4];
+    const int d = threadIdx.x & 255, g = threadIdx.x >> 8, lane = threadIdx.x & 63;
+    const int per = (blocks + 3) / 4, b0 = min(blocks, g * per), b1 = min(blocks, b0 + per);
+    int s = 0;
+#pragma unroll 8
+    for (int b = b0; b < b1; b++) s += count[b * 256 + d];
+    part[g][d] = s;
+    __syncthreads();
+    const int total = part[0][d] + part[1][d] + part[2][d] + part[3][d];
+    int x = total;   // inclusive scan over the digits: a wave's 64, then the waves before
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(x, o);
+        if (lane >= o) x += y;
+    }
+    if (lane == 63 && g == 0) wave_sum[d >> 6] = x;
+    __syncthreads();
+    int run = x - total;
+    for (int w = 0; w < (d >> 6); w++) run += wave_sum[w];
+    for (int k = 0; k < g; k++) run += part[k][d];
+#pragma unroll 8
+    for (int b = b0; b < b1; b++) {
+        const int c = count[b * 256 + d];
+        count[b * 256 + d] = run;
+        run += c;
+    }
+}
+
+// A wave takes a quarter of the block's tile in order: its digits' counts first,
+// then, with the waves' places known, 64 pairs at a time without a barrier.
+__global__ void __launch_bounds__(kST) k_sort_scatter(SortPass p) {
+    __shared__ int place[kST / 64][256];   // next free place per wave and digit
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (int w = 0; w < kST / 64; w++) place[w][threadIdx.x] = 0;
+    __syncthreads();
+    unsigned key[kSortPer];
+    int entry[kSortPer], digit[kSortPer];
+    const int first = blockIdx.x * kSortTile + wave * (kSortPer * 64) + lane;
+#pragma unroll
+    for (int r = 0; r < kSortPer; r++) {
+        const int i = first + 64 * r;
+        digit[r] = -1;
+        if (i < p.n) {
+            key[r] = p.key[i];
+            entry[r] = p.entry[i];
+            digit[r] = sort_digit(p, key[r], entry[r]);
+            atomicAdd(&place[wave][digit[r]], 1);
+        }
+    }
+    __syncthreads();
+    int run = p.count[blockIdx.x * 256 + threadIdx.x];
+    for (int w = 0; w < kST / 64; w++) {
+        const int c = place[w][threadIdx.x];
+        place[w][threadIdx.x] = run;
+        run += c;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kSortPer; r++) {
+        const bool act = digit[r] >= 0;
+        const int dg = act ? digit[r] : 0;
+        unsigned long long same = __ballot(act);   // the wave's lanes with this digit
+        for (int b = 0; b < 8; b++) {
+            const unsigned long long m = __ballot((dg >> b) & 1);
+            same &= (dg >> b) & 1 ? m : ~m;
+        }
+        const int rank = __popcll(same & ((1ull << lane) - 1));
+        const int at = place[wave][dg];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // every lane has read its place
+        __builtin_amdgcn_wave_barrier();
+        if (act) {
+            p.key_out[at + rank] = key[r];
+            p.entry_out[at + rank] = entry[r];
+            if (rank == 0) place[wave][dg] = at + __popcll(same);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+// Runs of equal keys, summed by their first entry's lane in FP64 in order: e
+// and d over all of a grid point's entries, an affinity map over the entries
+// of its own atoms.  Slots may coincide (an atom's map with e or d, e with d):
+// an entry then adds its map's, e's and d's term in that order.
+struct AdjParams {
+    const ScoreAtom *atoms;
+    int n;                      // entries, 8 per atom
+    unsigned P;
+    const unsigned *key;        // sorted by grid point
+    const int *entry;
+    const unsigned *mkey;       // sorted by map, then grid point
+    const int *mentry;
+    int e_slot, d_slot;
+    const float *dscore;
+    float *dmaps;
+};
+__device__ __forceinline__ float corner_weight(const ScoreAtom &at, int c) {
+    const float fx = at.gx - floorf(at.gx), fy = at.gy - floorf(at.gy), fz = at.gz - floorf(at.gz);
+    return ((c & 1) ? fx : 1.f - fx) * (((c >> 1) & 1) ? fy : 1.f - fy) * ((c >> 2) ? fz : 1.f - fz);
+}
+
+__global__ void __launch_bounds__(kST) k_score_adj(AdjParams p) {
+    const int i = blockIdx.x * kST + threadIdx.x;
+    if (i >= p.n) return;
+    if (blockIdx.y == 0) {
+        const unsigned pt = p.key[i];
+        if (pt >= p.P || (i > 0 && p.key[i - 1] == pt)) return;
+        double se = 0.0, sd = 0.0;
+        for (int k = i; k < p.n && p.key[k] == pt; k++) {
+            const int en = p.entry[k];
+            const ScoreAtom at = p.atoms[en >> 3];
+            const float w = corner_weight(at, en & 7);
+            const double g = (double)p.dscore[at.pose];
+            if (at.map == p.e_slot) se += (double)w * g;
+            se += (double)(w * at.q) * g;
+            if (p.d_slot == p.e_slot) {
+                se += (double)(w * fabsf(at.q)) * g;
+            } else {
+                if (at.map == p.d_slot) sd += (double)w * g;
+                sd += (double)(w * fabsf(at.q)) * g;
+            }
+        }
+        if (p.e_slot >= 0) p.dmaps[(size_t)p.e_slot * p.P + pt] = (float)se;
+        if (p.d_slot >= 0 && p.d_slot != p.e_slot) p.dmaps[(size_t)p.d_slot * p.P + pt] = (float)sd;
+    } else {
+        const unsigned pt = p.mkey[i];
+        const int m = p.atoms[p.mentry[i] >> 3].map;
+        if (pt >= p.P || m < 0 || m == p.e_slot || m == p.d_slot) return;
+        if (i > 0 && p.mkey[i - 1] == pt && p.atoms[p.mentry[i - 1] >> 3].map == m) return;
+        double s = 0.0;
+        for (int k = i; k < p.n && p.mkey[k] == pt; k++) {
+            const int en = p.mentry[k];
+            const ScoreAtom at = p.atoms[en >> 3];
+            if (at.map != m) break;
+            s += (double)corner_weight(at, en & 7) * (double)p.dscore[at.pose];
+        }
+        p.dmaps[(size_t)m * p.P + pt] = (float)s;
+    }
 }
 
 }  // namespace
@@ -131,85 +345,66 @@ struct ag_scorer {
     std::vector<int> pose_start;
     std::vector<int> map_index;
     std::vector<double> charge;
-    int n_rows = 0;
-    DevBuf atoms, pose_start_d, row_start, target, pose_of, val;
+    DevBuf atoms, pose_start_d, xyz, charge_d, map_d, pose_d;
+    DevBuf key[3], entry[3], count;
+    int by_point = 0, by_map = 0;   // buffers holding the two sorted lists
 };
 
 namespace agdev {
 
 static void scorer_positions(ag_scorer *s, const double *xyz) {
     const int n = s->n_atoms;
-    std::vector<ScoreAtom> h(std::max(n, 1));
-    struct Entry {
-        long long target;
-        int pose;
-        float val;
-    };
-    std::vector<Entry> ent;
-    ent.reserve((size_t)n * 24);
-    for (int p = 0; p < s->n_poses; p++)
-        for (int a = s->pose_start[p]; a < s->pose_start[p + 1]; a++) {
-            ScoreAtom &at = h[a];
-            double g[3];
-            bool inside = true;
-            for (int d = 0; d < 3; d++) {
-                if (!std::isfinite(xyz[3 * (size_t)a + d])) ag::fail(AG_ERR_BAD_INPUT, "ligand position is not finite");
-                g[d] = (xyz[3 * (size_t)a + d] + s->ne[d] * s->spacing) / s->spacing;
-                // the 8 corners must lie on the grid: 0 <= g < n1 - 1
-                inside = inside && g[d] >= 0.0 && g[d] < (double)(s->n1[d] - 1);
-            }
-            at.gx = (float)g[0];
-            at.gy = (float)g[1];
-            at.gz = (float)g[2];
-            // FP32 rounding may carry g onto n1 - 1: keep such atoms outside
-            inside = inside && at.gx < (float)(s->n1[0] - 1) && at.gy < (float)(s->n1[1] - 1) &&
-                     at.gz < (float)(s->n1[2] - 1);
-            at.q = (float)s->charge[a];
-            at.map = s->map_index[a];
-            at.pose = p;
-            at.inside = inside ? 1 : 0;
-            at.pad = 0;
-            if (!inside) continue;
-            // contributions to dL/dmaps, from the same FP32 weights k_score uses
-            const int i0 = (int)floorf(at.gx), j0 = (int)floorf(at.gy), k0 = (int)floorf(at.gz);
-            const float fx = at.gx - (float)i0, fy = at.gy - (float)j0, fz = at.gz - (float)k0;
-            for (int c = 0; c < 8; c++) {
-                const int dx = c & 1, dy = (c >> 1) & 1, dz = c >> 2;
-                const long long idx = (long long)(i0 + dx) +
-                                      (long long)s->n1[0] * ((long long)(j0 + dy) + (long long)s->n1[1] * (k0 + dz));
-                const float w = (dx ? fx : 1.f - fx) * (dy ? fy : 1.f - fy) * (dz ? fz : 1.f - fz);
-                if (at.map >= 0) ent.push_back({(long long)at.map * s->P + idx, p, w});
-                if (s->e_slot >= 0) ent.push_back({(long long)s->e_slot * s->P + idx, p, w * at.q});
-                if (s->d_slot >= 0) ent.push_back({(long long)s->d_slot * s->P + idx, p, w * std::fabs(at.q)});
-            }
-        }
-    std::stable_sort(ent.begin(), ent.end(), [](const Entry &x, const Entry &y) { return x.target < y.target; });
-    std::vector<int> rs, pose_of;
-    std::vector<long long> tg;
-    std::vector<float> val;
-    rs.reserve(ent.size() + 1);
-    for (size_t k = 0; k < ent.size(); k++) {
-        if (k == 0 || ent[k].target != ent[k - 1].target) {
-            rs.push_back((int)k);
-            tg.push_back(ent[k].target);
-        }
-        pose_of.push_back(ent[k].pose);
-        val.push_back(ent[k].val);
-    }
-    rs.push_back((int)ent.size());
-    if (ent.size() > (size_t)INT32_MAX) ag::fail(AG_ERR_UNSUPPORTED, "too many ligand atoms for one scorer");
-    s->n_rows = (int)tg.size();
+    for (size_t i = 0; i < 3 * (size_t)n; i++)
+        if (!std::isfinite(xyz[i])) ag::fail(AG_ERR_BAD_INPUT, "ligand position is not finite");
     hipStream_t st = s->ctx->stream;
-    auto up = [&](DevBuf &b, const void *src, size_t bytes) {
-        void *d = b.get(std::max<size_t>(bytes, 16));
-        if (bytes) HIP_CHECK(hipMemcpyAsync(d, src, bytes, hipMemcpyHostToDevice, st));
+    const size_t n8 = 8 * (size_t)n;
+    if (n8 > (size_t)INT32_MAX) ag::fail(AG_ERR_UNSUPPORTED, "too many ligand atoms for one scorer");
+    PlaceParams pp;
+    memset(&pp, 0, sizeof pp);
+    pp.xyz = (const double *)s->xyz.get(sizeof(double) * 3 * (size_t)n);
+    pp.charge = (const float *)s->charge_d.ptr;
+    pp.map = (const int *)s->map_d.ptr;
+    pp.pose = (const int *)s->pose_d.ptr;
+    pp.n = n;
+    for (int d = 0; d < 3; d++) {
+        pp.n1[d] = s->n1[d];
+        pp.shift[d] = s->ne[d] * s->spacing;
+    }
+    pp.spacing = s->spacing;
+    pp.P = (unsigned)s->P;
+    pp.atoms = (ScoreAtom *)s->atoms.get(sizeof(ScoreAtom) * (size_t)n);
+    const int blocks = (int)((n8 + kSortTile - 1) / kSortTile);
+    for (int k = 0; k < 3; k++) {
+        s->key[k].get(sizeof(unsigned) * n8);
+        s->entry[k].get(sizeof(int) * n8);
+    }
+    int *count = (int *)s->count.get(sizeof(int) * 256 * (size_t)std::max(blocks, 1));
+    if (n == 0) return;
+    // pinned staging: one DMA instead of the runtime's own staged copy
+    void *stage = s->ctx->stage.get(sizeof(double) * 3 * (size_t)n);
+    memcpy(stage, xyz, sizeof(double) * 3 * (size_t)n);
+    HIP_CHECK(hipMemcpyAsync(s->xyz.ptr, stage, sizeof(double) * 3 * (size_t)n, hipMemcpyHostToDevice, st));
+    pp.key = (unsigned *)s->key[0].ptr;
+    pp.entry = (int *)s->entry[0].ptr;
+    k_score_place<<<(n + kST - 1) / kST, kST, 0, st>>>(pp);
+    const auto pass = [&](int from, int to, int shift, bool by_map) {
+        SortPass sp{(const unsigned *)s->key[from].ptr, (const int *)s->entry[from].ptr, (unsigned *)s->key[to].ptr,
+                    (int *)s->entry[to].ptr, (int)n8, shift, by_map ? pp.atoms : nullptr, count};
+        k_sort_count<<<blocks, kST, 0, st>>>(sp);
+        k_sort_scan<<<1, 1024, 0, st>>>(count, blocks);
+        k_sort_scatter<<<blocks, kST, 0, st>>>(sp);
     };
-    up(s->atoms, h.data(), sizeof(ScoreAtom) * (size_t)n);
-    up(s->row_start, rs.data(), sizeof(int) * rs.size());
-    up(s->target, tg.data(), sizeof(long long) * tg.size());
-    up(s->pose_of, pose_of.data(), sizeof(int) * pose_of.size());
-    up(s->val, val.data(), sizeof(float) * val.size());
-    HIP_CHECK(hipStreamSynchronize(st));   // host vectors go out of scope
+    int cur = 0;
+    for (int shift = 0; shift < 32 && ((unsigned long long)s->P >> shift) > 0; shift += 8) {
+        pass(cur, 1 - cur, shift, false);
+        cur = 1 - cur;
+    }
+    s->by_point = cur;
+    // one more pass, by map: (map, grid point) order, from the sorted list
+    pass(cur, 2, 0, true);
+    s->by_map = 2;
+    HIP_CHECK(hipGetLastError());
+    HIP_CHECK(hipStreamSynchronize(st));   // the staging buffer is the context's
 }
 
 ag_scorer *scorer_create(ag_ctx *c, const ag_grid *grid, int n_maps, int elec_index, int dsolv_index, int n_poses,
@@ -249,9 +444,22 @@ ag_scorer *scorer_create(ag_ctx *c, const ag_grid *grid, int n_maps, int elec_in
     s->pose_start.assign(pose_start, pose_start + n_poses + 1);
     s->map_index.assign(map_index, map_index + n);
     s->charge.assign(charge, charge + n);
-    void *d = s->pose_start_d.get(sizeof(int) * (size_t)(n_poses + 1));
-    HIP_CHECK(hipMemcpyAsync(d, s->pose_start.data(), sizeof(int) * (size_t)(n_poses + 1), hipMemcpyHostToDevice,
-                             c->stream));
+    std::vector<float> q(std::max(n, 1));
+    std::vector<int> pose(std::max(n, 1));
+    for (int p = 0; p < n_poses; p++)
+        for (int a = pose_start[p]; a < pose_start[p + 1]; a++) {
+            q[a] = (float)charge[a];
+            pose[a] = p;
+        }
+    const auto up = [&](DevBuf &b, const void *src, size_t bytes) {
+        void *d = b.get(std::max<size_t>(bytes, 16));
+        if (bytes) HIP_CHECK(hipMemcpyAsync(d, src, bytes, hipMemcpyHostToDevice, c->stream));
+    };
+    up(s->pose_start_d, s->pose_start.data(), sizeof(int) * (size_t)(n_poses + 1));
+    up(s->charge_d, q.data(), sizeof(float) * (size_t)n);
+    up(s->map_d, s->map_index.data(), sizeof(int) * (size_t)n);
+    up(s->pose_d, pose.data(), sizeof(int) * (size_t)n);
+    HIP_CHECK(hipStreamSynchronize(c->stream));   // host vectors go out of scope
     scorer_positions(s.get(), xyz);
     return s.release();
 }
@@ -291,11 +499,13 @@ void scorer_adjoint(ag_scorer *s, const float *d_dscore, float *d_dmaps) {
     const long long total = s->P * s->n_maps;
     const unsigned zb = (unsigned)std::min<long long>((total + 255) / 256, 65536);
     k_score_zero<<<zb, 256, 0, st>>>(d_dmaps, total);
-    if (s->n_rows > 0)
-        k_score_adj<<<(s->n_rows + 255) / 256, 256, 0, st>>>(s->n_rows, (const int *)s->row_start.ptr,
-                                                             (const long long *)s->target.ptr,
-                                                             (const int *)s->pose_of.ptr, (const float *)s->val.ptr,
-                                                             d_dscore, d_dmaps);
+    if (s->n_atoms > 0) {
+        const int n8 = 8 * s->n_atoms;
+        AdjParams p{(const ScoreAtom *)s->atoms.ptr, n8, (unsigned)s->P, (const unsigned *)s->key[s->by_point].ptr,
+                    (const int *)s->entry[s->by_point].ptr, (const unsigned *)s->key[s->by_map].ptr,
+                    (const int *)s->entry[s->by_map].ptr, s->e_slot, s->d_slot, d_dscore, d_dmaps};
+        k_score_adj<<<dim3((unsigned)((n8 + kST - 1) / kST), 2), kST, 0, st>>>(p);
+    }
     HIP_CHECK(hipGetLastError());
     HIP_CHECK(hipStreamSynchronize(st));
 }
