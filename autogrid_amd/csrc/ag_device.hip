@@ -82,12 +82,12 @@ struct __align__(16) NearAtom {   // 96 bytes
     float qe;                     // charge * coeff_estat
     float vol;
     float solq;                   // solpar + solpar_q * |charge|
-    float dvol;                   // solpar_q * vol (d map)
+    float rv2sq;                  // |rv2|^2
     float rv[3];
     int meta;                     // type | hbond << 8 | rexp << 16 | disorder << 24
     float rv2[3];
     int index;                    // atom index in the receptor
-    float xE, yE, zE;             // the far kernel's coordinates (128 * coord, float)
+    float rv2xrv[3];              // rv2 x rv
     float pad;
 };
 static_assert(sizeof(NearAtom) == 96, "NearAtom layout");
@@ -172,6 +172,7 @@ struct NearParams {
     int out_slot[kMapSlots];      // output map of each slot, -1 if unused
     int e_slot, d_slot;           // -1 when not produced in this pass
     int has_affinity;             // any slot in use, or the d map
+    float solpar_q;
     int disorder_h, hydrogen_type;
     int *cmap;                    // constriction count per point, or null (pass 0 only)
     double ccut;                  // constriction distance cutoff (<= 8 A)
@@ -416,17 +417,18 @@ __global__ void k_gather(const int *nslots, const int *slot_atom, AtomSrc s, Nea
     a.qe = (float)(q * s.coeff_estat);
     a.vol = (float)s.vol[i];
     a.solq = (float)(s.solpar[i] + s.solpar_q * fabs(q));
-    a.dvol = (float)(s.solpar_q * s.vol[i]);
+    const double *u = s.rvec + 3 * (size_t)i, *v = s.rvec2 + 3 * (size_t)i;
+    a.rv2sq = (float)(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
+    a.rv2xrv[0] = (float)(v[1] * u[2] - v[2] * u[1]);
+    a.rv2xrv[1] = (float)(v[2] * u[0] - v[0] * u[2]);
+    a.rv2xrv[2] = (float)(v[0] * u[1] - v[1] * u[0]);
     for (int d = 0; d < 3; d++) {
-        a.rv[d] = (float)s.rvec[3 * i + d];
-        a.rv2[d] = (float)s.rvec2[3 * i + d];
+        a.rv[d] = (float)u[d];
+        a.rv2[d] = (float)v[d];
     }
     a.meta = (s.type[i] & 0xff) | ((s.hbond[i] & 0xff) << 8) | ((s.rexp[i] & 0xff) << 16) |
              ((s.disorder[i] ? 1 : 0) << 24);
     a.index = i;
-    a.xE = (float)(a.x * 128.0);
-    a.yE = (float)(a.y * 128.0);
-    a.zE = (float)(a.z * 128.0);
     a.pad = 0.f;
     out[k] = a;
 }
@@ -470,6 +472,12 @@ __device__ __forceinline__ double ref_dist(double ax, double ay, double az, doub
     dz = az - cz;
     return sqrt(dx * dx + dy * dy + dz * dz);
 }
+
+// Smaller and larger of two values neither of which is NaN, in one
+// instruction: fminf and fmaxf first quieten an operand that might be a
+// signalling NaN.
+__device__ __forceinline__ float min_of(float a, float b) { return __builtin_amdgcn_fmed3f(a, b, -__builtin_inff()); }
+__device__ __forceinline__ float max_of(float a, float b) { return __builtin_amdgcn_fmed3f(a, b, __builtin_inff()); }
 
 // Uniform per-atom values: every lane reads the same LDS record, so its
 // fields are moved to scalar registers and branches on them stay scalar.
@@ -729,7 +737,7 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
         qy += by * kBY;
         qz += bz * kBZ;
     };
-    float e_near = 0.f, d_acc = 0.f, dv_acc = 0.f, dq_acc = 0.f;
+    float e_near = 0.f, dv_acc = 0.f, dq_acc = 0.f;
     int ccount = 0;
     const bool want_cmap = GENERAL && p.cmap != nullptr;
     const float *tab = p.tab;
@@ -801,7 +809,7 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
                 if (r2 > 64.33f) continue;  // beyond 8.02 A: neither cutoff pass nor near e term
                 // hardware rsq: 128 r is good to ~3e-4 bins here, inside the guard band;
                 // the same rsq is 1/r for the near e term and the unit vector
-                const float r2c = fmaxf(r2, 1.0e-12f);
+                const float r2c = max_of(r2, 1.0e-12f);
                 float inv_r = __builtin_amdgcn_rsqf(r2c);
                 float r = r2c * inv_r;
                 const float g = r * 128.f;
@@ -870,17 +878,17 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
                 if (want_e) {
                     bool near_e = g < 1022.f;
                     if (g >= 1022.f && g <= 1027.f) {
-                        // the far kernel's point coordinates: run centre, offset in the run, y, z
+                        // the far kernel's coordinates of the atom and the point: run centre, offset in the run, y, z
                         int qx, qy, qz;
                         point_index(qx, qy, qz);
                         const int kxE = qx % kFarK;
-                        near_e = far_bin4(a.xE, a.yE, a.zE, far_cx(qx - kxE, nex, s128), kxE, s128,
+                        near_e = far_bin4((float)(ax * 128.0), (float)(ay * 128.0), (float)(az * 128.0), far_cx(qx - kxE, nex, s128), kxE, s128,
                                           (float)(qy - ney) * s128, (float)(qz - nez) * s128, far_floor(s128)) <
                                  4u * kFarBinMin;
                     }
                     // 1/max(r, 0.5) with r clamped at APPROX_ZERO; adding 0 leaves
                     // the sum as it is (it is never -0)
-                    const float inv_rmax = fminf(inv_r, 2.f);
+                    const float inv_rmax = min_of(inv_r, 2.f);
                     const float te = unif(a.qe) * inv_rmax * rsv.x;
                     e_near += near_e ? te : 0.f;
                 }
@@ -932,8 +940,7 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
                                 racc = rexp == 2 ? c2 : (rexp == 4 ? c2 * c2 : cos_t);
                                 if (aidx != best_idx) {
                                     float ct = hrv[0] * rv0 + hrv[1] * rv1 + hrv[2] * rv2;
-                                    ct = fminf(fmaxf(ct, -1.f), 1.f);
-                                    Hramp = 0.5f - 0.5f * cosf(acosf(ct) * (120.f / 90.f));
+                                    Hramp = hramp_value(__builtin_amdgcn_fmed3f(ct, -1.f, 1.f));
                                 }
                             }
                         } else {
@@ -941,23 +948,18 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
                             // y = (dn x rv2).rv / |dn x rv2|:
                             //   t0 = pi/2 - acos(x)         -> cos(t0) = sqrt(1 - x^2)
                             //   ti = |acos(y) - pi/2|       -> sin(2 ti) = 2|y| sqrt(1 - y^2)
-                            const float rw0 = unif(a.rv2[0]), rw1 = unif(a.rv2[1]), rw2 = unif(a.rv2[2]);
-                            float t0 = dn0 * rw0 + dn1 * rw1 + dn2 * rw2;
-                            t0 = fminf(fmaxf(t0, -1.f), 1.f);
-                            const float cos_t0 = __builtin_amdgcn_sqrtf(fmaxf(1.f - t0 * t0, 0.f));
+                            // and, from the record, (dn x rv2).rv = dn.(rv2 x rv),
+                            // |dn x rv2|^2 = |rv2|^2 - x^2 (dn a unit vector).
+                            const float x = dn0 * unif(a.rv2[0]) + dn1 * unif(a.rv2[1]) + dn2 * unif(a.rv2[2]);
+                            const float cos_t0 = __builtin_amdgcn_sqrtf(max_of(__builtin_fmaf(-x, x, 1.f), 0.f));
                             rdon = 0.f;
                             if (pos) {
-                                const float cr0 = dn1 * rw2 - dn2 * rw1;
-                                const float cr1 = dn2 * rw0 - dn0 * rw2;
-                                const float cr2 = dn0 * rw1 - dn1 * rw0;
-                                float rd2 = cr0 * cr0 + cr1 * cr1 + cr2 * cr2;
-                                if (rd2 < 1.0e-6f) rd2 = 1.0e-6f;
-                                const float inv_rd = __builtin_amdgcn_rsqf(rd2);
-                                float ti = (cr0 * inv_rd) * rv0 + (cr1 * inv_rd) * rv1 + (cr2 * inv_rd) * rv2;
-                                ti = fminf(fmaxf(ti, -1.f), 1.f);
-                                const float sin2ti =
-                                    2.f * fabsf(ti) * __builtin_amdgcn_sqrtf(fmaxf(1.f - ti * ti, 0.f));
-                                rdon = (0.9f + 0.1f * sin2ti) * cos_t0;
+                                const float rd2 = max_of(__builtin_fmaf(-x, x, unif(a.rv2sq)), 1.0e-6f);
+                                const float yn = dn0 * unif(a.rv2xrv[0]) + dn1 * unif(a.rv2xrv[1]) +
+                                                 dn2 * unif(a.rv2xrv[2]);
+                                const float y = min_of(fabsf(yn) * __builtin_amdgcn_rsqf(rd2), 1.f);
+                                const float s2 = y * __builtin_amdgcn_sqrtf(max_of(__builtin_fmaf(-y, y, 1.f), 0.f));
+                                rdon = __builtin_fmaf(0.2f, s2, 0.9f) * cos_t0;
                             } else if (cos_t >= -0.34202f) {
                                 const float u = 0.116978f - cos_t * cos_t;
                                 rdon = 562.25f * (u * u * u) * cos_t0;
@@ -993,22 +995,21 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
                 // H-bonding slots (main.cpp:3286-3374): the (probe, atom) case is a
                 // set of 0/1 coefficients chosen per atom class, uniform across
                 // the wave.  The plain table add is fma(c, E, acc) with c = 1 or
-                // 0 (bit for bit acc + E, or acc); the directional mix runs in a
-                // scalar branch for the classes that have one, with every slot's
-                // update written without a branch of its own, so the
-                // accumulators and min/max keep their registers through it.  A
-                // disordered partner uses the hydrogen-type row at r - 1.10 A
-                // (main.cpp:3313-3349), FP64 like the reference.
+                // 0 (bit for bit acc + E, or acc); the directional mix runs in
+                // scalar branches, one for the classes that have one and one per
+                // slot: acceptor atoms mix into the donor probe's slot alone, so
+                // three of four updates are skipped there.  A disordered partner
+                // uses the hydrogen-type row at r - 1.10 A (main.cpp:3313-3349),
+                // FP64 like the reference.
                 const int dsh = dis ? 4 : 0;
-                bool any_mix = false;
     #pragma unroll
                 for (int k = 0; k < kHbSlots; k++) {
                     const int code = (hw >> (8 * k + dsh)) & 15;
-                    any_mix |= (code & ~HC_PLAIN) != 0;
                     const float kP = __int_as_float((code & HC_PLAIN) ? 0x3f800000 : 0);
                     acc[kPlainSlots + k] = __builtin_fmaf(kP, E[kPlainSlots + k], acc[kPlainSlots + k]);
                 }
-                if (any_mix) {
+                constexpr unsigned kMixBits = (HC_HRAMP | HC_MINMAX) * 0x01010101u;
+                if ((hw >> dsh) & kMixBits) {
                     float Eh[kHbSlots] = {0.f, 0.f, 0.f, 0.f};
                     if (dis && p.hydrogen_type >= 0) {
                         double rdx, rdy, rdz;
@@ -1018,26 +1019,24 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
                             tab + ((size_t)p.hydrogen_type * AG_NEINT + hb_bin) * kMapSlots)[kPlainSlots / 4];
                         Eh[0] = v.x; Eh[1] = v.y; Eh[2] = v.z; Eh[3] = v.w;
                     }
-                    const float dfac = racc - rdon;
     #pragma unroll
                     for (int k = 0; k < kHbSlots; k++) {
                         const int m = kPlainSlots + k;
                         const int code = (hw >> (8 * k + dsh)) & 15;
+                        if (!(code & (HC_HRAMP | HC_MINMAX))) continue;   // scalar
                         const float e = E[m];
-                        // 0/1 coefficients as scalar float bit patterns
-                        const float kF = __int_as_float((code & HC_RACC) ? 0x3f800000 : 0);
-                        const float kH = __int_as_float((code & HC_HRAMP) ? 0x3f800000 : 0);
-                        const bool mm = (code & HC_MINMAX) != 0;
+                        const float f = (code & HC_RACC) ? racc : rdon;
                         const float rsph = __builtin_amdgcn_fmed3f(e * 0.01f, 0.f, 1.f);
-                        const float f = __builtin_fmaf(kF, dfac, rdon);
                         const float mix = __builtin_fmaf(1.f - f, rsph, f);
-                        acc[m] = __builtin_fmaf((kH * (dis ? Eh[k] : e)) * Hramp, mix, acc[m]);
-                        const float v = e * mix;
-                        hmin[k] = fminf(hmin[k], mm ? v : __builtin_inff());
-                        hmax[k] = fmaxf(hmax[k], mm ? v : -__builtin_inff());
+                        if (code & HC_HRAMP)
+                            acc[m] = __builtin_fmaf((dis ? Eh[k] : e) * Hramp, mix, acc[m]);
+                        if (code & HC_MINMAX) {
+                            const float v = e * mix;
+                            hmin[k] = min_of(hmin[k], v);
+                            hmax[k] = max_of(hmax[k], v);
+                        }
                     }
                 }
-                if (p.d_slot >= 0) d_acc += unif(a.dvol) * S;
             }
         }
         if constexpr (!PAGED) break;
@@ -1063,7 +1062,7 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
         if (want_e) maps[(long long)p.e_slot * P + pt] = e_near;
         if (cmap) cmap[pt] = ccount;
         if (p.collide) p.collide[cf.pt_off + pt] = collide ? 1 : 0;
-        if (p.d_slot >= 0) maps[(long long)p.d_slot * P + pt] = d_acc;
+        if (p.d_slot >= 0) maps[(long long)p.d_slot * P + pt] = p.solpar_q * dv_acc;   // solpar_q sum(vol S)
     }
 }
 
@@ -2213,6 +2212,7 @@ static ag_plan *plan_build(ag_ctx *c, int n, const ag_receptor *recs, const ag_g
     np.reps = d_reps;
     np.disorder_h = ms->disorder_h;
     np.hydrogen_type = ms->hydrogen_type;
+    np.solpar_q = (float)ms->solpar_q;
     np.status = (int *)p.status.ptr;
     for (int g = 0; g < p.groups; g++) {
         NearParams q = np;
