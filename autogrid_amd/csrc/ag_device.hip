@@ -53,6 +53,7 @@ namespace {
 
 constexpr int kBX = 8, kBY = 8, kBZ = 4;          // brick of the near kernel
 constexpr int kNearThreads = kBX * kBY * kBZ;     // 256
+constexpr int kStage = 3;                         // atoms per thread of a staging round
 constexpr int kMapSlots = 16;                     // maps per near-kernel pass
 constexpr int kPlainSlots = 12;                   // of which without H-bond terms
 constexpr int kHbSlots = kMapSlots - kPlainSlots; // of which H-bonding probes
@@ -82,13 +83,15 @@ struct __align__(16) NearAtom {   // 96 bytes
     float qe;                     // charge * coeff_estat
     float vol;
     float solq;                   // solpar + solpar_q * |charge|
+    int meta;                     // type | hbond << 8 | rexp << 16 | disorder << 24
+    int index;                    // atom index in the receptor
     float rv2sq;                  // |rv2|^2
     float rv[3];
-    int meta;                     // type | hbond << 8 | rexp << 16 | disorder << 24
+    float pad0;
     float rv2[3];
-    int index;                    // atom index in the receptor
+    float pad1;
     float rv2xrv[3];              // rv2 x rv
-    float pad;
+    float pad2;
 };
 static_assert(sizeof(NearAtom) == 96, "NearAtom layout");
 
@@ -99,6 +102,8 @@ struct ConfDev {
     int n1[3], ne[3];
     double spacing;
     float s128;                   // (float)(spacing * 128)
+    float near_band;              // far_band: half-width (bins) of the shell where the far kernel's bin decides
+    int near_share;               // near kernel: waves (1, 2 or 4) that share a cube's atoms
     int nb[3];                    // bricks per axis
     double cell_origin[3];
     int nc[3];
@@ -160,7 +165,8 @@ struct NearParams {
     const double *rvec64;         // [n][3]
     const double *rvec2_64;       // [n][3]
     // tables
-    const float *tab;             // [T][1024][kMapSlots] for this pass's maps
+    const float *tab;             // [T][1024][row slots] for this pass's maps (near_row)
+    unsigned zero_off;            // byte offset from tab of a row of zeros
     const float *sol;             // [1025]
     const float *reps;            // [8192] electrostatic factor (r_eps or 332/diel)
     // map slots of this pass: [0, kPlainSlots) maps without H-bond terms,
@@ -429,7 +435,7 @@ __global__ void k_gather(const int *nslots, const int *slot_atom, AtomSrc s, Nea
     a.meta = (s.type[i] & 0xff) | ((s.hbond[i] & 0xff) << 8) | ((s.rexp[i] & 0xff) << 16) |
              ((s.disorder[i] ? 1 : 0) << 24);
     a.index = i;
-    a.pad = 0.f;
+    a.pad0 = a.pad1 = a.pad2 = 0.f;
     out[k] = a;
 }
 
@@ -445,24 +451,6 @@ __global__ void k_far_atoms(int n, const double *coord, const double *charge, do
 // near kernel
 // ---------------------------------------------------------------------------
 
-// Block-wide ordered compaction helper: returns this thread's output position
-// among flagged threads and the block total (256 threads = 4 waves).
-__device__ __forceinline__ int block_compact(bool flag, int *wave_tot, int &total) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const unsigned long long m = __ballot(flag);
-    const int before = __popcll(m & ((1ull << lane) - 1ull));
-    if (lane == 0) wave_tot[wave] = __popcll(m);
-    __syncthreads();
-    int base = 0;
-    total = 0;
-    for (int w = 0; w < kNearThreads / 64; w++) {
-        if (w < wave) base += wave_tot[w];
-        total += wave_tot[w];
-    }
-    __syncthreads();
-    return base + before;
-}
-
 __device__ __forceinline__ double ref_dist(double ax, double ay, double az, double cx, double cy, double cz,
                                            double &dx, double &dy, double &dz) {
 #pragma clang fp contract(off)
@@ -473,11 +461,25 @@ __device__ __forceinline__ double ref_dist(double ax, double ay, double az, doub
     return sqrt(dx * dx + dy * dy + dz * dz);
 }
 
+// Orders a wave's own LDS accesses: its lanes see what the others wrote before.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // Smaller and larger of two values neither of which is NaN, in one
 // instruction: fminf and fmaxf first quieten an operand that might be a
 // signalling NaN.
-__device__ __forceinline__ float min_of(float a, float b) { return __builtin_amdgcn_fmed3f(a, b, -__builtin_inff()); }
-__device__ __forceinline__ float max_of(float a, float b) { return __builtin_amdgcn_fmed3f(a, b, __builtin_inff()); }
+__device__ __forceinline__ float min_of(float a, float b) {
+    float r;
+    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float max_of(float a, float b) {
+    float r;
+    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
 
 // Uniform per-atom values: every lane reads the same LDS record, so its
 // fields are moved to scalar registers and branches on them stay scalar.
@@ -486,14 +488,14 @@ __device__ __forceinline__ float unif(float v) {
     return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
 }
 
-// A thread's point inside the 8x8x4 brick: each wave takes an 8x8x1 slab
-// (CUBE false) or a 4x4x4 cube (CUBE true) of points.
+// A thread's point inside the brick: each wave takes a 4x4x4 cube, shared by
+// `share` consecutive waves, or (CUBE false, nothing shared) an 8x8x1 slab.
 template <bool CUBE>
-__device__ __forceinline__ void brick_lane(int tid, int &lx, int &ly, int &lz) {
-    if (CUBE) {
-        const int wave = tid >> 6, lane = tid & 63;
-        lx = (wave & 1) * 4 + (lane & 3);
-        ly = (wave >> 1) * 4 + ((lane >> 2) & 3);
+__device__ __forceinline__ void brick_lane(int tid, int share, int &lx, int &ly, int &lz) {
+    if (CUBE || share > 1) {
+        const int cube = (tid >> 6) / share, lane = tid & 63;
+        lx = (cube & 1) * 4 + (lane & 3);
+        ly = (cube >> 1) * 4 + ((lane >> 2) & 3);
         lz = lane >> 4;
     } else {
         lx = tid % kBX;
@@ -502,7 +504,23 @@ __device__ __forceinline__ void brick_lane(int tid, int &lx, int &ly, int &lz) {
     }
 }
 
-// CUBE selects the lane layout inside the 8x8x4 brick (brick_lane).  FORM:
+// Slots of a table row: NPLAIN == 4 keeps four plain and four H-bond slots (32
+// bytes), the others all sixteen (64 bytes).
+__host__ __device__ constexpr int near_row(int nplain) { return nplain == 4 ? 8 : 16; }
+
+// One value of a lane in each lane of its group of Q (2 or 4) neighbours, J the
+// lane's place in the group.
+template <int Q, int J>
+__device__ __forceinline__ int group_lane(int v) {
+    constexpr int ctrl = Q == 4 ? J * 0x55 : (J | J << 2 | (2 + J) << 4 | (2 + J) << 6);
+    return __builtin_amdgcn_mov_dpp(v, ctrl, 0xf, 0xf, true);
+}
+
+// Bound by its vector operations (issued in about 85 % of the cycles; 60 per
+// pair of a wave and a plain atom, 100 to 150 where the atom is directional),
+// then by the table reads.  5,000 atoms, 127^3 points: 13 Vina maps
+// 1,096 -> 712 us, 15 AutoDock maps 1,099 -> 812; 41^3 points and 1,000 atoms 157
+// -> 62.  CUBE selects the lane layout inside the brick (brick_lane).  FORM:
 //   kNearPlain   neither the tree build's queries, a constriction count
 //                nor disordered hydroxyls (their branches compiled out);
 //   kNearGeneral every map-set option;
@@ -513,25 +531,34 @@ __device__ __forceinline__ void brick_lane(int tid, int &lx, int &ly, int &lz) {
 // set again with the paged form (whose page loops keep state beside the
 // accumulators, with spills the common case should not pay for).
 enum : int { kNearPlain = 0, kNearGeneral = 1, kNearPaged = 2 };
+struct NearLists {
+    double hpos[kHCap][3];
+    int cand[kCandCap];
+    int hidx[kHCap];
+    float hrvs[kHCap][3];
+};
 template <int NPLAIN, bool CUBE, int FORM>
-__global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_eu(5))) k_near(NearParams p) {
+__global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_eu(FORM == kNearPlain ? 5 : 4))) k_near(NearParams p) {
     constexpr bool PAGED = FORM == kNearPaged;
     constexpr bool GENERAL = FORM != kNearPlain;
-    __shared__ int cand[kCandCap];
-    __shared__ int hcand[kHCap];
-    __shared__ double hpos[kHCap][3];
-    __shared__ int hidx[kHCap];
-    __shared__ float hrvs[kHCap][3];
+    __shared__ NearLists lists;   // reused at the end for the table sums
+    int *const cand = lists.cand, *const hidx = lists.hidx;
+    double(*const hpos)[3] = lists.hpos;
+    float(*const hrvs)[3] = lists.hrvs;
+    float *const scratch_f = reinterpret_cast<float *>(&lists);
+    static_assert(sizeof(NearLists) >= sizeof(float) * kNearThreads * (kMapSlots + 1), "room for the table sums");
     __shared__ float2 rs_s[kNearRepsLen];   // (electrostatic factor, sol_fn) per bin
-    __shared__ int wave_tot[kNearThreads / 64];
-    __shared__ int cell_off[kNearThreads + 1];
-    __shared__ int cstart_s[kNearThreads];
-    __shared__ int ncand_s, nh_s;
+    __shared__ int2 wave_tot[2][kStage][kNearThreads / 64];
 
     const int tid = threadIdx.x;
-    for (int k = tid; k < kNearRepsLen; k += kNearThreads) rs_s[k] = make_float2(p.reps[k], p.sol[min(k, AG_NEINT)]);
-    int lx, ly, lz;
-    brick_lane<CUBE>(tid, lx, ly, lz);
+    // read here, stored once the staging's own reads are on their way
+    constexpr int kRsPer = (kNearRepsLen + kNearThreads - 1) / kNearThreads;
+    float2 rs[kRsPer];
+#pragma unroll
+    for (int u = 0; u < kRsPer; u++) {
+        const int k = min(tid + u * kNearThreads, kNearRepsLen - 1);
+        rs[u] = make_float2(p.reps[k], p.sol[min(k, AG_NEINT)]);
+    }
 
     // one workgroup per brick of all conformations, in chunks of 16 bricks
     // spread over the XCDs: a brick's time follows the local atom density,
@@ -552,13 +579,22 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
     const int bx = brick % cf.nb[0];
     const int by = (brick / cf.nb[0]) % cf.nb[1];
     const int bz = brick / (cf.nb[0] * cf.nb[1]);
-    const int ix = bx * kBX + lx;
-    const int iy = by * kBY + ly;
-    const int iz = bz * kBZ + lz;
+    // With share > 1 the workgroup has a brick of 4 / share cubes of 4x4x4
+    // points, and the share waves of a cube hold the same points and take each
+    // share-th candidate (and donor H), the sums added up at the end.
+    const int share = cf.near_share;
+    const bool shared = share > 1;
+    const int first = uni((tid >> 6) & (share - 1));
+    const int ex = share > 2 ? kBX / 2 : kBX, ey = shared ? kBY / 2 : kBY;
+    const int ix0 = bx * ex, iy0 = by * ey, iz0 = bz * kBZ;
+    int lx, ly, lz;
+    brick_lane<CUBE>(tid, share, lx, ly, lz);
+    const int ix = ix0 + lx;
+    const int iy = iy0 + ly;
+    const int iz = iz0 + lz;
 
     // brick box in the grid frame
-    const int ix0 = bx * kBX, iy0 = by * kBY, iz0 = bz * kBZ;
-    const int ix1 = min(ix0 + kBX, n1x) - 1, iy1 = min(iy0 + kBY, n1y) - 1, iz1 = min(iz0 + kBZ, n1z) - 1;
+    const int ix1 = min(ix0 + ex, n1x) - 1, iy1 = min(iy0 + ey, n1y) - 1, iz1 = min(iz0 + kBZ, n1z) - 1;
     const double bmin[3] = {(ix0 - nex) * spacing, (iy0 - ney) * spacing, (iz0 - nez) * spacing};
     const double bmax[3] = {(ix1 - nex) * spacing, (iy1 - ney) * spacing, (iz1 - nez) * spacing};
 
@@ -582,94 +618,133 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
         c1[d] = min(c1[d], cf.nc[d] - 1);
     }
     const int ncx = c1[0] - c0[0] + 1, ncy = c1[1] - c0[1] + 1, ncz = c1[2] - c0[2] + 1;
-    const int ncell = (ncx > 0 && ncy > 0 && ncz > 0) ? ncx * ncy * ncz : 0;
+    // Cells along x follow each other in the sorted atoms, so the cells of one
+    // (y, z) are one run of slots: nrun runs, looked at 64 at a time, one per lane.
+    const int nrun = (ncx > 0 && ncy > 0 && ncz > 0) ? ncy * ncz : 0;
+    const int wave = tid >> 6, wlane = tid & 63;
     // Staging pass: the brick's candidates (atoms within 8.03 A of the box),
     // in cell order and slot order within a cell, are numbered from 0 as
     // found, and the donor H among them likewise.  Candidates numbered
     // cpage .. cpage + kCandCap - 1 go to cand[] and donor H numbered hpage ..
-    // hpage + kHCap - 1 to hcand[] (a negative page stores none); ncand_s
-    // and nh_s end as the totals.  A brick with more than fits is processed
+    // hpage + kHCap - 1 to the H lists (a negative page stores none); ncand
+    // and nh end as the totals.  A brick with more than fits is processed
     // page by page, each page staged by another pass, in the same order, so
-    // its sums are those one unbounded list would give.
+    // its sums are those one unbounded list would give.  Every wave scans
+    // the run lengths for itself, so the only exchange is each wave's count of
+    // what it found, one barrier per 256 atoms (two buffers: a wave may be one
+    // round ahead).
     const float r2cut = kNearRadius * kNearRadius;
+    const float lo_f[3] = {(float)bmin[0], (float)bmin[1], (float)bmin[2]};
+    const float hi_f[3] = {(float)bmax[0], (float)bmax[1], (float)bmax[2]};
+    int ncand = 0, nh = 0;
     auto stage = [&](int cpage, int hpage) {
-        if (tid == 0) { ncand_s = 0; nh_s = 0; }
-        __syncthreads();
-        for (int cbase = 0; cbase < ncell; cbase += kNearThreads) {
-            const int ci = cbase + tid;
-            int cstart = 0, ccount = 0;
-            if (ci < ncell) {
-                const int gx = c0[0] + ci % ncx, gy = c0[1] + (ci / ncx) % ncy, gz = c0[2] + ci / (ncx * ncy);
-                const int g = cf.cell_base + gx + cf.nc[0] * (gy + cf.nc[1] * gz);
-                cstart = p.cell_start[g];
-                ccount = p.cell_start[g + 1] - cstart;
+        int found = 0, found_h = 0, buf = 0;
+        for (int rbase = 0; rbase < nrun; rbase += 64) {
+            int rstart = 0, rcount = 0;
+            if (rbase + wlane < nrun) {
+                const int gy = c0[1] + (rbase + wlane) % ncy, gz = c0[2] + (rbase + wlane) / ncy;
+                const int g = cf.cell_base + c0[0] + cf.nc[0] * (gy + cf.nc[1] * gz);
+                rstart = p.cell_start[g];
+                rcount = p.cell_start[g + ncx] - rstart;
             }
-            cell_off[tid] = ccount;
-            __syncthreads();
-            for (int off = 1; off < kNearThreads; off <<= 1) {
-                int v = tid >= off ? cell_off[tid - off] : 0;
-                __syncthreads();
-                cell_off[tid] += v;
-                __syncthreads();
+            int rend = rcount;   // inclusive prefix
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const int v = __shfl_up(rend, o);
+                rend += wlane >= o ? v : 0;
             }
-            const int total = cell_off[kNearThreads - 1];
-            const int my_end = cell_off[tid];
-            __syncthreads();
-            cell_off[tid + 1] = my_end;
-            if (tid == 0) cell_off[0] = 0;
-            cstart_s[tid] = cstart;
-            __syncthreads();
-            for (int j0 = 0; j0 < total; j0 += kNearThreads) {
-                const int j = j0 + tid;
-                bool ok = false, is_h = false;
-                int slot = -1;
-                if (j < total) {
-                    int lo = 0, hi = kNearThreads;  // last cell with cell_off[c] <= j
-                    while (hi - lo > 1) {
-                        int mid = (lo + hi) >> 1;
-                        if (cell_off[mid] <= j) lo = mid; else hi = mid;
-                    }
-                    slot = cstart_s[lo] + (j - cell_off[lo]);
-                    const NearAtom &a = p.atoms[slot];
-                    float dd = 0.f;
-                    const double av[3] = {a.x, a.y, a.z};
-                    for (int d = 0; d < 3; d++) {
-                        double t = av[d] < bmin[d] ? bmin[d] - av[d] : (av[d] > bmax[d] ? av[d] - bmax[d] : 0.0);
-                        dd += (float)(t * t);
-                    }
-                    ok = dd <= r2cut;
-                    const int hb = (a.meta >> 8) & 0xff;
-                    is_h = ok && (hb == AG_HB_DS || hb == AG_HB_D1);
+            const int total = __shfl(rend, 63);
+            const int rslot = rstart - (rend - rcount);   // slot of the run's atom j is rslot + j
+            for (int j0 = 0; j0 < total; j0 += kStage * kNearThreads, buf ^= 1) {
+                bool ok[kStage], is_h[kStage];
+                int slot[kStage];
+#pragma unroll
+                for (int u = 0; u < kStage; u++) {
+                    const int j = j0 + u * kNearThreads + tid;
+                    int lo = 0;   // runs that end at or before j
+#pragma unroll
+                    for (int o = 32; o > 0; o >>= 1) lo += __shfl(rend, lo + o - 1) <= j ? o : 0;
+                    slot[u] = __shfl(rslot, lo) + j;
+                    ok[u] = j < total;
                 }
-                int tot;
-                const int pos = block_compact(ok, wave_tot, tot);
-                const int base = ncand_s;
-                const int cj = base + pos - cpage;
-                if (cpage >= 0 && ok && cj >= 0 && cj < kCandCap) cand[cj] = slot * (int)sizeof(NearAtom);
-                int htot;
-                const int hpos_i = block_compact(is_h, wave_tot, htot);
-                const int hbase = nh_s;
-                const int hj = hbase + hpos_i - hpage;
-                if (hpage >= 0 && is_h && hj >= 0 && hj < kHCap) hcand[hj] = slot;
+#pragma unroll
+                for (int u = 0; u < kStage; u++) {
+                    // an index past the last atom reads the first atom
+                    const NearAtom &a = p.atoms[ok[u] ? slot[u] : 0];
+                    // FP32: off by 1e-5 A at most, and an atom more than 8.02 A
+                    // away adds nothing
+                    const float av[3] = {(float)a.x, (float)a.y, (float)a.z};
+                    float dd = 0.f;
+                    for (int d = 0; d < 3; d++) {
+                        const float t = fmaxf(fmaxf(lo_f[d] - av[d], av[d] - hi_f[d]), 0.f);
+                        dd = __builtin_fmaf(t, t, dd);
+                    }
+                    ok[u] = ok[u] & (dd <= r2cut);
+                    const int hb = (a.meta >> 8) & 0xff;
+                    is_h[u] = ok[u] & ((hb == AG_HB_DS) | (hb == AG_HB_D1));
+                }
+                unsigned long long mo[kStage], mh[kStage];
+                const unsigned long long below = (1ull << wlane) - 1ull;
+#pragma unroll
+                for (int u = 0; u < kStage; u++) {
+                    mo[u] = __ballot(ok[u]);
+                    mh[u] = __ballot(is_h[u]);
+                    if (wlane == 0) wave_tot[buf][u][wave] = make_int2(__popcll(mo[u]), __popcll(mh[u]));
+                }
                 __syncthreads();
-                if (tid == 0) { ncand_s = base + tot; nh_s = hbase + htot; }
-                __syncthreads();
+#pragma unroll
+                for (int u = 0; u < kStage; u++) {
+                    int cj = found + __popcll(mo[u] & below) - cpage, hj = found_h + __popcll(mh[u] & below) - hpage;
+#pragma unroll
+                    for (int w = 0; w < kNearThreads / 64; w++) {
+                        const int2 n = wave_tot[buf][u][w];
+                        found += n.x;
+                        found_h += n.y;
+                        cj += w < wave ? n.x : 0;
+                        hj += w < wave ? n.y : 0;
+                    }
+                    if (cpage >= 0 && ok[u] && cj >= 0 && cj < kCandCap) cand[cj] = slot[u] * (int)sizeof(NearAtom);
+                    if (hpage >= 0 && is_h[u] && hj >= 0 && hj < kHCap) {
+                        const NearAtom &a = p.atoms[slot[u]];
+                        hpos[hj][0] = a.x; hpos[hj][1] = a.y; hpos[hj][2] = a.z;
+                        hidx[hj] = a.index;
+                        hrvs[hj][0] = a.rv[0]; hrvs[hj][1] = a.rv[1]; hrvs[hj][2] = a.rv[2];
+                    }
+                }
             }
         }
+        ncand = uni(found);
+        nh = uni(found_h);
     };
     stage(0, 0);
+#pragma unroll
+    for (int u = 0; u < kRsPer; u++)
+        if (tid + u * kNearThreads < kNearRepsLen) rs_s[tid + u * kNearThreads] = rs[u];
+    __syncthreads();
     if constexpr (!PAGED) {
-        if (ncand_s > kCandCap || nh_s > kHCap) {   // uniform per workgroup
+        if (ncand > kCandCap || nh > kHCap) {   // uniform per workgroup
             if (tid == 0) atomicOr(p.status, 1);
             return;
         }
     }
 
-    const int ncand = ncand_s, nh = nh_s;
-
-    float acc[kMapSlots];
+    // Table sums.  A table row is read by the Q lanes of a group together, 16
+    // bytes each: for each of the group's Q points in turn, lane c takes chunk c
+    // (four slots) of that point's row, and adds it to its own sums.  So accT[j]
+    // holds chunk c of point j; after the loop the group's lanes trade them.  The
+    // vector cache serves one 128-byte line per cycle, so a load whose 64 lanes
+    // read 64 rows took about 45 cycles and four of them 180 per candidate; now
+    // each touches 64 / Q rows (2.7e8 line reads instead of 7.4e8 in 13 maps of
+    // 127^3 points, 1,085 -> 712 us).  The H-bond slots of an atom whose class
+    // mixes there are read by the point's own lane (acc_hb).
+    constexpr int ROW = near_row(NPLAIN), Q = ROW / 4;
+    float accT[Q][4], acc_hb[kHbSlots];
 #pragma unroll
-    for (int m = 0; m < kMapSlots; m++) acc[m] = 0.f;
+    for (int j = 0; j < Q; j++)
+#pragma unroll
+        for (int s = 0; s < 4; s++) accT[j][s] = 0.f;
+#pragma unroll
+    for (int k = 0; k < kHbSlots; k++) acc_hb[k] = 0.f;
     // min/max of the H-bond pairs of each H-bonding slot (main.cpp:3300-3374)
     float hmin[kHbSlots], hmax[kHbSlots];
 #pragma unroll
@@ -687,42 +762,49 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
     double best_d2 = 999999.0 * 999999.0;
     int best_idx = 0x7fffffff;
     float hrv[3] = {0.f, 0.f, 0.f};   // bond vector of the closest H so far
+    const auto closer = [&](double d2, int index) {
+        if (d2 < best_d2 * (1.0 - 0x1p-49)) return true;
+        if (d2 > best_d2 * (1.0 + 0x1p-49)) return false;
+        const double r = sqrt(d2), rb = sqrt(best_d2);
+        return r < rb || (r == rb && index < best_idx);
+    };
     for (int h0 = 0; h0 < nh; h0 += kHCap) {   // pages of donor H
         if constexpr (PAGED) {
             if (h0 > 0) {
                 __syncthreads();
                 stage(-1, h0);
+                __syncthreads();
             }
         }
         const int hn = min(nh - h0, kHCap);
-        for (int h = tid; h < hn; h += kNearThreads) {
-            const NearAtom &a = p.atoms[hcand[h]];
-            hpos[h][0] = a.x; hpos[h][1] = a.y; hpos[h][2] = a.z;
-            hidx[h] = a.index;
-            hrvs[h][0] = a.rv[0]; hrvs[h][1] = a.rv[1]; hrvs[h][2] = a.rv[2];
-        }
-        __syncthreads();
-        for (int h = 0; h < hn; h++) {
+        for (int h = first; h < hn; h += share) {
 #pragma clang fp contract(off)
             const double dx = hpos[h][0] - cx, dy = hpos[h][1] - cy, dz = hpos[h][2] - cz;
             const double d2 = dx * dx + dy * dy + dz * dz;   // as ref_dist forms it
-            const int ix_h = hidx[h];
-            bool take;
-            if (d2 < best_d2 * (1.0 - 0x1p-49)) {
-                take = true;
-            } else if (d2 > best_d2 * (1.0 + 0x1p-49)) {
-                take = false;
-            } else {
-                const double r = sqrt(d2), rb = sqrt(best_d2);
-                take = r < rb || (r == rb && ix_h < best_idx);
-            }
-            if (take) {
+            if (closer(d2, hidx[h])) {
                 best_d2 = d2;
-                best_idx = ix_h;
+                best_idx = hidx[h];
                 hrv[0] = hrvs[h][0]; hrv[1] = hrvs[h][1]; hrv[2] = hrvs[h][2];
             }
         }
         if constexpr (!PAGED) break;
+    }
+    if (shared && nh > 0) {   // the closest of the sharing waves' (the order is total, so any split gives the same)
+        static_assert(kHCap == kNearThreads, "the donor-H lists hold one entry per thread");
+        double *const hd2 = &hpos[0][0];
+        __syncthreads();
+        hd2[tid] = best_d2;
+        hidx[tid] = best_idx;
+        hrvs[tid][0] = hrv[0]; hrvs[tid][1] = hrv[1]; hrvs[tid][2] = hrv[2];
+        __syncthreads();
+        for (int w = 0; w < share; w++) {
+            const int o = (wave - first + w) * 64 + wlane;
+            if (closer(hd2[o], hidx[o])) {
+                best_d2 = hd2[o];
+                best_idx = hidx[o];
+                hrv[0] = hrvs[o][0]; hrv[1] = hrvs[o][1]; hrv[2] = hrvs[o][2];
+            }
+        }
     }
 
     // The point indices are formed again from the thread index where they
@@ -732,16 +814,17 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
     const auto point_index = [&](int &qx, int &qy, int &qz) {
         int t = tid;
         asm volatile("" : "+v"(t));   // opaque at each use: not hoisted out of the loop
-        brick_lane<CUBE>(t, qx, qy, qz);
-        qx += bx * kBX;
-        qy += by * kBY;
-        qz += bz * kBZ;
+        brick_lane<CUBE>(t, share, qx, qy, qz);
+        qx += ix0;
+        qy += iy0;
+        qz += iz0;
     };
     float e_near = 0.f, dv_acc = 0.f, dq_acc = 0.f;
     int ccount = 0;
     const bool want_cmap = GENERAL && p.cmap != nullptr;
     const float *tab = p.tab;
     const bool want_e = p.e_slot >= 0;
+    const float band = cf.near_band;
     // cos and sin of 1.24791 rad, the disordered-hydroxyl offset angle
     const float cdis = 0.31936680f, sdis = 0.94763168f;
 
@@ -751,7 +834,8 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
     // top of a candidate iteration, where every lane of the wave is active:
     // a register reloaded from a spill under a partial exec mask would hold
     // stale values in the inactive lanes.
-    const int wlane = tid & 63;
+    const unsigned lane_chunk = 16u * (tid & (Q - 1));
+    const bool last_chunk = (tid & (Q - 1)) == Q - 1;
     const int hcw = wlane < 7 ? (p.hcode[0][wlane] | p.hcode[1][wlane] << 8 | p.hcode[2][wlane] << 16 |
                                  p.hcode[3][wlane] << 24)
                               : 0;
@@ -760,9 +844,11 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
             if (cpage > 0) {
                 __syncthreads();
                 stage(cpage, -1);
+                __syncthreads();
             }
         }
-        const int cn = min(ncand - cpage, kCandCap);
+        const int cpn = min(ncand - cpage, kCandCap);
+        const int cn = (cpn - first + share - 1) / share;   // this wave's: first, first + share, ...
         // candidate records go straight into scalar registers through the
         // constant address space (the atom array is read-only here).  The
         // wave holds 64 candidate indices in one register and loads the
@@ -777,11 +863,12 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
             return reinterpret_cast<const AG_CONST NearAtom *>(cbase + off);
         };
         for (int j0 = 0; j0 < cn; j0 += 64) {
-            const int vcand = cand[min(j0 + wlane, cn - 1)];
+            const int vcand = cand[min(j0 + wlane, cn - 1) * share + first];
             const int jn = min(64, cn - j0);
             unsigned off = (unsigned)__builtin_amdgcn_readlane(vcand, 0);
             double nx = rec(off)->x, ny = rec(off)->y, nz = rec(off)->z;
             int nmeta = rec(off)->meta, nindex = rec(off)->index;
+            float nqe = rec(off)->qe, nvol = rec(off)->vol, nsolq = rec(off)->solq;
             for (int jj = 0; jj < jn; jj++) {
                 // this record's address, formed once: its fields load from it
                 // with immediate offsets in whichever branch needs them
@@ -790,23 +877,31 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
                 const AG_CONST NearAtom &a = *ap;
                 const double ax = nx, ay = ny, az = nz;
                 const int ameta = nmeta, aindex = nindex;
+                const float aqe = nqe, avol = nvol, asolq = nsolq;
                 const unsigned hw = (unsigned)__builtin_amdgcn_readlane(hcw, (ameta >> 8) & 63);
                 unsigned noff = (unsigned)__builtin_amdgcn_readlane(vcand, min(jj + 1, jn - 1));
                 // the next loads may issue only once this record has arrived:
                 // scalar loads complete out of order, so the wait for this
                 // record would otherwise also wait for the next one
-                asm volatile("" : "+s"(noff) : "s"(ameta), "s"(aindex), "s"(ax), "s"(ay), "s"(az));
+                asm volatile("" : "+s"(noff) : "s"(ameta), "s"(aindex), "s"(ax), "s"(ay), "s"(az), "s"(aqe), "s"(avol), "s"(asolq));
                 nx = rec(noff)->x;
                 ny = rec(noff)->y;
                 nz = rec(noff)->z;
                 nmeta = rec(noff)->meta;
                 nindex = rec(noff)->index;
+                nqe = rec(noff)->qe;
+                nvol = rec(noff)->vol;
+                nsolq = rec(noff)->solq;
                 off = noff;   // a still names this record
                 // geometry: FP64 difference as the reference forms it, FP32 after
                 const double dx64 = ax - cx, dy64 = ay - cy, dz64 = az - cz;
                 const float dxf = (float)dx64, dyf = (float)dy64, dzf = (float)dz64;
                 const float r2 = __builtin_fmaf(dxf, dxf, __builtin_fmaf(dyf, dyf, dzf * dzf));
-                if (r2 > 64.33f) continue;  // beyond 8.02 A: neither cutoff pass nor near e term
+                // beyond 8.02 A: neither cutoff pass nor near e term.  A lane out of
+                // range goes along where another is in range (the table reads are
+                // shared) and adds zeros.
+                const bool in = r2 <= 64.33f;
+                if (!__ballot(in)) continue;
                 // hardware rsq: 128 r is good to ~3e-4 bins here, inside the guard band;
                 // the same rsq is 1/r for the near e term and the unit vector
                 const float r2c = max_of(r2, 1.0e-12f);
@@ -815,7 +910,7 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
                 const float g = r * 128.f;
                 int bin = (int)g;
                 bool cut = r > 8.0f;
-                if (fabsf(g - rintf(g)) < kGuardBins) {
+                if (in & (fabsf(g - rintf(g)) < kGuardBins)) {
                     double rdx, rdy, rdz;
                     const double r64 = ref_dist(ax, ay, az, cx, cy, cz, rdx, rdy, rdz);
                     bin = (int)(r64 * 128.0);
@@ -840,33 +935,51 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
                     rB = sqrtf(D);   // correctly rounded, as the tree's sqrt of a float
                     bin_bh = (int)((double)rB * 128.0);
                 }
-                // The pair's vdW/H-bond table row for the pass's slots, loaded
-                // here so that the loads are in flight during the constriction,
-                // electrostatic and directional work below.  The type's rows
-                // start at a scalar base, the bin's row is a 32-bit byte offset
-                // from it; the bin is the one Loop 2 uses (the tree build's FP32
-                // distance in that mode).  Every lane here has r < 8.03 A, so
-                // the row index stays inside the table.
-                const int indx_n = min(bh ? bin_bh : bin, AG_NEINT - 1);
-                float E[kMapSlots];
+                // The pairs' vdW/H-bond table rows, loaded here so that the loads
+                // are in flight during the constriction, electrostatic and
+                // directional work below.  The type's rows start at a scalar base,
+                // a bin's row is a 32-bit byte offset from it; the bin is the one
+                // Loop 2 uses (the tree build's FP32 distance in that mode).  A
+                // pair past the cutoff reads the row of zeros.
+                const int meta = ameta;
+                const int type = meta & 0xff, hb = (meta >> 8) & 0xff, rexp = (meta >> 16) & 0xff;
+                const bool dis = GENERAL && ((meta >> 24) & 1);
+                const bool skip_atom = !p.has_affinity || (p.disorder_h && dis && type == p.hydrogen_type);   // uniform
+                const bool sel = in & !(bh ? !in8 : cut) & !skip_atom;
+                // H-bonding slots (main.cpp:3286-3374): the (probe, atom) case is a
+                // set of 0/1 coefficients chosen per atom class, uniform across
+                // the wave.  For a class that mixes in some slot, each lane reads
+                // its own point's H-bond slots, and the lanes that would take that
+                // chunk for the group read zeros.
+                constexpr unsigned kMixBits = (HC_HRAMP | HC_MINMAX) * 0x01010101u;
+                const unsigned codes = hw >> (dis ? 4 : 0);
+                const bool mixes = (codes & kMixBits) != 0;   // uniform
+                float4 E[Q], Eo;
                 {
-                    const char *trow =
-                        reinterpret_cast<const char *>(tab + (size_t)(ameta & 0xff) * AG_NEINT * kMapSlots);
-                    const unsigned roff = (unsigned)indx_n * (unsigned)(kMapSlots * sizeof(float));
-    #pragma unroll
-                    for (int q4 = 0; q4 < kMapSlots / 4; q4++) {
-                        if (q4 < NPLAIN / 4 || q4 == kMapSlots / 4 - 1) {
-                            const float4 v = *reinterpret_cast<const float4 *>(trow + roff + 16u * q4);
-                            E[4 * q4] = v.x; E[4 * q4 + 1] = v.y; E[4 * q4 + 2] = v.z; E[4 * q4 + 3] = v.w;
-                        } else {
-                            E[4 * q4] = E[4 * q4 + 1] = E[4 * q4 + 2] = E[4 * q4 + 3] = 0.f;
-                        }
+                    constexpr unsigned kTypeBytes = AG_NEINT * ROW * sizeof(float);
+                    const char *trow = reinterpret_cast<const char *>(tab) + (size_t)type * kTypeBytes;
+                    const unsigned zero = p.zero_off - (unsigned)type * kTypeBytes;
+                    const unsigned roff =
+                        sel ? (unsigned)min(bh ? bin_bh : bin, AG_NEINT - 1) * (unsigned)(ROW * sizeof(float)) : zero;
+                    unsigned at[4];
+                    at[0] = (unsigned)group_lane<Q, 0>((int)roff) + lane_chunk;
+                    at[1] = (unsigned)group_lane<Q, 1>((int)roff) + lane_chunk;
+                    if constexpr (Q == 4) {
+                        at[2] = (unsigned)group_lane<Q, 2>((int)roff) + lane_chunk;
+                        at[3] = (unsigned)group_lane<Q, 3>((int)roff) + lane_chunk;
                     }
+                    if (mixes) {
+                        Eo = *reinterpret_cast<const float4 *>(trow + (roff + 16u * (Q - 1)));
+    #pragma unroll
+                        for (int j = 0; j < Q; j++) at[j] = last_chunk ? zero : at[j];
+                    }
+    #pragma unroll
+                    for (int j = 0; j < Q; j++) E[j] = *reinterpret_cast<const float4 *>(trow + at[j]);
                 }
                 // electrostatic factor and sol_fn of the bin, one LDS read
                 const float2 rsv = rs_s[min(bin, kNearRepsLen - 1)];
                 // constriction grid: atoms within the cutoff (main.cpp:2969-2973)
-                if (want_cmap && !bh) {
+                if (want_cmap && !bh && in) {
                     if (fabsf(r - (float)p.ccut) < 1.0e-5f) {
                         double rdx, rdy, rdz;
                         ccount += ref_dist(ax, ay, az, cx, cy, cz, rdx, rdy, rdz) <= p.ccut;
@@ -876,8 +989,8 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
                 }
                 // electrostatics of pairs the far kernel leaves out
                 if (want_e) {
-                    bool near_e = g < 1022.f;
-                    if (g >= 1022.f && g <= 1027.f) {
+                    bool near_e = g < (float)kFarBinMin;
+                    if (in & (fabsf(g - (float)kFarBinMin) <= band)) {
                         // the far kernel's coordinates of the atom and the point: run centre, offset in the run, y, z
                         int qx, qy, qz;
                         point_index(qx, qy, qz);
@@ -889,7 +1002,7 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
                     // 1/max(r, 0.5) with r clamped at APPROX_ZERO; adding 0 leaves
                     // the sum as it is (it is never -0)
                     const float inv_rmax = min_of(inv_r, 2.f);
-                    const float te = unif(a.qe) * inv_rmax * rsv.x;
+                    const float te = aqe * inv_rmax * rsv.x;
                     e_near += near_e ? te : 0.f;
                 }
                 // Loop 2 of the tree build takes the atoms its 8 A query returns,
@@ -900,15 +1013,10 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
                     bin = bin_bh;
                     inv_r = __builtin_amdgcn_rcpf(fmaxf(rB, 1.0e-6f));
                 }
-                if (cut || !p.has_affinity) continue;
-                const int meta = ameta;
-                const int type = meta & 0xff, hb = (meta >> 8) & 0xff, rexp = (meta >> 16) & 0xff;
-                const bool dis = GENERAL && ((meta >> 24) & 1);
-                if (p.disorder_h && dis && type == p.hydrogen_type) continue;
                 float racc = 1.f, rdon = 1.f, Hramp = 1.f;
                 // directional classes only (D1, A1, A2): the unit vector to the point
                 constexpr unsigned kDirClasses = (1u << AG_HB_D1) | (1u << AG_HB_A1) | (1u << AG_HB_A2);
-                if ((kDirClasses >> hb) & 1u) {
+                if (((kDirClasses >> hb) & 1u) && sel) {
                     const float dn0 = dxf * inv_r, dn1 = dyf * inv_r, dn2 = dzf * inv_r;
                     const float rv0 = unif(a.rv[0]), rv1 = unif(a.rv[1]), rv2 = unif(a.rv[2]);
                     const int aidx = aindex;
@@ -982,54 +1090,45 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
                         }
                     }
                 }  // directional classes
-                const float S = bh ? rs_s[min(bin, AG_NEINT)].y : rsv.y;   // sol_fn[min(bin, 1024)]
+                const float S = !sel ? 0.f : bh ? rs_s[min(bin, AG_NEINT)].y : rsv.y;   // sol_fn[min(bin, 1024)]
                 // desolvation (main.cpp:3375-3390): slot m gains
                 // (sp[m] vol + volp[m] solq) S per pair, i.e. sp[m] sum(vol S) +
                 // volp[m] sum(solq S) over the point's pairs: two sums per point
                 // instead of a term per slot, combined after the loop
-                dv_acc = __builtin_fmaf(unif(a.vol), S, dv_acc);
-                dq_acc = __builtin_fmaf(unif(a.solq), S, dq_acc);
-                // plain slots: the table value
+                dv_acc = __builtin_fmaf(avol, S, dv_acc);
+                dq_acc = __builtin_fmaf(asolq, S, dq_acc);
     #pragma unroll
-                for (int m = 0; m < NPLAIN; m++) acc[m] += E[m];
-                // H-bonding slots (main.cpp:3286-3374): the (probe, atom) case is a
-                // set of 0/1 coefficients chosen per atom class, uniform across
-                // the wave.  The plain table add is fma(c, E, acc) with c = 1 or
-                // 0 (bit for bit acc + E, or acc); the directional mix runs in
-                // scalar branches, one for the classes that have one and one per
-                // slot: acceptor atoms mix into the donor probe's slot alone, so
-                // three of four updates are skipped there.  A disordered partner
-                // uses the hydrogen-type row at r - 1.10 A (main.cpp:3313-3349),
-                // FP64 like the reference.
-                const int dsh = dis ? 4 : 0;
-    #pragma unroll
-                for (int k = 0; k < kHbSlots; k++) {
-                    const int code = (hw >> (8 * k + dsh)) & 15;
-                    const float kP = __int_as_float((code & HC_PLAIN) ? 0x3f800000 : 0);
-                    acc[kPlainSlots + k] = __builtin_fmaf(kP, E[kPlainSlots + k], acc[kPlainSlots + k]);
+                for (int j = 0; j < Q; j++) {
+                    accT[j][0] += E[j].x;
+                    accT[j][1] += E[j].y;
+                    accT[j][2] += E[j].z;
+                    accT[j][3] += E[j].w;
                 }
-                constexpr unsigned kMixBits = (HC_HRAMP | HC_MINMAX) * 0x01010101u;
-                if ((hw >> dsh) & kMixBits) {
+                // The mix runs in scalar branches, one per slot.  A disordered
+                // partner uses the hydrogen-type row at r - 1.10 A
+                // (main.cpp:3313-3349), FP64 like the reference.
+                if (mixes && sel) {
+                    const float e4[kHbSlots] = {Eo.x, Eo.y, Eo.z, Eo.w};
                     float Eh[kHbSlots] = {0.f, 0.f, 0.f, 0.f};
                     if (dis && p.hydrogen_type >= 0) {
                         double rdx, rdy, rdz;
                         const double r64 = bh ? (double)rB : ref_dist(ax, ay, az, cx, cy, cz, rdx, rdy, rdz);
                         const int hb_bin = min(max(0, (int)((r64 - 1.10) * 128.0)), AG_NEINT - 1);
                         const float4 v = reinterpret_cast<const float4 *>(
-                            tab + ((size_t)p.hydrogen_type * AG_NEINT + hb_bin) * kMapSlots)[kPlainSlots / 4];
+                            tab + ((size_t)p.hydrogen_type * AG_NEINT + hb_bin) * ROW)[Q - 1];
                         Eh[0] = v.x; Eh[1] = v.y; Eh[2] = v.z; Eh[3] = v.w;
                     }
     #pragma unroll
                     for (int k = 0; k < kHbSlots; k++) {
-                        const int m = kPlainSlots + k;
-                        const int code = (hw >> (8 * k + dsh)) & 15;
-                        if (!(code & (HC_HRAMP | HC_MINMAX))) continue;   // scalar
-                        const float e = E[m];
+                        const int code = (codes >> (8 * k)) & 15;   // scalar
+                        const float e = e4[k];
+                        if (code & HC_PLAIN) acc_hb[k] += e;
+                        if (!(code & (HC_HRAMP | HC_MINMAX))) continue;
                         const float f = (code & HC_RACC) ? racc : rdon;
                         const float rsph = __builtin_amdgcn_fmed3f(e * 0.01f, 0.f, 1.f);
                         const float mix = __builtin_fmaf(1.f - f, rsph, f);
                         if (code & HC_HRAMP)
-                            acc[m] = __builtin_fmaf((dis ? Eh[k] : e) * Hramp, mix, acc[m]);
+                            acc_hb[k] = __builtin_fmaf((dis ? Eh[k] : e) * Hramp, mix, acc_hb[k]);
                         if (code & HC_MINMAX) {
                             const float v = e * mix;
                             hmin[k] = min_of(hmin[k], v);
@@ -1042,27 +1141,90 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
         if constexpr (!PAGED) break;
     }
 
+    // each point's sums back to its lane, through LDS (the lists are done with)
+    float acc[kMapSlots];
+    {
+        __syncthreads();
+        constexpr int PITCH = ROW + 1, WAVE = 64 * PITCH;
+        float *const tr = scratch_f + wave * WAVE;
+        const int c = tid & (Q - 1), g0 = wlane - c;
+#pragma unroll
+        for (int j = 0; j < Q; j++)
+#pragma unroll
+            for (int s = 0; s < 4; s++) tr[(g0 + j) * PITCH + 4 * c + s] = accT[j][s];
+        wave_sync();
+#pragma unroll
+        for (int k = 0; k < kHbSlots; k++) tr[wlane * PITCH + ROW - 4 + k] += acc_hb[k];
+        if (shared) __syncthreads();
+        else wave_sync();
+#pragma unroll
+        for (int m = 0; m < kMapSlots; m++) {
+            if (m >= NPLAIN && m < kPlainSlots) continue;
+            const int at = wlane * PITCH + (m < kPlainSlots ? m : ROW - 4 + (m - kPlainSlots));
+            acc[m] = 0.f;
+            if (!shared) {
+                acc[m] = tr[at];
+            } else if ((m & (share - 1)) == first) {   // the maps this wave stores
+                for (int w = 0; w < share; w++) acc[m] += scratch_f[(wave - first + w) * WAVE + at];
+            }
+        }
+    }
+    if (shared) {   // the other sums of the sharing waves
+        constexpr int VALUES = 5 + 2 * kHbSlots;
+        static_assert(sizeof(NearLists) >= sizeof(float) * kNearThreads * VALUES, "room for the shared sums");
+        __syncthreads();
+        float *const mine = scratch_f + wave * (64 * VALUES) + wlane;
+        mine[0] = e_near;
+        mine[64] = dv_acc;
+        mine[128] = dq_acc;
+        mine[192] = __int_as_float(ccount);
+        mine[256] = __int_as_float(collide);
+#pragma unroll
+        for (int k = 0; k < kHbSlots; k++) {
+            mine[320 + 64 * k] = hmin[k];
+            mine[320 + 64 * (kHbSlots + k)] = hmax[k];
+        }
+        __syncthreads();
+        e_near = dv_acc = dq_acc = 0.f;
+        ccount = 0;
+        for (int w = 0; w < share; w++) {
+            const float *const v = scratch_f + (wave - first + w) * (64 * VALUES) + wlane;
+            e_near += v[0];
+            dv_acc += v[64];
+            dq_acc += v[128];
+            ccount += __float_as_int(v[192]);
+            collide |= __float_as_int(v[256]) != 0;
+#pragma unroll
+            for (int k = 0; k < kHbSlots; k++) {
+                hmin[k] = min_of(hmin[k], v[320 + 64 * k]);
+                hmax[k] = max_of(hmax[k], v[320 + 64 * (kHbSlots + k)]);
+            }
+        }
+    }
+
     int qx, qy, qz;
     point_index(qx, qy, qz);
     if (qx < n1x && qy < n1y && qz < n1z) {
         // output pointers are formed here, after the candidate loop, so they
-        // hold no registers during it
+        // hold no registers during it; each wave of a shared cube stores
+        // its part of the maps
         int *const cmap = p.cmap ? p.cmap + cf.pt_off : nullptr;
         float *const maps = p.maps + cf.map_off;
         const long long P = cf.P;
         const long long pt = (long long)qx + (long long)n1x * ((long long)qy + (long long)n1y * qz);
+        const auto stores = [&](int k) { return (k & (share - 1)) == first; };
 #pragma unroll
         for (int m = 0; m < kMapSlots; m++) {
-            if ((m >= NPLAIN && m < kPlainSlots) || p.out_slot[m] < 0) continue;
+            if ((m >= NPLAIN && m < kPlainSlots) || p.out_slot[m] < 0 || !stores(m)) continue;
             float v = acc[m] + __builtin_fmaf(p.sp[m], dv_acc, p.volp[m] * dq_acc);
             if (m >= kPlainSlots && hmin[m - kPlainSlots] < 999999.f)
                 v += hmin[m - kPlainSlots] + fmaxf(hmax[m - kPlainSlots], 0.f);
             maps[(long long)p.out_slot[m] * P + pt] = v;
         }
-        if (want_e) maps[(long long)p.e_slot * P + pt] = e_near;
-        if (cmap) cmap[pt] = ccount;
-        if (p.collide) p.collide[cf.pt_off + pt] = collide ? 1 : 0;
-        if (p.d_slot >= 0) maps[(long long)p.d_slot * P + pt] = p.solpar_q * dv_acc;   // solpar_q sum(vol S)
+        if (want_e && stores(0)) maps[(long long)p.e_slot * P + pt] = e_near;
+        if (cmap && stores(1)) cmap[pt] = ccount;
+        if (p.collide && stores(2)) p.collide[cf.pt_off + pt] = collide ? 1 : 0;
+        if (p.d_slot >= 0 && stores(3)) maps[(long long)p.d_slot * P + pt] = p.solpar_q * dv_acc;   // solpar_q sum(vol S)
     }
 }
 
@@ -1273,12 +1435,6 @@ __device__ __forceinline__ void far_pair(const PlainF4 &at, float py, float pz, 
 // A wave-uniform float moved to a scalar register.
 __device__ __forceinline__ float sreg(float v) {
     return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
-}
-
-// Orders a wave's own LDS accesses: its lanes see what the others wrote before.
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
 }
 
 // Chebyshev nodes of [-1, 1]: cos((2i + 1) pi / 2n), in increasing order.
@@ -1916,6 +2072,36 @@ static void launch_far(int blocks, const FarParams &fp, bool clamp, hipStream_t 
     HIP_CHECK(hipGetLastError());
 }
 
+// Waves of the near kernel that share a cube's atoms, from the number of 8x8x4
+// bricks of the grid.  The kernel is bound by its vector operations, so what
+// counts is that every SIMD has waves until the end: 256 CUs hold 1,280
+// workgroups at once.  Sharing by s cuts the list into s parts and makes s
+// times as many workgroups, whose staging and final sums are the cost.
+// Measured (us) at s = 1, 2, 4: 396 bricks (41^3 points) 147, 80, 62;
+// 1,024 (61^3) 201, 180, 170; 1,980 (47 x 83 x 119) 239, 215, 226; 2,541 (81^3)
+// 263, 231, 233 and twelve of these in a batch 5,137, 5,212, 5,397 in all; 8,448
+// (127^3) 810, 807, 935; 70,785 (257^3) 3,398, 3,817, 4,768.
+static int near_share(long long bricks) {
+    return bricks <= 1024 ? 4 : bricks <= 4096 ? 2 : 1;
+}
+
+// How far (bins) a pair's distance in the near kernel may lie from the far
+// kernel's bin limit and the two still disagree on which of them has it.  The
+// far kernel's coordinates are FP32 bins (2^-25 of the largest, an atom's and a
+// point's, three axes), its squared distance sums four products of up to
+// (limit + kFarMid s128)^2 with an error of 2^-24 each, the near kernel's
+// distance is good to 3e-4 bins; doubled.  At 0.375 A spacing and 96 A of grid
+// 0.01: the shell in which the near kernel repeats the far kernel's arithmetic
+// held some lane of 3 waves in 10 when it was 5 bins wide for every grid.
+static float far_band(const ag_grid &g) {
+    double edge = 0;
+    for (int d = 0; d < 3; d++) edge = std::max(edge, (double)std::max(g.ne[d], g.n1[d] - 1 - g.ne[d]));
+    const double s128 = g.spacing * 128.0, reach = kFarBinMin + kFarMid * s128;
+    const double coord = 6 * 0x1p-25 * (edge * s128 + 2 * kFarBinMin);
+    const double square = 4 * 0x1p-24 * 2 * reach * reach / (2.0 * kFarBinMin);
+    return (float)(2 * (coord + square + 3e-4));
+}
+
 // Per-conformation geometry, work prefixes and cell arrays for the plan's
 // cell size.
 static void plan_geometry(ag_plan &p, const ag_grid *grids, const int *natoms, const FarShape *far) {
@@ -1940,9 +2126,15 @@ static void plan_geometry(ag_plan &p, const ag_grid *grids, const int *natoms, c
         }
         cf.spacing = g.spacing;
         cf.s128 = (float)(g.spacing * 128.0);
-        cf.nb[0] = (g.n1[0] + kBX - 1) / kBX;
-        cf.nb[1] = (g.n1[1] + kBY - 1) / kBY;
-        cf.nb[2] = (g.n1[2] + kBZ - 1) / kBZ;
+        cf.near_band = far_band(g);
+        const int brick_edge[3] = {kBX, kBY, kBZ};
+        long long bricks = 1;
+        for (int d = 0; d < 3; d++) bricks *= (g.n1[d] + brick_edge[d] - 1) / brick_edge[d];
+        cf.near_share = near_share(bricks);
+        for (int d = 0; d < 3; d++) {
+            const int e = brick_edge[d] / (cf.near_share > (d == 0 ? 2 : 1) && d < 2 ? 2 : 1);
+            cf.nb[d] = (g.n1[d] + e - 1) / e;
+        }
         cf.cell_base = cell_base;
         cf.atom_base = atom_base;
         cf.n_atoms = natoms[c];
@@ -2156,8 +2348,6 @@ static ag_plan *plan_build(ag_ctx *c, int n, const ag_receptor *recs, const ag_g
     // the plain table add for every atom class (13 Vina maps: one pass).
     const int n_plain = (int)plain_maps.size(), n_hb = (int)hb_maps.size();
     p.groups = std::max({1, (n_hb + kHbSlots - 1) / kHbSlots, (n_plain + n_hb + kMapSlots - 1) / kMapSlots});
-    const size_t gstride = (size_t)(T > 0 ? T : 1) * AG_NEINT * kMapSlots;
-    std::vector<float> gtab(gstride * p.groups, 0.f);
     std::vector<std::array<int, kMapSlots>> slot_map(p.groups);
     std::vector<std::array<bool, kHbSlots>> hb_plain(p.groups);
     int nplain_max = 0;
@@ -2186,6 +2376,11 @@ static ag_plan *plan_build(ag_ctx *c, int n, const ag_receptor *recs, const ag_g
                 }
         if (!placed) ag::fail(AG_ERR_UNSUPPORTED, "near-kernel slot assignment left a map without a slot");
     }
+    p.nplain = nplain_max <= 4 ? 4 : (nplain_max <= 8 ? 8 : 12);
+    // rows of near_row slots per bin, and one row of zeros after the last group
+    const int row = near_row(p.nplain);
+    const size_t gstride = (size_t)(T > 0 ? T : 1) * AG_NEINT * row;
+    std::vector<float> gtab(gstride * p.groups + row, 0.f);
     for (int g = 0; g < p.groups; g++) {
         for (int t = 0; t < T; t++)
             for (int j = 0; j < kMapSlots; j++) {
@@ -2194,11 +2389,11 @@ static ag_plan *plan_build(ag_ctx *c, int n, const ag_receptor *recs, const ag_g
                 // zeros, so the kernel adds every slot's table value
                 if (m < 0 || !(map_role(ms, m) & ROLE_AFF)) continue;
                 const float *srcrow = tab->e_vdw_hb + ((size_t)t * M + m) * AG_NEINT;
-                float *dst = gtab.data() + g * gstride + (size_t)t * AG_NEINT * kMapSlots + j;
-                for (int k = 0; k < AG_NEINT; k++) dst[(size_t)k * kMapSlots] = srcrow[k];
+                const int at = j < kPlainSlots ? j : row - 4 + (j - kPlainSlots);
+                float *dst = gtab.data() + g * gstride + (size_t)t * AG_NEINT * row + at;
+                for (int k = 0; k < AG_NEINT; k++) dst[(size_t)k * row] = srcrow[k];
             }
     }
-    p.nplain = nplain_max <= 4 ? 4 : (nplain_max <= 8 ? 8 : 12);
     float *d_tab = upload(st, p.tab, gtab.data(), gtab.size());
     p.queue_d.get(sizeof(int) * kMaxChunks);
 
@@ -2251,6 +2446,7 @@ static ag_plan *plan_build(ag_ctx *c, int n, const ag_receptor *recs, const ag_g
             }
         }
         q.tab = d_tab + g * gstride;
+        q.zero_off = (unsigned)(sizeof(float) * gstride * (p.groups - g));
         q.e_slot = (g == 0 && !vina) ? ms->elec_index : -1;
         q.d_slot = (g == 0 && !vina) ? ms->dsolv_index : -1;
         q.has_affinity = used || q.d_slot >= 0;
