@@ -67,6 +67,8 @@ constexpr int kFarWaves = 4;                      // waves of a far-kernel workg
 constexpr int kFarThreads = 64 * kFarWaves;
 constexpr int kFarAtomChunk = 64;                 // Kahan block (at least)
 constexpr int kFarNx = 5, kFarNy = 4;             // interpolation nodes of a patch along x, and along y and z
+constexpr double kFarQRef = 0.85;                 // charge of level 0 over the conformation's rms charge
+constexpr int kFarLevels = 12;                    // charge levels, each with its own distance
 constexpr int kFarSplitMax = 8;                   // workgroups that may share a patch's atoms
 constexpr int kFarBinMin = 1025;                  // far kernel takes bins >= this
 constexpr float kGuardBins = 1.0e-3f;             // FP64 recompute band around bin edges
@@ -117,7 +119,8 @@ struct ConfDev {
     int far_npy, far_npz;         // patches along y and z
     int far_split;                // workgroups sharing each patch's atoms
     int far_clamp;                // far kernel: a direct pair may pass the table's end
-    float far_r2;                 // squared distance (bins^2) from a patch's box past which atoms are interpolated
+    float far_r2[kFarLevels];     // squared distances (bins^2) from a patch's box past which atoms are interpolated
+    float far_qscale;             // an atom's level is that of |its far charge| times this (far_level)
     long long part_off;           // far_split > 1: offset of its [far_split][P] partial e maps
 };
 
@@ -1475,6 +1478,13 @@ __device__ __forceinline__ void far_pair(const PlainF4 &at, float py, float pz, 
     for (int k = 0; k < kFarK; k++) part[k] = __builtin_fmaf(at.w, rs[k] * tv[k], part[k]);
 }
 
+// Level of an atom's charge over the conformation's: 0 for a ratio of sqrt(1/2)
+// or more, one more for each factor of sqrt(1/2), the last for all that are
+// smaller.
+__device__ __forceinline__ int far_level(float ratio) {
+    return min(max(126 - (int)(__float_as_uint(ratio * ratio) >> 23), 0), kFarLevels - 1);
+}
+
 // A wave-uniform float moved to a scalar register.
 __device__ __forceinline__ float sreg(float v) {
     return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
@@ -1511,14 +1521,14 @@ __device__ __forceinline__ void far_wy(double t, double w[4]) {
 // and a quarter of the part each (every fourth group of 64 atoms), and add
 // up in a fixed order through LDS.
 //
-// Atoms near the patch's box (closer than sqrt(far_r2)) go pair by pair
+// Atoms near the patch's box (closer than their level's sqrt(far_r2)) go pair by pair
 // through the dielectric table, as the reference sums them (main.cpp:2940-2982):
 // the table sits in LDS at address 0, so a bin's byte offset is its LDS
 // address, with zeros below bin 1025 for the pairs the near kernel takes.
 //
 // The others vary smoothly over the box (the host picks the distance so
 // that a table step there is below 6.5e-5 of its value and the box subtends a
-// small angle, far_radius): their sum is formed at 5 x 4 x 4 Chebyshev nodes of
+// small angle, and smaller distances for smaller charges, far_radii): their sum is formed at 5 x 4 x 4 Chebyshev nodes of
 // the box with the same table, and interpolated to its points.  An atom then
 // costs 80 terms instead of 1,024.  Four atoms go at once, one for each 16
 // lanes; a lane takes the five x-nodes of one (y, z) node.
@@ -1585,7 +1595,6 @@ __global__ void __launch_bounds__(kFarThreads) __attribute__((amdgpu_waves_per_e
         const float my = 0.5f * (float)(cf.far_py - 1), mz = 0.5f * (float)(cf.far_pz - 1);
         const float hy = sreg(my * s128), hz = sreg(mz * s128);
         const float by = sreg(((float)(iy0 - cf.ne[1]) + my) * s128), bz = sreg(((float)(iz0 - cf.ne[2]) + mz) * s128);
-        const float r2 = sreg(cf.far_r2);
         const float d1 = sreg(hx * far_node5(3)), d2 = sreg(hx * far_node5(4));
         const float d1q = sreg(d1 * d1), d2q = sreg(d2 * d2);
         float s[kFarK], c[kFarK], part[kFarK];
@@ -1595,6 +1604,10 @@ __global__ void __launch_bounds__(kFarThreads) __attribute__((amdgpu_waves_per_e
 #pragma unroll
         for (int i = 0; i < kFarNx; i++) ns[i] = np[i] = 0.f;
         float4 *const strip = reinterpret_cast<float4 *>(X) + 64 * wave;
+        float *const level_r2 = X + 4 * 64 * kFarWaves + kFarLevels * wave;   // the wave's copy
+        if (lane < kFarLevels) level_r2[lane] = reinterpret_cast<const float *>(&p.confs[ci].far_r2)[lane];
+        wave_sync();
+        const float qscale = sreg(cf.far_qscale);
         const float4 *const vatoms = p.atoms + cf.atom_base;
         const AG_CONST PlainF4 *atoms = as_const(reinterpret_cast<const PlainF4 *>(vatoms));   // scalar loads
         const int n_atoms = cf.n_atoms;
@@ -1608,7 +1621,8 @@ __global__ void __launch_bounds__(kFarThreads) __attribute__((amdgpu_waves_per_e
             if (a0 + step + lane < n_atoms) A = vatoms[a0 + step + lane];
             const float ex = fmaxf(fabsf(at.x - bx) - hx, 0.f), ey = fmaxf(fabsf(at.y - by) - hy, 0.f),
                         ez = fmaxf(fabsf(at.z - bz) - hz, 0.f);
-            const bool beyond = __builtin_fmaf(ex, ex, __builtin_fmaf(ey, ey, ez * ez)) >= r2;
+            const bool beyond =
+                __builtin_fmaf(ex, ex, __builtin_fmaf(ey, ey, ez * ez)) >= level_r2[far_level(at.w * qscale)];
             const int nb = min(64, n_atoms - a0);
             const unsigned long long all = nb == 64 ? ~0ull : ((1ull << nb) - 1);
             const unsigned long long far_set = __ballot(beyond) & all;
@@ -2014,62 +2028,95 @@ static void launch_near(const ag_plan &p, int grid, const NearParams &np, hipStr
 // share a patch's atoms.  All of it depends on the conformation and the
 // tables alone, so its maps are the same in a batch as in a plan of its own.
 struct FarShape {
-    float radius2 = 0.f;
+    float radius2[kFarLevels] = {};
+    float qscale = 0.f;
     bool clamp = false;
     int py = 8, pz = 8, split = 1;
 };
 
-// Smallest distance (A) past which an atom's term varies over a patch of a
-// grid of the given spacing the way 5 x 4 x 4 nodes follow: (a) no table step
-// beyond it exceeds 6.5e-5 of the value there, (b) 5 Chebyshev nodes over any
-// x-run's length beyond it reproduce the table to 1e-5, and (c) it is at least
-// 48.75 spacings, 6.5 half-lengths of an x-run, for the 1/r: 75 where the
-// table has no steps at all (constant dielectric), whose sum has no table
-// error beside the interpolation's.  Bins from 8191 on hold one value, so past
-// 64 A only (c) is asked for.
+// Least distance (A) of a level whatever the table (far_radii): 48.75 spacings,
+// 6.5 half-lengths of an x-run, for the 1/r, 75 where the table has no steps
+// at all (constant dielectric), whose sum has no table error beside the
+// interpolation's.  A level allows sqrt(2) times the error of the one
+// before: with five x-nodes 2^-0.1 of the distance from the run's centre, with
+// the Mehler-Solmajer dielectric's steps (they fall by e in 3.2 A) 1.1 A.  The
+// near kernel has the pairs up to 8.01 A.
+static double far_floor_radius(bool flat, double spacing, int level) {
+    const double half = 0.5 * (kFarK - 1) * spacing;
+    const double g = std::pow(2.0, -level / 10.0);
+    if (flat) return std::max({8.25, 20.0 * g, ((75.0 * spacing / half + 1.0) * g - 1.0) * half});
+    const double base = std::min(21.0, std::max(18.5, 26.0 - 20.0 * spacing)) - 1.1 * level;
+    return std::max({8.25, base, ((48.75 * spacing / half + 1.0) * g - 1.0) * half});
+}
+
+// Distances (A) past which an atom's term varies over a patch of a grid of
+// the given spacing the way 5 x 4 x 4 nodes follow, for each level of its charge.
+// Level 0: (a) no table step beyond it exceeds 6.5e-5 of the value there, (b)
+// 5 Chebyshev nodes over any x-run's length beyond it reproduce the table to
+// 1e-5, and (c) it is at least far_floor_radius.  An atom of level l has at
+// most 2^(-l/2) of the reference charge, so its term may be off by 2^(l/2)
+// times as much, and (a) and (b) ask for that.  Bins from 8191 on hold one
+// value, so past 64 A only (c) is asked for.
 // With the Mehler-Solmajer dielectric the steps decide: they leave 2e-7 of
 // the e map (2-norm, 5,000-atom protein) at 20 A, 5e-7 at 18 A and 8e-7 at 16 A,
-// beside the 7e-7 that FP32 bins of the direct pairs leave.  The floor keeps
-// the whole error below the all-pairs sum's at every spacing: 7.2e-7 for
-// 7.4e-7 at 0.25 A, 1.0e-6 for 1.1e-6 at 0.3 A, 9.3e-7 for 1.0e-6 at 0.375 A.
-static double far_radius(const std::vector<float> &reps, double spacing) {
+// beside the 7e-7 that FP32 bins of the direct pairs leave.  The floor and the
+// reference charge keep the whole error below the all-pairs sum's at every
+// spacing: 6.5e-7 for 7.0e-7 at 0.25 A, 8.4e-7 for 9.7e-7 at 0.3 A, 9.4e-7 for
+// 1.02e-6 at 0.375 A (5,000 atoms; 12,000: 1.19e-6 for 1.22e-6), 7.5e-7 for 1.5e-6 at
+// 0.5 A.  One distance for every charge: 3 % less error, 830 us instead of 772
+// for 5,000 atoms on 127^3 points, 460 instead of 430 for 3,000 on 81^3 in a constant
+// dielectric.
+static void far_radii(const std::vector<float> &reps, double spacing, double radius[kFarLevels]) {
     const bool flat = std::all_of(reps.begin() + kFarBinMin, reps.end(), [&](float v) { return v == reps.back(); });
-    const double floor_r = flat ? std::max(20.0, 75.0 * spacing)
-                                : std::max(std::min(21.0, std::max(18.5, 26.0 - 20.0 * spacing)), 48.75 * spacing);
     const double run = (kFarK - 1) * spacing * 128.0;   // bins along an x-run
     const auto g = [&](double bin) {                     // the table as a function, between bin centres
         const double y = std::min(std::max(bin - 0.5, 0.0), (double)(AG_NDIEL - 1));
         const int k = std::min((int)y, AG_NDIEL - 2);
         return reps[k] + (y - k) * ((double)reps[k + 1] - reps[k]);
     };
-    int first = AG_NDIEL - 1;   // bins from here on are smooth
-    while (first > kFarBinMin && std::fabs((double)reps[first - 1] - reps[first]) <= 6.5e-5 * std::fabs((double)reps[first]))
-        first--;
-    double ok = (AG_NDIEL - 1) / 128.0 + 1.0 / 64.0;
-    for (double r = AG_NDIEL - 1; r >= std::max<double>(first, floor_r * 128.0 - 64.0); r -= 32.0) {
+    double W[17][kFarNx];
+    for (int q = 0; q <= 16; q++)
+        for (int i = 0; i < kFarNx; i++) {
+            W[q][i] = 1.0;
+            for (int j = 0; j < kFarNx; j++)
+                if (j != i)
+                    W[q][i] *= (-1.0 + q / 8.0 - (double)far_node5(j)) / ((double)far_node5(i) - (double)far_node5(j));
+        }
+    double floor_r[kFarLevels], ok[kFarLevels];
+    for (int l = 0; l < kFarLevels; l++) {
+        floor_r[l] = far_floor_radius(flat, spacing, l);
+        ok[l] = (AG_NDIEL - 1) / 128.0 + 1.0 / 64.0;
+    }
+    // outwards in: a level's distance is the last before its first fault
+    int first = 0, bin = AG_NDIEL - 1;   // levels below first have ended
+    for (double r = AG_NDIEL - 1; first < kFarLevels; r -= 32.0) {
+        double step = 0.0, off = 0.0;
+        for (; bin > kFarBinMin && bin > r; bin--)
+            step = std::max(step, std::fabs((double)reps[bin - 1] - reps[bin]) / std::fabs((double)reps[bin]));
         double f[kFarNx];
         for (int i = 0; i < kFarNx; i++) f[i] = g(r + 0.5 * run * (1.0 + far_node5(i)));
-        bool good = true;
-        for (int q = 0; q <= 16 && good; q++) {
-            const double t = -1.0 + q / 8.0;
+        for (int q = 0; q <= 16; q++) {
             double v = 0.0;
-            for (int i = 0; i < kFarNx; i++) {
-                double w = 1.0;
-                for (int j = 0; j < kFarNx; j++)
-                    if (j != i) w *= (t - (double)far_node5(j)) / ((double)far_node5(i) - (double)far_node5(j));
-                v += w * f[i];
-            }
-            const double want = g(r + 0.5 * run * (1.0 + t));
-            good = std::fabs(v - want) <= 1.0e-5 * std::fabs(want);
+            for (int i = 0; i < kFarNx; i++) v += W[q][i] * f[i];
+            const double want = g(r + run * (q / 16.0));
+            off = std::max(off, std::fabs(v - want) / std::fabs(want));
         }
-        if (!good) break;
-        ok = r / 128.0;
+        for (int l = first; l < kFarLevels; l++) {
+            const bool good = step <= 6.5e-5 * std::pow(2.0, 0.5 * l) && off <= 1.0e-5 * std::pow(2.0, 0.5 * l);
+            if (good && r >= floor_r[l] * 128.0 - 64.0) ok[l] = r / 128.0;
+            else if (l == first) first++;   // the levels end in order
+        }
     }
-    return std::max(floor_r, ok);
+    for (int l = 0; l < kFarLevels; l++) radius[l] = std::max(floor_r[l], ok[l]);
 }
 
-static FarShape far_shape(const ag_grid &g, int n_atoms, double radius, const double *coord) {
+static FarShape far_shape(const ag_grid &g, int n_atoms, const double radius[kFarLevels], const double *coord,
+                          const double *charge, double coeff) {
     FarShape f;
+    double q2 = 0.0;
+    for (int a = 0; a < n_atoms; a++) q2 += charge[a] * charge[a];
+    const double ref = kFarQRef * std::sqrt(q2 / std::max(1, n_atoms)) * std::fabs(coeff) * 128.0;
+    f.qscale = ref > 0.0 ? (float)(1.0 / ref) : 0.f;
     // patches of 6 to 10 rows along y and what 64 lanes leave along z: the
     // shape that needs the fewest, the squarest of equals
     int best = INT32_MAX, best_d = 0;
@@ -2083,8 +2130,8 @@ static FarShape far_shape(const ag_grid &g, int n_atoms, double radius, const do
             f.pz = pz;
         }
     }
-    const double r = radius * 128.0, s = g.spacing * 128.0;
-    f.radius2 = (float)(r * r);
+    const double r = radius[0] * 128.0, s = g.spacing * 128.0;
+    for (int l = 0; l < kFarLevels; l++) f.radius2[l] = (float)(radius[l] * 128.0 * (radius[l] * 128.0));
     // the largest bin of a direct pair: its atom lies within the radius of the patch's box
     const double diag = s * std::sqrt((double)((kFarK - 1) * (kFarK - 1) + (f.py - 1) * (f.py - 1) +
                                                (f.pz - 1) * (f.pz - 1)));
@@ -2193,7 +2240,8 @@ static void plan_geometry(ag_plan &p, const ag_grid *grids, const int *natoms, c
         cf.far_npz = (g.n1[2] + fs.pz - 1) / fs.pz;
         cf.far_split = fs.split;
         cf.far_clamp = fs.clamp;
-        cf.far_r2 = fs.radius2;
+        for (int l = 0; l < kFarLevels; l++) cf.far_r2[l] = fs.radius2[l];
+        cf.far_qscale = fs.qscale;
         cf.part_off = part;
         if (fs.split > 1) part += fs.split * cf.P;
         p.brick_prefix[c] = (int)brick;
@@ -2527,10 +2575,11 @@ static ag_plan *plan_build(ag_ctx *c, int n, const ag_receptor *recs, const ag_g
         k_far_atoms<<<(N + 255) / 256, 256, 0, st>>>(N, d_coord, d_charge, ms->coeff_estat, d_far);
         HIP_CHECK(hipGetLastError());
         p.far_atoms_ready = true;
-        double radius = 0.0, spacing = -1.0;
+        double radius[kFarLevels] = {}, spacing = -1.0;
         for (int i = 0, o = 0; i < n; o += natoms[i], i++) {
-            if (grids[i].spacing != spacing) radius = far_radius(reps, spacing = grids[i].spacing);
-            far_shapes.push_back(far_shape(grids[i], natoms[i], radius, coord + 3 * (size_t)o));
+            if (grids[i].spacing != spacing) far_radii(reps, spacing = grids[i].spacing, radius);
+            far_shapes.push_back(
+                far_shape(grids[i], natoms[i], radius, coord + 3 * (size_t)o, charge + o, ms->coeff_estat));
         }
         FarParams &fp = p.far;
         memset(&fp, 0, sizeof fp);

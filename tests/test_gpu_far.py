@@ -59,7 +59,7 @@ def state(base, n_atoms, n1, spacing, radius, seed, r_eps=None, constant=None, o
     return st
 
 
-def check(st, got, seed=0, points=3000):
+def check(st, got, seed=0, points=3000, floor_charge=0.0):
     """e at sampled points (the grid's corners among them) against FP64."""
     rng = np.random.default_rng(seed)
     nx, ny, nz = st.n1
@@ -74,7 +74,8 @@ def check(st, got, seed=0, points=3000):
         t = st.charge[a:a + 4096] * st.coeff_estat * tab[np.minimum((r * 128.0).astype(np.int64), 8191)] / \
             np.maximum(r, 0.5)
         e += t.sum(1)
-        mag += np.abs(t).sum(1)
+        unit = abs(st.coeff_estat) * tab[np.minimum((r * 128.0).astype(np.int64), 8191)] / np.maximum(r, 0.5)
+        mag += (unit * np.maximum(np.abs(st.charge[a:a + 4096]), floor_charge)).sum(1)
         top = np.maximum(top, np.abs(t).max(1))
     err = np.abs(got.reshape(-1)[pick].astype(np.float64) - e)
     lim = 3e-5 * mag + 5e-3 * top
@@ -135,3 +136,28 @@ def test_dielectric_tables(base, table):
     else:
         tab[30 * 128:] = 0.0
     run(state(base, 2500, (40, 40, 40), 0.375, 45.0, 7, r_eps=tab))
+
+
+@pytest.mark.parametrize("charges", ["four decades", "one large", "all zero", "half zero"])
+@pytest.mark.parametrize("spacing", [0.25, 0.5])
+def test_charge_levels(base, charges, spacing):
+    """An atom of a small charge is interpolated from nearer, to the absolute
+    error of one of the reference charge (0.85 rms): the bound's first part
+    takes every charge as the rms at least."""
+    print(f"[gpu] far charges {charges} {spacing}", flush=True)
+    st = state(base, 2500, (40, 33, 41), spacing, 36.0, 9)
+    rng = np.random.default_rng(10)
+    q = st.charge
+    if charges == "four decades":
+        q = rng.choice([-1.0, 1.0], len(q)) * 10.0 ** rng.uniform(-4, 0, len(q))
+    elif charges == "one large":
+        q = np.where(np.arange(len(q)) == 7, 20.0, 0.01 * q)
+    elif charges == "all zero":
+        q = np.zeros(len(q))
+    else:
+        q = np.where(np.arange(len(q)) % 2, q, 0.0)
+    st = dataclasses.replace(st, charge=q, _keep=[])
+    with ag.Context(0) as ctx:
+        got = ctx.maps_plain(st)
+        assert np.array_equal(ctx.maps_plain(dataclasses.replace(st, charge=-q, _keep=[]))[0], -got[0])
+    check(st, got[0], floor_charge=float(np.sqrt(np.mean(q ** 2))))
