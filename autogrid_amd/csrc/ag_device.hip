@@ -191,13 +191,20 @@ struct NearParams {
     int *status;
 };
 
+// An atom of the far kernel: coordinates in bins (exact) and charge times the
+// electrostatic coefficient.
+struct __align__(16) FarAtom {
+    double x, y, z;
+    float w, pad;
+};
+
 struct FarParams {
     const ConfDev *confs;
     const int *tile_prefix;       // [nconf + 1], items: patches x x-runs x parts
     int nconf, total_tiles;
     int item_base, item_end;      // tiles [item_base, item_end) of this launch
     int *queue;                   // null: one tile per workgroup; else a persistent work counter
-    const float4 *atoms;          // (xE, yE, zE, w = q * coeff_estat * 128)
+    const FarAtom *atoms;
     const float *tab;             // [AG_NDIEL] electrostatic factor
     float *maps;                  // e map slot: in = near part, out = total
     float *part;                  // partial e maps of the conformations with far_split > 1
@@ -230,9 +237,13 @@ __device__ __forceinline__ unsigned bin4_of(float rb2, float rs) {
     return __float_as_uint(__builtin_fmaf(rb2, rs, kBinMagic)) & 0x7FFFFCu;
 }
 
-// Far-kernel geometry of a run of kFarK points along x.  The run's points
-// sit at cx + dk, dk = (k - kFarMid) s128 (k = 0..kFarK-1, cx the run's
-// centre, s128 = 128 spacing), and with u = ax - cx
+// Far-kernel geometry.  An atom and a patch's points are taken from the centre
+// of the patch's box: the difference is formed in FP64 and rounded once, so a
+// pair's bin does not depend on how far from the origin it lies (coordinates
+// rounded to FP32 before the difference put 20 to 90 % more variance into the
+// bins: 7.2e-7 of the e map for 6.1e-7 with 5,000 atoms, 9.0e-7 for 6.5e-7 with
+// 20,000).  Along x the box is a run of kFarK points at dk = (k - kFarMid) s128
+// (k = 0..kFarK-1), and with u the atom's x
 //   rb2 = (u - dk)^2 + dyz2,  dyz2 = max(dy^2 + dz^2, floor)
 //       = fma(u s128, 15 - 2k, fma(s128^2, (j + 1/2)^2, fma(u, u, dyz2))),
 // j = |k - kFarMid| - 1/2: the points k and kFarK-1-k share the middle
@@ -251,7 +262,14 @@ __device__ __forceinline__ float far_floor(float s128) {
     const float d = kFarMid * s128;
     return fmaxf(1.0e-3f, d * d * 0x1p-19f);
 }
-__device__ __forceinline__ float far_cx(int ix0, int ne0, float s128) { return ((float)(ix0 - ne0) + kFarMid) * s128; }
+// Centre (bins) of the n points from point i0 on.
+__device__ __forceinline__ double far_centre(int i0, int n, int ne, double spacing) {
+    return ((double)(i0 - ne) + 0.5 * (double)(n - 1)) * (spacing * 128.0);
+}
+// Offset of a box's j-th of n points from its centre.
+__device__ __forceinline__ float far_offset(int j, int n, float s128) {
+    return ((float)j - 0.5f * (float)(n - 1)) * s128;
+}
 // (j + 1/2)^2 for point k, and the factor 15 - 2k of u s128
 __device__ __forceinline__ constexpr float far_c2(int k) {
     return (k >= kFarK / 2 ? (float)(k - kFarK / 2) + 0.5f : (float)(kFarK / 2 - 1 - k) + 0.5f) *
@@ -259,19 +277,34 @@ __device__ __forceinline__ constexpr float far_c2(int k) {
 }
 __device__ __forceinline__ constexpr float far_m(int k) { return (float)(kFarK - 1 - 2 * k); }
 
-// The far kernel's per-pair table offset for point k of the run centred at
-// cx, reproduced bit for bit by the near kernel when it decides which atoms
+// The far kernel's table offset for an atom (in bins) and point (ix, iy, iz),
+// reproduced bit for bit by the near kernel when it decides which atoms
 // the far kernel left out, and by the audit (same operations in the same
 // order; the build turns off FP contraction).
-__device__ __forceinline__ unsigned far_bin4(float ax, float ay, float az, float cx, int k, float s128, float py,
-                                             float pz, float floor2) {
-    const float dy = ay - py, dz = az - pz;
-    const float dyz2 = fmaxf(__builtin_fmaf(dy, dy, dz * dz), floor2);
-    const float u = ax - cx;
+struct FarPatch {
+    int ne[3], py, pz;
+    double spacing;
+    float s128;
+};
+// An atom's y or z distance from row i, in patches of p rows.
+__device__ __forceinline__ float far_row(double a, int i, int p, int ne, double spacing, float s128) {
+    const int l = i % p;
+    return (float)(a - far_centre(i - l, p, ne, spacing)) - far_offset(l, p, s128);
+}
+// The offset from the distances along y and z and the atom's x from the run's centre.
+__device__ __forceinline__ unsigned far_bin4(float u, float dy, float dz, int k, float s128) {
+    const float dyz2 = fmaxf(__builtin_fmaf(dy, dy, dz * dz), far_floor(s128));
     const float U = __builtin_fmaf(u, u, dyz2);
     const float W = __builtin_fmaf(s128 * s128, far_c2(k), U);
     const float rb2 = __builtin_fmaf(u * s128, far_m(k), W);
     return bin4_of(rb2, __builtin_amdgcn_rsqf(rb2));
+}
+__device__ __forceinline__ unsigned far_bin4(double ax, double ay, double az, const FarPatch &f, int ix, int iy,
+                                             int iz) {
+    const int k = ix % kFarK;
+    return far_bin4((float)(ax - far_centre(ix - k, kFarK, f.ne[0], f.spacing)),
+                    far_row(ay, iy, f.py, f.ne[1], f.spacing, f.s128),
+                    far_row(az, iz, f.pz, f.ne[2], f.spacing, f.s128), k, f.s128);
 }
 
 // ---------------------------------------------------------------------------
@@ -443,11 +476,11 @@ __global__ void k_gather(const int *nslots, const int *slot_atom, AtomSrc s, Nea
 }
 
 __global__ void k_far_atoms(int n, const double *coord, const double *charge, double coeff_estat,
-                            float4 *out) {
+                            FarAtom *out) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    out[i] = make_float4((float)(coord[3 * i] * 128.0), (float)(coord[3 * i + 1] * 128.0),
-                         (float)(coord[3 * i + 2] * 128.0), (float)(charge[i] * coeff_estat * 128.0));
+    out[i] = FarAtom{coord[3 * i] * 128.0, coord[3 * i + 1] * 128.0, coord[3 * i + 2] * 128.0,
+                     (float)(charge[i] * coeff_estat * 128.0), 0.f};
 }
 
 // ---------------------------------------------------------------------------
@@ -994,13 +1027,18 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
                 if (want_e) {
                     bool near_e = g < (float)kFarBinMin;
                     if (in & (fabsf(g - (float)kFarBinMin) <= band)) {
-                        // the far kernel's coordinates of the atom and the point: run centre, offset in the run, y, z
-                        int qx, qy, qz;
-                        point_index(qx, qy, qz);
-                        const int kxE = qx % kFarK;
-                        near_e = far_bin4((float)(ax * 128.0), (float)(ay * 128.0), (float)(az * 128.0), far_cx(qx - kxE, nex, s128), kxE, s128,
-                                          (float)(qy - ney) * s128, (float)(qz - nez) * s128, far_floor(s128)) <
-                                 4u * kFarBinMin;
+                        // (one axis after the other: few registers beside the sums)
+                        int q, qy, qz, unused;
+                        point_index(unused, qy, unused);
+                        float dyE = far_row(ay * 128.0, qy, cf.far_py, ney, spacing, s128);
+                        asm volatile("" : "+v"(dyE));
+                        point_index(unused, unused, qz);
+                        float dzE = far_row(az * 128.0, qz, cf.far_pz, nez, spacing, s128);
+                        asm volatile("" : "+v"(dzE));
+                        point_index(q, unused, unused);
+                        const int k = q % kFarK;
+                        const float uE = (float)(ax * 128.0 - far_centre(q - k, kFarK, nex, spacing));
+                        near_e = far_bin4(uE, dyE, dzE, k, s128) < 4u * kFarBinMin;
                     }
                     // 1/max(r, 0.5) with r clamped at APPROX_ZERO; adding 0 leaves
                     // the sum as it is (it is never -0)
@@ -1377,10 +1415,8 @@ __global__ void k_fmin_atoms(int n, const double *coord, float4 *out) {
 //              kGuardBins of an integer, so a mismatch outside that band
 //              would be an unguarded flip (expected: none).
 struct AuditParams {
-    int n1[3], ne[3];
-    double spacing;
-    float s128;
-    const float4 *far_atoms;     // the far kernel's atoms
+    int n1[3];
+    FarPatch far;
     const double *coord;         // [n][3]
     int n_atoms;
     long long P;
@@ -1394,15 +1430,11 @@ __global__ void __launch_bounds__(256) k_audit(AuditParams p) {
         const int ix = (int)(pt % p.n1[0]);
         const int iy = (int)((pt / p.n1[0]) % p.n1[1]);
         const int iz = (int)(pt / ((long long)p.n1[0] * p.n1[1]));
-        const double cx = (double)(ix - p.ne[0]) * p.spacing, cy = (double)(iy - p.ne[1]) * p.spacing,
-                     cz = (double)(iz - p.ne[2]) * p.spacing;
-        const int kx = ix % kFarK;
-        const float cxE = far_cx(ix - kx, p.ne[0], p.s128);
-        const float pyE = (float)(iy - p.ne[1]) * p.s128, pzE = (float)(iz - p.ne[2]) * p.s128;
-        const float floorE = far_floor(p.s128);
+        const double cx = (double)(ix - p.far.ne[0]) * p.far.spacing, cy = (double)(iy - p.far.ne[1]) * p.far.spacing,
+                     cz = (double)(iz - p.far.ne[2]) * p.far.spacing;
         for (int a = 0; a < p.n_atoms; a++) {
-            const float4 at = p.far_atoms[a];
-            const int fb = (int)(far_bin4(at.x, at.y, at.z, cxE, kx, p.s128, pyE, pzE, floorE) >> 2);
+            const int fb = (int)(far_bin4(p.coord[3 * a] * 128.0, p.coord[3 * a + 1] * 128.0, p.coord[3 * a + 2] * 128.0,
+                                          p.far, ix, iy, iz) >> 2);
             double dx, dy, dz;
             const double r64 = ref_dist(p.coord[3 * a], p.coord[3 * a + 1], p.coord[3 * a + 2], cx, cy, cz, dx, dy, dz);
             const int b64 = min((int)(r64 * 128.0), AG_NDIEL - 1);
@@ -1450,13 +1482,12 @@ constexpr int kFarLastBin = AG_NDIEL - 1;
 // the bin's table offset in one fma and one and, the LDS read (CLAMP caps
 // the offset at the table's last entry).
 template <bool CLAMP>
-__device__ __forceinline__ void far_pair(const PlainF4 &at, float py, float pz, float cx, float floor2, float s128,
-                                         float s2, const float *T, float *part) {
+__device__ __forceinline__ void far_pair(const PlainF4 &at, float py, float pz, float floor2, float s128, float s2,
+                                         const float *T, float *part) {
     const float dy = at.y - py, dz = at.z - pz;
     const float dyz2 = fmaxf(__builtin_fmaf(dy, dy, dz * dz), floor2);
-    const float u = at.x - cx;
-    const float U = __builtin_fmaf(u, u, dyz2);
-    const float us = u * s128;
+    const float U = __builtin_fmaf(at.x, at.x, dyz2);
+    const float us = at.x * s128;
     float W[kFarK / 2];
 #pragma unroll
     for (int j = 0; j < kFarK / 2; j++) W[j] = __builtin_fmaf(s2, far_c2(kFarK / 2 + j), U);
@@ -1485,9 +1516,20 @@ __device__ __forceinline__ int far_level(float ratio) {
     return min(max(126 - (int)(__float_as_uint(ratio * ratio) >> 23), 0), kFarLevels - 1);
 }
 
-// A wave-uniform float moved to a scalar register.
+// A wave-uniform value moved to a scalar register.
 __device__ __forceinline__ float sreg(float v) {
     return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+}
+
+__device__ __forceinline__ double sreg(double v) {
+    const long long b = __double_as_longlong(v);
+    const unsigned lo = __builtin_amdgcn_readfirstlane((int)b), hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
+    return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
+}
+
+// Lane i's value, in a scalar register.
+__device__ __forceinline__ float lane_of(float v, int i) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), i));
 }
 
 // Chebyshev nodes of [-1, 1]: cos((2i + 1) pi / 2n), in increasing order.
@@ -1534,7 +1576,7 @@ __device__ __forceinline__ void far_wy(double t, double w[4]) {
 // lanes; a lane takes the five x-nodes of one (y, z) node.
 //
 // The split follows the wave: one lane tests one atom, a ballot gives the
-// direct atoms (a scalar loop, their records through scalar loads) and
+// direct atoms (a scalar loop, their records read from the lanes) and
 // packs the others into the wave's LDS strip, all in index order, so results
 // repeat and depend on the conformation alone.
 //
@@ -1587,14 +1629,14 @@ __global__ void __launch_bounds__(kFarThreads) __attribute__((amdgpu_waves_per_e
         const bool active = lz < cf.far_pz && iy0 + ly < cf.n1[1] && iz0 + lz < cf.n1[2];
         const int iy = iy0 + (active ? ly : 0), iz = iz0 + (active ? lz : 0);   // idle lanes: the patch's corner
         const float s128 = cf.s128;
-        const float py = (float)(iy - cf.ne[1]) * s128, pz = (float)(iz - cf.ne[2]) * s128;
-        const float cx = far_cx(ix0, cf.ne[0], s128);
+        const float py = far_offset(iy - iy0, cf.far_py, s128), pz = far_offset(iz - iz0, cf.far_pz, s128);
         const float floor2 = far_floor(s128), s2 = s128 * s128;
         // the patch's box (whole, also where the grid ends inside it): centre and half widths
-        const float hx = sreg(kFarMid * s128), bx = sreg(cx);
+        const double bx = sreg(far_centre(ix0, kFarK, cf.ne[0], cf.spacing)),
+                     by = sreg(far_centre(iy0, cf.far_py, cf.ne[1], cf.spacing)),
+                     bz = sreg(far_centre(iz0, cf.far_pz, cf.ne[2], cf.spacing));
         const float my = 0.5f * (float)(cf.far_py - 1), mz = 0.5f * (float)(cf.far_pz - 1);
-        const float hy = sreg(my * s128), hz = sreg(mz * s128);
-        const float by = sreg(((float)(iy0 - cf.ne[1]) + my) * s128), bz = sreg(((float)(iz0 - cf.ne[2]) + mz) * s128);
+        const float hx = sreg(kFarMid * s128), hy = sreg(my * s128), hz = sreg(mz * s128);
         const float d1 = sreg(hx * far_node5(3)), d2 = sreg(hx * far_node5(4));
         const float d1q = sreg(d1 * d1), d2q = sreg(d2 * d2);
         float s[kFarK], c[kFarK], part[kFarK];
@@ -1608,19 +1650,18 @@ __global__ void __launch_bounds__(kFarThreads) __attribute__((amdgpu_waves_per_e
         if (lane < kFarLevels) level_r2[lane] = reinterpret_cast<const float *>(&p.confs[ci].far_r2)[lane];
         wave_sync();
         const float qscale = sreg(cf.far_qscale);
-        const float4 *const vatoms = p.atoms + cf.atom_base;
-        const AG_CONST PlainF4 *atoms = as_const(reinterpret_cast<const PlainF4 *>(vatoms));   // scalar loads
+        const FarAtom *const atoms = p.atoms + cf.atom_base;
         const int n_atoms = cf.n_atoms;
         const int step = 64 * kFarWaves * cf.far_split;
         int n_part = 0, n_node = 0;   // atoms in part[] and np[] since they were last flushed
         const int a_first = 64 * (part_i * kFarWaves + wave);
-        float4 A = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (a_first + lane < n_atoms) A = vatoms[a_first + lane];
+        FarAtom A{};
+        if (a_first + lane < n_atoms) A = atoms[a_first + lane];
         for (int a0 = a_first; a0 < n_atoms; a0 += step) {
-            const float4 at = A;
-            if (a0 + step + lane < n_atoms) A = vatoms[a0 + step + lane];
-            const float ex = fmaxf(fabsf(at.x - bx) - hx, 0.f), ey = fmaxf(fabsf(at.y - by) - hy, 0.f),
-                        ez = fmaxf(fabsf(at.z - bz) - hz, 0.f);
+            const float4 at = make_float4((float)(A.x - bx), (float)(A.y - by), (float)(A.z - bz), A.w);
+            if (a0 + step + lane < n_atoms) A = atoms[a0 + step + lane];
+            const float ex = fmaxf(fabsf(at.x) - hx, 0.f), ey = fmaxf(fabsf(at.y) - hy, 0.f),
+                        ez = fmaxf(fabsf(at.z) - hz, 0.f);
             const bool beyond =
                 __builtin_fmaf(ex, ex, __builtin_fmaf(ey, ey, ez * ez)) >= level_r2[far_level(at.w * qscale)];
             const int nb = min(64, n_atoms - a0);
@@ -1631,19 +1672,19 @@ __global__ void __launch_bounds__(kFarThreads) __attribute__((amdgpu_waves_per_e
                 const int nf = __popcll(far_set);
                 if ((far_set >> lane) & 1) strip[__popcll(far_set & ((1ull << lane) - 1))] = at;
                 // the last four filled up with zero weights
-                if (lane >= nf && lane < ((nf + 3) & ~3)) strip[lane] = make_float4(bx + 4096.f, by, bz, 0.f);
+                if (lane >= nf && lane < ((nf + 3) & ~3)) strip[lane] = make_float4(4096.f, 0.f, 0.f, 0.f);
                 wave_sync();
                 // this lane's y and z node (formed here: no register holds it through the direct loop)
                 int jl = lane;
                 asm volatile("" : "+v"(jl));
                 const int jy = jl & 3, jz = (jl >> 2) & 3;
-                const float ny = by + hy * ((jy & 2 ? 1.f : -1.f) * ((jy == 0 || jy == 3) ? kNode4a : kNode4b));
-                const float nz = bz + hz * ((jz & 2 ? 1.f : -1.f) * ((jz == 0 || jz == 3) ? kNode4a : kNode4b));
+                const float ny = hy * ((jy & 2 ? 1.f : -1.f) * ((jy == 0 || jy == 3) ? kNode4a : kNode4b));
+                const float nz = hz * ((jz & 2 ? 1.f : -1.f) * ((jz == 0 || jz == 3) ? kNode4a : kNode4b));
                 for (int i = 0; i < nf; i += 4) {
                     const float4 q = strip[i + (jl >> 4)];
-                    const float dy = q.y - ny, dz = q.z - nz, u = q.x - bx;
-                    const float U = __builtin_fmaf(u, u, __builtin_fmaf(dy, dy, dz * dz));
-                    const float W1 = U + d1q, W2 = U + d2q, u2 = u + u;
+                    const float dy = q.y - ny, dz = q.z - nz;
+                    const float U = __builtin_fmaf(q.x, q.x, __builtin_fmaf(dy, dy, dz * dz));
+                    const float W1 = U + d1q, W2 = U + d2q, u2 = q.x + q.x;
                     const float rb2[kFarNx] = {__builtin_fmaf(u2, d2, W2), __builtin_fmaf(u2, d1, W1), U,
                                                __builtin_fmaf(-u2, d1, W1), __builtin_fmaf(-u2, d2, W2)};
                     float rs[kFarNx], tv[kFarNx];
@@ -1669,18 +1710,12 @@ __global__ void __launch_bounds__(kFarThreads) __attribute__((amdgpu_waves_per_e
             }
             if (dir_set) {
                 n_part += __popcll(dir_set);
-                PlainF4 nxt = ld4(atoms, a0 + __builtin_ctzll(dir_set));
-                dir_set &= dir_set - 1;
-                while (true) {
-                    const PlainF4 q = nxt;
-                    const bool more = dir_set != 0;
-                    if (more) {
-                        nxt = ld4(atoms, a0 + __builtin_ctzll(dir_set));
-                        dir_set &= dir_set - 1;
-                    }
-                    far_pair<CLAMP>(q, py, pz, cx, floor2, s128, s2, T, part);
-                    if (!more) break;
-                }
+                do {
+                    const int i = __builtin_ctzll(dir_set);
+                    dir_set &= dir_set - 1;
+                    const PlainF4 q{lane_of(at.x, i), lane_of(at.y, i), lane_of(at.z, i), lane_of(at.w, i)};
+                    far_pair<CLAMP>(q, py, pz, floor2, s128, s2, T, part);
+                } while (dir_set);
                 if (n_part >= kFarAtomChunk) {
                     n_part = 0;
 #pragma unroll
@@ -1838,7 +1873,6 @@ struct ag_plan {
     std::vector<int> zero_slots;       // output maps that are all zero (Vina e/d)
     FarParams far{};
     bool run_far = false;
-    bool far_atoms_ready = false;
     double coeff_estat = 0.0;
     int far_grid = 0;                  // persistent far-kernel grid
     bool paged = false;                // near kernel in its paged form (a brick overflowed one LDS list)
@@ -2059,11 +2093,11 @@ static double far_floor_radius(bool flat, double spacing, int level) {
 // value, so past 64 A only (c) is asked for.
 // With the Mehler-Solmajer dielectric the steps decide: they leave 2e-7 of
 // the e map (2-norm, 5,000-atom protein) at 20 A, 5e-7 at 18 A and 8e-7 at 16 A,
-// beside the 7e-7 that FP32 bins of the direct pairs leave.  The floor and the
-// reference charge keep the whole error below the all-pairs sum's at every
-// spacing: 6.5e-7 for 7.0e-7 at 0.25 A, 8.4e-7 for 9.7e-7 at 0.3 A, 9.4e-7 for
-// 1.02e-6 at 0.375 A (5,000 atoms; 12,000: 1.19e-6 for 1.22e-6), 7.5e-7 for 1.5e-6 at
-// 0.5 A.  One distance for every charge: 3 % less error, 830 us instead of 772
+// beside the 6e-7 that FP32 bins of the direct pairs leave.  The floor and the
+// reference charge keep the whole error below the all-pairs sum's (whose
+// coordinates were rounded in the grid's frame): 6.2e-7 for 6.9e-7 at 0.25 A (2,743
+// atoms), at 0.375 A 9.5e-7 for 1.07e-6 (5,000 atoms) and 1.28e-6 for 1.31e-6 (20,000,
+// 257^3 points).  One distance for every charge: 3 % less error, 830 us instead of 772
 // for 5,000 atoms on 127^3 points, 460 instead of 430 for 3,000 on 81^3 in a constant
 // dielectric.
 static void far_radii(const std::vector<float> &reps, double spacing, double radius[kFarLevels]) {
@@ -2177,17 +2211,15 @@ static int near_share(long long bricks) {
 
 // How far (bins) a pair's distance in the near kernel may lie from the far
 // kernel's bin limit and the two still disagree on which of them has it.  The
-// far kernel's coordinates are FP32 bins (2^-25 of the largest, an atom's and a
-// point's, three axes), its squared distance sums four products of up to
+// far kernel's distances from the patch's centre are good to 2^-25 of them on
+// each side, three times at most per axis, its squared distance sums four products of up to
 // (limit + kFarMid s128)^2 with an error of 2^-24 each, the near kernel's
-// distance is good to 3e-4 bins; doubled.  At 0.375 A spacing and 96 A of grid
-// 0.01: the shell in which the near kernel repeats the far kernel's arithmetic
-// held some lane of 3 waves in 10 when it was 5 bins wide for every grid.
+// distance is good to 3e-4 bins; doubled.  At 0.375 A spacing 0.003: the shell
+// in which the near kernel repeats the far kernel's arithmetic held some lane
+// of 3 waves in 10 when it was 5 bins wide for every grid.
 static float far_band(const ag_grid &g) {
-    double edge = 0;
-    for (int d = 0; d < 3; d++) edge = std::max(edge, (double)std::max(g.ne[d], g.n1[d] - 1 - g.ne[d]));
     const double s128 = g.spacing * 128.0, reach = kFarBinMin + kFarMid * s128;
-    const double coord = 6 * 0x1p-25 * (edge * s128 + 2 * kFarBinMin);
+    const double coord = 9 * 0x1p-25 * reach;
     const double square = 4 * 0x1p-24 * 2 * reach * reach / (2.0 * kFarBinMin);
     return (float)(2 * (coord + square + 3e-4));
 }
@@ -2571,10 +2603,9 @@ static ag_plan *plan_build(ag_ctx *c, int n, const ag_receptor *recs, const ag_g
     p.run_far = !vina && ms->elec_index >= 0 && N > 0;
     std::vector<FarShape> far_shapes;
     if (p.run_far) {
-        float4 *d_far = (float4 *)p.far_atoms.get(sizeof(float4) * (size_t)N);
+        FarAtom *d_far = (FarAtom *)p.far_atoms.get(sizeof(FarAtom) * (size_t)N);
         k_far_atoms<<<(N + 255) / 256, 256, 0, st>>>(N, d_coord, d_charge, ms->coeff_estat, d_far);
         HIP_CHECK(hipGetLastError());
-        p.far_atoms_ready = true;
         double radius[kFarLevels] = {}, spacing = -1.0;
         for (int i = 0, o = 0; i < n; o += natoms[i], i++) {
             if (grids[i].spacing != spacing) far_radii(reps, spacing = grids[i].spacing, radius);
@@ -3178,13 +3209,6 @@ void plan_audit(ag_plan *p, long long out[4]) {
     HIP_CHECK(hipSetDevice(c->device));
     hipStream_t st = c->stream;
     if (p->nconf != 1) ag::fail(AG_ERR_UNSUPPORTED, "the bin audit runs on single-conformation plans");
-    if (!p->far_atoms_ready) {
-        float4 *d_far = (float4 *)p->far_atoms.get(sizeof(float4) * (size_t)std::max(p->N, 1));
-        if (p->N > 0)
-            k_far_atoms<<<(p->N + 255) / 256, 256, 0, st>>>(p->N, (const double *)p->coord.ptr,
-                                                            (const double *)p->charge.ptr, p->coeff_estat, d_far);
-        p->far_atoms_ready = true;
-    }
     DevBuf acc;
     unsigned long long *d_out = (unsigned long long *)acc.get(4 * sizeof(unsigned long long));
     HIP_CHECK(hipMemsetAsync(d_out, 0, 4 * sizeof(unsigned long long), st));
@@ -3193,11 +3217,12 @@ void plan_audit(ag_plan *p, long long out[4]) {
     memset(&ap, 0, sizeof ap);
     for (int d = 0; d < 3; d++) {
         ap.n1[d] = cf.n1[d];
-        ap.ne[d] = cf.ne[d];
+        ap.far.ne[d] = cf.ne[d];
     }
-    ap.spacing = cf.spacing;
-    ap.s128 = cf.s128;
-    ap.far_atoms = (const float4 *)p->far_atoms.ptr;
+    ap.far.py = cf.far_py;
+    ap.far.pz = cf.far_pz;
+    ap.far.spacing = cf.spacing;
+    ap.far.s128 = cf.s128;
     ap.coord = (const double *)p->coord.ptr;
     ap.n_atoms = p->N;
     ap.P = cf.P;
