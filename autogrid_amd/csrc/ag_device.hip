@@ -423,20 +423,70 @@ __global__ void k_cell_scatter(int n, const int *atom_cell, const int *start, in
     slot_atom[pos] = i;
 }
 
-// Order each cell's atoms by atom index (insertion sort; cells hold few atoms).
-__global__ void k_cell_sort(int ncells, const int *start, int *slot_atom) {
-    int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= ncells) return;
-    int b = start[c], e = start[c + 1];
-    for (int i = b + 1; i < e; i++) {
-        int v = slot_atom[i];
-        int j = i - 1;
-        while (j >= b && slot_atom[j] > v) {
-            slot_atom[j + 1] = slot_atom[j];
-            j--;
-        }
-        slot_atom[j + 1] = v;
+// What one workgroup needs to make the cell list of a small plan by itself.
+struct CellParams {
+    const ConfDev *confs;
+    const int *atom_conf;         // null when there is one conformation
+    int n, ncells;
+    double cs;
+    const double *coord;
+    int *start, *atom_cell, *slot_atom;
+    int *status, *queue;
+    int nq;
+};
+
+// k_zero_cells, k_cell_count, k_scan and k_cell_scatter by one workgroup, the
+// counts (ncells + 1 of them) in its LDS.
+template <int THREADS>
+__device__ void cell_list(const CellParams &p, int *cnt, int *wave_sum) {
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    for (int k = t; k < p.ncells; k += THREADS) cnt[k] = 0;
+    for (int k = t; k < p.nq; k += THREADS) p.queue[k] = 0;
+    if (t == 0) *p.status = 0;
+    __syncthreads();
+    for (int i = t; i < p.n; i += THREADS) {
+        const int cell = cell_of(p.confs[p.atom_conf ? p.atom_conf[i] : 0], p.cs, p.coord + 3 * (size_t)i);
+        p.atom_cell[i] = cell;
+        if (cell >= 0) atomicAdd(&cnt[cell], 1);
     }
+    __syncthreads();
+    // exclusive scan: 64 consecutive cells per wave and round, the waves'
+    // parts one after the other
+    const int per = ((p.ncells + THREADS - 1) / THREADS) * 64;   // cells of a wave
+    const int c0 = w * per, c1 = min(c0 + per, p.ncells);
+    int sum = 0;
+    for (int c = c0 + lane; c < c1; c += 64) sum += cnt[c];
+    for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
+    if (lane == 0) wave_sum[w] = sum;
+    __syncthreads();
+    int run = 0;
+    for (int k = 0; k < w; k++) run += wave_sum[k];
+    for (int base = c0; base < c1; base += 64) {
+        const int c = base + lane, v = c < c1 ? cnt[c] : 0;
+        int x = v;
+        for (int off = 1; off < 64; off <<= 1) {
+            const int y = __shfl_up(x, off);
+            if (lane >= off) x += y;
+        }
+        if (c < c1) cnt[c] = p.start[c] = run + x - v;
+        run += __shfl(x, 63);
+    }
+    if (w == THREADS / 64 - 1 && lane == 0) p.start[p.ncells] = run;
+    __syncthreads();
+    for (int i = t; i < p.n; i += THREADS) {
+        const int cell = p.atom_cell[i];
+        if (cell >= 0) p.slot_atom[atomicAdd(&cnt[cell], 1)] = i;
+    }
+}
+
+// The cell list in one launch.  Its four parts take 2 to 4 us each, most of that
+// the launch, and as much again between them: 1,000 atoms 11.4 us in all and 4.9
+// here, 5,000 atoms 13.9 and 14.9, 20,000 atoms 21 and 69 (the gaps not counted).
+constexpr int kCellsOne = 32768, kCellsOneAtoms = 6144;
+__global__ void __launch_bounds__(1024) k_cells(CellParams p) {
+    __shared__ int cnt[kCellsOne];
+    __shared__ int wave_sum[16];
+    cell_list<1024>(p, cnt, wave_sum);
 }
 
 struct AtomSrc {
@@ -446,11 +496,16 @@ struct AtomSrc {
     double coeff_estat, solpar_q;
 };
 
-// nslots = start[ncells], the number of atoms that landed in a cell.
-__global__ void k_gather(const int *nslots, const int *slot_atom, AtomSrc s, NearAtom *out) {
-    int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= *nslots) return;
-    int i = slot_atom[k];
+// The atoms' records in cell order, by atom index within a cell (a cell holds
+// few atoms: each counts those before it).
+__global__ void k_gather(int ncells, const int *atom_cell, const int *start, const int *slot_atom, AtomSrc s,
+                         NearAtom *out) {
+    const int slot = blockIdx.x * blockDim.x + threadIdx.x;
+    if (slot >= start[ncells]) return;
+    const int i = slot_atom[slot], cell = atom_cell[i];
+    const int b = start[cell], e = start[cell + 1];
+    int k = b;
+    for (int j = b; j < e; j++) k += slot_atom[j] < i;
     NearAtom a;
     a.x = s.coord[3 * i];
     a.y = s.coord[3 * i + 1];
@@ -2718,18 +2773,23 @@ static void enqueue(ag_plan *p, float *d_maps, float *d_fmap, int32_t *d_cmap, b
     const unsigned cgrid = (unsigned)((p->total_cells + tpb - 1) / tpb);
     if (events) HIP_CHECK(hipEventRecord(c->ev[0], st));
     if (part != kPartFar) {
-    k_zero_cells<<<std::max(cgrid, (unsigned)((kMaxChunks + tpb - 1) / tpb)), tpb, 0, st>>>(
-        d_count, d_cursor, p->total_cells, d_status, d_queue, kMaxChunks);
+    const int *atom_conf = p->nconf > 1 ? (const int *)p->atom_conf_d.ptr : nullptr;
+    const ConfDev *d_confs = (const ConfDev *)p->confs_d.ptr;
+    if (N <= kCellsOneAtoms && p->total_cells <= kCellsOne) {
+        k_cells<<<1, 1024, 0, st>>>({d_confs, atom_conf, N, p->total_cells, p->tune.cell_size,
+                                     (const double *)p->coord.ptr, d_start, d_atom_cell, d_slot_atom, d_status, d_queue,
+                                     kMaxChunks});
+    } else {
+        k_zero_cells<<<std::max(cgrid, (unsigned)((kMaxChunks + tpb - 1) / tpb)), tpb, 0, st>>>(
+            d_count, d_cursor, p->total_cells, d_status, d_queue, kMaxChunks);
+        if (N > 0)
+            k_cell_count<<<(N + tpb - 1) / tpb, tpb, 0, st>>>(d_confs, atom_conf, N, p->tune.cell_size,
+                                                              (const double *)p->coord.ptr, d_atom_cell, d_count);
+        k_scan<<<1, 1024, 0, st>>>(d_count, d_start, p->total_cells);
+        if (N > 0) k_cell_scatter<<<(N + tpb - 1) / tpb, tpb, 0, st>>>(N, d_atom_cell, d_start, d_cursor, d_slot_atom);
+    }
     if (N > 0)
-        k_cell_count<<<(N + tpb - 1) / tpb, tpb, 0, st>>>((const ConfDev *)p->confs_d.ptr,
-                                                          p->nconf > 1 ? (const int *)p->atom_conf_d.ptr : nullptr, N,
-                                                          p->tune.cell_size, (const double *)p->coord.ptr,
-                                                          d_atom_cell, d_count);
-    k_scan<<<1, 1024, 0, st>>>(d_count, d_start, p->total_cells);
-    if (N > 0) k_cell_scatter<<<(N + tpb - 1) / tpb, tpb, 0, st>>>(N, d_atom_cell, d_start, d_cursor, d_slot_atom);
-    k_cell_sort<<<cgrid, tpb, 0, st>>>(p->total_cells, d_start, d_slot_atom);
-    if (N > 0)
-        k_gather<<<(N + tpb - 1) / tpb, tpb, 0, st>>>(d_start + p->total_cells, d_slot_atom, p->src,
+        k_gather<<<(N + tpb - 1) / tpb, tpb, 0, st>>>(p->total_cells, d_atom_cell, d_start, d_slot_atom, p->src,
                                                       (NearAtom *)p->near_atoms.ptr);
     HIP_CHECK(hipGetLastError());
     }
