@@ -357,7 +357,7 @@ class Context:
         return Plan(self, st, potential)
 
     def timing(self) -> dict:
-        """HIP-event milliseconds of the last plan execution on this context."""
+        """Milliseconds of the last plan execution on this context (ag_context_timing)."""
         ms = (C.c_float * 4)()
         check(lib().ag_context_timing(self._h, ms))
         return {"cell_ms": ms[0], "near_ms": ms[1], "far_ms": ms[2], "total_ms": ms[3]}

@@ -173,6 +173,39 @@ __device__ __forceinline__ float hramp_value(float ct) {
     return (1.f - h) * q;
 }
 
+// What the kernels of a map set report, in pinned host memory that they write
+// themselves: a copy after the map set cost 10 us of a 41^3-point one, and events
+// between its kernels as much again.
+struct MapReport {
+    int overflow = 0;                  // a brick of the near kernel overflowed its LDS lists
+    unsigned long long start[4] = {0, 0, 0, 0};   // wall_clock64 at the start of its phases
+};
+
+// The reports of a context's plans: one page, allocated with the first and
+// freed with the last owner.  A plan that finds none free goes without.
+class StatusPage {
+    static constexpr int kReports = 64;
+    std::mutex mu;
+    HostStage page;
+    unsigned long long used = 0;
+
+  public:
+    MapReport *take() {
+        std::lock_guard<std::mutex> lk(mu);
+        if (used == ~0ull) return nullptr;
+        const int k = __builtin_ctzll(~used);
+        MapReport *r = reinterpret_cast<MapReport *>((char *)page.get(64 * kReports) + 64 * k);
+        *r = MapReport{};
+        used |= 1ull << k;
+        return r;
+    }
+    void give_back(MapReport *r) {
+        std::lock_guard<std::mutex> lk(mu);
+        used &= ~(1ull << (((char *)r - (char *)page.get(64 * kReports)) / 64));
+    }
+};
+static_assert(sizeof(MapReport) <= 64, "one report per line");
+
 struct ag_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -186,7 +219,8 @@ struct ag_ctx {
     std::shared_ptr<DevPool> pool = std::make_shared<DevPool>();   // blocks of destroyed plans
     DevBuf maps;                       // output staging of ag_maps_plain
     HostStage stage;                   // receptor arrays of a plan on their way up
-    HostStage status_word;             // pinned target of a plan's status flag after each map set
+    std::shared_ptr<StatusPage> status_page = std::make_shared<StatusPage>();   // its plans' reports
+    double clock_khz = 1.0e5;          // rate of the device's wall clock
     void *scratch = nullptr;           // this device's allocation-free scratch (ag_maps_plain_noalloc)
     hipEvent_t ev[4] = {};
     float last_ms[4] = {0, 0, 0, 0};   // cell list, near, far, total of the last execute

@@ -155,6 +155,11 @@ __device__ __forceinline__ int find_conf(const AG_CONST int *prefix, int nconf, 
     return lo;
 }
 
+// When a kernel began, by its first thread (wall_clock64; null: not wanted).
+__device__ __forceinline__ void stamp_start(unsigned long long *stamp) {
+    if (stamp && blockIdx.x == 0 && threadIdx.x == 0) *stamp = wall_clock64();
+}
+
 struct NearParams {
     // conformations and work distribution
     const ConfDev *confs;
@@ -188,7 +193,9 @@ struct NearParams {
     int bhtree;                   // ag_mapset.bhtree: Loop 2 and cmap by the tree's FP32 test
     unsigned char *collide;       // tree build, collisions tested: 1 per point within 1.5 A of an atom (pass 0)
     float *maps;
+    const float *far_part;        // the far kernel's parts of the e map when it has run before, or null
     int *status;
+    unsigned long long *stamp;
 };
 
 // An atom of the far kernel: coordinates in bins (exact) and charge times the
@@ -209,6 +216,7 @@ struct FarParams {
     float *maps;                  // e map slot: in = near part, out = total
     float *part;                  // partial e maps of the conformations with far_split > 1
     int e_slot;
+    unsigned long long *stamp;
 };
 
 // Consecutive workgroup ids go round-robin over the 8 XCDs; here XCD x takes
@@ -332,7 +340,9 @@ __global__ void k_cell_count(const ConfDev *confs, const int *atom_conf, int n, 
 // Clears the cell counts and cursors [0, n), the status word and the nq
 // work counters of one map set, in one launch: a kernel rather than memset
 // nodes, since a plan's map set is captured in a graph.
-__global__ void k_zero_cells(int *count, int *cursor, int n, int *status, int *queue, int nq) {
+__global__ void k_zero_cells(int *count, int *cursor, int n, int *status, int *queue, int nq,
+                             unsigned long long *stamp) {
+    stamp_start(stamp);
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) {
         count[i] = 0;
@@ -433,6 +443,7 @@ struct CellParams {
     int *start, *atom_cell, *slot_atom;
     int *status, *queue;
     int nq;
+    unsigned long long *stamp;
 };
 
 // k_zero_cells, k_cell_count, k_scan and k_cell_scatter by one workgroup, the
@@ -440,6 +451,7 @@ struct CellParams {
 template <int THREADS>
 __device__ void cell_list(const CellParams &p, int *cnt, int *wave_sum) {
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    stamp_start(p.stamp);
     for (int k = t; k < p.ncells; k += THREADS) cnt[k] = 0;
     for (int k = t; k < p.nq; k += THREADS) p.queue[k] = 0;
     if (t == 0) *p.status = 0;
@@ -499,7 +511,8 @@ struct AtomSrc {
 // The atoms' records in cell order, by atom index within a cell (a cell holds
 // few atoms: each counts those before it).
 __global__ void k_gather(int ncells, const int *atom_cell, const int *start, const int *slot_atom, AtomSrc s,
-                         NearAtom *out) {
+                         NearAtom *out, unsigned long long *stamp) {
+    stamp_start(stamp);
     const int slot = blockIdx.x * blockDim.x + threadIdx.x;
     if (slot >= start[ncells]) return;
     const int i = slot_atom[slot], cell = atom_cell[i];
@@ -642,6 +655,7 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
     __shared__ int2 wave_tot[2][kStage][kNearThreads / 64];
 
     const int tid = threadIdx.x;
+    stamp_start(p.stamp);
     // read here, stored once the staging's own reads are on their way
     constexpr int kRsPer = (kNearRepsLen + kNearThreads - 1) / kNearThreads;
     float2 rs[kRsPer];
@@ -814,7 +828,7 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
     __syncthreads();
     if constexpr (!PAGED) {
         if (ncand > kCandCap || nh > kHCap) {   // uniform per workgroup
-            if (tid == 0) atomicOr(p.status, 1);
+            if (tid == 0) __hip_atomic_store(p.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);   // host memory
             return;
         }
     }
@@ -1317,7 +1331,14 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
                 v += hmin[m - kPlainSlots] + fmaxf(hmax[m - kPlainSlots], 0.f);
             maps[(long long)p.out_slot[m] * P + pt] = v;
         }
-        if (want_e && stores(0)) maps[(long long)p.e_slot * P + pt] = e_near;
+        if (want_e && stores(0)) {
+            if (p.far_part) {   // as k_far_sum adds them
+                double v = e_near;
+                for (int q = 0; q < cf.far_split; q++) v += (double)p.far_part[cf.part_off + q * P + pt];
+                e_near = (float)v;
+            }
+            maps[(long long)p.e_slot * P + pt] = e_near;
+        }
         if (cmap && stores(1)) cmap[pt] = ccount;
         if (p.collide && stores(2)) p.collide[cf.pt_off + pt] = collide ? 1 : 0;
         if (p.d_slot >= 0 && stores(3)) maps[(long long)p.d_slot * P + pt] = p.solpar_q * dv_acc;   // solpar_q sum(vol S)
@@ -1646,10 +1667,19 @@ __device__ __forceinline__ void far_wy(double t, double w[4]) {
 // CLAMP caps the direct pairs' table offsets at bin 8191: for launches where
 // a conformation's direct pairs may pass it (spacings of about 1 A and more;
 // the cap changes no other pair's value).
-template <bool CLAMP>
-__global__ void __launch_bounds__(kFarThreads) __attribute__((amdgpu_waves_per_eu(4))) k_far(FarParams p) {
+// CELLS: the launch's first workgroup makes the plan's cell list, which the
+// near kernel will want (small plans, whose parts the near kernel adds up).
+constexpr int kFarLds = AG_NDIEL + 2 * 64 * kFarK;
+template <bool CLAMP, bool CELLS>
+__global__ void __launch_bounds__(kFarThreads) __attribute__((amdgpu_waves_per_eu(4))) k_far(FarParams p, CellParams cp) {
     // 40 KiB: four workgroups per CU
-    __shared__ float lds[AG_NDIEL + 2 * 64 * kFarK];
+    __shared__ float lds[kFarLds];
+    if (CELLS && blockIdx.x == 0) {
+        int *const cnt = reinterpret_cast<int *>(lds);
+        cell_list<kFarThreads>(cp, cnt + kFarWaves, cnt);
+        return;
+    }
+    if (!CELLS) stamp_start(p.stamp);
     float *const T = lds, *const X = lds + AG_NDIEL;
     static_assert(kFarBinMin == AG_NEINT + 1, "the table's zeros below end one bin into a float4");
     for (int i = threadIdx.x; i < AG_NDIEL / 4; i += kFarThreads) {
@@ -1666,7 +1696,7 @@ __global__ void __launch_bounds__(kFarThreads) __attribute__((amdgpu_waves_per_e
         __syncthreads();
         item = reinterpret_cast<int *>(X)[0];
     } else {
-        item = p.item_base + xcd_chunked<16>(blockIdx.x, gridDim.x);
+        item = p.item_base + (CELLS ? xcd_chunked<16>(blockIdx.x - 1, gridDim.x - 1) : xcd_chunked<16>(blockIdx.x, gridDim.x));
     }
     __syncthreads();
     item = __builtin_amdgcn_readfirstlane(item);
@@ -1938,6 +1968,8 @@ struct ag_plan {
     // empty when far_split == nconf)
     hipGraphExec_t graph = nullptr, graph_far = nullptr, graph_far2 = nullptr;
     int far_split = 0;
+    std::shared_ptr<StatusPage> status_page;   // owner of report, if any
+    MapReport *report = nullptr;       // pinned: what the kernels of a map set report
     float *g_maps = nullptr, *g_fmap = nullptr;
     int32_t *g_cmap = nullptr;
     void drop_graphs() {
@@ -1946,7 +1978,12 @@ struct ag_plan {
         if (graph_far2) (void)hipGraphExecDestroy(graph_far2);
         graph = graph_far = graph_far2 = nullptr;
     }
-    ~ag_plan() { drop_graphs(); }
+    int *overflow_flag() const { return report ? &report->overflow : (int *)status.ptr; }
+    unsigned long long *stamp(int phase) const { return report && !persistent ? &report->start[phase] : nullptr; }
+    ~ag_plan() {
+        drop_graphs();
+        if (report) status_page->give_back(report);
+    }
 };
 
 namespace agdev {
@@ -1984,6 +2021,9 @@ ag_status context_create(ag_ctx **out, int device) {
     for (auto &e : c->ev) HIP_CHECK(hipEventCreate(&e));
     for (auto &e : c->chunk_ev) HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     HIP_CHECK(hipDeviceGetAttribute(&c->n_cu, hipDeviceAttributeMultiprocessorCount, device));
+    int khz = 0;
+    HIP_CHECK(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device));
+    c->clock_khz = khz > 0 ? khz : 100000.0;
     c->scratch = scratch_address(device);
     *out = c;
     return AG_OK;
@@ -2246,8 +2286,14 @@ static FarShape far_shape(const ag_grid &g, int n_atoms, const double radius[kFa
 }
 
 static void launch_far(int blocks, const FarParams &fp, bool clamp, hipStream_t st) {
-    if (clamp) k_far<true><<<blocks, kFarThreads, 0, st>>>(fp);
-    else k_far<false><<<blocks, kFarThreads, 0, st>>>(fp);
+    if (clamp) k_far<true, false><<<blocks, kFarThreads, 0, st>>>(fp, CellParams{});
+    else k_far<false, false><<<blocks, kFarThreads, 0, st>>>(fp, CellParams{});
+    HIP_CHECK(hipGetLastError());
+}
+// The same with the cell list in one more workgroup.
+static void launch_far_cells(int blocks, const FarParams &fp, const CellParams &cp, bool clamp, hipStream_t st) {
+    if (clamp) k_far<true, true><<<blocks + 1, kFarThreads, 0, st>>>(fp, cp);
+    else k_far<false, true><<<blocks + 1, kFarThreads, 0, st>>>(fp, cp);
     HIP_CHECK(hipGetLastError());
 }
 
@@ -2389,7 +2435,7 @@ static void plan_geometry(ag_plan &p, const ag_grid *grids, const int *natoms, c
     p.far.nconf = n;
     p.far.total_tiles = p.total_tiles;
     int occ = 0;
-    HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, reinterpret_cast<const void *>(&k_far<true>),
+    HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, reinterpret_cast<const void *>(&k_far<true, false>),
                                                            kFarThreads, 0));
     p.far_grid = std::max(1, std::min(p.total_tiles, std::max(occ, 1) * p.ctx->n_cu));
 }
@@ -2498,7 +2544,12 @@ static ag_plan *plan_build(ag_ctx *c, int n, const ag_receptor *recs, const ag_g
     if ((unsigned long long)N * sizeof(NearAtom) > UINT32_MAX)
         ag::fail(AG_ERR_UNSUPPORTED, "too many atoms in one plan for the near kernel (at most 44,739,242)");
     p.near_atoms.get(sizeof(NearAtom) * (size_t)N);
-    p.status.get(sizeof(int));
+    // an arena pool allocates no pinned memory: its plans keep the flag on the device
+    if (!p.pool->arena) {
+        p.status_page = c->status_page;
+        p.report = p.status_page->take();
+    }
+    if (!p.report) p.status.get(sizeof(int));
 
     // electrostatic factor per bin: 332/eps for the distance-dependent
     // dielectric, 332/diel for a constant one (main.cpp:2960-2978)
@@ -2586,7 +2637,7 @@ static ag_plan *plan_build(ag_ctx *c, int n, const ag_receptor *recs, const ag_g
     np.disorder_h = ms->disorder_h;
     np.hydrogen_type = ms->hydrogen_type;
     np.solpar_q = (float)ms->solpar_q;
-    np.status = (int *)p.status.ptr;
+    np.status = p.overflow_flag();
     for (int g = 0; g < p.groups; g++) {
         NearParams q = np;
         bool used = false;
@@ -2746,6 +2797,17 @@ static std::vector<std::pair<int, int>> plan_chunks(const ag_plan &p, int want, 
 }
 
 enum : int { kPartAll = 0, kPartNear = 1, kPartFar = 2 };
+// Phases of MapReport::start: the first kernel (the cell list, or with it the
+// far field), the gather behind a far field that went first, the near field,
+// the far field in its usual place.
+enum : int { kStampFirst = 0, kStampGather = 1, kStampNear = 2, kStampFar = 3 };
+
+// One conformation whose far field is in parts, with a cell list that one
+// workgroup makes in the far kernel's LDS before the others are done.
+static bool far_goes_first(const ag_plan &p) {
+    return !p.persistent && p.nconf == 1 && p.run_far && p.confs[0].far_split > 1 && p.N <= kCellsOneAtoms &&
+           p.total_cells <= kFarLds - kFarWaves;
+}
 
 // Enqueue one map set on the context's stream, conformation chunk by chunk.
 // With events, HIP events bracket the cell list, the near-field and the
@@ -2765,35 +2827,49 @@ static void enqueue(ag_plan *p, float *d_maps, float *d_fmap, int32_t *d_cmap, b
     int *d_atom_cell = (int *)p->atom_cell.ptr, *d_count = (int *)p->cell_count.ptr;
     int *d_start = (int *)p->cell_start.ptr, *d_cursor = (int *)p->cell_cursor.ptr;
     int *d_slot_atom = (int *)p->slot_atom.ptr;
-    int *d_status = (int *)p->status.ptr;
+    int *d_status = p->overflow_flag();
     int *d_queue = (int *)p->queue_d.ptr;
     const int nchunks = (int)chunks.size();
     if (nchunks < 1 || nchunks > kMaxChunks) ag::fail(AG_ERR_BAD_INPUT, "bad chunking of the batch");
     if (part != kPartAll && (nchunks != 1 || host)) ag::fail(AG_ERR_BAD_INPUT, "bad chunking of the batch");
     const unsigned cgrid = (unsigned)((p->total_cells + tpb - 1) / tpb);
     if (events) HIP_CHECK(hipEventRecord(c->ev[0], st));
+    // A small plan's far field, in parts, goes first with the cell list in one
+    // of its workgroups, and the near kernel adds the parts: 3 launches instead
+    // of 5.  (With one part the far kernel adds to the near field's e map, and
+    // a copy to the host overlaps the far field behind it.)
+    const bool far_first = far_goes_first(*p) && part == kPartAll && !skip_far && !host && !mark_near && nchunks == 1;
+    const bool stamps = events && p->report && !p->persistent && !skip_far;
+    const auto stamp = [&](int phase) { return stamps ? p->stamp(phase) : nullptr; };
     if (part != kPartFar) {
-    const int *atom_conf = p->nconf > 1 ? (const int *)p->atom_conf_d.ptr : nullptr;
-    const ConfDev *d_confs = (const ConfDev *)p->confs_d.ptr;
-    if (N <= kCellsOneAtoms && p->total_cells <= kCellsOne) {
-        k_cells<<<1, 1024, 0, st>>>({d_confs, atom_conf, N, p->total_cells, p->tune.cell_size,
-                                     (const double *)p->coord.ptr, d_start, d_atom_cell, d_slot_atom, d_status, d_queue,
-                                     kMaxChunks});
-    } else {
-        k_zero_cells<<<std::max(cgrid, (unsigned)((kMaxChunks + tpb - 1) / tpb)), tpb, 0, st>>>(
-            d_count, d_cursor, p->total_cells, d_status, d_queue, kMaxChunks);
+        const int *atom_conf = p->nconf > 1 ? (const int *)p->atom_conf_d.ptr : nullptr;
+        const ConfDev *d_confs = (const ConfDev *)p->confs_d.ptr;
+        const CellParams cp{d_confs, atom_conf, N, p->total_cells, p->tune.cell_size, (const double *)p->coord.ptr,
+                            d_start, d_atom_cell, d_slot_atom, d_status, d_queue, kMaxChunks, stamp(kStampFirst)};
+        if (far_first) {
+            FarParams fp = p->far;
+            fp.maps = d_maps;
+            fp.item_end = p->total_tiles;
+            launch_far_cells(p->total_tiles, fp, cp, p->confs[0].far_clamp, st);
+        } else if (N <= kCellsOneAtoms && p->total_cells <= kCellsOne) {
+            k_cells<<<1, 1024, 0, st>>>(cp);
+        } else {
+            k_zero_cells<<<std::max(cgrid, (unsigned)((kMaxChunks + tpb - 1) / tpb)), tpb, 0, st>>>(
+                d_count, d_cursor, p->total_cells, d_status, d_queue, kMaxChunks, stamp(kStampFirst));
+            if (N > 0)
+                k_cell_count<<<(N + tpb - 1) / tpb, tpb, 0, st>>>(d_confs, atom_conf, N, p->tune.cell_size,
+                                                                  (const double *)p->coord.ptr, d_atom_cell, d_count);
+            k_scan<<<1, 1024, 0, st>>>(d_count, d_start, p->total_cells);
+            if (N > 0)
+                k_cell_scatter<<<(N + tpb - 1) / tpb, tpb, 0, st>>>(N, d_atom_cell, d_start, d_cursor, d_slot_atom);
+        }
         if (N > 0)
-            k_cell_count<<<(N + tpb - 1) / tpb, tpb, 0, st>>>(d_confs, atom_conf, N, p->tune.cell_size,
-                                                              (const double *)p->coord.ptr, d_atom_cell, d_count);
-        k_scan<<<1, 1024, 0, st>>>(d_count, d_start, p->total_cells);
-        if (N > 0) k_cell_scatter<<<(N + tpb - 1) / tpb, tpb, 0, st>>>(N, d_atom_cell, d_start, d_cursor, d_slot_atom);
+            k_gather<<<(N + tpb - 1) / tpb, tpb, 0, st>>>(p->total_cells, d_atom_cell, d_start, d_slot_atom, p->src,
+                                                          (NearAtom *)p->near_atoms.ptr,
+                                                          far_first ? stamp(kStampGather) : nullptr);
+        HIP_CHECK(hipGetLastError());
     }
-    if (N > 0)
-        k_gather<<<(N + tpb - 1) / tpb, tpb, 0, st>>>(p->total_cells, d_atom_cell, d_start, d_slot_atom, p->src,
-                                                      (NearAtom *)p->near_atoms.ptr);
-    HIP_CHECK(hipGetLastError());
-    }
-    if (events) HIP_CHECK(hipEventRecord(c->ev[1], st));
+    if (events && !stamps) HIP_CHECK(hipEventRecord(c->ev[1], st));
     // The near field (near kernel, floating grid, covalent and zero maps) of
     // conformations [c0, c1) on stream s.
     auto near_pass = [&](int c0, int c1, hipStream_t s) {
@@ -2803,6 +2879,8 @@ static void enqueue(ag_plan *p, float *d_maps, float *d_fmap, int32_t *d_cmap, b
             np.maps = d_maps;
             np.cmap = (g == 0 && p->want_cmap) ? d_cmap : nullptr;
             np.item_base = b0;
+            np.far_part = far_first ? p->far.part : nullptr;
+            np.stamp = g == 0 ? stamp(kStampNear) : nullptr;
             if (!(np.has_affinity || np.e_slot >= 0 || np.cmap) || b1 <= b0) continue;
             launch_near(*p, b1 - b0, np, s);
         }
@@ -2849,9 +2927,10 @@ static void enqueue(ag_plan *p, float *d_maps, float *d_fmap, int32_t *d_cmap, b
     // build's collision rule after it, on stream s.
     auto far_pass = [&](int k, int c0, int c1, hipStream_t s) {
         const int t0 = p->tile_prefix[c0], t1 = p->tile_prefix[c1];
-        if (p->run_far && !skip_far && t1 > t0) {
+        if (p->run_far && !skip_far && !far_first && t1 > t0) {
             FarParams fp = p->far;
             fp.maps = d_maps;
+            fp.stamp = stamp(kStampFar);
             fp.item_base = t0;
             fp.item_end = t1;
             fp.queue = p->persistent ? d_queue + queue_base + k : nullptr;
@@ -2913,7 +2992,7 @@ static void enqueue(ag_plan *p, float *d_maps, float *d_fmap, int32_t *d_cmap, b
     } else {
         for (int k = 0; k < nchunks; k++) {
             if (part != kPartFar) near_pass(chunks[k].first, chunks[k].second, st_main);
-            if (events && k == nchunks - 1) HIP_CHECK(hipEventRecord(c->ev[2], st_main));
+            if (events && !stamps && k == nchunks - 1) HIP_CHECK(hipEventRecord(c->ev[2], st_main));
             if (mark_near && k == nchunks - 1) HIP_CHECK(hipEventRecord(c->near_ev, st_main));
             if (part != kPartNear) far_pass(k, chunks[k].first, chunks[k].second, st_main);
             if (host) copy_out(k, chunks[k].first, chunks[k].second, st_main);
@@ -2937,13 +3016,14 @@ static void enqueue(ag_plan *p, float *d_maps, float *d_fmap, int32_t *d_cmap, b
 // Whether a brick of the last map set overflowed the near kernel's LDS lists
 // (syncs the context's stream).
 static bool overflowed(ag_plan *p) {
-    // into pinned memory: a direct copy, not a staged one (a plan on an
-    // arena pool allocates no pinned word and copies into the stack)
-    int local = 0;
-    int *status = p->pool->arena ? &local : (int *)p->ctx->status_word.get(sizeof(int));
-    HIP_CHECK(hipMemcpyAsync(status, p->status.ptr, sizeof(int), hipMemcpyDeviceToHost, p->ctx->stream));
+    if (p->report) {   // written by the kernels themselves
+        HIP_CHECK(hipStreamSynchronize(p->ctx->stream));
+        return __atomic_load_n(&p->report->overflow, __ATOMIC_ACQUIRE) != 0;
+    }
+    int status = 0;
+    HIP_CHECK(hipMemcpyAsync(&status, p->status.ptr, sizeof(int), hipMemcpyDeviceToHost, p->ctx->stream));
     HIP_CHECK(hipStreamSynchronize(p->ctx->stream));
-    return (*status & 1) != 0;
+    return status != 0;
 }
 
 // Runs one map set of p through `run` and checks the overflow word: when a
@@ -3100,11 +3180,12 @@ static hipGraphExec_t capture(ag_plan *p, float *d_maps, float *d_fmap, int32_t 
     return exec;
 }
 
-static void launch_mapset(ag_plan *p, float *d_maps, float *d_fmap, int32_t *d_cmap) {
+static void launch_mapset(ag_plan *p, float *d_maps, float *d_fmap, int32_t *d_cmap, bool mark_near) {
     ag_ctx *c = p->ctx;
     hipStream_t st = c->stream;
     if (!p->persistent) {
-        enqueue(p, d_maps, d_fmap, d_cmap, true, false, true);
+        if (p->report) *p->report = MapReport{};   // (the plan's last map set was waited for)
+        enqueue(p, d_maps, d_fmap, d_cmap, true, false, mark_near);
         return;
     }
     if (!p->graph || p->g_maps != d_maps || p->g_fmap != d_fmap || p->g_cmap != d_cmap) {
@@ -3133,21 +3214,38 @@ static void launch_mapset(ag_plan *p, float *d_maps, float *d_fmap, int32_t *d_c
 
 static void read_timing(ag_plan *p) {
     ag_ctx *c = p->ctx;
-    if (!p->persistent) {
+    float total = 0.f;
+    HIP_CHECK(hipEventElapsedTime(&total, c->ev[0], c->ev[3]));
+    if (p->persistent) {
+        c->last_ms[0] = c->last_ms[1] = c->last_ms[2] = -1.f;
+    } else if (p->report) {
+        // the phases' starts by the device's clock; the last one ends with the total
+        const unsigned long long *const t = p->report->start;
+        const auto span = [&](int from, int to) {
+            return t[from] && t[to] > t[from] ? (float)((double)(t[to] - t[from]) / c->clock_khz) : 0.f;
+        };
+        if (t[kStampGather]) {   // the far field went first
+            c->last_ms[2] = span(kStampFirst, kStampGather);
+            c->last_ms[0] = span(kStampGather, kStampNear);
+            c->last_ms[1] = std::max(0.f, total - c->last_ms[0] - c->last_ms[2]);
+        } else {
+            c->last_ms[0] = span(kStampFirst, kStampNear);
+            c->last_ms[1] = t[kStampFar] ? span(kStampNear, kStampFar) : std::max(0.f, total - c->last_ms[0]);
+            c->last_ms[2] = std::max(0.f, total - c->last_ms[0] - c->last_ms[1]);
+        }
+    } else {
         HIP_CHECK(hipEventElapsedTime(&c->last_ms[0], c->ev[0], c->ev[1]));
         HIP_CHECK(hipEventElapsedTime(&c->last_ms[1], c->ev[1], c->ev[2]));
         HIP_CHECK(hipEventElapsedTime(&c->last_ms[2], c->ev[2], c->ev[3]));
-    } else {
-        c->last_ms[0] = c->last_ms[1] = c->last_ms[2] = -1.f;
     }
-    HIP_CHECK(hipEventElapsedTime(&c->last_ms[3], c->ev[0], c->ev[3]));
+    c->last_ms[3] = total;
 }
 
 void plan_execute(ag_plan *p, float *d_maps, float *d_fmap, int32_t *d_cmap) {
     if ((p->want_fmap && !d_fmap) || (p->want_cmap && !d_cmap))
         ag::fail(AG_ERR_BAD_INPUT, "the map set asks for a floating/constriction grid but no output was given");
     HIP_CHECK(hipSetDevice(p->ctx->device));
-    run_checked(p, [&] { launch_mapset(p, d_maps, d_fmap, d_cmap); });
+    run_checked(p, [&] { launch_mapset(p, d_maps, d_fmap, d_cmap, false); });
     read_timing(p);
 }
 
@@ -3178,7 +3276,7 @@ void plan_execute_host(ag_plan *p, float *d_maps, float *d_fmap, int32_t *d_cmap
         if (bytes) HIP_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, cs));
     };
     run_checked(p, [&] {
-        launch_mapset(p, d_maps, d_fmap, d_cmap);
+        launch_mapset(p, d_maps, d_fmap, d_cmap, true);
         HIP_CHECK(hipStreamWaitEvent(cs, c->near_ev, 0));
         for (int i = 0; i < p->nconf; i++) {
             const ConfDev &cf = p->confs[i];

@@ -307,9 +307,10 @@ typedef struct ag_audit {
 } ag_audit;
 ag_status ag_plan_audit(ag_plan *plan, ag_audit *out);
 
-/* Milliseconds of the last execute on ctx, from HIP events recorded on ctx's
- * stream: [0] cell list, [1] near-field kernel(s), [2] far-field kernel,
- * [3] total. */
+/* Milliseconds of the last execute on ctx: [0] cell list, [1] near-field
+ * kernel(s), [2] far-field kernel, by the device's clock (a small plan makes
+ * its cell list inside the far-field kernel), [3] total, from HIP events on
+ * ctx's stream. */
 ag_status ag_context_timing(ag_ctx *ctx, float ms[4]);
 
 /* ------------------------------------------------------------------------ */

@@ -3,6 +3,7 @@ the same records in the same order, so the same maps bit for bit.  A receptor
 alone takes the first, and in a batch beside a large one the second."""
 from __future__ import annotations
 
+import ctypes as C
 import dataclasses
 import os
 
@@ -26,6 +27,28 @@ def base(tmp_path_factory):
         return ag.Job(gpf).prepare().state()
     finally:
         os.chdir(cwd)
+
+
+class Dev:
+    """A device buffer through the engine's own HIP runtime."""
+
+    def __init__(self, nbytes):
+        self.hip, self.p = C.CDLL("libamdhip64.so"), C.c_void_p()
+        assert self.hip.hipMalloc(C.byref(self.p), C.c_size_t(nbytes)) == 0
+
+    def put(self, a):
+        assert self.hip.hipMemcpy(self.p, a.ctypes.data_as(C.c_void_p), C.c_size_t(a.nbytes), 1) == 0
+
+    def get(self, n):
+        a = np.empty(n, np.float32)
+        assert self.hip.hipMemcpy(a.ctypes.data_as(C.c_void_p), self.p, C.c_size_t(a.nbytes), 2) == 0
+        return a
+
+    def __enter__(self):
+        return self
+
+    def __exit__(self, *exc):
+        assert self.hip.hipFree(self.p) == 0
 
 
 def state(base, n, n1, edge, seed):
@@ -55,3 +78,51 @@ def test_one_workgroup(base, n, n1, edge):
         beside = ctx.maps_batch([st, large], tune={"cell_size": 4.0, "cube": True})
     assert np.array_equal(np.asarray(alone).reshape(-1), np.asarray(beside[0]).reshape(-1))
     assert np.isfinite(alone).all()
+
+
+@pytest.mark.parametrize("n, n1, edge", [
+    (600, (33, 33, 33), 25.0),       # two parts: the far field first, the cell list in it
+    (2500, (25, 31, 17), 33.0),      # eight parts, ragged patches
+    (5000, (5, 5, 5), 42.0),         # one patch
+    (ONE, (41, 41, 41), 44.0),
+    (600, (33, 33, 157), 25.0),      # more cells than fit beside the far kernel's other workgroups
+    (200, (33, 33, 33), 18.0),       # one part: the usual order
+])
+def test_far_field_first(base, n, n1, edge):
+    """A map set on the device and one copied to the host take the far field
+    in other places of the same sum."""
+    print(f"[gpu] far first {n} {n1}", flush=True)
+    st = state(base, n, n1, edge, n)
+    with ag.Context(0) as ctx:
+        host = np.asarray(ctx.maps_plain(st)).reshape(-1)
+        blank = np.full(host.size, np.nan, np.float32)
+        with ctx.plan(st) as plan, Dev(host.nbytes) as out:
+            for _ in range(3):
+                out.put(blank)
+                plan.execute(out.p.value)
+                assert np.array_equal(out.get(host.size), host)
+            t = ctx.timing()
+    assert all(v >= 0.0 for v in t.values()) and max(t.values()) < 1e3
+
+
+def test_more_plans_than_reports(base):
+    """Plans past the 64 that a context has reports for keep their flag on the
+    device; a report given back is used again."""
+    print("[gpu] plans without reports", flush=True)
+    st = state(base, 300, (17, 17, 17), 20.0, 3)
+    n = st.n_maps * st.points
+    with ag.Context(0) as ctx, Dev(4 * n) as out:
+        def run(plan):
+            out.put(np.full(n, np.nan, np.float32))
+            plan.execute(out.p.value)
+            return out.get(n)
+
+        plans = [ctx.plan(st) for _ in range(66)]
+        first = run(plans[0])
+        assert np.isfinite(first).all()
+        assert all(np.array_equal(run(p), first) for p in plans[1:])
+        plans[3].close()
+        plans.append(ctx.plan(st))
+        assert np.array_equal(run(plans[-1]), first)
+        for p in plans:
+            p.close()
