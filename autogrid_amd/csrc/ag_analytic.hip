@@ -1408,9 +1408,11 @@ struct ag_analytic {
     std::vector<ag::BondRecipe> recipes;
     std::vector<int> h_atoms, atom_list;
     // device
-    DevBuf d_atoms, d_by_index, d_rv, d_cells, d_pairs, d_near_pairs, d_eatoms, d_closest, d_amin, d_amax, d_vh, d_hout,
-        d_hatoms, d_alist, d_aout, d_partial, d_eout, d_fatoms, d_epart, d_gcount, d_gpack, d_vcount, d_vpack,
-        d_gmask;
+    DevBuf d_up, d_eup, d_closest, d_amin, d_amax, d_vh, d_hout, d_aout, d_partial, d_eout, d_epart, d_gcount, d_gpack,
+        d_vcount, d_vpack, d_gmask;
+    HostStage stage;                   // pinned: parameters up, gradients' sums down
+    const AAtom *by_index = nullptr;   // in d_up
+    const int *hatoms_d = nullptr, *alist_d = nullptr;
     int eK = 16;                       // run length of the forward e kernel
     AParams ap{};
     EParams ep{};
@@ -1521,12 +1523,102 @@ void analytic_set(ag_analytic *a, const double *coord, const double *charge, con
     a->uploaded = false;
 }
 
-// Host precompute and upload of everything the kernels read.
-static void analytic_upload(ag_analytic *a) {
-    ag_ctx *c = a->ctx;
-    hipStream_t st = c->stream;
+// Arrays on their way up, packed one after the other in pinned memory and
+// copied to one device block.
+struct UploadPack {
+    char *host, *dev;
+    size_t used = 0;
+    static size_t padded(size_t bytes) { return (bytes + 255) & ~(size_t)255; }
+    template <typename T>
+    T *add(size_t n, const T **on_device) {
+        T *h = reinterpret_cast<T *>(host + used);
+        *on_device = reinterpret_cast<const T *>(dev + used);
+        used += padded(sizeof(T) * n);
+        return h;
+    }
+    void copy(hipStream_t st) const {
+        if (used) HIP_CHECK(hipMemcpyAsync(dev, host, used, hipMemcpyHostToDevice, st));
+    }
+};
+
+static void cell_grid(const ag_grid &g, float corg[3], int nc[3]) {   // over the box padded by 8 A
+    for (int d = 0; d < 3; d++) {
+        const double lo = -g.ne[d] * g.spacing - 8.1, hi = (g.n1[d] - 1 - g.ne[d]) * g.spacing + 8.1;
+        corg[d] = (float)lo;
+        nc[d] = (int)std::ceil((hi - lo) / kCellA) + 1;
+    }
+}
+
+// Bytes that upload_e and upload_near pack at most.
+static size_t upload_e_bytes(const ag_analytic *a) {
+    return 2 * UploadPack::padded(sizeof(float4) * (size_t)std::max(a->N, 1));
+}
+static size_t upload_near_bytes(const ag_analytic *a) {
+    const size_t n = (size_t)std::max(a->N, 1), t = (size_t)std::max(a->T, 1), k = (size_t)std::max(a->naff, 1);
+    float corg[3];
+    int nc[3];
+    cell_grid(a->grid, corg, nc);
+    const auto pad = UploadPack::padded;
+    return 2 * pad(sizeof(AAtom) * n) + pad(sizeof(float) * 3 * n) +
+           pad(sizeof(int) * ((size_t)nc[0] * nc[1] * nc[2] + 1)) + pad(sizeof(APair) * k * t) +
+           pad(sizeof(ANearType) * t) + 2 * pad(sizeof(int) * n);
+}
+
+static void check_pairs(const ag_analytic *a) {
+    for (int k = 0; k < a->naff; k++)
+        for (int t = 0; t < a->T; t++) {
+            const ag_pair &pf = a->pair_form[(size_t)a->aff_slot[k] * a->T + t];
+            if (pf.xA == pf.xB || pf.xA <= 0 || pf.xB <= 0)
+                ag::fail(AG_ERR_BAD_INPUT, "pair exponents must differ and be positive");
+        }
+}
+
+// What the electrostatic kernels read: needs the coordinates and charges only.
+static void upload_e(ag_analytic *a, UploadPack up) {
+    const int N = a->N;
+    const ag_grid &g = a->grid;
+    EParams &e = a->ep;
+    memset(&e, 0, sizeof e);
+    float4 *const eat = up.add<float4>(std::max(N, 1), &e.atoms);
+    for (int i = 0; i < N; i++)
+        eat[i] = make_float4((float)a->coord[3 * i], (float)a->coord[3 * i + 1], (float)a->coord[3 * i + 2],
+                             (float)(a->charge[i] * a->w[2]));
+    // the forward's atoms: coordinates scaled by cs, weights with the
+    // electrostatic constants (k_an_e)
+    const double cs = a->dddiel ? (double)kMsLB * 1.4426950408889634 : 1.0;
+    const double wk = a->dddiel ? 332.0 * cs : a->inv_diel;
+    float4 *const fat = up.add<float4>(std::max(N, 1), &e.fatoms);
+    for (int i = 0; i < N; i++)
+        fat[i] = make_float4((float)(cs * a->coord[3 * i]), (float)(cs * a->coord[3 * i + 1]),
+                             (float)(cs * a->coord[3 * i + 2]), (float)(a->charge[i] * a->w[2] * wk));
+    for (int d = 0; d < 3; d++) {
+        e.n1[d] = g.n1[d];
+        e.ne[d] = g.ne[d];
+    }
+    e.h = (float)g.spacing;
+    e.P = a->P;
+    e.n_atoms = N;
+    e.dddiel = a->dddiel;
+    e.inv_diel = (float)a->inv_diel;
+    e.sc = (float)(cs * g.spacing);
+    e.rcap = (float)(2.0 / cs);
+    e.echunk = std::max(kEAtoms, (N + kEMaxChunks - 1) / kEMaxChunks);
+    e.nechunks = std::max(1, (N + e.echunk - 1) / e.echunk);
+    e.epart = (float *)a->d_epart.get(sizeof(float) * (size_t)e.nechunks * (size_t)a->P);
+    // run length: 13 or 16 points, whichever leaves fewer idle run slots
+    a->eK = 13 * ((g.n1[0] + 12) / 13) < 16 * ((g.n1[0] + 15) / 16) ? 13 : 16;
+    a->nchunks = (int)((a->P + kEAdjChunk - 1) / kEAdjChunk);
+    e.nchunks = a->nchunks;
+    e.partial = (float4 *)a->d_partial.get(sizeof(float4) * (size_t)a->nchunks * std::max(N, 1));
+    up.copy(a->ctx->stream);
+}
+
+// Host precompute and upload of everything the near kernel and the adjoint read.
+static void upload_near(ag_analytic *a, UploadPack up) {
     const int N = a->N, T = a->T;
     const ag_grid &g = a->grid;
+    AParams &p = a->ap;
+    memset(&p, 0, sizeof p);
     // bond vectors with their construction recipes
     a->rexp.assign(N, 0);
     a->rv.assign(3 * (size_t)N, 0.0);
@@ -1535,17 +1627,14 @@ static void analytic_upload(ag_analytic *a) {
     a->recipes.assign(N, ag::BondRecipe{});
     ag::build_bond_vectors(a->setup, N, a->coord.data(), a->type.data(), a->hbond.data(), a->rexp.data(),
                            a->rv.data(), a->rv2.data(), a->dis.data(), nullptr, a->recipes.data());
-    // cells over the box padded by 8 A
     float corg[3];
     int nc[3];
-    for (int d = 0; d < 3; d++) {
-        const double lo = -g.ne[d] * g.spacing - 8.1, hi = (g.n1[d] - 1 - g.ne[d]) * g.spacing + 8.1;
-        corg[d] = (float)lo;
-        nc[d] = (int)std::ceil((hi - lo) / kCellA) + 1;
-    }
+    cell_grid(g, corg, nc);
     const int ncells = nc[0] * nc[1] * nc[2];
-    std::vector<int> cell_of(N, -1), count(ncells + 1, 0);
-    std::vector<AAtom> by_index(N);
+    std::vector<int> cell_of(N, -1);
+    int *const count = up.add<int>(ncells + 1, &p.cell_start);
+    std::fill(count, count + ncells + 1, 0);
+    AAtom *const by_index = up.add<AAtom>(N, &a->by_index);
     for (int i = 0; i < N; i++) {
         AAtom &t = by_index[i];
         memset(&t, 0, sizeof t);
@@ -1574,26 +1663,25 @@ static void analytic_upload(ag_analytic *a) {
         }
     }
     for (int k = 0; k < ncells; k++) count[k + 1] += count[k];
-    std::vector<AAtom> sorted(count[ncells]);
+    AAtom *const sorted = up.add<AAtom>(count[ncells], &p.atoms);
     {
-        std::vector<int> cur(count.begin(), count.end() - 1);
+        std::vector<int> cur(count, count + ncells);
         for (int i = 0; i < N; i++)   // atom index order within each cell
             if (cell_of[i] >= 0) sorted[cur[cell_of[i]]++] = by_index[i];
     }
-    std::vector<float> rvf(3 * (size_t)std::max(N, 1), 0.f);
+    float *const rvf = up.add<float>(3 * (size_t)std::max(N, 1), &p.rv_by_index);
     for (size_t k = 0; k < 3 * (size_t)N; k++) rvf[k] = (float)a->rv[k];
     // pair potentials of the affinity maps, effective eps
-    std::vector<APair> pairs((size_t)std::max(a->naff, 1) * std::max(T, 1));
+    const size_t npairs = (size_t)std::max(a->naff, 1) * std::max(T, 1);
+    APair *const pairs = up.add<APair>(npairs, &p.pairs);
+    memset(pairs, 0, sizeof(APair) * npairs);
     for (int k = 0; k < a->naff; k++)
         for (int t = 0; t < T; t++) {
             const int m = a->aff_slot[k];
             const ag_pair &pf = a->pair_form[(size_t)m * T + t];
             APair &pp = pairs[(size_t)k * T + t];
-            memset(&pp, 0, sizeof pp);
             pp.a = pf.xA;
             pp.b = pf.xB;
-            if (pf.xA == pf.xB || pf.xA <= 0 || pf.xB <= 0)
-                ag::fail(AG_ERR_BAD_INPUT, "pair exponents must differ and be positive");
             if (pf.cA == 0 && pf.cB == 0) {
                 pp.R = (float)a->rij[(size_t)m * T + t];
                 pp.eps = (float)(a->eps0[(size_t)m * T + t] * (pf.hbonder ? a->w[1] : a->w[0]));
@@ -1606,8 +1694,8 @@ static void analytic_upload(ag_analytic *a) {
                 pp.expl = 1;
             }
         }
-    std::vector<ANearType> near_pairs((size_t)std::max(T, 1));
-    memset(near_pairs.data(), 0, sizeof(ANearType) * near_pairs.size());
+    ANearType *const near_pairs = up.add<ANearType>(std::max(T, 1), &p.near_pairs);
+    memset(near_pairs, 0, sizeof(ANearType) * std::max(T, 1));
     for (int k = 0; k < a->naff; k++)
         for (int t = 0; t < T; t++) {
             const APair &pp = pairs[(size_t)k * T + t];
@@ -1622,18 +1710,6 @@ static void analytic_upload(ag_analytic *a) {
             nt.b[k] = pp.b;
             nt.form |= (pp.a == 12 && pp.b == 6 ? 0 : pp.a == 12 && pp.b == 10 ? 1 : 2) << (2 * k);
         }
-    std::vector<float4> eat(std::max(N, 1));
-    for (int i = 0; i < N; i++)
-        eat[i] = make_float4((float)a->coord[3 * i], (float)a->coord[3 * i + 1], (float)a->coord[3 * i + 2],
-                             (float)(a->charge[i] * a->w[2]));
-    // the forward's atoms: coordinates scaled by cs, weights with the
-    // electrostatic constants (k_an_e)
-    const double cs = a->dddiel ? (double)kMsLB * 1.4426950408889634 : 1.0;
-    const double wk = a->dddiel ? 332.0 * cs : a->inv_diel;
-    std::vector<float4> fat(std::max(N, 1));
-    for (int i = 0; i < N; i++)
-        fat[i] = make_float4((float)(cs * a->coord[3 * i]), (float)(cs * a->coord[3 * i + 1]),
-                             (float)(cs * a->coord[3 * i + 2]), (float)(a->charge[i] * a->w[2] * wk));
     // donor H atoms and atoms whose 8 A sphere meets the box (adjoint work lists)
     a->h_atoms.clear();
     a->atom_list.clear();
@@ -1647,13 +1723,8 @@ static void analytic_upload(ag_analytic *a) {
         a->atom_list.push_back(i);
         if (a->hbond[i] == AG_HB_D1 || a->hbond[i] == AG_HB_DS) a->h_atoms.push_back(i);
     }
-    auto up = [&](DevBuf &b, const void *src, size_t bytes) {
-        void *d = b.get(bytes);
-        if (bytes) HIP_CHECK(hipMemcpyAsync(d, src, bytes, hipMemcpyHostToDevice, st));
-        return d;
-    };
-    AParams &p = a->ap;
-    memset(&p, 0, sizeof p);
+    std::copy(a->h_atoms.begin(), a->h_atoms.end(), up.add<int>(a->h_atoms.size(), &a->hatoms_d));
+    std::copy(a->atom_list.begin(), a->atom_list.end(), up.add<int>(a->atom_list.size(), &a->alist_d));
     for (int d = 0; d < 3; d++) {
         p.n1[d] = g.n1[d];
         p.ne[d] = g.ne[d];
@@ -1662,10 +1733,6 @@ static void analytic_upload(ag_analytic *a) {
     }
     p.h = (float)g.spacing;
     p.P = a->P;
-    p.cell_start = (const int *)up(a->d_cells, count.data(), sizeof(int) * count.size());
-    p.atoms = (const AAtom *)up(a->d_atoms, sorted.data(), sizeof(AAtom) * sorted.size());
-    up(a->d_by_index, by_index.data(), sizeof(AAtom) * by_index.size());
-    p.rv_by_index = (const float *)up(a->d_rv, rvf.data(), sizeof(float) * rvf.size());
     p.n_atoms = N;
     p.naff = a->naff;
     for (int k = 0; k < a->naff; k++) {
@@ -1682,8 +1749,6 @@ static void analytic_upload(ag_analytic *a) {
     p.cov_hw = a->cov_hw;
     p.cov_barrier = a->cov_barrier;
     p.d_slot = a->dsolv;
-    p.pairs = (const APair *)up(a->d_pairs, pairs.data(), sizeof(APair) * pairs.size());
-    p.near_pairs = (const ANearType *)up(a->d_near_pairs, near_pairs.data(), sizeof(ANearType) * near_pairs.size());
     for (int h = 0; h < 7; h++)
         for (int k = 0; k < a->naff; k++) p.case_word[h] |= a->cases[k][h] << (2 * k);
     p.T = T;
@@ -1694,33 +1759,7 @@ static void analytic_upload(ag_analytic *a) {
     p.amin = (int *)a->d_amin.get(sizeof(int) * (size_t)a->P * std::max(a->naff, 1));
     p.amax = (int *)a->d_amax.get(sizeof(int) * (size_t)a->P * std::max(a->naff, 1));
     p.vh = (float *)a->d_vh.get(sizeof(float) * 3 * (size_t)a->P);
-    EParams &e = a->ep;
-    memset(&e, 0, sizeof e);
-    for (int d = 0; d < 3; d++) {
-        e.n1[d] = g.n1[d];
-        e.ne[d] = g.ne[d];
-    }
-    e.h = (float)g.spacing;
-    e.P = a->P;
-    e.atoms = (const float4 *)up(a->d_eatoms, eat.data(), sizeof(float4) * eat.size());
-    e.n_atoms = N;
-    e.dddiel = a->dddiel;
-    e.inv_diel = (float)a->inv_diel;
-    e.fatoms = (const float4 *)up(a->d_fatoms, fat.data(), sizeof(float4) * fat.size());
-    e.sc = (float)(cs * g.spacing);
-    e.rcap = (float)(2.0 / cs);
-    e.echunk = std::max(kEAtoms, (N + kEMaxChunks - 1) / kEMaxChunks);
-    e.nechunks = std::max(1, (N + e.echunk - 1) / e.echunk);
-    e.epart = (float *)a->d_epart.get(sizeof(float) * (size_t)e.nechunks * (size_t)a->P);
-    // run length: 13 or 16 points, whichever leaves fewer idle run slots
-    a->eK = 13 * ((g.n1[0] + 12) / 13) < 16 * ((g.n1[0] + 15) / 16) ? 13 : 16;
-    a->nchunks = (int)((a->P + kEAdjChunk - 1) / kEAdjChunk);
-    e.nchunks = a->nchunks;
-    e.partial = (float4 *)a->d_partial.get(sizeof(float4) * (size_t)a->nchunks * std::max(N, 1));
-    up(a->d_hatoms, a->h_atoms.data(), sizeof(int) * a->h_atoms.size());
-    up(a->d_alist, a->atom_list.data(), sizeof(int) * a->atom_list.size());
-    HIP_CHECK(hipStreamSynchronize(st));   // host staging goes out of scope
-    a->uploaded = true;
+    up.copy(a->ctx->stream);
 }
 
 static unsigned cube_count(const ag_grid &g) {
@@ -1729,20 +1768,24 @@ static unsigned cube_count(const ag_grid &g) {
     return n;
 }
 
+// The e map needs the coordinates and charges only, so its kernels run while
+// the host makes the bond vectors, cells and pair tables of new parameters
+// (0.5 ms of host work for 5,000 atoms that the device waited for).
 void analytic_forward(ag_analytic *a, float *d_maps) {
     ag_ctx *c = a->ctx;
     HIP_CHECK(hipSetDevice(c->device));
-    if (!a->uploaded) analytic_upload(a);
     hipStream_t st = c->stream;
-    AParams p = a->ap;
-    p.maps = d_maps;
-    const unsigned cubes = cube_count(a->grid);
+    const bool fresh = !a->uploaded;
+    UploadPack eup{}, up{};
+    if (fresh) {
+        check_pairs(a);
+        const size_t eb = upload_e_bytes(a), nb = upload_near_bytes(a);
+        char *stage = (char *)a->stage.get(eb + nb);   // free: every call waits for its copies
+        eup = UploadPack{stage, (char *)a->d_eup.get(eb)};
+        up = UploadPack{stage + eb, (char *)a->d_up.get(nb)};
+        upload_e(a, eup);
+    }
     HIP_CHECK(hipEventRecord(c->ev[0], st));
-    if (a->naff <= 4) k_an_near<4><<<cubes, kAT, 0, st>>>(p);
-    else if (a->naff <= 6) k_an_near<6><<<cubes, kAT, 0, st>>>(p);
-    else k_an_near<8><<<cubes, kAT, 0, st>>>(p);
-    HIP_CHECK(hipGetLastError());
-    HIP_CHECK(hipEventRecord(c->ev[1], st));
     if (a->elec >= 0) {
         EParams e = a->ep;
         e.emap = d_maps + (size_t)a->elec * a->P;
@@ -1758,11 +1801,26 @@ void analytic_forward(ag_analytic *a, float *d_maps) {
         k_an_esum<<<(unsigned)((a->P + 255) / 256), 256, 0, st>>>(e.epart, e.nechunks, a->P, e.emap);
         HIP_CHECK(hipGetLastError());
     }
+    HIP_CHECK(hipEventRecord(c->ev[1], st));
+    try {
+        if (fresh) upload_near(a, up);
+    } catch (...) {
+        (void)hipStreamSynchronize(st);   // the e kernels write the caller's maps
+        throw;
+    }
+    AParams p = a->ap;
+    p.maps = d_maps;
+    const unsigned cubes = cube_count(a->grid);
     HIP_CHECK(hipEventRecord(c->ev[2], st));
+    if (a->naff <= 4) k_an_near<4><<<cubes, kAT, 0, st>>>(p);
+    else if (a->naff <= 6) k_an_near<6><<<cubes, kAT, 0, st>>>(p);
+    else k_an_near<8><<<cubes, kAT, 0, st>>>(p);
+    HIP_CHECK(hipGetLastError());
     HIP_CHECK(hipEventRecord(c->ev[3], st));
     HIP_CHECK(hipStreamSynchronize(st));
-    HIP_CHECK(hipEventElapsedTime(&c->last_ms[1], c->ev[0], c->ev[1]));
-    HIP_CHECK(hipEventElapsedTime(&c->last_ms[2], c->ev[1], c->ev[2]));
+    a->uploaded = true;
+    HIP_CHECK(hipEventElapsedTime(&c->last_ms[1], c->ev[2], c->ev[3]));
+    HIP_CHECK(hipEventElapsedTime(&c->last_ms[2], c->ev[0], c->ev[1]));
     HIP_CHECK(hipEventElapsedTime(&c->last_ms[3], c->ev[0], c->ev[3]));
     c->last_ms[0] = 0.f;
     a->last_maps = d_maps;
@@ -1791,14 +1849,14 @@ void analytic_adjoint(ag_analytic *a, const float *d_dmaps, double *g_coord, dou
         int *counts = (int *)a->d_vcount.get(sizeof(int) * (2 * (size_t)nblk + 1));
         int *vlist = (int *)a->d_vpack.get(sizeof(int) * (size_t)a->P);
         pack_points(NonzeroVh{p.vh}, a->P, counts, counts + nblk, vlist, st);
-        HsumParams hp{p.closest_h, p.vh, vlist, counts + 2 * nblk, (const int *)a->d_hatoms.ptr, d_hout};
+        HsumParams hp{p.closest_h, p.vh, vlist, counts + 2 * nblk, a->hatoms_d, d_hout};
         k_an_hsum<<<nh, kAT, 0, st>>>(hp);
     }
     if (nl > 0) {
         AtomAdjParams q;
         q.a = p;
-        q.by_index = (const AAtom *)a->d_by_index.ptr;
-        q.atom_list = (const int *)a->d_alist.ptr;
+        q.by_index = a->by_index;
+        q.atom_list = a->alist_d;
         q.out = d_aout;
         q.words = (a->grid.n1[0] + 63) / 64;
         const long long words = (long long)q.words * a->grid.n1[1] * a->grid.n1[2];
@@ -1810,7 +1868,16 @@ void analytic_adjoint(ag_analytic *a, const float *d_dmaps, double *g_coord, dou
         else k_an_atom<8><<<nl, kAT, 0, st>>>(q);
     }
     HIP_CHECK(hipGetLastError());
+    // the near sums go to the host, and are worked off there, beside the e adjoint
     const bool want_e = a->elec >= 0 && N > 0;
+    const size_t hb = UploadPack::padded(sizeof(float) * 3 * (size_t)nh), ab = UploadPack::padded(sizeof(float) * kAtomOut * (size_t)nl);
+    char *const stage = (char *)a->stage.get(hb + ab + sizeof(double) * 4 * (size_t)std::max(N, 1));
+    const float *const hout = (const float *)stage, *const aout = (const float *)(stage + hb);
+    const double *const eout = (const double *)(stage + hb + ab);
+    HIP_CHECK(hipEventRecord(c->near_ev, st));
+    HIP_CHECK(hipStreamWaitEvent(c->copy_stream, c->near_ev, 0));
+    if (nh) HIP_CHECK(hipMemcpyAsync(stage, d_hout, sizeof(float) * 3 * (size_t)nh, hipMemcpyDeviceToHost, c->copy_stream));
+    if (nl) HIP_CHECK(hipMemcpyAsync(stage + hb, d_aout, sizeof(float) * kAtomOut * (size_t)nl, hipMemcpyDeviceToHost, c->copy_stream));
     if (want_e) {
         EParams e = a->ep;
         e.ge = d_dmaps + (size_t)a->elec * a->P;
@@ -1826,20 +1893,20 @@ void analytic_adjoint(ag_analytic *a, const float *d_dmaps, double *g_coord, dou
         HIP_CHECK(hipGetLastError());
     }
     HIP_CHECK(hipEventRecord(c->ev[3], st));
-    std::vector<float> hout(3 * (size_t)nh), aout((size_t)kAtomOut * nl);
-    std::vector<double> eout(4 * (size_t)N, 0.0);
-    if (nh) HIP_CHECK(hipMemcpyAsync(hout.data(), d_hout, sizeof(float) * hout.size(), hipMemcpyDeviceToHost, st));
-    if (nl) HIP_CHECK(hipMemcpyAsync(aout.data(), d_aout, sizeof(float) * aout.size(), hipMemcpyDeviceToHost, st));
-    if (want_e) HIP_CHECK(hipMemcpyAsync(eout.data(), d_eout, sizeof(double) * eout.size(), hipMemcpyDeviceToHost, st));
-    HIP_CHECK(hipStreamSynchronize(st));
-    HIP_CHECK(hipEventElapsedTime(&c->last_ms[3], c->ev[0], c->ev[3]));
+    if (want_e) HIP_CHECK(hipMemcpyAsync(stage + hb + ab, d_eout, sizeof(double) * 4 * (size_t)N, hipMemcpyDeviceToHost, st));
+    // (an exception would leave the e adjoint's copy without its target)
+    struct Join {
+        hipStream_t st;
+        ~Join() { (void)hipStreamSynchronize(st); }
+    } join{st};
+    HIP_CHECK(hipStreamSynchronize(c->copy_stream));
     // assemble in FP64
     std::vector<double> gx(3 * (size_t)N, 0.0), grv(3 * (size_t)N, 0.0), grv2(3 * (size_t)N, 0.0), gq(N, 0.0);
     std::vector<double> gR((size_t)M * T, 0.0), gE((size_t)M * T, 0.0);
     double gwd = 0.0;
     for (int l = 0; l < nl; l++) {
         const int i = a->atom_list[l];
-        const float *o = aout.data() + (size_t)l * kAtomOut;
+        const float *o = aout + (size_t)l * kAtomOut;
         for (int k = 0; k < 3; k++) {
             gx[3 * i + k] += o[k];
             grv[3 * i + k] += o[3 + k];
@@ -1857,16 +1924,18 @@ void analytic_adjoint(ag_analytic *a, const float *d_dmaps, double *g_coord, dou
         const int h = a->h_atoms[l];
         for (int k = 0; k < 3; k++) grv[3 * h + k] += hout[3 * l + k];
     }
+    // bond vectors -> coordinates
+    ag::bond_vectors_vjp(N, a->coord.data(), a->recipes.data(), grv.data(), grv2.data(), gx.data());
+    HIP_CHECK(hipStreamSynchronize(st));
+    HIP_CHECK(hipEventElapsedTime(&c->last_ms[3], c->ev[0], c->ev[3]));
     double gwe = 0.0;
-    for (int i = 0; i < N; i++) {
+    for (int i = 0; want_e && i < N; i++) {
         // eout: d/dx of sum_p g q w f (the float4 weight holds q w), and
         // sum_p g f
         for (int k = 0; k < 3; k++) gx[3 * i + k] += eout[4 * i + k];
         gq[i] += a->w[2] * eout[4 * i + 3];
         gwe += a->charge[i] * eout[4 * i + 3];
     }
-    // bond vectors -> coordinates
-    ag::bond_vectors_vjp(N, a->coord.data(), a->recipes.data(), grv.data(), grv2.data(), gx.data());
     // effective eps -> unweighted eps and the vdW / H-bond weights
     double gwv = 0.0, gwh = 0.0;
     for (int m = 0; m < M; m++)
