@@ -14,7 +14,7 @@
 //   k_score      one workgroup per pose, lanes over its atoms: per-atom
 //                energy and gradient dE/dx, the pose's sum reduced in FP64
 //                in a fixed order;
-//   k_score_place, k_sort_count / _scan / _scatter
+//   k_score_place, k_sort_zero / _scan / _scatter
 //                new positions: each atom's place on the grid, and its eight
 //                corners sorted by grid point and by (map, grid point), a
 //                stable radix sort, so equal keys stay in atom order;
@@ -109,6 +109,48 @@ __global__ void k_score_zero(float *out, long long n) {
         out[i] = 0.f;
 }
 
+// One pass of a stable radix sort of (key, entry) pairs by eight bits: with the
+// tiles' digit counts known, each pair's place is that of its digit (a digit's
+// tiles follow each other).  A digit comes from the key, or from the entry's
+// atom's map (map + 1, so that atoms without one go first).  Whoever places a
+// pair counts it for the next pass, so a pass is one launch, which up to
+// kSortScanned tiles also adds up the counts itself (each workgroup all of
+// them, from the L2 cache).  10,000 atoms, 80,000 pairs: 39 us for all four
+// passes; as three launches each (count, scan, scatter) 66 us and the gaps
+// between.  (Pairs a workgroup has spread go out one cache line a clock: 40
+// workgroups of 2,048 take 9.5 us a pass, ten of 8,192 15.)  The host's sort of the 250,000 contributions and their upload took
+// 5.4 ms.
+constexpr int kSortThreads = 512, kSortPer = 4;
+constexpr int kSortTile = kSortThreads * kSortPer;   // pairs of a workgroup
+constexpr int kSortScanned = 64;
+
+// The digits of a pass and its counts.
+struct SortDigit {
+    const ScoreAtom *by_map;    // null: the digit is (key >> shift) & 255
+    int shift;
+    int *count;                 // [tiles][256]; null: no pass
+};
+struct SortPass {
+    const uint2 *pair;          // (key, entry)
+    uint2 *pair_out;
+    int n, tiles;
+    int scanned;                // the counts have been through k_sort_scan
+    SortDigit digit, next;
+    int *clear;                 // the counts of the pass before, left clear for the next sort
+};
+__device__ __forceinline__ int sort_digit(const SortDigit &p, uint2 pair) {
+    return p.by_map ? p.by_map[pair.y >> 3].map + 1 : (int)((pair.x >> p.shift) & 255u);
+}
+__device__ __forceinline__ void sort_count(const SortDigit &p, uint2 pair, int place) {
+    atomicAdd(&p.count[place / kSortTile * 256 + sort_digit(p, pair)], 1);
+}
+
+// Clears the counts of all passes, before a scorer's first sort.
+__global__ void __launch_bounds__(kST) k_sort_zero(int *count, int n) {
+    const int i = blockIdx.x * kST + threadIdx.x;
+    if (i < n) count[i] = 0;
+}
+
 struct PlaceParams {
     const double *xyz;          // [n][3]
     const float *charge;
@@ -118,12 +160,15 @@ struct PlaceParams {
     double shift[3], spacing;   // ne * spacing
     unsigned P;                 // grid points; the key of an atom off the grid
     ScoreAtom *atoms;
-    unsigned *key;              // [8 n] corner's grid point
-    int *entry;                 // [8 n] atom * 8 + corner
+    uint2 *pair;                // [8 n] (corner's grid point, atom * 8 + corner)
+    SortDigit first;            // of the sort
+    int *clear;                 // counts of the last sort's last pass, 256 per 256 atoms
 };
 
 __global__ void __launch_bounds__(kST) k_score_place(PlaceParams p) {
     const int a = blockIdx.x * kST + threadIdx.x;
+    static_assert(kSortTile == 8 * kST && kST == 256, "a workgroup's corners are a tile");
+    p.clear[a] = 0;
     if (a >= p.n) return;
     double g[3];
     bool inside = true;
@@ -150,44 +195,10 @@ __global__ void __launch_bounds__(kST) k_score_place(PlaceParams p) {
                                          (unsigned)p.n1[0] * ((unsigned)(j0 + ((c >> 1) & 1)) +
                                                               (unsigned)p.n1[1] * (unsigned)(k0 + (c >> 2)))
                                    : p.P;
-        p.key[8 * (size_t)a + c] = pt;
-        p.entry[8 * (size_t)a + c] = 8 * a + c;
+        const uint2 pair = make_uint2(pt, 8u * a + c);
+        p.pair[8 * (size_t)a + c] = pair;
+        sort_count(p.first, pair, 8 * a + c);
     }
-}
-
-// One pass of a stable radix sort of (key, entry) pairs by eight bits: the
-// blocks' digit counts, their places in the output (a digit's blocks follow
-// each other), and the scatter.  A digit comes from the key, or from the entry's
-// atom's map (map + 1, so that atoms without one go first).  10,000 atoms, 80,000
-// pairs: about 11 us a pass, launches and their latency; the host's sort of the
-// 250,000 contributions and their upload took 5.4 ms.
-constexpr int kSortTile = 2048;   // pairs per block
-constexpr int kSortPer = kSortTile / kST;
-
-struct SortPass {
-    const unsigned *key;
-    const int *entry;
-    unsigned *key_out;
-    int *entry_out;
-    int n, shift;
-    const ScoreAtom *by_map;    // null: the digit is (key >> shift) & 255
-    int *count;                 // [blocks][256], then the first place of each
-};
-__device__ __forceinline__ int sort_digit(const SortPass &p, unsigned key, int entry) {
-    return p.by_map ? p.by_map[entry >> 3].map + 1 : (int)((key >> p.shift) & 255u);
-}
-
-__global__ void __launch_bounds__(kST) k_sort_count(SortPass p) {
-    __shared__ int bin[256];
-    bin[threadIdx.x] = 0;
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < kSortPer; r++) {
-        const int i = blockIdx.x * kSortTile + r * kST + threadIdx.x;
-        if (i < p.n) atomicAdd(&bin[sort_digit(p, p.key[i], p.entry[i])], 1);
-    }
-    __syncthreads();
-    p.count[blockIdx.x * 256 + threadIdx.x] = bin[threadIdx.x];
 }
 
 // count[b][d] -> pairs of smaller digits plus digit d's of earlier blocks.  One
@@ -220,34 +231,72 @@ __global__ void __launch_bounds__(1024) k_sort_scan(int *count, int blocks) {
     }
 }
 
-// A wave takes a quarter of the block's tile in order: its digits' counts first,
+// A wave takes its part of the workgroup's tile in order: its digits' counts first,
 // then, with the waves' places known, 64 pairs at a time without a barrier.
-__global__ void __launch_bounds__(kST) k_sort_scatter(SortPass p) {
-    __shared__ int place[kST / 64][256];   // next free place per wave and digit
+__global__ void __launch_bounds__(kSortThreads) k_sort_scatter(SortPass p) {
+    constexpr int kWaves = kSortThreads / 64;
+    __shared__ int place[kWaves][256];   // next free place per wave and digit
+    __shared__ int wave_sum[kWaves];
+    __shared__ int2 other[256];
+    // counts for the next pass: many pairs may share one (few digits, or one
+    // map's atoms), so they are added up here before they go to memory
+    __shared__ int ahead[kSortScanned * 256];
+    const bool gather_ahead = p.next.count && p.tiles <= kSortScanned;
+    if (p.clear && threadIdx.x < 256) p.clear[blockIdx.x * 256 + threadIdx.x] = 0;
+    if (gather_ahead)
+        for (int k = threadIdx.x; k < p.tiles * 256; k += kSortThreads) ahead[k] = 0;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (int w = 0; w < kST / 64; w++) place[w][threadIdx.x] = 0;
+    const int d = threadIdx.x & 255;
+    for (int w = threadIdx.x >> 8; w < kWaves; w += kSortThreads / 256) place[w][d] = 0;
+    int run = 0;   // the tile's first place of digit d
+    if (p.scanned) {
+        run = p.digit.count[blockIdx.x * 256 + d];
+    } else {
+        // two threads per digit, every other tile each
+        static_assert(kSortThreads == 512, "two threads per digit");
+        const int half = threadIdx.x >> 8;
+        int total = 0;
+#pragma unroll 16
+        for (int b = half; b < p.tiles; b += 2) {
+            const int c = p.digit.count[b * 256 + d];
+            total += c;
+            run += b < (int)blockIdx.x ? c : 0;
+        }
+        if (half) other[d] = make_int2(total, run);
+        __syncthreads();
+        total += other[d].x;
+        run += other[d].y;
+        int x = total;   // (the lower half's; the upper half's are not used)
+        for (int o = 1; o < 64; o <<= 1) {
+            const int y = __shfl_up(x, o);
+            if (lane >= o) x += y;
+        }
+        if (lane == 63 && !half) wave_sum[wave] = x;
+        __syncthreads();
+        run += x - total;
+        for (int w = 0; w < (d >> 6); w++) run += wave_sum[w];
+    }
     __syncthreads();
-    unsigned key[kSortPer];
-    int entry[kSortPer], digit[kSortPer];
+    uint2 pair[kSortPer];
+    int digit[kSortPer];
     const int first = blockIdx.x * kSortTile + wave * (kSortPer * 64) + lane;
 #pragma unroll
     for (int r = 0; r < kSortPer; r++) {
         const int i = first + 64 * r;
         digit[r] = -1;
         if (i < p.n) {
-            key[r] = p.key[i];
-            entry[r] = p.entry[i];
-            digit[r] = sort_digit(p, key[r], entry[r]);
+            pair[r] = p.pair[i];
+            digit[r] = sort_digit(p.digit, pair[r]);
             atomicAdd(&place[wave][digit[r]], 1);
         }
     }
     __syncthreads();
-    int run = p.count[blockIdx.x * 256 + threadIdx.x];
-    for (int w = 0; w < kST / 64; w++) {
-        const int c = place[w][threadIdx.x];
-        place[w][threadIdx.x] = run;
-        run += c;
-    }
+    if (threadIdx.x < 256)
+        for (int w = 0; w < kWaves; w++) {
+            const int c = place[w][d];
+            place[w][d] = run;
+            run += c;
+        }
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < kSortPer; r++) {
@@ -263,12 +312,20 @@ __global__ void __launch_bounds__(kST) k_sort_scatter(SortPass p) {
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // every lane has read its place
         __builtin_amdgcn_wave_barrier();
         if (act) {
-            p.key_out[at + rank] = key[r];
-            p.entry_out[at + rank] = entry[r];
+            p.pair_out[at + rank] = pair[r];
+            if (gather_ahead)
+                atomicAdd(&ahead[(at + rank) / kSortTile * 256 + sort_digit(p.next, pair[r])], 1);
+            else if (p.next.count)
+                sort_count(p.next, pair[r], at + rank);
             if (rank == 0) place[wave][dg] = at + __popcll(same);
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
+    }
+    if (gather_ahead) {
+        __syncthreads();
+        for (int k = threadIdx.x; k < p.tiles * 256; k += kSortThreads)
+            if (ahead[k]) atomicAdd(&p.next.count[k], ahead[k]);
     }
 }
 
@@ -280,10 +337,8 @@ struct AdjParams {
     const ScoreAtom *atoms;
     int n;                      // entries, 8 per atom
     unsigned P;
-    const unsigned *key;        // sorted by grid point
-    const int *entry;
-    const unsigned *mkey;       // sorted by map, then grid point
-    const int *mentry;
+    const uint2 *pair;          // (grid point, entry) sorted by grid point
+    const uint2 *mpair;         // sorted by map, then grid point
     int e_slot, d_slot;
     const float *dscore;
     float *dmaps;
@@ -297,11 +352,11 @@ __global__ void __launch_bounds__(kST) k_score_adj(AdjParams p) {
     const int i = blockIdx.x * kST + threadIdx.x;
     if (i >= p.n) return;
     if (blockIdx.y == 0) {
-        const unsigned pt = p.key[i];
-        if (pt >= p.P || (i > 0 && p.key[i - 1] == pt)) return;
+        const unsigned pt = p.pair[i].x;
+        if (pt >= p.P || (i > 0 && p.pair[i - 1].x == pt)) return;
         double se = 0.0, sd = 0.0;
-        for (int k = i; k < p.n && p.key[k] == pt; k++) {
-            const int en = p.entry[k];
+        for (int k = i; k < p.n && p.pair[k].x == pt; k++) {
+            const int en = (int)p.pair[k].y;
             const ScoreAtom at = p.atoms[en >> 3];
             const float w = corner_weight(at, en & 7);
             const double g = (double)p.dscore[at.pose];
@@ -317,13 +372,13 @@ __global__ void __launch_bounds__(kST) k_score_adj(AdjParams p) {
         if (p.e_slot >= 0) p.dmaps[(size_t)p.e_slot * p.P + pt] = (float)se;
         if (p.d_slot >= 0 && p.d_slot != p.e_slot) p.dmaps[(size_t)p.d_slot * p.P + pt] = (float)sd;
     } else {
-        const unsigned pt = p.mkey[i];
-        const int m = p.atoms[p.mentry[i] >> 3].map;
+        const unsigned pt = p.mpair[i].x;
+        const int m = p.atoms[p.mpair[i].y >> 3].map;
         if (pt >= p.P || m < 0 || m == p.e_slot || m == p.d_slot) return;
-        if (i > 0 && p.mkey[i - 1] == pt && p.atoms[p.mentry[i - 1] >> 3].map == m) return;
+        if (i > 0 && p.mpair[i - 1].x == pt && p.atoms[p.mpair[i - 1].y >> 3].map == m) return;
         double s = 0.0;
-        for (int k = i; k < p.n && p.mkey[k] == pt; k++) {
-            const int en = p.mentry[k];
+        for (int k = i; k < p.n && p.mpair[k].x == pt; k++) {
+            const int en = (int)p.mpair[k].y;
             const ScoreAtom at = p.atoms[en >> 3];
             if (at.map != m) break;
             s += (double)corner_weight(at, en & 7) * (double)p.dscore[at.pose];
@@ -346,7 +401,8 @@ struct ag_scorer {
     std::vector<int> map_index;
     std::vector<double> charge;
     DevBuf atoms, pose_start_d, xyz, charge_d, map_d, pose_d;
-    DevBuf key[3], entry[3], count;
+    DevBuf pair[3], count;
+    bool counts_clear = false;      // every pass's counts but the last's are clear
     int by_point = 0, by_map = 0;   // buffers holding the two sorted lists
 };
 
@@ -375,36 +431,45 @@ static void scorer_positions(ag_scorer *s, const double *xyz) {
     pp.atoms = (ScoreAtom *)s->atoms.get(sizeof(ScoreAtom) * (size_t)n);
     const int blocks = (int)((n8 + kSortTile - 1) / kSortTile);
     for (int k = 0; k < 3; k++) {
-        s->key[k].get(sizeof(unsigned) * n8);
-        s->entry[k].get(sizeof(int) * n8);
+        s->pair[k].get(sizeof(uint2) * n8);
     }
-    int *count = (int *)s->count.get(sizeof(int) * 256 * (size_t)std::max(blocks, 1));
+    // the passes: by grid point, eight bits at a time, then by map
+    SortDigit digit[6] = {};
+    int passes = 0;
+    const size_t counts = 256 * (size_t)std::max(blocks, 1);
+    int *count = (int *)s->count.get(sizeof(int) * counts * 5);
+    for (int shift = 0; shift < 32 && ((unsigned long long)s->P >> shift) > 0; shift += 8)
+        digit[passes++] = SortDigit{nullptr, shift, nullptr};
+    digit[passes++] = SortDigit{pp.atoms, 0, nullptr};
+    for (int k = 0; k < passes; k++) digit[k].count = count + counts * k;
     if (n == 0) return;
     // pinned staging: one DMA instead of the runtime's own staged copy
     void *stage = s->ctx->stage.get(sizeof(double) * 3 * (size_t)n);
     memcpy(stage, xyz, sizeof(double) * 3 * (size_t)n);
     HIP_CHECK(hipMemcpyAsync(s->xyz.ptr, stage, sizeof(double) * 3 * (size_t)n, hipMemcpyHostToDevice, st));
-    pp.key = (unsigned *)s->key[0].ptr;
-    pp.entry = (int *)s->entry[0].ptr;
+    pp.pair = (uint2 *)s->pair[0].ptr;
+    pp.first = digit[0];
+    pp.clear = digit[passes - 1].count;
+    if (!s->counts_clear)
+        k_sort_zero<<<(unsigned)((counts * passes + kST - 1) / kST), kST, 0, st>>>(count, (int)(counts * passes));
+    s->counts_clear = false;
     k_score_place<<<(n + kST - 1) / kST, kST, 0, st>>>(pp);
-    const auto pass = [&](int from, int to, int shift, bool by_map) {
-        SortPass sp{(const unsigned *)s->key[from].ptr, (const int *)s->entry[from].ptr, (unsigned *)s->key[to].ptr,
-                    (int *)s->entry[to].ptr, (int)n8, shift, by_map ? pp.atoms : nullptr, count};
-        k_sort_count<<<blocks, kST, 0, st>>>(sp);
-        k_sort_scan<<<1, 1024, 0, st>>>(count, blocks);
-        k_sort_scatter<<<blocks, kST, 0, st>>>(sp);
-    };
-    int cur = 0;
-    for (int shift = 0; shift < 32 && ((unsigned long long)s->P >> shift) > 0; shift += 8) {
-        pass(cur, 1 - cur, shift, false);
-        cur = 1 - cur;
+    // each pass but the last (by map, from the list by grid point) goes to
+    // and fro between two buffers
+    const bool scan = blocks > kSortScanned;
+    for (int k = 0, from = 0; k < passes; k++, from = 1 - from) {
+        const bool last = k + 1 == passes;
+        const int to = last ? 2 : 1 - from;
+        if (scan) k_sort_scan<<<1, 1024, 0, st>>>(digit[k].count, blocks);
+        k_sort_scatter<<<blocks, kSortThreads, 0, st>>>(SortPass{
+            (const uint2 *)s->pair[from].ptr, (uint2 *)s->pair[to].ptr, (int)n8, blocks, scan, digit[k], digit[k + 1],
+            k > 0 ? digit[k - 1].count : nullptr});
+        if (last) s->by_point = from;
     }
-    s->by_point = cur;
-    // one more pass, by map: (map, grid point) order, from the sorted list
-    pass(cur, 2, 0, true);
     s->by_map = 2;
     HIP_CHECK(hipGetLastError());
     HIP_CHECK(hipStreamSynchronize(st));   // the staging buffer is the context's
+    s->counts_clear = true;
 }
 
 ag_scorer *scorer_create(ag_ctx *c, const ag_grid *grid, int n_maps, int elec_index, int dsolv_index, int n_poses,
@@ -501,9 +566,8 @@ void scorer_adjoint(ag_scorer *s, const float *d_dscore, float *d_dmaps) {
     k_score_zero<<<zb, 256, 0, st>>>(d_dmaps, total);
     if (s->n_atoms > 0) {
         const int n8 = 8 * s->n_atoms;
-        AdjParams p{(const ScoreAtom *)s->atoms.ptr, n8, (unsigned)s->P, (const unsigned *)s->key[s->by_point].ptr,
-                    (const int *)s->entry[s->by_point].ptr, (const unsigned *)s->key[s->by_map].ptr,
-                    (const int *)s->entry[s->by_map].ptr, s->e_slot, s->d_slot, d_dscore, d_dmaps};
+        AdjParams p{(const ScoreAtom *)s->atoms.ptr, n8, (unsigned)s->P, (const uint2 *)s->pair[s->by_point].ptr,
+                    (const uint2 *)s->pair[s->by_map].ptr, s->e_slot, s->d_slot, d_dscore, d_dmaps};
         k_score_adj<<<dim3((unsigned)((n8 + kST - 1) / kST), 2), kST, 0, st>>>(p);
     }
     HIP_CHECK(hipGetLastError());

@@ -124,3 +124,12 @@ def test_moved_positions():
     b = _poses(st, 900, 30, np.random.default_rng(5), spread=1.2)   # some of them off the grid
     moved = [(p[0], p[1], r[2]) for p, r in zip(a, b)]
     _check(st, a, moved=moved)
+
+
+@pytest.mark.parametrize("n", [64 * 256, 64 * 256 + 1])
+def test_sort_tiles(n):
+    """Tiles of 2,048 corners: up to 64 of them, each workgroup adds up the
+    counts itself, and for more a launch of its own does."""
+    print(f"[gpu] scorer lists, {n} atoms", flush=True)
+    st = Grid((41, 43, 47), 5, 3, 4)
+    _check(st, _poses(st, n, 300, np.random.default_rng(n), spread=1.05))
