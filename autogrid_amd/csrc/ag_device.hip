@@ -34,7 +34,6 @@
 #include <cstdio>
 #include <cstring>
 #include <functional>
-#include <type_traits>
 #include <memory>
 #include <string>
 #include <thread>
@@ -1553,11 +1552,20 @@ __global__ void __launch_bounds__(256) k_audit(AuditParams p) {
 // the index there (main.cpp:2956).
 constexpr int kFarLastBin = AG_NDIEL - 1;
 
+// How a far-kernel launch reads its table.
+//   kFarTable   a bin's entry from LDS;
+//   kFarClamped the same, offsets capped at the last entry: for launches where a
+//               conformation's direct pairs may pass it (spacings of about 1 A
+//               and more; the cap changes no other pair's value);
+//   kFarFlat    one value from bin 1025 on (constant dielectric): no table, only
+//               the test for the pairs the near kernel takes, and that only for
+//               atoms near the patch (kFarFlatBeyond: pairs of the others).
+enum : int { kFarTable = 0, kFarClamped = 1, kFarFlat = 2, kFarFlatBeyond = 3 };
+
 // One pair of an atom with the 16 points of a lane's run, accumulated into
 // part[]: the squared distance in bins^2 by the run-centre expansion, rsq,
-// the bin's table offset in one fma and one and, the LDS read (CLAMP caps
-// the offset at the table's last entry).
-template <bool CLAMP>
+// the bin's table offset in one fma and one and, the LDS read.
+template <int KIND>
 __device__ __forceinline__ void far_pair(const PlainF4 &at, float py, float pz, float floor2, float s128, float s2,
                                          const float *T, float *part) {
     const float dy = at.y - py, dz = at.z - pz;
@@ -1574,8 +1582,14 @@ __device__ __forceinline__ void far_pair(const PlainF4 &at, float py, float pz, 
         const int j = k >= kFarK / 2 ? k - kFarK / 2 : kFarK / 2 - 1 - k;
         const float rb2 = __builtin_fmaf(us, far_m(k), W[j]);
         rs[k] = __builtin_amdgcn_rsqf(rb2);
-        off[k] = bin4_of(rb2, rs[k]);
-        if (CLAMP) off[k] = min(off[k], 4u * kFarLastBin);
+        if (KIND == kFarFlat) rs[k] = bin4_of(rb2, rs[k]) >= 4u * kFarBinMin ? rs[k] : 0.f;
+        if (KIND < kFarFlat) off[k] = bin4_of(rb2, rs[k]);
+        if (KIND == kFarClamped) off[k] = min(off[k], 4u * kFarLastBin);
+    }
+    if (KIND >= kFarFlat) {   // the weight holds the table's value
+#pragma unroll
+        for (int k = 0; k < kFarK; k++) part[k] = __builtin_fmaf(at.w, rs[k], part[k]);
+        return;
     }
     float tv[kFarK];
 #pragma unroll
@@ -1664,13 +1678,12 @@ __device__ __forceinline__ void far_wy(double t, double w[4]) {
 // busy) and the table reads in LDS (60 %, 3.9 conflict cycles each) together.
 // Eight waves per workgroup instead of four: 0.94 ms, 9.7 ms on 257^3.
 //
-// CLAMP caps the direct pairs' table offsets at bin 8191: for launches where
-// a conformation's direct pairs may pass it (spacings of about 1 A and more;
-// the cap changes no other pair's value).
+// KIND: kFarTable, kFarClamped or kFarFlat.  Without the table 3,000 atoms on 81^3
+// points take 336 us for 444.
 // CELLS: the launch's first workgroup makes the plan's cell list, which the
 // near kernel will want (small plans, whose parts the near kernel adds up).
 constexpr int kFarLds = AG_NDIEL + 2 * 64 * kFarK;
-template <bool CLAMP, bool CELLS>
+template <int KIND, bool CELLS>
 __global__ void __launch_bounds__(kFarThreads) __attribute__((amdgpu_waves_per_eu(4))) k_far(FarParams p, CellParams cp) {
     // 40 KiB: four workgroups per CU
     __shared__ float lds[kFarLds];
@@ -1682,7 +1695,9 @@ __global__ void __launch_bounds__(kFarThreads) __attribute__((amdgpu_waves_per_e
     if (!CELLS) stamp_start(p.stamp);
     float *const T = lds, *const X = lds + AG_NDIEL;
     static_assert(kFarBinMin == AG_NEINT + 1, "the table's zeros below end one bin into a float4");
-    for (int i = threadIdx.x; i < AG_NDIEL / 4; i += kFarThreads) {
+    constexpr bool FLAT = KIND == kFarFlat;
+    const float flat = FLAT ? as_const(p.tab)[kFarLastBin] : 1.f;
+    for (int i = threadIdx.x; !FLAT && i < AG_NDIEL / 4; i += kFarThreads) {
         float4 v = reinterpret_cast<const float4 *>(p.tab)[i];
         if (i <= AG_NEINT / 4) v.x = 0.f;
         if (i < AG_NEINT / 4) v.y = v.z = v.w = 0.f;
@@ -1734,7 +1749,7 @@ __global__ void __launch_bounds__(kFarThreads) __attribute__((amdgpu_waves_per_e
         float *const level_r2 = X + 4 * 64 * kFarWaves + kFarLevels * wave;   // the wave's copy
         if (lane < kFarLevels) level_r2[lane] = reinterpret_cast<const float *>(&p.confs[ci].far_r2)[lane];
         wave_sync();
-        const float qscale = sreg(cf.far_qscale);
+        const float qscale = sreg(FLAT ? cf.far_qscale / flat : cf.far_qscale);   // (zero charges: any level)
         const FarAtom *const atoms = p.atoms + cf.atom_base;
         const int n_atoms = cf.n_atoms;
         const int step = 64 * kFarWaves * cf.far_split;
@@ -1743,15 +1758,17 @@ __global__ void __launch_bounds__(kFarThreads) __attribute__((amdgpu_waves_per_e
         FarAtom A{};
         if (a_first + lane < n_atoms) A = atoms[a_first + lane];
         for (int a0 = a_first; a0 < n_atoms; a0 += step) {
-            const float4 at = make_float4((float)(A.x - bx), (float)(A.y - by), (float)(A.z - bz), A.w);
+            const float4 at = make_float4((float)(A.x - bx), (float)(A.y - by), (float)(A.z - bz), FLAT ? A.w * flat : A.w);
             if (a0 + step + lane < n_atoms) A = atoms[a0 + step + lane];
             const float ex = fmaxf(fabsf(at.x) - hx, 0.f), ey = fmaxf(fabsf(at.y) - hy, 0.f),
                         ez = fmaxf(fabsf(at.z) - hz, 0.f);
-            const bool beyond =
-                __builtin_fmaf(ex, ex, __builtin_fmaf(ey, ey, ez * ez)) >= level_r2[far_level(at.w * qscale)];
+            const float box2 = __builtin_fmaf(ex, ex, __builtin_fmaf(ey, ey, ez * ez));
+            const bool beyond = box2 >= level_r2[far_level(at.w * qscale)];
             const int nb = min(64, n_atoms - a0);
             const unsigned long long all = nb == 64 ? ~0ull : ((1ull << nb) - 1);
             const unsigned long long far_set = __ballot(beyond) & all;
+            const unsigned long long past =
+                FLAT ? __ballot(box2 >= (float)(kFarBinMin + 1) * (float)(kFarBinMin + 1)) : 0;
             unsigned long long dir_set = ~far_set & all;
             if (far_set) {
                 const int nf = __popcll(far_set);
@@ -1776,11 +1793,12 @@ __global__ void __launch_bounds__(kFarThreads) __attribute__((amdgpu_waves_per_e
 #pragma unroll
                     for (int j = 0; j < kFarNx; j++) {
                         rs[j] = __builtin_amdgcn_rsqf(rb2[j]);
+                        if (FLAT) continue;
                         const unsigned off = min(bin4_of(rb2[j], rs[j]), 4u * kFarLastBin);
                         tv[j] = *reinterpret_cast<const float *>(reinterpret_cast<const char *>(T) + off);
                     }
 #pragma unroll
-                    for (int j = 0; j < kFarNx; j++) np[j] = __builtin_fmaf(q.w, rs[j] * tv[j], np[j]);
+                    for (int j = 0; j < kFarNx; j++) np[j] = __builtin_fmaf(q.w, FLAT ? rs[j] : rs[j] * tv[j], np[j]);
                 }
                 wave_sync();   // the strip is rewritten for the next 64 atoms
                 n_node += nf;
@@ -1799,7 +1817,9 @@ __global__ void __launch_bounds__(kFarThreads) __attribute__((amdgpu_waves_per_e
                     const int i = __builtin_ctzll(dir_set);
                     dir_set &= dir_set - 1;
                     const PlainF4 q{lane_of(at.x, i), lane_of(at.y, i), lane_of(at.z, i), lane_of(at.w, i)};
-                    far_pair<CLAMP>(q, py, pz, floor2, s128, s2, T, part);
+                    // (no point of the box within a bin of the near kernel's pairs)
+                    if (FLAT && ((past >> i) & 1)) far_pair<kFarFlatBeyond>(q, py, pz, floor2, s128, s2, T, part);
+                    else far_pair<KIND>(q, py, pz, floor2, s128, s2, T, part);
                 } while (dir_set);
                 if (n_part >= kFarAtomChunk) {
                     n_part = 0;
@@ -1958,6 +1978,7 @@ struct ag_plan {
     std::vector<int> zero_slots;       // output maps that are all zero (Vina e/d)
     FarParams far{};
     bool run_far = false;
+    bool far_flat = false;             // the electrostatic factor is one value from the far kernel's bins on
     double coeff_estat = 0.0;
     int far_grid = 0;                  // persistent far-kernel grid
     bool paged = false;                // near kernel in its paged form (a brick overflowed one LDS list)
@@ -2178,6 +2199,10 @@ static double far_floor_radius(bool flat, double spacing, int level) {
     return std::max({8.25, base, ((48.75 * spacing / half + 1.0) * g - 1.0) * half});
 }
 
+static bool flat_table(const std::vector<float> &reps) {
+    return std::all_of(reps.begin() + kFarBinMin, reps.end(), [&](float v) { return v == reps.back(); });
+}
+
 // Distances (A) past which an atom's term varies over a patch of a grid of
 // the given spacing the way 5 x 4 x 4 nodes follow, for each level of its charge.
 // Level 0: (a) no table step beyond it exceeds 6.5e-5 of the value there, (b)
@@ -2196,7 +2221,7 @@ static double far_floor_radius(bool flat, double spacing, int level) {
 // for 5,000 atoms on 127^3 points, 460 instead of 430 for 3,000 on 81^3 in a constant
 // dielectric.
 static void far_radii(const std::vector<float> &reps, double spacing, double radius[kFarLevels]) {
-    const bool flat = std::all_of(reps.begin() + kFarBinMin, reps.end(), [&](float v) { return v == reps.back(); });
+    const bool flat = flat_table(reps);
     const double run = (kFarK - 1) * spacing * 128.0;   // bins along an x-run
     const auto g = [&](double bin) {                     // the table as a function, between bin centres
         const double y = std::min(std::max(bin - 0.5, 0.0), (double)(AG_NDIEL - 1));
@@ -2285,16 +2310,27 @@ static FarShape far_shape(const ag_grid &g, int n_atoms, const double radius[kFa
     return f;
 }
 
-static void launch_far(int blocks, const FarParams &fp, bool clamp, hipStream_t st) {
-    if (clamp) k_far<true, false><<<blocks, kFarThreads, 0, st>>>(fp, CellParams{});
-    else k_far<false, false><<<blocks, kFarThreads, 0, st>>>(fp, CellParams{});
+// The far kernel with, if cp is given, the cell list in one more workgroup.
+static void launch_far(int blocks, const FarParams &fp, int kind, const CellParams *cp, hipStream_t st) {
+#define AG_FAR(K)                                                                              \
+    case K:                                                                                    \
+        if (cp) k_far<K, true><<<blocks + 1, kFarThreads, 0, st>>>(fp, *cp);                   \
+        else k_far<K, false><<<blocks, kFarThreads, 0, st>>>(fp, CellParams{});                \
+        break
+    switch (kind) {
+        AG_FAR(kFarTable);
+        AG_FAR(kFarClamped);
+        AG_FAR(kFarFlat);
+    }
+#undef AG_FAR
     HIP_CHECK(hipGetLastError());
 }
-// The same with the cell list in one more workgroup.
-static void launch_far_cells(int blocks, const FarParams &fp, const CellParams &cp, bool clamp, hipStream_t st) {
-    if (clamp) k_far<true, true><<<blocks + 1, kFarThreads, 0, st>>>(fp, cp);
-    else k_far<false, true><<<blocks + 1, kFarThreads, 0, st>>>(fp, cp);
-    HIP_CHECK(hipGetLastError());
+// The kind of a launch of conformations [c0, c1).
+static int far_kind(const ag_plan &p, int c0, int c1) {
+    if (p.far_flat) return kFarFlat;
+    for (int ci = c0; ci < c1; ci++)
+        if (p.confs[ci].far_clamp) return kFarClamped;
+    return kFarTable;
 }
 
 // Waves of the near kernel that share a cube's atoms, from the number of 8x8x4
@@ -2435,7 +2471,7 @@ static void plan_geometry(ag_plan &p, const ag_grid *grids, const int *natoms, c
     p.far.nconf = n;
     p.far.total_tiles = p.total_tiles;
     int occ = 0;
-    HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, reinterpret_cast<const void *>(&k_far<true, false>),
+    HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, reinterpret_cast<const void *>(&k_far<kFarClamped, false>),
                                                            kFarThreads, 0));
     p.far_grid = std::max(1, std::min(p.total_tiles, std::max(occ, 1) * p.ctx->n_cu));
 }
@@ -2707,6 +2743,7 @@ static ag_plan *plan_build(ag_ctx *c, int n, const ag_receptor *recs, const ag_g
 
     // far kernel (e map)
     p.run_far = !vina && ms->elec_index >= 0 && N > 0;
+    p.far_flat = flat_table(reps) && std::isfinite(reps.back());   // (its pairs are weighted before they are left out)
     std::vector<FarShape> far_shapes;
     if (p.run_far) {
         FarAtom *d_far = (FarAtom *)p.far_atoms.get(sizeof(FarAtom) * (size_t)N);
@@ -2850,7 +2887,7 @@ static void enqueue(ag_plan *p, float *d_maps, float *d_fmap, int32_t *d_cmap, b
             FarParams fp = p->far;
             fp.maps = d_maps;
             fp.item_end = p->total_tiles;
-            launch_far_cells(p->total_tiles, fp, cp, p->confs[0].far_clamp, st);
+            launch_far(p->total_tiles, fp, far_kind(*p, 0, 1), &cp, st);
         } else if (N <= kCellsOneAtoms && p->total_cells <= kCellsOne) {
             k_cells<<<1, 1024, 0, st>>>(cp);
         } else {
@@ -2935,9 +2972,7 @@ static void enqueue(ag_plan *p, float *d_maps, float *d_fmap, int32_t *d_cmap, b
             fp.item_end = t1;
             fp.queue = p->persistent ? d_queue + queue_base + k : nullptr;
             const int blocks = p->persistent ? std::min(p->far_grid, t1 - t0) : t1 - t0;
-            bool clamp = false;
-            for (int ci = c0; ci < c1; ci++) clamp = clamp || p->confs[ci].far_clamp;
-            launch_far(blocks, fp, clamp, s);
+            launch_far(blocks, fp, far_kind(*p, c0, c1), nullptr, s);
             long long most = 0;   // points of the largest conformation with parts to add
             for (int ci = c0; ci < c1; ci++)
                 if (p->confs[ci].far_split > 1) most = std::max(most, p->confs[ci].P);

@@ -161,3 +161,21 @@ def test_charge_levels(base, charges, spacing):
         got = ctx.maps_plain(st)
         assert np.array_equal(ctx.maps_plain(dataclasses.replace(st, charge=-q, _keep=[]))[0], -got[0])
     check(st, got[0], floor_charge=float(np.sqrt(np.mean(q ** 2))))
+
+
+@pytest.mark.parametrize("n1, spacing, constant, offset", [
+    ((1, 1, 1), 0.375, 1.0, 0.0), ((33, 41, 17), 0.25, 4.0, 0.0), ((35, 21, 27), 0.9, 80.0, 3.0),
+    ((30, 21, 20), 2.0, 4.0, 0.0), ((33, 33, 33), 0.375, 2.5, 90.0)])
+def test_constant_dielectric(base, n1, spacing, constant, offset):
+    """One value past the near kernel's pairs: summed without the table, at
+    any spacing, with atoms at and inside the near limit of a patch."""
+    print(f"[gpu] far constant {n1} {spacing} {constant}", flush=True)
+    run(state(base, 1600, n1, spacing, 30.0, 11, constant=constant, offset=offset))
+
+
+def test_zero_past_the_near_limit(base):
+    """A table that is zero from bin 1025 on: the far kernel adds nothing."""
+    print("[gpu] far zero table", flush=True)
+    tab = base.r_eps.copy()
+    tab[1025:] = 0.0
+    run(state(base, 1600, (33, 33, 33), 0.375, 30.0, 12, r_eps=tab))
