@@ -179,3 +179,25 @@ def test_zero_past_the_near_limit(base):
     tab = base.r_eps.copy()
     tab[1025:] = 0.0
     run(state(base, 1600, (33, 33, 33), 0.375, 30.0, 12, r_eps=tab))
+
+
+@pytest.mark.parametrize("n_atoms, n1, spacing, constant", [
+    (9000, (97, 65, 66), 0.375, None),     # boxes of 4 x 4 patches, ragged ones at the ends
+    (9001, (33, 60, 140), 0.375, None),    # one x-run past a box; patches not 8 x 8
+    (12000, (90, 90, 90), 0.3, None),
+    (16000, (60, 61, 63), 0.6, None),      # wide boxes: a longer distance
+    (20000, (97, 65, 66), 0.375, 4.0),     # no table
+])
+def test_coarse_boxes(base, n_atoms, n1, spacing, constant):
+    """Atoms beyond a box of patches are summed at the box's nodes; alone and
+    in a batch the same bits."""
+    print(f"[gpu] far boxes {n_atoms} {n1}", flush=True)
+    radius = (n_atoms / 0.068 * 0.75 / np.pi) ** (1 / 3)
+    st = state(base, n_atoms, n1, spacing, radius, n_atoms, constant=constant, offset=0.4 * radius)
+    small = state(base, 700, (17, 18, 19), spacing, 17.0, 13, constant=constant)
+    with ag.Context(0) as ctx:
+        got = ctx.maps_plain(st)
+        assert np.array_equal(got, ctx.maps_plain(st))
+        beside = ctx.maps_batch([small, st], tune={"cell_size": 4.0, "cube": True})
+    assert np.array_equal(np.asarray(beside[1]).reshape(-1), np.asarray(got).reshape(-1))
+    check(st, got[0])
