@@ -1297,8 +1297,7 @@ static void pack_points(Pred pred, long long P, int *counts, int *offs, int *pac
 // One wave per (64 atoms, chunk of kEAdjChunk packed points): per atom
 // sum_p g f(r) and sum_p g d(q w f(r))/d(atom position), f = 332 / (eps(r)
 // max(r, 0.5)) (inv_diel / max(r, 0.5) for a constant dielectric), with
-// hardware rsq / exp2 / rcp.  Chunks past the packed count write zeros, so
-// k_an_ered's fixed-order sum needs no count.
+// hardware rsq / exp2 / rcp.  Chunks past the packed count write nothing.
 template <bool DD>
 __global__ void __launch_bounds__(64) k_an_eadj(EParams p, const int *packed, const int *count) {
     __shared__ float4 sp[256];
@@ -1307,6 +1306,7 @@ __global__ void __launch_bounds__(64) k_an_eadj(EParams p, const int *packed, co
     const float4 at = act ? p.atoms[ai] : make_float4(0.f, 0.f, 0.f, 0.f);
     const int npk = *count;
     const int p0 = blockIdx.y * kEAdjChunk, p1 = min(npk, p0 + kEAdjChunk);
+    if (p0 >= p1) return;   // uniform; k_an_ered reads the chunks with points
     float gx = 0.f, gy = 0.f, gz = 0.f, gq = 0.f;
     constexpr float cs = kMsLB * 1.44269504088896341f;      // exp(-lambda B r) = 2^(-cs r)
     constexpr float dk = -kMsB * kMsK * kMsLB;             // d(1/eps)/dr = dk e y^2 (see below)
@@ -1360,18 +1360,34 @@ __global__ void __launch_bounds__(64) k_an_eadj(EParams p, const int *packed, co
     if (act) p.partial[(long long)blockIdx.y * p.n_atoms + ai] = make_float4(gx, gy, gz, gq);
 }
 
-__global__ void k_an_ered(const float4 *partial, int n_atoms, int nchunks, double *out) {
-    const int ai = blockIdx.x * blockDim.x + threadIdx.x;
-    if (ai >= n_atoms) return;
+// Each atom's chunks added up in FP64: 16 atoms per workgroup and 16 threads
+// per atom, each every 16th chunk with points, the threads' sums in order.  (One
+// thread per atom, all chunks: 20 workgroups for 5,000 atoms, 77 us; now 4.2.)
+constexpr int kRedAtoms = 16;
+__global__ void __launch_bounds__(256) k_an_ered(const float4 *partial, int n_atoms, const int *count, double *out) {
+    constexpr int kParts = 256 / kRedAtoms;
+    __shared__ double sum[kParts][kRedAtoms][4];
+    const int a = threadIdx.x % kRedAtoms, part = threadIdx.x / kRedAtoms;
+    const int ai = blockIdx.x * kRedAtoms + a;
+    const int nchunks = (*count + kEAdjChunk - 1) / kEAdjChunk;
     double s[4] = {0, 0, 0, 0};
-    for (int c = 0; c < nchunks; c++) {
-        const float4 v = partial[(long long)c * n_atoms + ai];
-        s[0] += v.x;
-        s[1] += v.y;
-        s[2] += v.z;
-        s[3] += v.w;
+    if (ai < n_atoms)
+        for (int c = part; c < nchunks; c += kParts) {
+            const float4 v = partial[(long long)c * n_atoms + ai];
+            s[0] += v.x;
+            s[1] += v.y;
+            s[2] += v.z;
+            s[3] += v.w;
+        }
+    for (int k = 0; k < 4; k++) sum[part][a][k] = s[k];
+    __syncthreads();
+    if (threadIdx.x < kRedAtoms * 4) {
+        const int b = threadIdx.x / 4, k = threadIdx.x % 4;
+        double v = 0.0;
+        for (int q = 0; q < kParts; q++) v += sum[q][b][k];
+        const int bi = blockIdx.x * kRedAtoms + b;
+        if (bi < n_atoms) out[4 * bi + k] = v;
     }
-    for (int k = 0; k < 4; k++) out[4 * ai + k] = s[k];
 }
 
 }  // namespace
@@ -1889,7 +1905,7 @@ void analytic_adjoint(ag_analytic *a, const float *d_dmaps, double *g_coord, dou
         const dim3 eg((unsigned)((N + 63) / 64), (unsigned)a->nchunks);
         if (a->dddiel) k_an_eadj<true><<<eg, 64, 0, st>>>(e, packed, offs + nblk);
         else k_an_eadj<false><<<eg, 64, 0, st>>>(e, packed, offs + nblk);
-        k_an_ered<<<(N + 255) / 256, 256, 0, st>>>(e.partial, N, a->nchunks, d_eout);
+        k_an_ered<<<(N + kRedAtoms - 1) / kRedAtoms, 256, 0, st>>>(e.partial, N, offs + nblk, d_eout);
         HIP_CHECK(hipGetLastError());
     }
     HIP_CHECK(hipEventRecord(c->ev[3], st));
