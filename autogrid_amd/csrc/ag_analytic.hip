@@ -722,6 +722,12 @@ __global__ void __launch_bounds__(kAT) k_an_near(AParams p) {
     }
 }
 
+// Orders a wave's own LDS accesses: its lanes see what the others wrote before.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 struct EParams {
     int n1[3], ne[3];
     float h;
@@ -737,6 +743,14 @@ struct EParams {
     float rcap;               // 2 / cs
     int echunk, nechunks;     // atoms per chunk, chunks
     float *epart;             // [nechunks][P] partial sums
+    // forward with boxes (k_an_ebox, k_an_epatch): patches of K x 8 x 8 points, boxes
+    // of 2 x 2 of them
+    int npatch[3], nbox[3];
+    int box_parts;            // workgroups sharing a box's atoms; 0: no boxes
+    int split;                // workgroups sharing a patch's atoms
+    float box_r2;             // squared distance (scaled) past which a box takes an atom
+    double *box_sums;         // [box][part][512]
+    unsigned long long *box_mask;   // [box][groups of 64 atoms]: the atoms it takes
     // adjoint
     const float *ge;          // cotangent of the e map
     float4 *partial;          // [chunks][n_atoms]: dx, dy, dz, dq
@@ -754,6 +768,31 @@ struct ERun {
     static __device__ __forceinline__ constexpr float c2(int k) { return ((float)k - mid) * ((float)k - mid); }
     static __device__ __forceinline__ constexpr float m(int k) { return (float)(K - 1 - 2 * k); }
 };
+
+// An atom's share of the e map at K points along x.
+template <int K, bool DD>
+__device__ __forceinline__ void e_pair(const EAtom &at, float py, float pz, float cx, float sc, float s2, float bias,
+                                       float rcap, float *part) {
+    const float dy = at.y - py, dz = at.z - pz;
+    const float dyz2 = __builtin_fmaf(dy, dy, __builtin_fmaf(dz, dz, bias));
+    const float u = at.x - cx;
+    const float U = __builtin_fmaf(u, u, dyz2);
+    const float us = u * sc;
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+        const float rb2 = __builtin_fmaf(us, ERun<K>::m(k), __builtin_fmaf(s2, ERun<K>::c2(k), U));
+        const float rs = __builtin_amdgcn_rsqf(rb2);
+        const float h = fminf(rs, rcap);
+        if (DD) {
+            const float e2 = __builtin_amdgcn_exp2f(-(rb2 * rs));
+            const float den = __builtin_fmaf(kMsK, e2, 1.f);
+            const float g = den * __builtin_amdgcn_rcpf(__builtin_fmaf(kMsA, den, kMsB));
+            part[k] = __builtin_fmaf(at.w, h * g, part[k]);
+        } else {
+            part[k] = __builtin_fmaf(at.w, h, part[k]);
+        }
+    }
+}
 
 template <int K, bool DD>
 __global__ void __launch_bounds__(64) k_an_e(EParams p) {
@@ -787,25 +826,7 @@ __global__ void __launch_bounds__(64) k_an_e(EParams p) {
         for (int a = a0; a < a1; a++) {
             const EAtom at = nxt;
             nxt = ld(min(a + 1, a1 - 1));
-            const float dy = at.y - py, dz = at.z - pz;
-            const float dyz2 = __builtin_fmaf(dy, dy, __builtin_fmaf(dz, dz, bias));
-            const float u = at.x - cx;
-            const float U = __builtin_fmaf(u, u, dyz2);
-            const float us = u * sc;
-#pragma unroll
-            for (int k = 0; k < K; k++) {
-                const float rb2 = __builtin_fmaf(us, ERun<K>::m(k), __builtin_fmaf(s2, ERun<K>::c2(k), U));
-                const float rs = __builtin_amdgcn_rsqf(rb2);
-                const float h = fminf(rs, rcap);
-                if (DD) {
-                    const float e2 = __builtin_amdgcn_exp2f(-(rb2 * rs));
-                    const float den = __builtin_fmaf(kMsK, e2, 1.f);
-                    const float g = den * __builtin_amdgcn_rcpf(__builtin_fmaf(kMsA, den, kMsB));
-                    part[k] = __builtin_fmaf(at.w, h * g, part[k]);
-                } else {
-                    part[k] = __builtin_fmaf(at.w, h, part[k]);
-                }
-            }
+            e_pair<K, DD>(at, py, pz, cx, sc, s2, bias, rcap, part);
         }
     }
     if (active) {
@@ -813,6 +834,213 @@ __global__ void __launch_bounds__(64) k_an_e(EParams p) {
 #pragma unroll
         for (int k = 0; k < K; k++)
             if (ix0 + k < p.n1[0]) out[k] = part[k];
+    }
+}
+
+// The e map of larger receptors.  1 / (eps(r) r) is smooth away from the atom, so
+// a box of 2 x 2 patches (about 16 x 16 x 16 points) takes the atoms beyond
+// box_r2 at 8 x 8 x 8 Chebyshev nodes, and its points interpolate; only the
+// atoms around it go pair by pair.  The distance, 2.6 half-edges, leaves
+// 3e-7 of a term at its nearest (2 rho^-8, rho = z + sqrt(z^2 - 1), z = 3.6);
+// the map's own error is 2e-5 (2-norm), from points on atoms.  Bound by the
+// pairs' and nodes' transcendentals (rsq, exp2, rcp), as the all-pairs kernel:
+// 5,000 atoms, 65^3 points 595 -> 257 us (boxes 158, patches 95, sum 4).
+constexpr int kEBoxN = 8, kEBoxNodes = kEBoxN * kEBoxN * kEBoxN, kEPatch = 8, kEWaves = 4;
+__host__ __device__ __forceinline__ constexpr double e_node(int i) {   // Chebyshev nodes, increasing
+    constexpr double c[4] = {0.98078528040323044913, 0.83146961230254523708, 0.55557023301960222474,
+                             0.19509032201612826785};
+    return i < 4 ? -c[i] : c[7 - i];
+}
+__host__ __device__ __forceinline__ constexpr double e_node_den(int i) {
+    double d = 1.0;
+    for (int m = 0; m < kEBoxN; m++)
+        if (m != i) d *= e_node(i) - e_node(m);
+    return d;
+}
+// The eight Lagrange weights at t.
+__device__ __forceinline__ constexpr void e_weights(double t, double w[kEBoxN]) {
+    double before[kEBoxN] = {1.0}, after = 1.0;
+    for (int m = 1; m < kEBoxN; m++) before[m] = before[m - 1] * (t - e_node(m - 1));
+    for (int m = kEBoxN - 1; m >= 0; m--) {
+        w[m] = before[m] * after * (1.0 / e_node_den(m));
+        after *= t - e_node(m);
+    }
+}
+
+// The sums at a box's nodes of one part of the atoms beyond it, and which atoms
+// those are: a lane has the eight x-nodes of one (y, z) node.
+template <int K, bool DD>
+__global__ void __launch_bounds__(64 * kEWaves) k_an_ebox(EParams p) {
+    __shared__ double XD[(kEWaves - 1) * kEBoxNodes];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
+    const int part = blockIdx.x % p.box_parts, box = blockIdx.x / p.box_parts;
+    const int bx = box % p.nbox[0], by = box / p.nbox[0] % p.nbox[1], bz = box / p.nbox[0] / p.nbox[1];
+    const float sc = p.sc;
+    const float hx = ERun<K>::mid * sc, hr = ((float)kEPatch - 0.5f) * sc;
+    const float mx = ((float)(bx * K - p.ne[0]) + ERun<K>::mid) * sc;
+    const float my = ((float)(by * 2 * kEPatch - p.ne[1]) + (float)kEPatch - 0.5f) * sc;
+    const float mz = ((float)(bz * 2 * kEPatch - p.ne[2]) + (float)kEPatch - 0.5f) * sc;
+    float cy = 0.f, cz = 0.f;
+#pragma unroll
+    for (int i = 0; i < kEBoxN; i++) {
+        cy = (lane & 7) == i ? my + hr * (float)e_node(i) : cy;
+        cz = lane >> 3 == i ? mz + hr * (float)e_node(i) : cz;
+    }
+    double sum[kEBoxN];
+    float acc[kEBoxN];
+#pragma unroll
+    for (int j = 0; j < kEBoxN; j++) {
+        sum[j] = 0.;
+        acc[j] = 0.f;
+    }
+    const int groups = (p.n_atoms + 63) / 64;
+    unsigned long long *const mask = p.box_mask + (size_t)box * groups;
+    const AN_CONST EAtom *atoms = (const AN_CONST EAtom *)p.fatoms;   // scalar loads
+    int n_acc = 0;
+    for (int a0 = 64 * (part * kEWaves + wave); a0 < p.n_atoms; a0 += 64 * kEWaves * p.box_parts) {
+        const float4 v = p.fatoms[min(a0 + lane, p.n_atoms - 1)];
+        const float ex = fmaxf(fabsf(v.x - mx) - hx, 0.f), ey = fmaxf(fabsf(v.y - my) - hr, 0.f),
+                    ez = fmaxf(fabsf(v.z - mz) - hr, 0.f);
+        unsigned long long set = __ballot(a0 + lane < p.n_atoms &&
+                                          __builtin_fmaf(ex, ex, __builtin_fmaf(ey, ey, ez * ez)) >= p.box_r2);
+        if (lane == 0) mask[a0 / 64] = set;
+        n_acc += __popcll(set);
+        while (set) {
+            const AN_CONST EAtom &at = atoms[a0 + __builtin_ctzll(set)];
+            set &= set - 1;
+            const float dy = at.y - cy, dz = at.z - cz, u = at.x - mx, w = at.w;
+            const float U = __builtin_fmaf(u, u, __builtin_fmaf(dy, dy, dz * dz)), u2 = u + u;
+#pragma unroll
+            for (int j = 0; j < kEBoxN; j++) {
+                const float d = hx * (float)e_node(j);
+                const float rb2 = __builtin_fmaf(-u2, d, __builtin_fmaf(d, d, U));
+                const float rs = __builtin_amdgcn_rsqf(rb2);
+                if (DD) {
+                    const float e2 = __builtin_amdgcn_exp2f(-(rb2 * rs));
+                    const float den = __builtin_fmaf(kMsK, e2, 1.f);
+                    const float g = den * __builtin_amdgcn_rcpf(__builtin_fmaf(kMsA, den, kMsB));
+                    acc[j] = __builtin_fmaf(w, rs * g, acc[j]);
+                } else {
+                    acc[j] = __builtin_fmaf(w, rs, acc[j]);
+                }
+            }
+        }
+        if (n_acc >= kEAtoms) {
+            n_acc = 0;
+#pragma unroll
+            for (int j = 0; j < kEBoxN; j++) {
+                sum[j] += (double)acc[j];
+                acc[j] = 0.f;
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < kEBoxN; j++) sum[j] += (double)acc[j];
+    if (wave > 0) {
+#pragma unroll
+        for (int j = 0; j < kEBoxN; j++) XD[((wave - 1) * kEBoxN + j) * 64 + lane] = sum[j];
+    }
+    __syncthreads();
+    if (wave == 0) {
+        double *const out = p.box_sums + (size_t)blockIdx.x * kEBoxNodes;
+#pragma unroll
+        for (int j = 0; j < kEBoxN; j++) {
+            for (int q = 0; q < kEWaves - 1; q++) sum[j] += XD[(q * kEBoxN + j) * 64 + lane];
+            out[j * 64 + lane] = sum[j];
+        }
+    }
+}
+
+// One patch, and one of its parts of the atoms its box leaves, a run of K
+// points per lane; each wave also interpolates a quarter of the box's nodes (in
+// the first part).  The waves' sums meet in LDS, in order.
+template <int K, bool DD>
+__global__ void __launch_bounds__(64 * kEWaves) k_an_epatch(EParams p) {
+    __shared__ double XD[(kEWaves - 1) * K * 64];
+    __shared__ double V[kEWaves][kEBoxNodes / kEWaves];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
+    const int part = blockIdx.x % p.split, patch = blockIdx.x / p.split;
+    const int px = patch % p.npatch[0], pyi = patch / p.npatch[0] % p.npatch[1], pzi = patch / p.npatch[0] / p.npatch[1];
+    const int box = px + p.nbox[0] * (pyi / 2 + p.nbox[1] * (pzi / 2));
+    const int ix0 = px * K, iy = pyi * kEPatch + lane % kEPatch, iz = pzi * kEPatch + lane / kEPatch;
+    const bool active = iy < p.n1[1] && iz < p.n1[2];
+    const float sc = p.sc;
+    const float py = (float)(iy - p.ne[1]) * sc, pz = (float)(iz - p.ne[2]) * sc;
+    const float cx = ((float)(ix0 - p.ne[0]) + ERun<K>::mid) * sc;
+    const float s2 = sc * sc, bias = fmaxf(1.0e-12f, ERun<K>::mid * ERun<K>::mid * s2 * 0x1p-19f), rcap = p.rcap;
+    const int groups = (p.n_atoms + 63) / 64;
+    const AN_CONST unsigned long long *mask = (const AN_CONST unsigned long long *)p.box_mask + (size_t)box * groups;
+    const AN_CONST EAtom *atoms = (const AN_CONST EAtom *)p.fatoms;   // scalar loads
+    float sum[K];
+#pragma unroll
+    for (int k = 0; k < K; k++) sum[k] = 0.f;
+    for (int a0 = 64 * (part * kEWaves + wave); a0 < p.n_atoms; a0 += 64 * kEWaves * p.split) {
+        const int nb = min(64, p.n_atoms - a0);
+        unsigned long long set = (nb == 64 ? ~0ull : (1ull << nb) - 1) & ~mask[a0 / 64];
+        if (!set) continue;
+        const auto ld = [&](int i) {
+            const AN_CONST EAtom &q = atoms[a0 + i];
+            return EAtom{q.x, q.y, q.z, q.w};
+        };
+        EAtom nxt = ld(__builtin_ctzll(set));
+        while (set) {
+            const EAtom at = nxt;
+            set &= set - 1;
+            if (set) nxt = ld(__builtin_ctzll(set));
+            e_pair<K, DD>(at, py, pz, cx, sc, s2, bias, rcap, sum);
+        }
+    }
+    double f[K];
+#pragma unroll
+    for (int k = 0; k < K; k++) f[k] = (double)sum[k];
+    if (part == 0) {
+        constexpr int kOwn = 64 / kEWaves;   // (y, z) nodes of a wave: two rows of eight
+        for (int t = lane; t < kOwn * kEBoxN; t += 64) {
+            double v = 0.;
+            for (int q = 0; q < p.box_parts; q++)
+                v += p.box_sums[((size_t)box * p.box_parts + q) * kEBoxNodes + t / kOwn * 64 + wave * kOwn + t % kOwn];
+            V[wave][t % kOwn * kEBoxN + t / kOwn] = v;
+        }
+        wave_sync();
+        constexpr double half = kEPatch - 0.5;
+        double wy[kEBoxN], wz[kEBoxN];
+        e_weights(((double)((pyi & 1) * kEPatch + lane % kEPatch) - half) / half, wy);
+        e_weights(((double)((pzi & 1) * kEPatch + lane / kEPatch) - half) / half, wz);
+        double wz0 = wz[0], wz1 = wz[1];
+#pragma unroll
+        for (int q = 1; q < kEWaves; q++) {
+            wz0 = wave == q ? wz[2 * q] : wz0;
+            wz1 = wave == q ? wz[2 * q + 1] : wz1;
+        }
+        double g[kEBoxN];
+#pragma unroll
+        for (int j = 0; j < kEBoxN; j++) g[j] = 0.;
+#pragma unroll
+        for (int l = 0; l < kOwn; l++) {
+            const double w = wy[l & 7] * (l < 8 ? wz0 : wz1);
+#pragma unroll
+            for (int j = 0; j < kEBoxN; j++) g[j] = __builtin_fma(w, V[wave][l * kEBoxN + j], g[j]);
+        }
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            double wx[kEBoxN];
+            e_weights(((double)k - 0.5 * (K - 1)) / (0.5 * (K - 1)), wx);
+#pragma unroll
+            for (int j = 0; j < kEBoxN; j++) f[k] = __builtin_fma(wx[j], g[j], f[k]);
+        }
+    }
+    if (wave > 0) {
+#pragma unroll
+        for (int k = 0; k < K; k++) XD[((wave - 1) * K + k) * 64 + lane] = f[k];
+    }
+    __syncthreads();
+    if (wave == 0 && active) {
+        float *const out = p.epart + (long long)part * p.P + ix0 + (long long)p.n1[0] * (iy + (long long)p.n1[1] * iz);
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            for (int q = 0; q < kEWaves - 1; q++) f[k] += XD[(q * K + k) * 64 + lane];
+            if (ix0 + k < p.n1[0]) out[k] = (float)f[k];
+        }
     }
 }
 
@@ -905,12 +1133,6 @@ __global__ void __launch_bounds__(kAT) k_an_vh(AParams p) {
     }
     if (wave == 0 && q.inside)
         for (int k = 0; k < 3; k++) p.vh[3 * pt + k] = v[k];
-}
-
-// Orders a wave's own LDS accesses: its lanes see what the others wrote before.
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
 }
 
 // Block reduction of n floats per lane (fixed order): lane 0 of the block
@@ -1424,7 +1646,7 @@ struct ag_analytic {
     std::vector<ag::BondRecipe> recipes;
     std::vector<int> h_atoms, atom_list;
     // device
-    DevBuf d_up, d_eup, d_closest, d_amin, d_amax, d_vh, d_hout, d_aout, d_partial, d_eout, d_epart, d_gcount, d_gpack,
+    DevBuf d_up, d_eup, d_ebox, d_closest, d_amin, d_amax, d_vh, d_hout, d_aout, d_partial, d_eout, d_epart, d_gcount, d_gpack,
         d_vcount, d_vpack, d_gmask;
     HostStage stage;                   // pinned: parameters up, gradients' sums down
     const AAtom *by_index = nullptr;   // in d_up
@@ -1589,6 +1811,33 @@ static void check_pairs(const ag_analytic *a) {
         }
 }
 
+// Boxes for the e map's forward where they pay: a box's 512 nodes stand for its
+// about 4,096 points, at two more launches (15 us).  At protein density (0.068
+// atoms / A^3) the atoms within the distance of a box are pairs as before, so
+// a receptor has to hold twice as many, and what is saved at 2.4e12 terms/s has
+// to be worth the launches.  (1,000 atoms on 41^3 points stay with 69 us.)
+static void e_boxes(ag_analytic *a) {
+    EParams &e = a->ep;
+    const ag_grid &g = a->grid;
+    const int edge[3] = {a->eK, 2 * kEPatch, 2 * kEPatch}, rows[3] = {a->eK, kEPatch, kEPatch};
+    double boxes = 1.0, patches = 1.0;
+    for (int d = 0; d < 3; d++) {
+        e.npatch[d] = (g.n1[d] + rows[d] - 1) / rows[d];
+        e.nbox[d] = (g.n1[d] + edge[d] - 1) / edge[d];
+        boxes *= e.nbox[d];
+        patches *= e.npatch[d];
+    }
+    // (1 A: past the point where max(r, 0.5) has its kink)
+    const double half = 0.5 * (2 * kEPatch - 1) * g.spacing, r = std::max(2.6 * half, 1.0), w = 2.0 * half;
+    const double inside = 0.068 * (w * w * w + r * (6 * w * w + M_PI * r * (3 * w + 4. / 3. * r)));
+    const double pairs = patches * 64 * a->eK;
+    if (a->N < 2.0 * inside || (a->N - inside) * (pairs - boxes * kEBoxNodes) < 2.4e8) return;
+    e.box_parts = (int)std::max(1.0, std::min({1024 / boxes, a->N / 256.0, 16.0}));
+    e.split = (int)std::max(1.0, std::min({1536 / patches, a->N / 256.0, 8.0}));
+    const double cs = e.sc / g.spacing;   // coordinates of fatoms are scaled by it
+    e.box_r2 = (float)(cs * r * (cs * r));
+}
+
 // What the electrostatic kernels read: needs the coordinates and charges only.
 static void upload_e(ag_analytic *a, UploadPack up) {
     const int N = a->N;
@@ -1620,9 +1869,18 @@ static void upload_e(ag_analytic *a, UploadPack up) {
     e.rcap = (float)(2.0 / cs);
     e.echunk = std::max(kEAtoms, (N + kEMaxChunks - 1) / kEMaxChunks);
     e.nechunks = std::max(1, (N + e.echunk - 1) / e.echunk);
-    e.epart = (float *)a->d_epart.get(sizeof(float) * (size_t)e.nechunks * (size_t)a->P);
     // run length: 13 or 16 points, whichever leaves fewer idle run slots
     a->eK = 13 * ((g.n1[0] + 12) / 13) < 16 * ((g.n1[0] + 15) / 16) ? 13 : 16;
+    e_boxes(a);
+    if (e.box_parts) {
+        const size_t boxes = (size_t)e.nbox[0] * e.nbox[1] * e.nbox[2];
+        const size_t sums = sizeof(double) * boxes * e.box_parts * kEBoxNodes;
+        char *const block = (char *)a->d_ebox.get(sums + sizeof(unsigned long long) * boxes * ((N + 63) / 64));
+        e.box_sums = (double *)block;
+        e.box_mask = (unsigned long long *)(block + sums);
+        e.nechunks = e.split;
+    }
+    e.epart = (float *)a->d_epart.get(sizeof(float) * (size_t)e.nechunks * (size_t)a->P);
     a->nchunks = (int)((a->P + kEAdjChunk - 1) / kEAdjChunk);
     e.nchunks = a->nchunks;
     e.partial = (float4 *)a->d_partial.get(sizeof(float4) * (size_t)a->nchunks * std::max(N, 1));
@@ -1784,6 +2042,26 @@ static unsigned cube_count(const ag_grid &g) {
     return n;
 }
 
+template <int K>
+static void launch_e(const ag_analytic &a, const EParams &e, hipStream_t st) {
+    if (e.box_parts) {
+        const unsigned boxes = (unsigned)(e.nbox[0] * e.nbox[1] * e.nbox[2] * e.box_parts);
+        const unsigned patches = (unsigned)(e.npatch[0] * e.npatch[1] * e.npatch[2] * e.split);
+        if (a.dddiel) {
+            k_an_ebox<K, true><<<boxes, 64 * kEWaves, 0, st>>>(e);
+            k_an_epatch<K, true><<<patches, 64 * kEWaves, 0, st>>>(e);
+        } else {
+            k_an_ebox<K, false><<<boxes, 64 * kEWaves, 0, st>>>(e);
+            k_an_epatch<K, false><<<patches, 64 * kEWaves, 0, st>>>(e);
+        }
+        return;
+    }
+    const long long nruns = (long long)a.grid.n1[1] * a.grid.n1[2] * ((a.grid.n1[0] + K - 1) / K);
+    const dim3 eg((unsigned)((nruns + 63) / 64), (unsigned)e.nechunks);
+    if (a.dddiel) k_an_e<K, true><<<eg, 64, 0, st>>>(e);
+    else k_an_e<K, false><<<eg, 64, 0, st>>>(e);
+}
+
 // The e map needs the coordinates and charges only, so its kernels run while
 // the host makes the bond vectors, cells and pair tables of new parameters
 // (0.5 ms of host work for 5,000 atoms that the device waited for).
@@ -1805,15 +2083,8 @@ void analytic_forward(ag_analytic *a, float *d_maps) {
     if (a->elec >= 0) {
         EParams e = a->ep;
         e.emap = d_maps + (size_t)a->elec * a->P;
-        const long long nruns = (long long)a->grid.n1[1] * a->grid.n1[2] * ((a->grid.n1[0] + a->eK - 1) / a->eK);
-        const dim3 eg((unsigned)((nruns + 63) / 64), (unsigned)e.nechunks);
-        if (a->eK == 13) {
-            if (a->dddiel) k_an_e<13, true><<<eg, 64, 0, st>>>(e);
-            else k_an_e<13, false><<<eg, 64, 0, st>>>(e);
-        } else {
-            if (a->dddiel) k_an_e<16, true><<<eg, 64, 0, st>>>(e);
-            else k_an_e<16, false><<<eg, 64, 0, st>>>(e);
-        }
+        if (a->eK == 13) launch_e<13>(*a, e, st);
+        else launch_e<16>(*a, e, st);
         k_an_esum<<<(unsigned)((a->P + 255) / 256), 256, 0, st>>>(e.epart, e.nechunks, a->P, e.emap);
         HIP_CHECK(hipGetLastError());
     }
