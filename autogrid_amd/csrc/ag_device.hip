@@ -74,7 +74,7 @@ constexpr int kBoxNodes = kBoxN * kBoxN * kBoxN;
 constexpr int kFarNodes = kFarNx * kFarNy * kFarNy;  // of a patch
 constexpr int kBoxRuns = 2, kBoxRows = 32;        // a coarse box: x-runs, and rows along y and z (whole patches, about)
 constexpr int kFarBinMin = 1025;                  // far kernel takes bins >= this
-constexpr float kGuardBins = 1.0e-3f;             // FP64 recompute band around bin edges
+constexpr float kGuardBins = 4.0e-4f;             // FP64 recompute band around bin edges
 
 // Map roles.
 enum : int { ROLE_NONE = 0, ROLE_AFF = 1, ROLE_DES = 2, ROLE_COV = 4 };
@@ -1020,7 +1020,9 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
                 // shared) and adds zeros.
                 const bool in = r2 <= 64.33f;
                 if (!__ballot(in)) continue;
-                // hardware rsq: 128 r is good to ~3e-4 bins here, inside the guard band;
+                // hardware rsq (1 ulp): 128 r is good to 5.5 x 2^-24 of itself, 3.4e-4
+                // bins here, inside the guard band (a 1e-3 band sent 13 % of the
+                // wave's atoms through FP64 for some lane, 4e-4 sends 5 %);
                 // the same rsq is 1/r for the near e term and the unit vector
                 const float r2c = max_of(r2, 1.0e-12f);
                 float inv_r = __builtin_amdgcn_rsqf(r2c);
