@@ -59,7 +59,12 @@ constexpr int kHbSlots = kMapSlots - kPlainSlots; // of which H-bonding probes
 constexpr int kCandCap = 2048;                    // candidates per brick
 constexpr int kHCap = 256;                        // donor-H candidates per brick
 constexpr int kChunk = 128;                       // candidate records staged per pass
-constexpr int kNearRepsLen = 1040;                // electrostatic bins used by the near kernel
+// The near kernel's bins, as rows of its tables: 0 to 1023, whose rows hold
+// values; 1024 to 1039, past the 8 A cutoff, whose rows are zeros (a distance is
+// clamped to 1039.5 bins), so a lane out of range needs no test; the pair at 8 A
+// exactly (bin 1024, not past the cutoff: the last value row); and bin 1025 as
+// the near field's, where the far kernel's bin is 1024.
+constexpr int kNearZeroRow = 1039, kNearExactRow = 1040, kNearEdgeRow = 1041, kNearRows = 1042;
 constexpr float kNearRadius = 8.03f;              // staging radius (A)
 constexpr int kFarK = 16;                         // points per lane, far kernel
 constexpr int kFarWaves = 4;                      // waves of a far-kernel workgroup: parts of the atom list
@@ -183,8 +188,7 @@ struct NearParams {
     const double *rvec64;         // [n][3]
     const double *rvec2_64;       // [n][3]
     // tables
-    const float *tab;             // [T][1024][row slots] for this pass's maps (near_row)
-    unsigned zero_off;            // byte offset from tab of a row of zeros
+    const float *tab;             // [T][kNearRows][row slots] for this pass's maps (near_row)
     const float *sol;             // [1025]
     const float *reps;            // [8192] electrostatic factor (r_eps or 332/diel)
     // map slots of this pass: [0, kPlainSlots) maps without H-bond terms,
@@ -598,6 +602,18 @@ __device__ __forceinline__ float max_of(float a, float b) {
     return r;
 }
 
+// min(g, 1039.5) and min(inv_r, 2), the limit in the instruction.
+__device__ __forceinline__ float clamp_bins(float g) {
+    float r;
+    asm("v_min_f32 %0, 0x4481f000, %1" : "=v"(r) : "v"(g));
+    return r;
+}
+__device__ __forceinline__ float half_at_least(float inv_r) {
+    float r;
+    asm("v_min_f32 %0, 2.0, %1" : "=v"(r) : "v"(inv_r));
+    return r;
+}
+
 // Uniform per-atom values: every lane reads the same LDS record, so its
 // fields are moved to scalar registers and branches on them stay scalar.
 __device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
@@ -664,18 +680,20 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
     float(*const hrvs)[3] = lists.hrvs;
     float *const scratch_f = reinterpret_cast<float *>(&lists);
     static_assert(sizeof(NearLists) >= sizeof(float) * kNearThreads * (kMapSlots + 1), "room for the table sums");
-    __shared__ float2 rs_s[kNearRepsLen];   // (electrostatic factor, sol_fn) per bin
+    __shared__ float2 rs_s[kNearRows];   // (electrostatic factor, sol_fn) per row; zeros past the near field's
     __shared__ int2 wave_tot[2][kStage][kNearThreads / 64];
 
     const int tid = threadIdx.x;
     stamp_start(p.stamp);
     // read here, stored once the staging's own reads are on their way
-    constexpr int kRsPer = (kNearRepsLen + kNearThreads - 1) / kNearThreads;
+    constexpr int kRsPer = (kNearRows + kNearThreads - 1) / kNearThreads;
     float2 rs[kRsPer];
 #pragma unroll
     for (int u = 0; u < kRsPer; u++) {
-        const int k = min(tid + u * kNearThreads, kNearRepsLen - 1);
-        rs[u] = make_float2(p.reps[k], p.sol[min(k, AG_NEINT)]);
+        const int k = min(tid + u * kNearThreads, kNearRows - 1);
+        const int bin = k == kNearExactRow ? AG_NEINT : k == kNearEdgeRow ? kFarBinMin : min(k, kFarBinMin);
+        rs[u] = make_float2(k < kFarBinMin || k > kNearZeroRow ? p.reps[bin] : 0.f,
+                            k < AG_NEINT || k == kNearExactRow ? p.sol[min(bin, AG_NEINT)] : 0.f);
     }
 
     // one workgroup per brick of all conformations, in chunks of 16 bricks
@@ -837,7 +855,7 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
     stage(0, 0);
 #pragma unroll
     for (int u = 0; u < kRsPer; u++)
-        if (tid + u * kNearThreads < kNearRepsLen) rs_s[tid + u * kNearThreads] = rs[u];
+        if (tid + u * kNearThreads < kNearRows) rs_s[tid + u * kNearThreads] = rs[u];
     __syncthreads();
     if constexpr (!PAGED) {
         if (ncand > kCandCap || nh > kHCap) {   // uniform per workgroup
@@ -1014,7 +1032,8 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
                 // geometry: FP64 difference as the reference forms it, FP32 after
                 const double dx64 = ax - cx, dy64 = ay - cy, dz64 = az - cz;
                 const float dxf = (float)dx64, dyf = (float)dy64, dzf = (float)dz64;
-                const float r2 = __builtin_fmaf(dxf, dxf, __builtin_fmaf(dyf, dyf, dzf * dzf));
+                // (1e-14 A^2 keeps the root's argument positive)
+                const float r2 = __builtin_fmaf(dxf, dxf, __builtin_fmaf(dyf, dyf, __builtin_fmaf(dzf, dzf, 1.0e-14f)));
                 // beyond 8.02 A: neither cutoff pass nor near e term.  A lane out of
                 // range goes along where another is in range (the table reads are
                 // shared) and adds zeros.
@@ -1024,19 +1043,40 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
                 // bins here, inside the guard band (a 1e-3 band sent 13 % of the
                 // wave's atoms through FP64 for some lane, 4e-4 sends 5 %);
                 // the same rsq is 1/r for the near e term and the unit vector
-                const float r2c = max_of(r2, 1.0e-12f);
-                float inv_r = __builtin_amdgcn_rsqf(r2c);
-                float r = r2c * inv_r;
-                const float g = r * 128.f;
+                float inv_r = __builtin_amdgcn_rsqf(r2);
+                float r = r2 * inv_r;
+                const float g = clamp_bins(r * 128.f);
                 int bin = (int)g;
                 bool cut = r > 8.0f;
-                if (in & (fabsf(g - rintf(g)) < kGuardBins)) {
+                if (fabsf(g - rintf(g)) < kGuardBins) {
                     double rdx, rdy, rdz;
                     const double r64 = ref_dist(ax, ay, az, cx, cy, cz, rdx, rdy, rdz);
-                    bin = (int)(r64 * 128.0);
                     cut = r64 > 8.0;
+                    bin = (int)(r64 * 128.0);
+                    if (bin == AG_NEINT && !cut) bin = kNearExactRow;
                     r = (float)r64;
                     inv_r = __builtin_amdgcn_rcpf(fmaxf(r, 1.0e-6f));
+                }
+                // which of the pairs at 1,025 bins are the near kernel's: the far
+                // kernel's own bin says
+                bool no_e = false;   // (general forms, at spacings where the band reaches below 8 A)
+                if (want_e && fabsf(g - (float)kFarBinMin) <= band) {
+                    // the far kernel's coordinates of the atom and the point: run centre, offset in the run, y, z
+                    // (one axis after the other: few registers beside the sums)
+                    int q, qy, qz, unused;
+                    point_index(unused, qy, unused);
+                    float dyE = far_row(ay * 128.0, qy, cf.far_py, ney, spacing, s128);
+                    asm volatile("" : "+v"(dyE));
+                    point_index(unused, unused, qz);
+                    float dzE = far_row(az * 128.0, qz, cf.far_pz, nez, spacing, s128);
+                    asm volatile("" : "+v"(dzE));
+                    point_index(q, unused, unused);
+                    const int k = q % kFarK;
+                    const float uE = (float)(ax * 128.0 - far_centre(q - k, kFarK, nex, spacing));
+                    const bool near_e = far_bin4(uE, dyE, dzE, k, s128) < 4u * kFarBinMin;
+                    if (!GENERAL || (bin >= AG_NEINT && bin != kNearExactRow))
+                        bin = !near_e ? kNearZeroRow : bin >= kFarBinMin ? kNearEdgeRow : bin;
+                    else no_e = !near_e;
                 }
                 // the tree build's radius queries (bhtree.cpp:341-362): FP32 point
                 // and atom, each component within the radius, then the rounded
@@ -1065,7 +1105,13 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
                 const int type = meta & 0xff, hb = (meta >> 8) & 0xff, rexp = (meta >> 16) & 0xff;
                 const bool dis = GENERAL && ((meta >> 24) & 1);
                 const bool skip_atom = !p.has_affinity || (p.disorder_h && dis && type == p.hydrogen_type);   // uniform
-                const bool sel = in & !(bh ? !in8 : cut) & !skip_atom;
+                // whether the pair has terms (the plain form asks only where a class has
+                // directional terms or mixes: its other rows are zeros)
+                const auto selected = [&] {
+                    return GENERAL ? in & !(bh ? !in8 : cut) & !skip_atom : (bin < AG_NEINT) | (bin == kNearExactRow);
+                };
+                const int row = !GENERAL ? bin : !selected() ? kNearZeroRow
+                                : !bh ? bin : bin_bh >= AG_NEINT ? kNearExactRow : bin_bh;
                 // H-bonding slots (main.cpp:3286-3374): the (probe, atom) case is a
                 // set of 0/1 coefficients chosen per atom class, uniform across
                 // the wave.  For a class that mixes in some slot, each lane reads
@@ -1076,11 +1122,10 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
                 const bool mixes = (codes & kMixBits) != 0;   // uniform
                 float4 E[Q], Eo;
                 {
-                    constexpr unsigned kTypeBytes = AG_NEINT * ROW * sizeof(float);
+                    constexpr unsigned kTypeBytes = kNearRows * ROW * sizeof(float);
                     const char *trow = reinterpret_cast<const char *>(tab) + (size_t)type * kTypeBytes;
-                    const unsigned zero = p.zero_off - (unsigned)type * kTypeBytes;
-                    const unsigned roff =
-                        sel ? (unsigned)min(bh ? bin_bh : bin, AG_NEINT - 1) * (unsigned)(ROW * sizeof(float)) : zero;
+                    constexpr unsigned zero = kNearZeroRow * ROW * sizeof(float);
+                    const unsigned roff = (unsigned)row * (unsigned)(ROW * sizeof(float));
                     unsigned at[4];
                     at[0] = (unsigned)group_lane<Q, 0>((int)roff) + lane_chunk;
                     at[1] = (unsigned)group_lane<Q, 1>((int)roff) + lane_chunk;
@@ -1097,7 +1142,7 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
                     for (int j = 0; j < Q; j++) E[j] = *reinterpret_cast<const float4 *>(trow + at[j]);
                 }
                 // electrostatic factor and sol_fn of the bin, one LDS read
-                const float2 rsv = rs_s[min(bin, kNearRepsLen - 1)];
+                const float2 rsv = rs_s[bin];
                 // constriction grid: atoms within the cutoff (main.cpp:2969-2973)
                 if (want_cmap && !bh && in) {
                     if (fabsf(r - (float)p.ccut) < 1.0e-5f) {
@@ -1109,39 +1154,20 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
                 }
                 // electrostatics of pairs the far kernel leaves out
                 if (want_e) {
-                    bool near_e = g < (float)kFarBinMin;
-                    if (in & (fabsf(g - (float)kFarBinMin) <= band)) {
-                        // (one axis after the other: few registers beside the sums)
-                        int q, qy, qz, unused;
-                        point_index(unused, qy, unused);
-                        float dyE = far_row(ay * 128.0, qy, cf.far_py, ney, spacing, s128);
-                        asm volatile("" : "+v"(dyE));
-                        point_index(unused, unused, qz);
-                        float dzE = far_row(az * 128.0, qz, cf.far_pz, nez, spacing, s128);
-                        asm volatile("" : "+v"(dzE));
-                        point_index(q, unused, unused);
-                        const int k = q % kFarK;
-                        const float uE = (float)(ax * 128.0 - far_centre(q - k, kFarK, nex, spacing));
-                        near_e = far_bin4(uE, dyE, dzE, k, s128) < 4u * kFarBinMin;
-                    }
-                    // 1/max(r, 0.5) with r clamped at APPROX_ZERO; adding 0 leaves
-                    // the sum as it is (it is never -0)
-                    const float inv_rmax = min_of(inv_r, 2.f);
-                    const float te = aqe * inv_rmax * rsv.x;
-                    e_near += near_e ? te : 0.f;
+                    // 1/max(r, 0.5) with r clamped at APPROX_ZERO
+                    const float te = aqe * half_at_least(inv_r);
+                    e_near = __builtin_fmaf(GENERAL && no_e ? 0.f : te, rsv.x, e_near);
                 }
                 // Loop 2 of the tree build takes the atoms its 8 A query returns,
                 // at their FP32 distance (main.cpp:3019-3028)
                 if (bh) {
-                    cut = !in8;
                     r = rB;
-                    bin = bin_bh;
                     inv_r = __builtin_amdgcn_rcpf(fmaxf(rB, 1.0e-6f));
                 }
                 float racc = 1.f, rdon = 1.f, Hramp = 1.f;
                 // directional classes only (D1, A1, A2): the unit vector to the point
                 constexpr unsigned kDirClasses = (1u << AG_HB_D1) | (1u << AG_HB_A1) | (1u << AG_HB_A2);
-                if (((kDirClasses >> hb) & 1u) && sel) {
+                if (((kDirClasses >> hb) & 1u) && selected()) {
                     const float dn0 = dxf * inv_r, dn1 = dyf * inv_r, dn2 = dzf * inv_r;
                     const float rv0 = unif(a.rv[0]), rv1 = unif(a.rv[1]), rv2 = unif(a.rv[2]);
                     const int aidx = aindex;
@@ -1215,7 +1241,7 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
                         }
                     }
                 }  // directional classes
-                const float S = !sel ? 0.f : bh ? rs_s[min(bin, AG_NEINT)].y : rsv.y;   // sol_fn[min(bin, 1024)]
+                const float S = !GENERAL ? rsv.y : !selected() ? 0.f : rs_s[row].y;   // sol_fn[min(bin, 1024)]
                 // desolvation (main.cpp:3375-3390): slot m gains
                 // (sp[m] vol + volp[m] solq) S per pair, i.e. sp[m] sum(vol S) +
                 // volp[m] sum(solq S) over the point's pairs: two sums per point
@@ -1232,7 +1258,7 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
                 // The mix runs in scalar branches, one per slot.  A disordered
                 // partner uses the hydrogen-type row at r - 1.10 A
                 // (main.cpp:3313-3349), FP64 like the reference.
-                if (mixes && sel) {
+                if (mixes && selected()) {
                     const float e4[kHbSlots] = {Eo.x, Eo.y, Eo.z, Eo.w};
                     float Eh[kHbSlots] = {0.f, 0.f, 0.f, 0.f};
                     if (dis && p.hydrogen_type >= 0) {
@@ -1240,7 +1266,7 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
                         const double r64 = bh ? (double)rB : ref_dist(ax, ay, az, cx, cy, cz, rdx, rdy, rdz);
                         const int hb_bin = min(max(0, (int)((r64 - 1.10) * 128.0)), AG_NEINT - 1);
                         const float4 v = reinterpret_cast<const float4 *>(
-                            tab + ((size_t)p.hydrogen_type * AG_NEINT + hb_bin) * ROW)[Q - 1];
+                            tab + ((size_t)p.hydrogen_type * kNearRows + hb_bin) * ROW)[Q - 1];
                         Eh[0] = v.x; Eh[1] = v.y; Eh[2] = v.z; Eh[3] = v.w;
                     }
     #pragma unroll
@@ -1534,7 +1560,7 @@ __global__ void __launch_bounds__(256) k_audit(AuditParams p) {
                 far_flips += min(fb, AG_NDIEL - 1) != b64;
             } else {
                 const float dxf = (float)dx, dyf = (float)dy, dzf = (float)dz;
-                const float r2 = fmaxf(__builtin_fmaf(dxf, dxf, __builtin_fmaf(dyf, dyf, dzf * dzf)), 1.0e-12f);
+                const float r2 = __builtin_fmaf(dxf, dxf, __builtin_fmaf(dyf, dyf, __builtin_fmaf(dzf, dzf, 1.0e-14f)));
                 const float g = r2 * __builtin_amdgcn_rsqf(r2) * 128.f;
                 if (fabsf(g - rintf(g)) >= kGuardBins && min((int)g, AG_NDIEL - 1) != b64) near_bad++;
             }
@@ -2401,10 +2427,12 @@ static int hb_case(int mh, int ah) {
 }
 
 static void launch_near(const ag_plan &p, int grid, const NearParams &np, hipStream_t st) {
+    // the plain form takes a band that stays past 8 A (spacings up to about 50 A)
+    const bool wide = std::any_of(p.confs.begin(), p.confs.end(), [](const ConfDev &c) { return c.near_band > 0.9f; });
 #define AG_NEAR(NP, CB)                                                                 \
     do {                                                                                \
         if (p.paged) k_near<NP, CB, kNearPaged><<<grid, kNearThreads, 0, st>>>(np);     \
-        else if (np.bhtree || np.cmap || p.any_disorder)                                \
+        else if (np.bhtree || np.cmap || p.any_disorder || wide)                        \
             k_near<NP, CB, kNearGeneral><<<grid, kNearThreads, 0, st>>>(np);            \
         else k_near<NP, CB, kNearPlain><<<grid, kNearThreads, 0, st>>>(np);             \
     } while (0)
@@ -2956,10 +2984,11 @@ static ag_plan *plan_build(ag_ctx *c, int n, const ag_receptor *recs, const ag_g
         if (!placed) ag::fail(AG_ERR_UNSUPPORTED, "near-kernel slot assignment left a map without a slot");
     }
     p.nplain = nplain_max <= 4 ? 4 : (nplain_max <= 8 ? 8 : 12);
-    // rows of near_row slots per bin, and one row of zeros after the last group
+    // rows of near_row slots: the bins, zeros past the cutoff, and the last bin's
+    // again for 8 A exactly
     const int row = near_row(p.nplain);
-    const size_t gstride = (size_t)(T > 0 ? T : 1) * AG_NEINT * row;
-    std::vector<float> gtab(gstride * p.groups + row, 0.f);
+    const size_t gstride = (size_t)(T > 0 ? T : 1) * kNearRows * row;
+    std::vector<float> gtab(gstride * p.groups, 0.f);
     for (int g = 0; g < p.groups; g++) {
         for (int t = 0; t < T; t++)
             for (int j = 0; j < kMapSlots; j++) {
@@ -2969,8 +2998,9 @@ static ag_plan *plan_build(ag_ctx *c, int n, const ag_receptor *recs, const ag_g
                 if (m < 0 || !(map_role(ms, m) & ROLE_AFF)) continue;
                 const float *srcrow = tab->e_vdw_hb + ((size_t)t * M + m) * AG_NEINT;
                 const int at = j < kPlainSlots ? j : row - 4 + (j - kPlainSlots);
-                float *dst = gtab.data() + g * gstride + (size_t)t * AG_NEINT * row + at;
+                float *dst = gtab.data() + g * gstride + (size_t)t * kNearRows * row + at;
                 for (int k = 0; k < AG_NEINT; k++) dst[(size_t)k * row] = srcrow[k];
+                dst[(size_t)kNearExactRow * row] = srcrow[AG_NEINT - 1];
             }
     }
     float *d_tab = upload(st, p.tab, gtab.data(), gtab.size());
@@ -3025,7 +3055,6 @@ static ag_plan *plan_build(ag_ctx *c, int n, const ag_receptor *recs, const ag_g
             }
         }
         q.tab = d_tab + g * gstride;
-        q.zero_off = (unsigned)(sizeof(float) * gstride * (p.groups - g));
         q.e_slot = (g == 0 && !vina) ? ms->elec_index : -1;
         q.d_slot = (g == 0 && !vina) ? ms->dsolv_index : -1;
         q.has_affinity = used || q.d_slot >= 0;
