@@ -309,8 +309,9 @@ ag_status ag_plan_audit(ag_plan *plan, ag_audit *out);
 
 /* Milliseconds of the last execute on ctx: [0] cell list, [1] near-field
  * kernel(s), [2] far-field kernel, by the device's clock (a small plan makes
- * its cell list inside the far-field kernel), [3] total, from HIP events on
- * ctx's stream. */
+ * its cell list inside the far-field kernel, and where near and far field run
+ * beside each other, in a constant dielectric, [1] is both), [3] total, from
+ * HIP events on ctx's stream. */
 ag_status ag_context_timing(ag_ctx *ctx, float ms[4]);
 
 /* ------------------------------------------------------------------------ */

@@ -126,3 +126,18 @@ def test_more_plans_than_reports(base):
         assert np.array_equal(run(plans[-1]), first)
         for p in plans:
             p.close()
+
+
+@pytest.mark.parametrize("n, n1", [(500, (41, 42, 43)), (1500, (81, 33, 80)), (9000, (97, 65, 66))])
+def test_far_field_beside(base, n, n1):
+    """In a constant dielectric the far field runs beside the near one for a map
+    set on the device, and behind it for one copied to the host."""
+    print(f"[gpu] far beside {n} {n1}", flush=True)
+    st = dataclasses.replace(state(base, n, n1, (n / 0.068) ** (1 / 3), n), dddiel=0, inv_diel_cal=332.0 / 4.0, _keep=[])
+    with ag.Context(0) as ctx:
+        host = np.asarray(ctx.maps_plain(st)).reshape(-1)
+        with ctx.plan(st) as plan, Dev(host.nbytes) as out:
+            for _ in range(3):
+                out.put(np.full(host.size, np.nan, np.float32))
+                plan.execute(out.p.value)
+                assert np.array_equal(out.get(host.size), host)
