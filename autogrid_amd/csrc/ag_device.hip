@@ -355,17 +355,14 @@ __global__ void k_cell_count(const ConfDev *confs, const int *atom_conf, int n, 
     if (cell >= 0) atomicAdd(&count[cell], 1);
 }
 
-// Clears the cell counts and cursors [0, n), the status word and the nq
+// Clears the cell counts [0, n), the status word and the nq
 // work counters of one map set, in one launch: a kernel rather than memset
 // nodes, since a plan's map set is captured in a graph.
-__global__ void k_zero_cells(int *count, int *cursor, int n, int *status, int *queue, int nq,
+__global__ void k_zero_cells(int *count, int n, int *status, int *queue, int nq,
                              unsigned long long *stamp) {
     stamp_start(stamp);
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) {
-        count[i] = 0;
-        cursor[i] = 0;
-    }
+    if (i < n) count[i] = 0;
     if (i < nq) queue[i] = 0;
     if (i == 0) *status = 0;
 }
@@ -442,12 +439,13 @@ __global__ void __launch_bounds__(1024) k_scan(const int *count, int *start, int
     if (t == 0) start[n] = carry;
 }
 
-__global__ void k_cell_scatter(int n, const int *atom_cell, const int *start, int *cursor, int *slot_atom) {
+// Counts the cells down again (k_gather finds the order within a cell).
+__global__ void k_cell_scatter(int n, const int *atom_cell, const int *start, int *count, int *slot_atom) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     int cell = atom_cell[i];
     if (cell < 0) return;
-    int pos = start[cell] + atomicAdd(&cursor[cell], 1);
+    int pos = start[cell] + atomicSub(&count[cell], 1) - 1;
     slot_atom[pos] = i;
 }
 
@@ -2244,7 +2242,7 @@ struct ag_plan {
     DevBuf confs_d{pool}, brick_prefix_d{pool}, tile_prefix_d{pool}, atom_conf_d{pool}, queue_d{pool};
     DevBuf coord{pool}, charge{pool}, vol{pool}, solpar{pool}, rvec{pool}, rvec2{pool}, type{pool}, hbond{pool},
         rexp{pool}, disorder{pool};
-    DevBuf atom_cell{pool}, cell_count{pool}, cell_start{pool}, cell_cursor{pool}, slot_atom{pool},
+    DevBuf atom_cell{pool}, cell_count{pool}, cell_start{pool}, slot_atom{pool},
         near_atoms{pool}, far_atoms{pool}, fmin_atoms{pool};
     DevBuf tab{pool}, sol{pool}, reps{pool}, far_part{pool}, far_box{pool}, far_wide{pool}, status{pool};
     DevBuf collide{pool};              // tree build: collision mask per point
@@ -2772,7 +2770,6 @@ static void plan_geometry(ag_plan &p, const ag_grid *grids, const int *natoms, c
     }
     p.cell_count.get(sizeof(int) * (size_t)p.total_cells);
     p.cell_start.get(sizeof(int) * ((size_t)p.total_cells + 1));
-    p.cell_cursor.get(sizeof(int) * (size_t)p.total_cells);
     p.confs_d.get(sizeof(ConfDev) * p.confs.size());
     p.brick_prefix_d.get(sizeof(int) * p.brick_prefix.size());
     p.tile_prefix_d.get(sizeof(int) * p.tile_prefix.size());
@@ -3218,7 +3215,7 @@ static void enqueue(ag_plan *p, float *d_maps, float *d_fmap, int32_t *d_cmap, b
     const int N = p->N;
     const int tpb = 256;
     int *d_atom_cell = (int *)p->atom_cell.ptr, *d_count = (int *)p->cell_count.ptr;
-    int *d_start = (int *)p->cell_start.ptr, *d_cursor = (int *)p->cell_cursor.ptr;
+    int *d_start = (int *)p->cell_start.ptr;
     int *d_slot_atom = (int *)p->slot_atom.ptr;
     int *d_status = p->overflow_flag();
     int *d_queue = (int *)p->queue_d.ptr;
@@ -3254,13 +3251,13 @@ static void enqueue(ag_plan *p, float *d_maps, float *d_fmap, int32_t *d_cmap, b
             k_cells<<<1, 1024, 0, st>>>(cp);
         } else {
             k_zero_cells<<<std::max(cgrid, (unsigned)((kMaxChunks + tpb - 1) / tpb)), tpb, 0, st>>>(
-                d_count, d_cursor, p->total_cells, d_status, d_queue, kMaxChunks, stamp(kStampFirst));
+                d_count, p->total_cells, d_status, d_queue, kMaxChunks, stamp(kStampFirst));
             if (N > 0)
                 k_cell_count<<<(N + tpb - 1) / tpb, tpb, 0, st>>>(d_confs, atom_conf, N, p->tune.cell_size,
                                                                   (const double *)p->coord.ptr, d_atom_cell, d_count);
             k_scan<<<1, 1024, 0, st>>>(d_count, d_start, p->total_cells);
             if (N > 0)
-                k_cell_scatter<<<(N + tpb - 1) / tpb, tpb, 0, st>>>(N, d_atom_cell, d_start, d_cursor, d_slot_atom);
+                k_cell_scatter<<<(N + tpb - 1) / tpb, tpb, 0, st>>>(N, d_atom_cell, d_start, d_count, d_slot_atom);
         }
         if (N > 0)
             k_gather<<<(N + tpb - 1) / tpb, tpb, 0, st>>>(p->total_cells, d_atom_cell, d_start, d_slot_atom, p->src,
