@@ -58,7 +58,6 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 FP32_PEAK_TFLOPS = 157.3          # MI355X FP32 vector, packed
-FP32_PEAK_NONPACKED_TFLOPS = 78.6
 FLOPS_PER_PAIR_E = 16
 
 
@@ -215,17 +214,17 @@ def cpu_leg(st, gpu_maps, map_files, large: bool = True, vina=None) -> dict:
 TRAFFIC_PROFILE = "profiles/full_mapset_5000atoms_127cubed.md"
 
 
-def profiled_traffic():
-    """HBM bytes per k_far launch on the full workload, from the committed
-    rocprofv3 FETCH_SIZE / WRITE_SIZE runs (calibrated by a device copy);
-    None when the summary is missing."""
+def profiled(name):
+    """A figure of k_far on the full workload from the committed rocprofv3
+    summary (HBM bytes per launch from FETCH_SIZE / WRITE_SIZE, calibrated by
+    a device copy; the issuing share from SQ_INSTS_VALU); None when missing."""
     import re
     try:
         with open(os.path.join(ROOT, TRAFFIC_PROFILE)) as f:
-            m = re.search(r"traffic_bytes_per_launch k_far: (\d+)", f.read())
+            m = re.search(re.escape(name) + r": ([0-9.]+)", f.read())
     except OSError:
         return None
-    return int(m.group(1)) if m else None
+    return float(m.group(1)) if m else None
 
 
 def batched_leg(reps: int = 2) -> dict:
@@ -393,7 +392,7 @@ def large_leg(reps: int = 3) -> dict:
                                                "far": far},
             "far_pairs": far_pairs,
             "pair_evals_per_s": far_pairs / (far * 1e-3),
-            "far_tflops": FLOPS_PER_PAIR_E * far_pairs / (far * 1e-3) / 1e12}
+            "far_equivalent_tflops": FLOPS_PER_PAIR_E * far_pairs / (far * 1e-3) / 1e12}
 
 
 def protein_leg(reps: int = 5) -> dict:
@@ -719,7 +718,7 @@ def main():
         t_k = sum(cell_ms) / len(cell_ms) + sum(near_ms) / len(near_ms) + far_avg
         ach = ms_flops / (t_k * 1e-3) / 1e12
         map_set_roofline = {"achieved": ach, "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
-                            "frac": ach / FP32_PEAK_TFLOPS, "frac_nonpacked_peak": ach / FP32_PEAK_NONPACKED_TFLOPS,
+                            "frac": None,   # an equivalent rate, as the far kernel's
                             "flops": ms_flops, "kernels_ms": t_k,
                             "flops_rule": f"16 W_E + F_A W_A, W_E = P*N, W_A = pairs within 8 A (oracle count), "
                                           f"F_A = 16 + 4*{n_aff} maps" + (" + 2 (d map)" if st.dsolv_index >= 0 else "")}
@@ -735,13 +734,17 @@ def main():
                    "atoms": N, "points": P, "maps": st.n_maps},
         "roofline": {"bound": "valu", "kernel": "k_far (electrostatics, all atoms beyond the near field)",
                      "achieved": achieved, "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
-                     "frac": achieved / FP32_PEAK_TFLOPS,
-                     "frac_nonpacked_peak": achieved / FP32_PEAK_NONPACKED_TFLOPS,
+                     "frac": None,
+                     "achieved_is": "an equivalent rate: the all-pairs rule's FLOPs over the launch. Atoms away "
+                                    "from a patch are summed at its nodes and interpolated, so the rate may pass "
+                                    "the peak and is no fraction of it; valu_issue_frac is the share of the "
+                                    "launch in which the vector unit issues, from the committed counters",
+                     "valu_issue_frac": profiled("valu_issue_fraction k_far") if args.workload == "full" else None,
                      "flops_per_launch": flops,
                      "flops_rule": "16 per far-field (point, atom) pair: the audit's far_pairs, FP32 bin >= 1025 "
                                    "(the near-field pairs the kernel passes over are not counted)",
                      "avg_launch_ms": far_avg,
-                     "traffic": profiled_traffic() if args.workload == "full" else None,
+                     "traffic": profiled("traffic_bytes_per_launch k_far") if args.workload == "full" else None,
                      "traffic_source": TRAFFIC_PROFILE if args.workload == "full" else None},
         "map_set_roofline": map_set_roofline,
         "kernels_ms": {"cell_list": sum(cell_ms) / len(cell_ms), "near": sum(near_ms) / len(near_ms),
