@@ -165,11 +165,8 @@ struct PlaceParams {
     int *clear;                 // counts of the last sort's last pass, 256 per 256 atoms
 };
 
-__global__ void __launch_bounds__(kST) k_score_place(PlaceParams p) {
-    const int a = blockIdx.x * kST + threadIdx.x;
-    static_assert(kSortTile == 8 * kST && kST == 256, "a workgroup's corners are a tile");
-    p.clear[a] = 0;
-    if (a >= p.n) return;
+// An atom's place on the grid and its eight corners' pairs.
+__device__ __forceinline__ void place_atom(const PlaceParams &p, int a, int *bin) {
     double g[3];
     bool inside = true;
     for (int d = 0; d < 3; d++) {
@@ -197,8 +194,21 @@ __global__ void __launch_bounds__(kST) k_score_place(PlaceParams p) {
                                    : p.P;
         const uint2 pair = make_uint2(pt, 8u * a + c);
         p.pair[8 * (size_t)a + c] = pair;
-        sort_count(p.first, pair, 8 * a + c);
+        atomicAdd(&bin[sort_digit(p.first, pair)], 1);
     }
+}
+
+__global__ void __launch_bounds__(kST) k_score_place(PlaceParams p) {
+    const int a = blockIdx.x * kST + threadIdx.x;
+    static_assert(kSortTile == 8 * kST && kST == 256, "a workgroup's corners are a tile");
+    // the tile's digits for the first pass, counted in LDS
+    __shared__ int bin[256];
+    bin[threadIdx.x] = 0;
+    p.clear[a] = 0;
+    __syncthreads();
+    if (a < p.n) place_atom(p, a, bin);
+    __syncthreads();
+    p.first.count[a] = bin[threadIdx.x];
 }
 
 // count[b][d] -> pairs of smaller digits plus digit d's of earlier blocks.  One
