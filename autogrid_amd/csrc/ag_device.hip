@@ -240,8 +240,8 @@ struct FarParams {
 // Consecutive workgroup ids go round-robin over the 8 XCDs; here XCD x takes
 // chunks x, x + 8, x + 16, ... of C consecutive items, so that every XCD
 // gets items from all over the grid (the work per item varies with the
-// local atom density, and in the far kernel's table-free path with the
-// distance to the atoms) while the items of a chunk share its L2.  Ids past
+// local atom density, and in the far kernel with the distance to the
+// atoms) while the items of a chunk share its L2.  Ids past
 // the last whole round of 8 chunks map to themselves.
 template <int C>
 __device__ __forceinline__ int xcd_chunked(int bid, int nblocks) {
@@ -355,7 +355,7 @@ __global__ void k_cell_count(const ConfDev *confs, const int *atom_conf, int n, 
     if (cell >= 0) atomicAdd(&count[cell], 1);
 }
 
-// Clears the cell counts [0, n), the status word and the nq
+// Clears the cell counts [0, n), the overflow word and the nq
 // work counters of one map set, in one launch: a kernel rather than memset
 // nodes, since a plan's map set is captured in a graph.
 __global__ void k_zero_cells(int *count, int n, int *status, int *queue, int nq,
@@ -648,18 +648,18 @@ __device__ __forceinline__ int group_lane(int v) {
     return __builtin_amdgcn_mov_dpp(v, ctrl, 0xf, 0xf, true);
 }
 
-// Bound by its vector operations (issued in about 85 % of the cycles; 60 per
-// pair of a wave and a plain atom, 100 to 150 where the atom is directional),
-// then by the table reads.  5,000 atoms, 127^3 points: 13 Vina maps
-// 1,096 -> 712 us, 15 AutoDock maps 1,099 -> 812; 41^3 points and 1,000 atoms 157
-// -> 62.  CUBE selects the lane layout inside the brick (brick_lane).  FORM:
+// With 32-byte rows bound by its vector operations (49 per pair of a wave and a
+// plain atom, 90 to 140 where the atom is directional), with 64-byte rows by the
+// vector caches: 13 Vina maps make 4.3e8 accesses, 0.70 ms at one per clock and
+// CU.  5,000 atoms, 127^3 points: 13 Vina maps 1,096 -> 746 us, 15 AutoDock maps
+// 1,099 -> 854; 41^3 points and 1,000 atoms 157 -> 61.  CUBE selects the lane layout inside the brick (brick_lane).  FORM:
 //   kNearPlain   neither the tree build's queries, a constriction count
 //                nor disordered hydroxyls (their branches compiled out);
 //   kNearGeneral every map-set option;
 //   kNearPaged   every option, and candidate / donor-H lists longer than
 //                one LDS page.
 // The unpaged forms leave a brick whose candidates (or donor H) do not fit
-// one LDS list: they set the status word, and the host runs the whole map
+// one LDS list: they set the overflow word, and the host runs the whole map
 // set again with the paged form (whose page loops keep state beside the
 // accumulators, with spills the common case should not pay for).
 enum : int { kNearPlain = 0, kNearGeneral = 1, kNearPaged = 2 };
