@@ -942,6 +942,18 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
         }
     }
 
+    // With 64-byte rows a lane keeps its H's bond vector in the H list, which is
+    // done with, for the donor hydrogens among the candidates: in registers two of
+    // its components went to scratch (whole map set of 127^3 points 1,618 -> 1,600
+    // us).  With 32-byte rows there are registers for it (47 x 83 x 119 points 428 us,
+    // 435 from LDS).
+    constexpr bool H_IN_LDS = NPLAIN > 4;
+    if constexpr (H_IN_LDS) {
+        static_assert(kHCap >= kNearThreads, "a bond vector per thread");
+        __syncthreads();
+        hrvs[tid][0] = hrv[0]; hrvs[tid][1] = hrv[1]; hrvs[tid][2] = hrv[2];
+    }
+
     // The point indices are formed again from the thread index where they
     // are needed after this point (a rare branch of the candidate loop and
     // the stores), so three indices do not stay live across the loop: one
@@ -1197,7 +1209,8 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
                                 const float c2 = cos_t * cos_t;
                                 racc = rexp == 2 ? c2 : (rexp == 4 ? c2 * c2 : cos_t);
                                 if (aidx != best_idx) {
-                                    float ct = hrv[0] * rv0 + hrv[1] * rv1 + hrv[2] * rv2;
+                                    const float *const h = H_IN_LDS ? hrvs[tid] : hrv;
+                                    float ct = h[0] * rv0 + h[1] * rv1 + h[2] * rv2;
                                     Hramp = hramp_value(__builtin_amdgcn_fmed3f(ct, -1.f, 1.f));
                                 }
                             }
