@@ -1661,6 +1661,13 @@ struct ag_analytic {
 
 namespace agdev {
 
+// The adjoint's work is on all three of the context's streams.
+static void wait_streams(ag_ctx *c) {
+    (void)hipStreamSynchronize(c->stream);
+    (void)hipStreamSynchronize(c->stream2);
+    (void)hipStreamSynchronize(c->copy_stream);
+}
+
 // (probe class, atom class) -> case of main.cpp:3286-3374 without disorder.
 static int an_case(int mh, int ah) {
     const bool atom_don = (ah == 1 || ah == 2 || ah == 6);
@@ -1743,7 +1750,7 @@ ag_analytic *analytic_create(ag_ctx *c, const ag_receptor *rec, const ag_grid *g
 void analytic_destroy(ag_analytic *a) {
     if (!a) return;
     (void)hipSetDevice(a->ctx->device);
-    (void)hipStreamSynchronize(a->ctx->stream);
+    wait_streams(a->ctx);
     delete a;
 }
 
@@ -2122,14 +2129,37 @@ void analytic_adjoint(ag_analytic *a, const float *d_dmaps, double *g_coord, dou
     if (!a->uploaded || !a->last_maps) ag::fail(AG_ERR_BAD_INPUT, "ag_analytic_adjoint needs a forward first");
     hipStream_t st = c->stream;
     const int N = a->N, T = a->T, M = a->M;
-    const unsigned grid = (unsigned)((a->P + kAT - 1) / kAT);
     AParams p = a->ap;
     p.dmaps = d_dmaps;
-    HIP_CHECK(hipEventRecord(c->ev[0], st));
     const int nh = (int)a->h_atoms.size(), nl = (int)a->atom_list.size();
+    const bool want_e = a->elec >= 0 && N > 0;
+    // all buffers before the first launch: a failed allocation leaves no kernel
+    // behind that reads the caller's cotangent
     float *d_hout = (float *)a->d_hout.get(sizeof(float) * 3 * (size_t)std::max(nh, 1));
     float *d_aout = (float *)a->d_aout.get(sizeof(float) * kAtomOut * (size_t)std::max(nl, 1));
     double *d_eout = (double *)a->d_eout.get(sizeof(double) * 4 * (size_t)std::max(N, 1));
+    const size_t hb = UploadPack::padded(sizeof(float) * 3 * (size_t)nh), ab = UploadPack::padded(sizeof(float) * kAtomOut * (size_t)nl);
+    char *const stage = (char *)a->stage.get(hb + ab + sizeof(double) * 4 * (size_t)std::max(N, 1));
+    const float *const hout = (const float *)stage, *const aout = (const float *)(stage + hb);
+    const double *const eout = (const double *)(stage + hb + ab);
+    const int row_words = (a->grid.n1[0] + 63) / 64;
+    const long long words = (long long)row_words * a->grid.n1[1] * a->grid.n1[2];
+    const int nblk = (int)((a->P + kGPack - 1) / kGPack);   // packing blocks
+    const size_t pack_counts = sizeof(int) * (2 * (size_t)nblk + 1), packed_points = sizeof(int) * (size_t)a->P;
+    unsigned long long *const bits = nl > 0 ? (unsigned long long *)a->d_gmask.get(sizeof(unsigned long long) * (size_t)words) : nullptr;
+    int *const vcounts = nh > 0 ? (int *)a->d_vcount.get(pack_counts) : nullptr;
+    int *const vlist = nh > 0 ? (int *)a->d_vpack.get(packed_points) : nullptr;
+    int *const gcounts = want_e ? (int *)a->d_gcount.get(pack_counts) : nullptr;
+    int *const packed = want_e ? (int *)a->d_gpack.get(packed_points) : nullptr;
+    // whatever else throws, no stream is left working on the caller's cotangent
+    // or the staging buffer
+    struct Join {
+        ag_ctx *c;
+        ~Join() {
+            if (c) wait_streams(c);
+        }
+    } join{c};
+    HIP_CHECK(hipEventRecord(c->ev[0], st));
     // Two independent chains: the atom gather, which waits for scattered reads
     // most of its time, and beside it on the second stream the bond-vector
     // cotangent and the e map's adjoint (one after the other they took 860 us of a
@@ -2138,20 +2168,13 @@ void analytic_adjoint(ag_analytic *a, const float *d_dmaps, double *g_coord, dou
     const hipStream_t s2 = c->stream2;
     HIP_CHECK(hipEventRecord(c->cells_ev, st));
     HIP_CHECK(hipStreamWaitEvent(s2, c->cells_ev, 0));
-    const bool want_e = a->elec >= 0 && N > 0;
-    const size_t hb = UploadPack::padded(sizeof(float) * 3 * (size_t)nh), ab = UploadPack::padded(sizeof(float) * kAtomOut * (size_t)nl);
-    char *const stage = (char *)a->stage.get(hb + ab + sizeof(double) * 4 * (size_t)std::max(N, 1));
-    const float *const hout = (const float *)stage, *const aout = (const float *)(stage + hb);
-    const double *const eout = (const double *)(stage + hb + ab);
     if (nl > 0) {
         AtomAdjParams q;
         q.a = p;
         q.by_index = a->by_index;
         q.atom_list = a->alist_d;
         q.out = d_aout;
-        q.words = (a->grid.n1[0] + 63) / 64;
-        const long long words = (long long)q.words * a->grid.n1[1] * a->grid.n1[2];
-        unsigned long long *bits = (unsigned long long *)a->d_gmask.get(sizeof(unsigned long long) * (size_t)words);
+        q.words = row_words;
         k_an_gmask<<<(unsigned)((words + kAT / 64 - 1) / (kAT / 64)), kAT, 0, st>>>(p, q.words, bits);
         q.bits = bits;
         if (a->naff <= 4) k_an_atom<4><<<nl, kAT, 0, st>>>(q);
@@ -2161,22 +2184,16 @@ void analytic_adjoint(ag_analytic *a, const float *d_dmaps, double *g_coord, dou
     HIP_CHECK(hipEventRecord(c->near_ev, st));
     if (nh > 0) {
         k_an_vh<<<cube_count(a->grid), kAT, 0, s2>>>(p);
-        const int nblk = (int)((a->P + kGPack - 1) / kGPack);
-        int *counts = (int *)a->d_vcount.get(sizeof(int) * (2 * (size_t)nblk + 1));
-        int *vlist = (int *)a->d_vpack.get(sizeof(int) * (size_t)a->P);
-        pack_points(NonzeroVh{p.vh}, a->P, counts, counts + nblk, vlist, s2);
-        HsumParams hp{p.closest_h, p.vh, vlist, counts + 2 * nblk, a->hatoms_d, d_hout};
+        pack_points(NonzeroVh{p.vh}, a->P, vcounts, vcounts + nblk, vlist, s2);
+        HsumParams hp{p.closest_h, p.vh, vlist, vcounts + 2 * nblk, a->hatoms_d, d_hout};
         k_an_hsum<<<nh, kAT, 0, s2>>>(hp);
     }
     HIP_CHECK(hipEventRecord(c->far_ev, s2));
     if (want_e) {
         EParams e = a->ep;
         e.ge = d_dmaps + (size_t)a->elec * a->P;
-        const int nblk = (int)((a->P + kGPack - 1) / kGPack);
-        int *counts = (int *)a->d_gcount.get(sizeof(int) * (2 * (size_t)nblk + 1));
-        int *offs = counts + nblk;
-        int *packed = (int *)a->d_gpack.get(sizeof(int) * (size_t)a->P);
-        pack_points(NonzeroE{e.ge}, a->P, counts, offs, packed, s2);
+        int *const offs = gcounts + nblk;
+        pack_points(NonzeroE{e.ge}, a->P, gcounts, offs, packed, s2);
         const dim3 eg((unsigned)((N + 63) / 64), (unsigned)a->nchunks);
         if (a->dddiel) k_an_eadj<true><<<eg, 64, 0, s2>>>(e, packed, offs + nblk);
         else k_an_eadj<false><<<eg, 64, 0, s2>>>(e, packed, offs + nblk);
@@ -2192,11 +2209,6 @@ void analytic_adjoint(ag_analytic *a, const float *d_dmaps, double *g_coord, dou
     if (nh) HIP_CHECK(hipMemcpyAsync(stage, d_hout, sizeof(float) * 3 * (size_t)nh, hipMemcpyDeviceToHost, c->copy_stream));
     HIP_CHECK(hipStreamWaitEvent(c->copy_stream, c->near_ev, 0));
     if (nl) HIP_CHECK(hipMemcpyAsync(stage + hb, d_aout, sizeof(float) * kAtomOut * (size_t)nl, hipMemcpyDeviceToHost, c->copy_stream));
-    // (an exception would leave the e adjoint's copy without its target)
-    struct Join {
-        hipStream_t st;
-        ~Join() { (void)hipStreamSynchronize(st); }
-    } join{st};
     HIP_CHECK(hipStreamSynchronize(c->copy_stream));
     // assemble in FP64
     std::vector<double> gx(3 * (size_t)N, 0.0), grv(3 * (size_t)N, 0.0), grv2(3 * (size_t)N, 0.0), gq(N, 0.0);
@@ -2224,7 +2236,8 @@ void analytic_adjoint(ag_analytic *a, const float *d_dmaps, double *g_coord, dou
     }
     // bond vectors -> coordinates
     ag::bond_vectors_vjp(N, a->coord.data(), a->recipes.data(), grv.data(), grv2.data(), gx.data());
-    HIP_CHECK(hipStreamSynchronize(st));
+    HIP_CHECK(hipStreamSynchronize(st));   // and with it stream2
+    join.c = nullptr;
     HIP_CHECK(hipEventElapsedTime(&c->last_ms[3], c->ev[0], c->ev[3]));
     double gwe = 0.0;
     for (int i = 0; want_e && i < N; i++) {
