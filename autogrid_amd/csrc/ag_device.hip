@@ -1999,11 +1999,11 @@ __global__ void __launch_bounds__(kFarThreads) __attribute__((amdgpu_waves_per_e
         const float d1 = sreg(hx * far_node5(3)), d2 = sreg(hx * far_node5(4));
         const float d1q = sreg(d1 * d1), d2q = sreg(d2 * d2);
         float s[kFarK], c[kFarK], part[kFarK];
-        float ns[kFarNx], np[kFarNx];
+        double ns[kFarNx];
 #pragma unroll
         for (int k = 0; k < kFarK; k++) s[k] = c[k] = part[k] = 0.f;
 #pragma unroll
-        for (int i = 0; i < kFarNx; i++) ns[i] = np[i] = 0.f;
+        for (int i = 0; i < kFarNx; i++) ns[i] = 0.;
         float4 *const strip = reinterpret_cast<float4 *>(X) + 64 * wave;
         float *const level_r2 = X + 4 * 64 * kFarWaves + kFarLevels * wave;   // the wave's copy
         if (lane < kFarLevels) level_r2[lane] = reinterpret_cast<const float *>(&p.confs[ci].far_r2)[lane];
@@ -2012,7 +2012,7 @@ __global__ void __launch_bounds__(kFarThreads) __attribute__((amdgpu_waves_per_e
         const FarAtom *const atoms = p.atoms + cf.atom_base;
         const int n_atoms = cf.n_atoms;
         const int step = 64 * kFarWaves * cf.far_split;
-        int n_part = 0, n_node = 0;   // atoms in part[] and np[] since they were last flushed
+        int n_part = 0;   // atoms in part[] since it was last flushed
         const int a_first = 64 * (part_i * kFarWaves + wave);
         // the coarse box's atoms are in its own sums
         const unsigned long long *box_mask = nullptr;
@@ -2061,6 +2061,9 @@ __global__ void __launch_bounds__(kFarThreads) __attribute__((amdgpu_waves_per_e
                     const int jy = jl & 3, jz = (jl >> 2) & 3;
                     const float ny = hy * ((jy & 2 ? 1.f : -1.f) * ((jy == 0 || jy == 3) ? kNode4a : kNode4b));
                     const float nz = hz * ((jz & 2 ? 1.f : -1.f) * ((jz == 0 || jz == 3) ? kNode4a : kNode4b));
+                    float np[kFarNx];
+#pragma unroll
+                    for (int j = 0; j < kFarNx; j++) np[j] = 0.f;
                     for (int i = 0; i < nf; i += 4) {
                         const float4 q = strip[i + (jl >> 4)];
                         const float dy = q.y - ny, dz = q.z - nz;
@@ -2080,15 +2083,10 @@ __global__ void __launch_bounds__(kFarThreads) __attribute__((amdgpu_waves_per_e
                         for (int j = 0; j < kFarNx; j++) np[j] = __builtin_fmaf(q.w, FLAT ? rs[j] : rs[j] * tv[j], np[j]);
                     }
                     wave_sync();   // the strip is rewritten for the next 64 atoms
-                    n_node += nf;
-                    if (n_node >= 4 * kFarAtomChunk) {
-                        n_node = 0;
+                    // (16 atoms of a lane at most: what a node's value loses here, the
+                    // points near the patch's ends get up to three times over)
 #pragma unroll
-                        for (int j = 0; j < kFarNx; j++) {
-                            ns[j] += np[j];
-                            np[j] = 0.f;
-                        }
-                    }
+                    for (int j = 0; j < kFarNx; j++) ns[j] += (double)np[j];
                 }
                 if (dir_set) {
                     n_part += __popcll(dir_set);
@@ -2122,7 +2120,7 @@ __global__ void __launch_bounds__(kFarThreads) __attribute__((amdgpu_waves_per_e
             double v[kFarNx];
 #pragma unroll
             for (int j = 0; j < kFarNx; j++) {
-                v[j] = (double)ns[j] + (double)np[j];
+                v[j] = ns[j];
                 v[j] += __shfl_xor(v[j], 16);
                 v[j] += __shfl_xor(v[j], 32);
             }
