@@ -2488,10 +2488,9 @@ struct FarShape {
 // the Mehler-Solmajer dielectric's steps (they fall by e in 3.2 A) 1.1 A.  The
 // near kernel has the pairs up to 8.01 A.
 static double far_floor_radius(bool flat, double spacing, int level, int nodes, double half_points) {
-    // coarse boxes: rho = z + sqrt(z^2 - 1) of the run's 7.5 (11) half-lengths to
-    // the power 5/8, for the same rho^-n
+    // (coarse boxes: far_boxes adds what their nodes need)
     const double half = half_points * spacing, g = std::pow(2.0, -level / (2.0 * nodes));
-    const double z = nodes == kBoxN ? (flat ? 3.52 : 2.80) : (flat ? 11.0 : 7.5);
+    const double z = nodes == kBoxN ? 1.0 : flat ? 11.0 : 7.5;
     if (flat) return std::max({8.25, 20.0 * g, (z * g - 1.0) * half});
     const double base = std::min(21.0, std::max(18.5, 26.0 - 20.0 * spacing)) - 1.1 * level;
     return std::max({8.25, base, (z * g - 1.0) * half});
@@ -2563,6 +2562,86 @@ static void far_radii(const std::vector<float> &reps, double spacing, int nodes,
     for (int l = 0; l < kFarLevels; l++) radius[l] = std::max(floor_r[l], ok[l]);
 }
 
+// The table as a function of the distance (A), over the distance.
+static double far_term(const std::vector<float> &reps, double r) {
+    const double y = std::min(std::max(r * 128.0 - 0.5, 0.0), (double)(AG_NDIEL - 1));
+    const int k = std::min((int)y, AG_NDIEL - 2);
+    return (reps[k] + (y - k) * ((double)reps[k + 1] - reps[k])) / r;
+}
+
+// Error of the interpolation from the given nodes over an axis of half-length
+// `half` (A), for an atom r off the box: ahead of it, beside its middle and beside its
+// end.
+static double far_axis_error(const std::vector<float> &reps, double r, double half, const double *node, int nodes) {
+    double worst = 0.0;
+    for (int place = 0; place < 3; place++) {
+        const auto f = [&](double t) {
+            return far_term(reps, place == 0 ? r + half * (1.0 + t) : std::hypot(r, half * (place == 1 ? t : 1.0 + t)));
+        };
+        double v[kBoxN];
+        for (int i = 0; i < nodes; i++) v[i] = f(node[i]);
+        for (int q = 0; q <= nodes; q++) {   // the ends and between the nodes
+            const double t = q == 0 ? -1.0 : q == nodes ? 1.0 : 0.5 * (node[q - 1] + node[q]);
+            double s = 0.0;
+            for (int i = 0; i < nodes; i++) {
+                double w = 1.0;
+                for (int j = 0; j < nodes; j++)
+                    if (j != i) w *= (t - node[j]) / (node[i] - node[j]);
+                s += w * v[i];
+            }
+            worst = std::max(worst, std::fabs(s - f(t)));
+        }
+    }
+    return worst;
+}
+
+// What interpolating an atom of unit charge leaves of its term, by its distance
+// from the box: the steps (a third of one each way) and the nodes' error.
+struct FarError {
+    const std::vector<float> &reps;
+    std::vector<float> step;      // largest step beyond k / 2 A, over the distance
+    explicit FarError(const std::vector<float> &tab) : reps(tab), step(129, 0.f) {
+        for (int k = 127; k >= 0; k--) {
+            float s = 0.f;
+            for (int b = std::max(64 * k, 1); b < 64 * (k + 1); b++) s = std::max(s, std::fabs(tab[b] - tab[b - 1]));
+            step[k] = std::max(step[k + 1], s / std::max(0.5f, 0.5f * (float)k));
+        }
+    }
+    double steps(double r) const { return step[std::min((int)(2.0 * r), 128)]; }
+};
+
+// The nodes' error of a box whose axes have the given half-lengths and nodes, and
+// with the steps' (a third of one each way), for an atom r off it.
+static double far_nodes_error(const FarError &e, double r, const double half[2], const int nodes[2]) {
+    static const double n4[4] = {-kNode4a, -kNode4b, kNode4b, kNode4a};
+    double nd[kBoxN], worst = 0.0;
+    for (int a = 0; a < 2; a++) {
+        for (int i = 0; i < nodes[a]; i++)
+            nd[i] = nodes[a] == kBoxN ? box_node(i) : nodes[a] == kFarNx ? (double)far_node5(i) : n4[i];
+        worst = std::max(worst, far_axis_error(e.reps, r, half[a], nd, nodes[a]));
+        if (nodes[1] == nodes[0]) break;   // (a box is as good as a cube)
+    }
+    return worst;
+}
+static double far_error(const FarError &e, double r, const double half[2], const int nodes[2]) {
+    return std::hypot(e.steps(r) / std::sqrt(12.0), far_nodes_error(e, r, half, nodes));
+}
+
+// Distances at which error(r) keeps to h0 2^(-n/2), h0 2^(-(n-1)/2), ...: from
+// `most` inwards to r0, so that nothing beyond a distance is worse.
+template <typename F>
+static void far_distances(F &&error, double r0, double most, double hop, double h0, int n, int levels, double *radius) {
+    for (int l = 0; l < levels; l++) radius[l] = std::max(most, r0);
+    int first = 0;   // levels before it have ended
+    for (double r = most; r > r0 && first < levels; r -= hop) {
+        const double h = error(r);
+        for (int l = first; l < levels; l++) {
+            if (h <= h0 * std::pow(2.0, 0.5 * (l - n))) radius[l] = r;
+            else if (l == first) first++;
+        }
+    }
+}
+
 static FarShape far_shape(const ag_grid &g, int n_atoms, const double radius[kFarLevels], const double *coord,
                           const double *charge, double coeff) {
     FarShape f;
@@ -2616,15 +2695,27 @@ static FarShape far_shape(const ag_grid &g, int n_atoms, const double radius[kFa
 // hold half as many again before a part of it worth the launches is beyond.
 // (5,000 atoms on 127^3 points, where that is 5,470: 794 us with boxes for 807; a
 // batch of twelve conformations of 1,500 to 6,000 atoms 5.19 ms for 4.96.)
-static void far_boxes(FarShape &f, const ag_grid &g, int n_atoms, const std::vector<float> &reps) {
+static void far_boxes(FarShape &f, const ag_grid &g, int n_atoms, const std::vector<float> &reps, const FarError &err) {
     f.box_py = std::max(1, (kBoxRows + f.py / 2) / f.py);
     f.box_pz = std::max(1, (kBoxRows + f.pz / 2) / f.pz);
     const int edge = std::max({kBoxRuns * kFarK, f.box_py * f.py, f.box_pz * f.pz});
     const double a = edge * g.spacing;
     const auto dilated = [&](double r) { return a * a * a + r * (6 * a * a + M_PI * r * (3 * a + 4. / 3. * r)); };
     if (n_atoms < 1.5 * 0.068 * dilated(18.5)) return;   // (no distance is less)
-    double radius[kFarLevels];
-    far_radii(reps, g.spacing, kBoxN, 0.5 * (edge - 1), radius);
+    // as far_radii has it for the table, and where its nodes leave half of what a
+    // level allows a patch.  (What counts is the atom ahead of a face: the two
+    // axes along it see the pole of 1/r beside them, at 1.8 half-edges 2.6e-5 of
+    // the term where a patch's run leaves 5e-6.)
+    const double patch_half[2] = {kFarMid * g.spacing, 0.5 * (std::max(f.py, f.pz) - 1) * g.spacing};
+    const double half[2] = {0.5 * (edge - 1) * g.spacing, 0.5 * (edge - 1) * g.spacing};
+    const int patch_nodes[2] = {kFarNx, kFarNy}, nodes[2] = {kBoxN, kBoxN};
+    const double r0 = std::sqrt((double)f.radius2[0]) / 128.0;   // a patch's level 0
+    double table[kFarLevels], radius[kFarLevels];
+    far_radii(reps, g.spacing, kBoxN, 0.5 * (edge - 1), table);
+    far_distances([&](double r) { return 2.0 * far_nodes_error(err, r, half, nodes); }, 8.25,
+                  std::max(30.0, 8.0 * half[0]), std::max(1.5, half[0] / 4.0), far_error(err, r0, patch_half, patch_nodes),
+                  0, kFarLevels, radius);
+    for (int l = 0; l < kFarLevels; l++) radius[l] = std::max(radius[l], table[l]);
     const double beyond = n_atoms - 0.068 * dilated(radius[0]);
     const double patches = (double)((g.n1[0] + kFarK - 1) / kFarK) * ((g.n1[1] + f.py - 1) / f.py) *
                            ((g.n1[2] + f.pz - 1) / f.pz);
@@ -3112,12 +3203,13 @@ static ag_plan *plan_build(ag_ctx *c, int n, const ag_receptor *recs, const ag_g
         FarAtom *d_far = (FarAtom *)p.far_atoms.get(sizeof(FarAtom) * (size_t)N);
         k_far_atoms<<<(N + 255) / 256, 256, 0, st>>>(N, d_coord, d_charge, ms->coeff_estat, d_far);
         HIP_CHECK(hipGetLastError());
+        const FarError err(reps);
         double radius[kFarLevels] = {}, spacing = -1.0;
         for (int i = 0, o = 0; i < n; o += natoms[i], i++) {
             if (grids[i].spacing != spacing) far_radii(reps, spacing = grids[i].spacing, kFarNx, kFarMid, radius);
             far_shapes.push_back(
                 far_shape(grids[i], natoms[i], radius, coord + 3 * (size_t)o, charge + o, ms->coeff_estat));
-            far_boxes(far_shapes.back(), grids[i], natoms[i], reps);
+            far_boxes(far_shapes.back(), grids[i], natoms[i], reps, err);
         }
         FarParams &fp = p.far;
         memset(&fp, 0, sizeof fp);

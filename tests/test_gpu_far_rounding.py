@@ -7,6 +7,8 @@ independent roundings of the terms add up to a multiple of it.
 """
 from __future__ import annotations
 
+import dataclasses
+
 import numpy as np
 import pytest
 
@@ -56,3 +58,34 @@ def test_node_sums(base, n_atoms, spacing):  # noqa: F811
     err, t = np.std(got - want), np.sqrt(np.mean(sq))
     out = 0.42 * U * np.sqrt(np.mean(want ** 2))      # the result's own rounding
     assert err <= np.hypot(2.05 * t, out), f"{err / t:.2f} u T"
+
+
+@pytest.mark.parametrize("spacing, constant", [(0.9, None), (0.75, 4.0)])
+def test_box_nodes(base, spacing, constant):  # noqa: F811
+    """One charge ahead of a coarse box's face, at the distances from which the box
+    takes it: its nodes leave no more than a patch's own at the distance from
+    which that interpolates (6.5 half-lengths of a run, 10 without table steps),
+    5.2e-6 of the term there (8.4e-7), once for each axis."""
+    print(f"[gpu] far box nodes {spacing} {constant}", flush=True)
+    n = 40000
+    st = state(base, n, (64, 64, 64), spacing, 50.0, n, constant=constant)
+    edge = 0.5 * 31 * spacing                               # half of a box of 32 points
+    far = (10.0 if constant else 6.5) * 7.5 * spacing
+    tab = np.asarray(st.r_eps if st.dddiel else np.full(8192, st.inv_diel_cal), np.float64)
+    q = np.zeros(n)
+    q[n // 2] = 1.0
+    pts = grid_points(st)
+    allowed = 3 * (8.4e-7 if constant else 5.2e-6) * abs(st.coeff_estat) * tab[min(int(128 * far), 8191)] / far
+    with ag.Context(0) as ctx:
+        for d in np.arange(1.3, 3.6, 0.15) * edge:          # from the face, in half-edges
+            x = st.coord.copy()
+            x[n // 2] = [edge - 32 * spacing, -32 * spacing - d, edge - 32 * spacing]
+            one = dataclasses.replace(st, coord=x, charge=q, _keep=[])
+            got = ctx.maps_plain(one)[0].reshape(-1)
+            box = np.all(pts < -0.5 * spacing, axis=1)      # the first box's points
+            r = np.linalg.norm(pts[box] - x[n // 2], axis=1)
+            b = np.minimum((128 * r).astype(int), 8190)
+            want = st.coeff_estat * tab[b] / r
+            off = st.coeff_estat * np.abs(tab[b] - tab[b + 1]) / r + 3e-7 * np.abs(want)   # a table step; FP32
+            err = np.abs(got[box] - want)
+            assert np.all(err <= allowed + np.abs(off)), (d, float((err / (allowed + np.abs(off))).max()))
