@@ -73,6 +73,8 @@ constexpr int kFarAtomChunk = 64;                 // Kahan block (at least)
 constexpr int kFarNx = 5, kFarNy = 4;             // interpolation nodes of a patch along x, and along y and z
 constexpr double kFarQRef = 0.85;                 // charge of level 0 over the conformation's rms charge
 constexpr int kFarLevels = 12;                    // charge levels, each with its own distance
+constexpr int kFarStrict = 20;                    // stricter levels before them, for patches far from the atoms
+constexpr int kReachTab = 256;                    // distances (half A) of k_far_reach's table
 constexpr int kFarSplitMax = 8;                   // workgroups that may share a patch's atoms
 constexpr int kBoxN = 8;                          // interpolation nodes of a coarse box along each axis
 constexpr int kBoxNodes = kBoxN * kBoxN * kBoxN;
@@ -127,13 +129,14 @@ struct ConfDev {
     int far_npy, far_npz;         // patches along y and z
     int far_split;                // workgroups sharing each patch's atoms
     int far_clamp;                // far kernel: a direct pair may pass the table's end
-    float far_r2[kFarLevels];     // squared distances (bins^2) from a patch's box past which atoms are interpolated
+    float far_r2[kFarStrict + kFarLevels];   // squared distances (bins^2) from a patch's box past which atoms are interpolated
     float far_qscale;             // an atom's level is that of |its far charge| times this (far_level)
     long long part_off;           // far_split > 1: offset of its [far_split][P] partial e maps
     int box_parts;                // coarse boxes: workgroups sharing one's atoms; 0: no coarse boxes
     int box_py, box_pz;           // patches of a box along y and z
     int box_n[3];                 // boxes per axis
-    float box_r2[kFarLevels];     // as far_r2, from a box
+    float box_r2[kFarStrict + kFarLevels];   // as far_r2, from a box
+    long long reach_off;          // offset of its patches' shifts (k_far_reach)
     long long box_off;            // offsets of its boxes' node sums ([box][part][kBoxNodes] doubles), of their
     long long box_mask_off;       // atom sets ([box][groups of 64 atoms]) and of its patches' node values
     long long box_patch_off;      // ([patch][kFarNodes] doubles)
@@ -233,6 +236,7 @@ struct FarParams {
     double *box_sums;             // coarse boxes (ConfDev::box_*)
     unsigned long long *box_mask;
     double *box_patch;
+    const unsigned char *shift;   // per patch, how many levels stricter its distances are (k_far_reach)
     int e_slot;
     unsigned long long *stamp;
 };
@@ -1653,11 +1657,12 @@ __device__ __forceinline__ void far_pair(const PlainF4 &at, float py, float pz, 
     for (int k = 0; k < kFarK; k++) part[k] = __builtin_fmaf(at.w, rs[k] * tv[k], part[k]);
 }
 
-// Level of an atom's charge over the conformation's: 0 for a ratio of sqrt(1/2)
-// or more, one more for each factor of sqrt(1/2), the last for all that are
-// smaller.
+// Place among the levels of an atom's charge over the conformation's: level 0
+// for ratios from sqrt(1/2) to 2 sqrt(2), one more for each factor of sqrt(1/2) below,
+// the last for all that are smaller, and one stricter for each factor of sqrt(2) above.
 __device__ __forceinline__ int far_level(float ratio) {
-    return min(max(126 - (int)(__float_as_uint(ratio * ratio) >> 23), 0), kFarLevels - 1);
+    const int l = 126 - (int)(__float_as_uint(ratio * ratio) >> 23);
+    return min(max(l > 0 ? l : min(l + 3, 0), -kFarStrict) + kFarStrict, kFarStrict + kFarLevels - 1);
 }
 
 // A wave-uniform value moved to a scalar register.
@@ -1737,20 +1742,30 @@ __device__ __forceinline__ double box_weight(int j, double t) {
 // atoms go one after the other, as the far kernel's direct pairs do.
 template <bool FLAT>
 __global__ void __launch_bounds__(kFarThreads) __attribute__((amdgpu_waves_per_eu(4))) k_far_boxes(FarParams p, int conf) {
-    __shared__ float T[FLAT ? kFarLevels : AG_NDIEL];
+    __shared__ float T[FLAT ? kFarStrict + kFarLevels : AG_NDIEL];
     __shared__ double XD[2 * kBoxNodes];   // 40 KiB in all: four workgroups per CU
     const AG_CONST ConfDev &cf = as_const(p.confs)[conf];
     const float flat = FLAT ? as_const(p.tab)[kFarLastBin] : 1.f;
     // the bins below the far kernel's are not read: the distances are there instead
     float *const level_r2 = T;
-    static_assert(kFarLevels <= kFarBinMin / 4 * 4, "room for the distances");
+    static_assert(kFarStrict + kFarLevels <= kFarBinMin / 4 * 4, "room for the distances");
     for (int i = kFarBinMin / 4 + threadIdx.x; !FLAT && i < AG_NDIEL / 4; i += kFarThreads)
         reinterpret_cast<float4 *>(T)[i] = reinterpret_cast<const float4 *>(p.tab)[i];
-    if (threadIdx.x < kFarLevels) level_r2[threadIdx.x] = reinterpret_cast<const float *>(&p.confs[conf].box_r2)[threadIdx.x];
-    __syncthreads();
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
     const int part = blockIdx.x % cf.box_parts, box = blockIdx.x / cf.box_parts;
     const int ibx = box % cf.box_n[0], iby = box / cf.box_n[0] % cf.box_n[1], ibz = box / cf.box_n[0] / cf.box_n[1];
+    // as strict as its strictest patch (every wave for itself; at most 2 x 5 x 5 patches)
+    int shift = 0;
+    {
+        const int r = ibx * kBoxRuns + lane % kBoxRuns, y = iby * cf.box_py + lane / kBoxRuns % cf.box_py,
+                  z = ibz * cf.box_pz + lane / (kBoxRuns * cf.box_py);
+        if (lane < kBoxRuns * cf.box_py * cf.box_pz && r < cf.runs_per_row && y < cf.far_npy && z < cf.far_npz)
+            shift = p.shift[cf.reach_off + r + (long long)cf.runs_per_row * (y + (long long)cf.far_npy * z)];
+        for (int o = 32; o > 0; o >>= 1) shift = max(shift, __shfl_xor(shift, o));
+    }
+    if (threadIdx.x < kFarStrict + kFarLevels)
+        level_r2[threadIdx.x] = reinterpret_cast<const float *>(&p.confs[conf].box_r2)[max((int)threadIdx.x - shift, 0)];
+    __syncthreads();
     const int nx = kBoxRuns * kFarK, ny = cf.box_py * cf.far_py, nz = cf.box_pz * cf.far_pz;   // points of the box
     const double bx = sreg(far_centre(ibx * nx, nx, cf.ne[0], cf.spacing)),
                  by = sreg(far_centre(iby * ny, ny, cf.ne[1], cf.spacing)),
@@ -1906,6 +1921,60 @@ __global__ void __launch_bounds__(64) k_far_down(FarParams p, int conf) {
     }
 }
 
+// How much stricter a patch's distances have to be.  Interpolation replaces the
+// table's steps by their mean, an error of a third of a step a pair, where the
+// sum pair by pair only puts one pair in 6,000 on the wrong side of a step.
+// Beside the pairs around a patch in or near the receptor that is nothing: their
+// steps are larger by more than that.  Away from it, it shows: in the shell 12
+// to 30 A outside, distances meant for the inside left up to 20 times the error
+// of the all-pairs sum.  So each patch finds the largest error a pair summed there
+// may have, max over the atoms of |charge| G(distance), and goes as many levels
+// of 2^(-1/2) stricter as that is below what level 0 leaves (far_shape makes the
+// table, 2 log2(level 0 / G) at each half A from the patch's centre).  A
+// workgroup takes 16 patches, each 16 lanes' group of its 1,024 threads another of
+// the atoms; once, when the plan is made, as it depends on the conformation
+// alone (20,000 atoms, 18,513 patches: 193 us, 5,000 and 2,048: 17).
+constexpr int kReachThreads = 1024, kReachPatches = 16;
+__global__ void __launch_bounds__(kReachThreads) k_far_reach(FarParams p, int conf, const float *tables, unsigned char *shift) {
+    constexpr int kParts = kReachThreads / kReachPatches;
+    __shared__ float table[kReachTab];
+    __shared__ float4 list[kReachThreads];   // x, y, z, level of the charge
+    __shared__ float least_s[kParts][kReachPatches];
+    const AG_CONST ConfDev &cf = as_const(p.confs)[conf];
+    const int own = threadIdx.x % kReachPatches, part = threadIdx.x / kReachPatches;
+    const int patches = cf.runs_per_row * cf.far_npy * cf.far_npz, mine = blockIdx.x * kReachPatches + own;
+    const int patch = min(mine, patches - 1);
+    const int prow = patch / cf.runs_per_row, pzi = prow / cf.far_npy;
+    const float cx = (float)far_centre((patch - prow * cf.runs_per_row) * kFarK, kFarK, cf.ne[0], cf.spacing),
+                cy = (float)far_centre((prow - pzi * cf.far_npy) * cf.far_py, cf.far_py, cf.ne[1], cf.spacing),
+                cz = (float)far_centre(pzi * cf.far_pz, cf.far_pz, cf.ne[2], cf.spacing);
+    if (threadIdx.x < kReachTab) table[threadIdx.x] = tables[(size_t)conf * kReachTab + threadIdx.x];
+    const FarAtom *const atoms = p.atoms + cf.atom_base;
+    float least = (float)kFarStrict;
+    for (int a0 = 0; a0 < cf.n_atoms; a0 += kReachThreads) {
+        const int n = min(kReachThreads, cf.n_atoms - a0);
+        __syncthreads();   // the last atoms' readers are done
+        if ((int)threadIdx.x < n) {
+            const FarAtom q = atoms[a0 + threadIdx.x];
+            list[threadIdx.x] = make_float4((float)q.x, (float)q.y, (float)q.z,
+                                            -2.f * __builtin_amdgcn_logf(fabsf(q.w) * cf.far_qscale));
+        }
+        __syncthreads();
+        for (int i = part; i < n; i += kParts) {
+            const float4 q = list[i];
+            const float dx = q.x - cx, dy = q.y - cy, dz = q.z - cz;
+            const float d = __builtin_amdgcn_sqrtf(__builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz))) * (2.f / 128.f);
+            least = fminf(least, table[(int)fminf(d, (float)(kReachTab - 1))] + q.w);   // (no charge: infinite, or NaN, which fminf drops)
+        }
+    }
+    least_s[part][own] = least;
+    __syncthreads();
+    if (part == 0 && mine < patches) {
+        for (int k = 1; k < kParts; k++) least = fminf(least, least_s[k][own]);
+        shift[cf.reach_off + patch] = (unsigned char)(int)ceilf(fmaxf(least, 0.f));
+    }
+}
+
 // Far-field electrostatics.  An item is one patch of rows (far_py x far_pz,
 // one per lane of a wave) times one x-run of 16 points, and one of far_split
 // parts of the atom list; the workgroup's four waves take the same points
@@ -1919,7 +1988,8 @@ __global__ void __launch_bounds__(64) k_far_down(FarParams p, int conf) {
 //
 // The others vary smoothly over the box (the host picks the distance so
 // that a table step there is below 6.5e-5 of its value and the box subtends a
-// small angle, and smaller distances for smaller charges, far_radii): their sum is formed at 5 x 4 x 4 Chebyshev nodes of
+// small angle, smaller distances for smaller charges, far_radii, and larger ones
+// away from the atoms, k_far_reach): their sum is formed at 5 x 4 x 4 Chebyshev nodes of
 // the box with the same table, and interpolated to its points.  An atom then
 // costs 80 terms instead of 1,024.  Four atoms go at once, one for each 16
 // lanes; a lane takes the five x-nodes of one (y, z) node.
@@ -2005,8 +2075,11 @@ __global__ void __launch_bounds__(kFarThreads) __attribute__((amdgpu_waves_per_e
 #pragma unroll
         for (int i = 0; i < kFarNx; i++) ns[i] = 0.;
         float4 *const strip = reinterpret_cast<float4 *>(X) + 64 * wave;
-        float *const level_r2 = X + 4 * 64 * kFarWaves + kFarLevels * wave;   // the wave's copy
-        if (lane < kFarLevels) level_r2[lane] = reinterpret_cast<const float *>(&p.confs[ci].far_r2)[lane];
+        static_assert(kFarStrict + kFarLevels <= 64, "a lane for each level");
+        float *const level_r2 = X + 4 * 64 * kFarWaves + 64 * wave;   // the wave's copy, as strict as the patch is
+        if (lane < kFarStrict + kFarLevels)
+            level_r2[lane] = reinterpret_cast<const float *>(
+                &p.confs[ci].far_r2)[max(lane - (int)p.shift[cf.reach_off + patch], 0)];
         wave_sync();
         const float qscale = sreg(FLAT ? cf.far_qscale / flat : cf.far_qscale);   // (zero charges: any level)
         const FarAtom *const atoms = p.atoms + cf.atom_base;
@@ -2255,7 +2328,7 @@ struct ag_plan {
         rexp{pool}, disorder{pool};
     DevBuf atom_cell{pool}, cell_count{pool}, cell_start{pool}, slot_atom{pool},
         near_atoms{pool}, far_atoms{pool}, fmin_atoms{pool};
-    DevBuf tab{pool}, sol{pool}, reps{pool}, far_part{pool}, far_box{pool}, far_wide{pool}, status{pool};
+    DevBuf tab{pool}, sol{pool}, reps{pool}, far_part{pool}, far_box{pool}, far_reach{pool}, far_wide{pool}, status{pool};
     DevBuf collide{pool};              // tree build: collision mask per point
     bool want_collide = false;
     int e_index = -1;                  // e map slot, -1 if none
@@ -2280,6 +2353,7 @@ struct ag_plan {
     // empty when far_split == nconf)
     hipGraphExec_t graph = nullptr, graph_far = nullptr, graph_far2 = nullptr;
     int far_split = 0;
+    std::vector<float> reach_tables;   // k_far_reach's, on their way up
     std::shared_ptr<StatusPage> status_page;   // owner of report, if any
     MapReport *report = nullptr;       // pinned: what the kernels of a map set report
     float *g_maps = nullptr, *g_fmap = nullptr;
@@ -2471,13 +2545,15 @@ static void launch_near(const ag_plan &p, int grid, const NearParams &np, hipStr
 // share a patch's atoms.  All of it depends on the conformation and the
 // tables alone, so its maps are the same in a batch as in a plan of its own.
 struct FarShape {
-    float radius2[kFarLevels] = {};
+    float radius2[kFarStrict + kFarLevels] = {};
+    float reach[kReachTab] = {};   // k_far_reach's table
     float qscale = 0.f;
     bool clamp = false;
+    int clamp_from = kFarStrict + 1;   // least shift of a patch at which it is needed (plan_build)
     int py = 8, pz = 8, split = 1;
     // coarse boxes (ConfDev::box_*): parts (0: none), patches along y and z
     int box_parts = 0, box_py = 4, box_pz = 4;
-    float box_radius2[kFarLevels] = {};
+    float box_radius2[kFarStrict + kFarLevels] = {};
 };
 
 // Least distance (A) of a level whatever the table (far_radii): 48.75 spacings,
@@ -2569,34 +2645,47 @@ static double far_term(const std::vector<float> &reps, double r) {
     return (reps[k] + (y - k) * ((double)reps[k + 1] - reps[k])) / r;
 }
 
-// Error of the interpolation from the given nodes over an axis of half-length
-// `half` (A), for an atom r off the box: ahead of it, beside its middle and beside its
-// end.
-static double far_axis_error(const std::vector<float> &reps, double r, double half, const double *node, int nodes) {
+// The interpolation along an axis: its nodes, and their weights at the ends and
+// between them, where it is furthest off.
+struct FarNodes {
+    int n;
+    double node[kBoxN], at[kBoxN + 1], weight[kBoxN + 1][kBoxN];
+    explicit FarNodes(int count) : n(count) {
+        const double four[4] = {-kNode4a, -kNode4b, kNode4b, kNode4a};
+        for (int i = 0; i < n; i++) node[i] = n == kBoxN ? box_node(i) : n == kFarNx ? (double)far_node5(i) : four[i];
+        for (int q = 0; q <= n; q++) {
+            at[q] = q == 0 ? -1.0 : q == n ? 1.0 : 0.5 * (node[q - 1] + node[q]);
+            for (int i = 0; i < n; i++) {
+                weight[q][i] = 1.0;
+                for (int j = 0; j < n; j++)
+                    if (j != i) weight[q][i] *= (at[q] - node[j]) / (node[i] - node[j]);
+            }
+        }
+    }
+};
+static const FarNodes kFarAxisX(kFarNx), kFarAxisY(kFarNy), kBoxAxis(kBoxN);
+
+// Its error over an axis of half-length `half` (A), for an atom r off the box: ahead
+// of it, beside its middle and beside its end.
+static double far_axis_error(const std::vector<float> &reps, double r, double half, const FarNodes &x) {
     double worst = 0.0;
     for (int place = 0; place < 3; place++) {
         const auto f = [&](double t) {
-            return far_term(reps, place == 0 ? r + half * (1.0 + t) : std::hypot(r, half * (place == 1 ? t : 1.0 + t)));
+            const double a = half * (place == 1 ? t : 1.0 + t);
+            return far_term(reps, place == 0 ? r + a : std::sqrt(r * r + a * a));
         };
         double v[kBoxN];
-        for (int i = 0; i < nodes; i++) v[i] = f(node[i]);
-        for (int q = 0; q <= nodes; q++) {   // the ends and between the nodes
-            const double t = q == 0 ? -1.0 : q == nodes ? 1.0 : 0.5 * (node[q - 1] + node[q]);
+        for (int i = 0; i < x.n; i++) v[i] = f(x.node[i]);
+        for (int q = 0; q <= x.n; q++) {
             double s = 0.0;
-            for (int i = 0; i < nodes; i++) {
-                double w = 1.0;
-                for (int j = 0; j < nodes; j++)
-                    if (j != i) w *= (t - node[j]) / (node[i] - node[j]);
-                s += w * v[i];
-            }
-            worst = std::max(worst, std::fabs(s - f(t)));
+            for (int i = 0; i < x.n; i++) s += x.weight[q][i] * v[i];
+            worst = std::max(worst, std::fabs(s - f(x.at[q])));
         }
     }
     return worst;
 }
 
-// What interpolating an atom of unit charge leaves of its term, by its distance
-// from the box: the steps (a third of one each way) and the nodes' error.
+// The largest table step beyond a distance, over that distance.
 struct FarError {
     const std::vector<float> &reps;
     std::vector<float> step;      // largest step beyond k / 2 A, over the distance
@@ -2610,40 +2699,49 @@ struct FarError {
     double steps(double r) const { return step[std::min((int)(2.0 * r), 128)]; }
 };
 
-// The nodes' error of a box whose axes have the given half-lengths and nodes, and
-// with the steps' (a third of one each way), for an atom r off it.
-static double far_nodes_error(const FarError &e, double r, const double half[2], const int nodes[2]) {
-    static const double n4[4] = {-kNode4a, -kNode4b, kNode4b, kNode4a};
-    double nd[kBoxN], worst = 0.0;
-    for (int a = 0; a < 2; a++) {
-        for (int i = 0; i < nodes[a]; i++)
-            nd[i] = nodes[a] == kBoxN ? box_node(i) : nodes[a] == kFarNx ? (double)far_node5(i) : n4[i];
-        worst = std::max(worst, far_axis_error(e.reps, r, half[a], nd, nodes[a]));
-        if (nodes[1] == nodes[0]) break;   // (a box is as good as a cube)
-    }
-    return worst;
-}
-static double far_error(const FarError &e, double r, const double half[2], const int nodes[2]) {
-    return std::hypot(e.steps(r) / std::sqrt(12.0), far_nodes_error(e, r, half, nodes));
+// What a patch leaves of the term of an atom r off it: half of the steps each way and
+// the nodes' error, the half-lengths of its axes given.
+static double far_error(const FarError &e, double r, const double half[2]) {
+    const double nodes = std::max(far_axis_error(e.reps, r, half[0], kFarAxisX), far_axis_error(e.reps, r, half[1], kFarAxisY));
+    return std::hypot(e.steps(r) / std::sqrt(12.0), nodes);
 }
 
 // Distances at which error(r) keeps to h0 2^(-n/2), h0 2^(-(n-1)/2), ...: from
-// `most` inwards to r0, so that nothing beyond a distance is worse.
+// `most` inwards to r0, so that nothing beyond a distance is worse, between two hops
+// as the error's logarithm has it.
 template <typename F>
 static void far_distances(F &&error, double r0, double most, double hop, double h0, int n, int levels, double *radius) {
     for (int l = 0; l < levels; l++) radius[l] = std::max(most, r0);
     int first = 0;   // levels before it have ended
+    double outer = 0.0;
     for (double r = most; r > r0 && first < levels; r -= hop) {
         const double h = error(r);
         for (int l = first; l < levels; l++) {
-            if (h <= h0 * std::pow(2.0, 0.5 * (l - n))) radius[l] = r;
-            else if (l == first) first++;
+            const double allowed = h0 * std::pow(2.0, 0.5 * (l - n));
+            if (h <= allowed) {
+                radius[l] = r;
+            } else if (l == first) {
+                const double x = std::log(h / allowed) / std::log(h / outer);
+                if (r < most && x >= 0.0 && x < 1.0) radius[l] = r + hop * x;
+                first++;
+            }
         }
+        outer = h;
     }
 }
 
-static FarShape far_shape(const ag_grid &g, int n_atoms, const double radius[kFarLevels], const double *coord,
-                          const double *charge, double coeff) {
+// Share of the pairs that an all-pairs sum in FP32 puts on the wrong side of a
+// table step (5,000 atoms on 127^3 points, 0.375 A; fewer on finer grids), and levels
+// between one such pair and a patch's sum over many, chosen so that the error is
+// the all-pairs sum's or less in the shells around receptors of 600 to 20,000
+// atoms: 16 to 20 A outside 5,000 atoms 0.8 to 1.0 times it (with 3, 0.95 to 1.3;
+// without the stricter levels 13 to 16 times).  20,000 atoms on 257^3 points, two
+// thirds of them outside the receptor: 11.0 ms, with 3 10.2, without 7.9; boxes of
+// which little is outside take the same time.
+constexpr double kFarFlips = 1.6e-4, kFarMargin = 4.0;
+
+static FarShape far_shape(const ag_grid &g, int n_atoms, const double radius[kFarLevels], const FarError &err,
+                          const double *coord, const double *charge, double coeff) {
     FarShape f;
     double q2 = 0.0;
     for (int a = 0; a < n_atoms; a++) q2 += charge[a] * charge[a];
@@ -2662,13 +2760,41 @@ static FarShape far_shape(const ag_grid &g, int n_atoms, const double radius[kFa
             f.pz = pz;
         }
     }
-    const double r = radius[0] * 128.0, s = g.spacing * 128.0;
-    for (int l = 0; l < kFarLevels; l++) f.radius2[l] = (float)(radius[l] * 128.0 * (radius[l] * 128.0));
-    // the largest bin of a direct pair: its atom lies within the radius of the patch's box
+    // the stricter levels, and the pair sum's error over the distance
+    const double half[2] = {kFarMid * g.spacing, 0.5 * (std::max(f.py, f.pz) - 1) * g.spacing};
+    const double h0 = far_error(err, radius[0], half);
+    double strict[kFarStrict];
+    const double s = g.spacing * 128.0;
     const double diag = s * std::sqrt((double)((kFarK - 1) * (kFarK - 1) + (f.py - 1) * (f.py - 1) +
                                                (f.pz - 1) * (f.pz - 1)));
+    // up to where direct pairs reach the table's end, if not 17 half-lengths
+    const double inside = (kFarLastBin - 5.0 - diag) / 128.0;
+    far_distances([&](double r) { return far_error(err, r, half); }, radius[0], std::max(inside, 17.0 * half[0]),
+                  std::max(4.0, half[0] / 2.0), h0, kFarStrict, kFarStrict, strict);
+    const double flips = kFarFlips * std::min(1.0, std::pow(g.spacing / 0.375, 4));
+    for (int k = 0; k < kReachTab; k++) {
+        const double d = std::max(1.0, 0.5 * k), step = std::sqrt(flips) * err.steps(std::max(d, 8.0)),
+                     round = 6.0e-8 * std::fabs(far_term(err.reps, d));
+        f.reach[k] = (float)(2.0 * std::log2(std::max(h0, 1e-300) / std::max(std::hypot(step, round), 1e-300)) + kFarMargin);
+    }
+    for (int l = 0; l < kFarStrict + kFarLevels; l++) {
+        const double d = 128.0 * (l < kFarStrict ? strict[l] : radius[l - kFarStrict]);
+        f.radius2[l] = (float)(d * d);
+    }
+    // how many levels stricter than 0 the largest charge is (far_level)
+    double q_max = 0.0;
+    for (int a = 0; a < n_atoms; a++) q_max = std::max(q_max, std::fabs(charge[a]));
+    int large = 0;
+    if (ref > 0.0 && q_max > 0.0)
+        large = (int)std::min(std::max(std::floor(2.0 * std::log2(q_max * std::fabs(coeff) * 128.0 / ref) + 1e-5) - 2.0, 0.0),
+                              (double)kFarStrict);
+    if (!std::isfinite(q2) || !std::isfinite(f.qscale)) large = kFarStrict;
+    // the largest bin of a direct pair: its atom lies within the radius of the patch's box
+    int passes = kFarStrict + 1;   // least level past 0 with which one may pass the table's end
+    for (int q = kFarStrict; q >= 0; q--)
+        if (std::sqrt(f.radius2[kFarStrict - q]) + diag + 4.0 >= kFarLastBin) passes = q;
     double rmax = 0.0;
-    if (r + diag + 4.0 >= kFarLastBin)
+    if (passes <= kFarStrict)
         for (int a = 0; a < n_atoms; a++) {
             double q = 0.0;
             for (int d = 0; d < 3; d++) {
@@ -2679,7 +2805,8 @@ static FarShape far_shape(const ag_grid &g, int n_atoms, const double radius[kFa
             }
             rmax = std::max(rmax, q);
         }
-    f.clamp = std::sqrt(rmax) * 128.0 + 20.0 * s + 4.0 >= kFarLastBin;
+    if (std::sqrt(rmax) * 128.0 + 20.0 * s + 4.0 >= kFarLastBin) f.clamp_from = std::max(0, passes - large);
+    f.clamp = f.clamp_from == 0;
     // a grid of few patches shares each among workgroups until there are
     // about four workgroups per CU, at least 256 atoms each (one group of 64
     // per wave)
@@ -2703,20 +2830,21 @@ static void far_boxes(FarShape &f, const ag_grid &g, int n_atoms, const std::vec
     const auto dilated = [&](double r) { return a * a * a + r * (6 * a * a + M_PI * r * (3 * a + 4. / 3. * r)); };
     if (n_atoms < 1.5 * 0.068 * dilated(18.5)) return;   // (no distance is less)
     // as far_radii has it for the table, and where its nodes leave half of what a
-    // level allows a patch.  (What counts is the atom ahead of a face: the two
-    // axes along it see the pole of 1/r beside them, at 1.8 half-edges 2.6e-5 of
-    // the term where a patch's run leaves 5e-6.)
+    // level allows; the stricter levels no nearer than a patch's.  (What counts is the
+    // atom ahead of a face: the two axes along it see the pole of 1/r beside them,
+    // at 1.8 half-edges 2.6e-5 of the term where a patch's run leaves 5e-6.)
+    constexpr int kLevels = kFarStrict + kFarLevels;
     const double patch_half[2] = {kFarMid * g.spacing, 0.5 * (std::max(f.py, f.pz) - 1) * g.spacing};
-    const double half[2] = {0.5 * (edge - 1) * g.spacing, 0.5 * (edge - 1) * g.spacing};
-    const int patch_nodes[2] = {kFarNx, kFarNy}, nodes[2] = {kBoxN, kBoxN};
-    const double r0 = std::sqrt((double)f.radius2[0]) / 128.0;   // a patch's level 0
-    double table[kFarLevels], radius[kFarLevels];
+    const double half = 0.5 * (edge - 1) * g.spacing;
+    const double r0 = std::sqrt((double)f.radius2[kFarStrict]) / 128.0;   // a patch's level 0
+    double table[kFarLevels], radius[kLevels];
     far_radii(reps, g.spacing, kBoxN, 0.5 * (edge - 1), table);
-    far_distances([&](double r) { return 2.0 * far_nodes_error(err, r, half, nodes); }, 8.25,
-                  std::max(30.0, 8.0 * half[0]), std::max(1.5, half[0] / 4.0), far_error(err, r0, patch_half, patch_nodes),
-                  0, kFarLevels, radius);
-    for (int l = 0; l < kFarLevels; l++) radius[l] = std::max(radius[l], table[l]);
-    const double beyond = n_atoms - 0.068 * dilated(radius[0]);
+    far_distances([&](double r) { return 2.0 * far_axis_error(err.reps, r, half, kBoxAxis); }, 8.25,
+                  std::max(30.0, 8.0 * half), std::max(3.0, half / 2.0), far_error(err, r0, patch_half), kFarStrict,
+                  kLevels, radius);
+    for (int l = 0; l < kLevels; l++)
+        radius[l] = std::max(radius[l], l < kFarStrict ? std::sqrt((double)f.radius2[l]) / 128.0 : table[l - kFarStrict]);
+    const double beyond = n_atoms - 0.068 * dilated(radius[kFarStrict]);
     const double patches = (double)((g.n1[0] + kFarK - 1) / kFarK) * ((g.n1[1] + f.py - 1) / f.py) *
                            ((g.n1[2] + f.pz - 1) / f.pz);
     const double boxes = std::ceil(g.n1[0] / (double)(kBoxRuns * kFarK)) * std::ceil(g.n1[1] / (double)(f.box_py * f.py)) *
@@ -2724,7 +2852,7 @@ static void far_boxes(FarShape &f, const ag_grid &g, int n_atoms, const std::vec
     if (beyond < n_atoms / 3.0 || beyond * (kFarNodes * patches - kBoxNodes * boxes) < 8e7) return;
     // about eight workgroups per CU, at least 256 atoms each
     f.box_parts = (int)std::max(1.0, std::min({2048 / boxes, n_atoms / 256.0, 16.0}));
-    for (int l = 0; l < kFarLevels; l++) f.box_radius2[l] = (float)(radius[l] * 128.0 * (radius[l] * 128.0));
+    for (int l = 0; l < kLevels; l++) f.box_radius2[l] = (float)(radius[l] * 128.0 * (radius[l] * 128.0));
 }
 
 // The far kernel with, if cp is given, the cell list in one more workgroup.
@@ -2789,7 +2917,7 @@ static void plan_geometry(ag_plan &p, const ag_grid *grids, const int *natoms, c
     p.confs.assign(n, ConfDev{});
     p.brick_prefix.assign(n + 1, 0);
     p.tile_prefix.assign(n + 1, 0);
-    long long brick = 0, tile = 0, moff = 0, poff = 0, part = 0, box_sums = 0, box_mask = 0, box_patch = 0;
+    long long brick = 0, tile = 0, moff = 0, poff = 0, part = 0, box_sums = 0, box_mask = 0, box_patch = 0, reach = 0;
     int cell_base = 0, atom_base = 0;
     for (int c = 0; c < n; c++) {
         ConfDev &cf = p.confs[c];
@@ -2829,7 +2957,7 @@ static void plan_geometry(ag_plan &p, const ag_grid *grids, const int *natoms, c
         cf.far_npz = (g.n1[2] + fs.pz - 1) / fs.pz;
         cf.far_split = fs.split;
         cf.far_clamp = fs.clamp;
-        for (int l = 0; l < kFarLevels; l++) cf.far_r2[l] = fs.radius2[l];
+        for (int l = 0; l < kFarStrict + kFarLevels; l++) cf.far_r2[l] = fs.radius2[l];
         cf.far_qscale = fs.qscale;
         cf.part_off = part;
         cf.box_parts = fs.box_parts;
@@ -2838,7 +2966,9 @@ static void plan_geometry(ag_plan &p, const ag_grid *grids, const int *natoms, c
         cf.box_n[0] = (cf.runs_per_row + kBoxRuns - 1) / kBoxRuns;
         cf.box_n[1] = (cf.far_npy + fs.box_py - 1) / fs.box_py;
         cf.box_n[2] = (cf.far_npz + fs.box_pz - 1) / fs.box_pz;
-        for (int l = 0; l < kFarLevels; l++) cf.box_r2[l] = fs.box_radius2[l];
+        for (int l = 0; l < kFarStrict + kFarLevels; l++) cf.box_r2[l] = fs.box_radius2[l];
+        cf.reach_off = reach;
+        reach += far_patch_count(cf);
         if (cf.box_parts) {
             const long long boxes = far_box_count(cf);
             cf.box_off = box_sums;
@@ -2875,6 +3005,8 @@ static void plan_geometry(ag_plan &p, const ag_grid *grids, const int *natoms, c
     p.confs_d.get(sizeof(ConfDev) * p.confs.size());
     p.brick_prefix_d.get(sizeof(int) * p.brick_prefix.size());
     p.tile_prefix_d.get(sizeof(int) * p.tile_prefix.size());
+    const size_t reach_tables = sizeof(float) * kReachTab * (size_t)n;
+    unsigned char *const d_reach = far ? (unsigned char *)p.far_reach.get(reach_tables + (size_t)reach) : nullptr;
     // the partial e maps come last: where a fixed arena has no room left for
     // them, no patch is shared
     if (part && p.pool->arena && !p.pool->fits(sizeof(float) * (size_t)part)) {
@@ -2927,6 +3059,16 @@ static void plan_geometry(ag_plan &p, const ag_grid *grids, const int *natoms, c
     HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, reinterpret_cast<const void *>(&k_far<kFarClamped, false>),
                                                            kFarThreads, 0));
     p.far_grid = std::max(1, std::min(p.total_tiles, std::max(occ, 1) * p.ctx->n_cu));
+    if (far) {
+        p.reach_tables.clear();
+        for (int c = 0; c < n; c++) p.reach_tables.insert(p.reach_tables.end(), far[c].reach, far[c].reach + kReachTab);
+        HIP_CHECK(hipMemcpyAsync(d_reach, p.reach_tables.data(), reach_tables, hipMemcpyHostToDevice, st));
+        p.far.shift = d_reach + reach_tables;
+        for (int c = 0; c < n; c++)
+            k_far_reach<<<(unsigned)((far_patch_count(p.confs[c]) + kReachPatches - 1) / kReachPatches), kReachThreads, 0, st>>>(
+                p.far, c, (const float *)d_reach, d_reach + reach_tables);
+        HIP_CHECK(hipGetLastError());
+    }
 }
 
 // Build a plan over n conformations (a single plan is n = 1).
@@ -3208,7 +3350,7 @@ static ag_plan *plan_build(ag_ctx *c, int n, const ag_receptor *recs, const ag_g
         for (int i = 0, o = 0; i < n; o += natoms[i], i++) {
             if (grids[i].spacing != spacing) far_radii(reps, spacing = grids[i].spacing, kFarNx, kFarMid, radius);
             far_shapes.push_back(
-                far_shape(grids[i], natoms[i], radius, coord + 3 * (size_t)o, charge + o, ms->coeff_estat));
+                far_shape(grids[i], natoms[i], radius, err, coord + 3 * (size_t)o, charge + o, ms->coeff_estat));
             far_boxes(far_shapes.back(), grids[i], natoms[i], reps, err);
         }
         FarParams &fp = p.far;
@@ -3241,7 +3383,22 @@ static ag_plan *plan_build(ag_ctx *c, int n, const ag_receptor *recs, const ag_g
         }
         p.far_split = split;
     }
+    // whether some patch's direct pairs may pass the table's end (spacings past
+    // 0.48 A, patches far from the atoms)
+    bool ask = false;
+    for (int i = 0; i < n && p.run_far && !p.far_flat; i++)
+        ask = ask || (far_shapes[i].clamp_from > 0 && far_shapes[i].clamp_from <= kFarStrict);
+    std::vector<unsigned char> shift;
+    if (ask) {
+        shift.resize((size_t)(p.confs[n - 1].reach_off + far_patch_count(p.confs[n - 1])));
+        HIP_CHECK(hipMemcpyAsync(shift.data(), p.far.shift, shift.size(), hipMemcpyDeviceToHost, st));
+    }
     HIP_CHECK(hipStreamSynchronize(st));   // host staging vectors go out of scope
+    for (int i = 0; i < n && ask; i++) {
+        const auto first = shift.begin() + p.confs[i].reach_off;
+        const int most = *std::max_element(first, first + far_patch_count(p.confs[i]));
+        p.confs[i].far_clamp = most >= far_shapes[i].clamp_from;
+    }
     return pl.release();
 }
 

@@ -20,8 +20,8 @@ pytestmark = pytest.mark.gpu
 U = 2.0 ** -24
 
 
-def terms(st, points, flips=0.0):
-    """(sum of the terms, mean square error that rounding each to U and putting
+def terms(st, points, rounds=1.0, flips=0.0):
+    """(sum of the terms, mean square error that `rounds` roundings of each and putting
     `flips` of the pairs on the wrong side of a table step leaves) at points, FP64."""
     tab = np.asarray(st.r_eps if st.dddiel else np.full(8192, st.inv_diel_cal), np.float32).astype(np.float64)
     step = np.abs(np.diff(tab, append=tab[-1]))
@@ -32,7 +32,7 @@ def terms(st, points, flips=0.0):
         b = np.minimum((r * 128.0).astype(np.int64), 8191)
         w = q[a:a + 2048] / np.maximum(r, 0.5)
         e += (w * tab[b]).sum(1)
-        sq += ((w * tab[b] * U) ** 2 + flips * (w * step[b]) ** 2).sum(1)
+        sq += ((w * tab[b] * U * rounds) ** 2 + flips * (w * step[b]) ** 2).sum(1)
     return e, sq
 
 
@@ -89,3 +89,48 @@ def test_box_nodes(base, spacing, constant):  # noqa: F811
             off = st.coeff_estat * np.abs(tab[b] - tab[b + 1]) / r + 3e-7 * np.abs(want)   # a table step; FP32
             err = np.abs(got[box] - want)
             assert np.all(err <= allowed + np.abs(off)), (d, float((err / (allowed + np.abs(off))).max()))
+
+
+# Share of the pairs that FP32 distances put on the wrong side of a table step,
+# where all are summed pair by pair: 128 r is good to some 1e-4 of a step.
+FLIPS = 1.6e-4
+
+
+def shell_error(st, got):
+    """(rms error, rms error that rounded terms and flipped bins leave) by
+    distance from the nearest atom, in shells of 4 A from 8 A on, at sampled points."""
+    pick = np.random.default_rng(st.n_atoms).choice(st.points, 9000, replace=False)
+    pts, got = grid_points(st)[pick], got[pick]
+    want, sq = terms(st, pts, 2.0, FLIPS)
+    near = np.full(len(pts), np.inf)
+    for a in range(0, st.n_atoms, 2048):
+        near = np.minimum(near, np.linalg.norm(pts[:, None, :] - st.coord[None, a:a + 2048], axis=2).min(1))
+    out = []
+    for lo in np.arange(8.0, 64.0, 4.0):
+        m = (near >= lo) & (near < lo + 4.0)
+        if m.sum() >= 200:
+            out.append((lo, np.sqrt(np.mean((got[m] - want[m]) ** 2)), np.sqrt(np.mean(sq[m]))))
+    return out
+
+
+@pytest.mark.parametrize("n_atoms, spacing, charges", [
+    (30, 0.375, "all"), (600, 0.375, "all"), (5000, 0.375, "all"), (5000, 0.375, "one"), (5000, 0.375, "ion"),
+    (2500, 0.5, "all"), (1200, 1.0, "all"), (12000, 0.375, "all")])
+def test_shells_outside_the_receptor(base, n_atoms, spacing, charges):  # noqa: F811
+    """The shells 8 to 60 A outside: no table step there is hidden by larger ones
+    nearer.  Against what a sum pair by pair leaves (its rounded terms 2 u each,
+    FLIPS of the pairs one table step off), three times as much: flips are few
+    and a shell is a small sample of them."""
+    print(f"[gpu] far shells {n_atoms} {spacing} {charges}", flush=True)
+    radius = (n_atoms / 0.068 * 0.75 / np.pi) ** (1 / 3)
+    n1 = (97, 33, 33) if spacing < 0.5 else (81, 33, 33)
+    st = state(base, n_atoms, n1, spacing, radius, n_atoms, offset=-(radius + 4.0 + 0.5 * (n1[0] - 1) * spacing))
+    if charges != "all":     # one charge alone, or an ion's among the others
+        q = 1e-3 * st.charge if charges == "one" else st.charge.copy()
+        q[n_atoms // 2] = 2.0
+        st = dataclasses.replace(st, charge=q, _keep=[])
+    with ag.Context(0) as ctx:
+        got = ctx.maps_plain(st)[0].reshape(-1)
+    worst = [(lo, err / left) for lo, err, left in shell_error(st, got)]
+    print(" ".join(f"{lo:.0f}:{x:.2f}" for lo, x in worst), flush=True)
+    assert len(worst) >= 4 and all(x <= 3.0 for _, x in worst), worst
