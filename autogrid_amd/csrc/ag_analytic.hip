@@ -840,11 +840,12 @@ __global__ void __launch_bounds__(64) k_an_e(EParams p) {
 // The e map of larger receptors.  1 / (eps(r) r) is smooth away from the atom, so
 // a box of 2 x 2 patches (about 16 x 16 x 16 points) takes the atoms beyond
 // box_r2 at 8 x 8 x 8 Chebyshev nodes, and its points interpolate; only the
-// atoms around it go pair by pair.  The distance, 2.6 half-edges, leaves
-// 3e-7 of a term at its nearest (2 rho^-8, rho = z + sqrt(z^2 - 1), z = 3.6);
-// the map's own error is 2e-5 (2-norm), from points on atoms.  Bound by the
-// pairs' and nodes' transcendentals (rsq, exp2, rcp), as the all-pairs kernel:
-// 5,000 atoms, 65^3 points 595 -> 257 us (boxes 158, patches 95, sum 4).
+// atoms around it go pair by pair.  The worst place for an atom is ahead of a
+// face, the pole of 1/r beside the two axes along it; evaluated there, eight nodes
+// leave 1e-7 of the term on each axis at 4.5 half-edges (2e-7 at 4, 4e-6 at 2.6),
+// 8e-8 at 3.5 in a constant dielectric (8e-7 at 2.6): an FP32 term's own roundings.
+// Bound by the pairs' and nodes' transcendentals (rsq, exp2, rcp), as the all-pairs
+// kernel: 5,000 atoms, 65^3 points 595 -> 368 us (boxes 148, patches 216, sum 4).
 constexpr int kEBoxN = 8, kEBoxNodes = kEBoxN * kEBoxN * kEBoxN, kEPatch = 8, kEWaves = 4;
 __host__ __device__ __forceinline__ constexpr double e_node(int i) {   // Chebyshev nodes, increasing
     constexpr double c[4] = {0.98078528040323044913, 0.83146961230254523708, 0.55557023301960222474,
@@ -1835,7 +1836,8 @@ static void e_boxes(ag_analytic *a) {
         patches *= e.npatch[d];
     }
     // (1 A: past the point where max(r, 0.5) has its kink)
-    const double half = 0.5 * (2 * kEPatch - 1) * g.spacing, r = std::max(2.6 * half, 1.0), w = 2.0 * half;
+    const double half = 0.5 * (2 * kEPatch - 1) * g.spacing, w = 2.0 * half;
+    const double r = std::max((a->dddiel ? 4.5 : 3.5) * half, 1.0);
     const double inside = 0.068 * (w * w * w + r * (6 * w * w + M_PI * r * (3 * w + 4. / 3. * r)));
     const double pairs = patches * 64 * a->eK;
     if (a->N < 2.0 * inside || (a->N - inside) * (pairs - boxes * kEBoxNodes) < 2.4e8) return;

@@ -1,0 +1,77 @@
+"""The analytic e map's accuracy where its nearest atoms do not hide it.
+
+Unit: u = 2^-24, the most that one FP32 operation loses, relatively (0.42 u rms).
+T = sqrt(sum over atoms of term^2)."""
+from __future__ import annotations
+
+import dataclasses
+
+import numpy as np
+import pytest
+
+import autogrid_amd as ag
+from test_gpu_analytic import Dev
+from test_gpu_analytic_boxes import base, state  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+U = 2.0 ** -24
+
+
+def forward(st):
+    d = Dev(4 * st.n_maps * st.points)
+    try:
+        with ag.Context(0) as ctx, ag.Analytic(ctx, st) as an:
+            an.forward(d.p.value)
+            return d.get(st.n_maps * st.points).reshape(st.n_maps, -1)[st.elec_index].astype(np.float64)
+    finally:
+        d.free()
+
+
+def place(st, pt):
+    nx, ny, _ = st.n1
+    return (np.stack([pt % nx, pt // nx % ny, pt // (nx * ny)], 1) - np.array(st.ne)) * st.spacing
+
+
+def sums(st, xyz):
+    """(sum of the terms, sum of their squares, distance of the nearest atom) in
+    FP64, the pairs' squared distance with the half-run's 2^-19 added, as the kernels
+    have it."""
+    nx = st.n1[0]
+    run = 13 if 13 * -(-nx // 13) < 16 * -(-nx // 16) else 16
+    added = (0.5 * (run - 1) * st.spacing) ** 2 * 2.0 ** -19
+    e, sq, near = np.zeros(len(xyz)), np.zeros(len(xyz)), np.full(len(xyz), np.inf)
+    for a in range(0, st.n_atoms, 2048):
+        r2 = np.sum((xyz[:, None] - st.coord[None, a:a + 2048]) ** 2, axis=2)
+        near = np.minimum(near, np.sqrt(r2.min(1)))
+        r = np.sqrt(r2 + added)
+        f = 332.0 / (-8.5525 + 86.9525 / (1.0 + 7.7839 * np.exp(-0.003627 * 86.9525 * r))) if st.dddiel else \
+            np.full_like(r, st.inv_diel_cal)
+        t = st.charge[a:a + 2048] * st.weights[2] * f / r
+        e += t.sum(1)
+        sq += (t * t).sum(1)
+    return e, sq, near
+
+
+@pytest.mark.parametrize("spacing, constant", [(0.375, None), (0.25, None), (0.6, None), (0.375, 4.0)])
+def test_box_nodes(base, spacing, constant):  # noqa: F811
+    """One charge ahead of a box's face, from where boxes might take it to where
+    they do: eight nodes leave at most 1.2e-7 of the term on each of three axes; a
+    term's roundings and those of the places (20 A, 8 A apart) 12 u at most."""
+    print(f"[gpu] analytic box nodes {spacing} {constant}", flush=True)
+    n = 12000
+    st = state(base, n, (48, 48, 48), spacing, 5, constant)
+    edge = 7.5 * spacing
+    pts = place(st, np.arange(st.points))
+    box = np.all(pts < (-8.5) * spacing, axis=1)            # the first box's points
+    q = np.zeros(n)
+    q[n // 2] = 1.0
+    for d in np.arange(2.0, 6.0, 0.25) * edge:
+        x = st.coord.copy()
+        x[n // 2] = [edge - 24 * spacing, -24 * spacing - d, edge - 24 * spacing]
+        one = dataclasses.replace(st, coord=x, charge=q, _keep=[])
+        got = forward(one)[box]
+        want, _, _ = sums(dataclasses.replace(one, coord=x[n // 2:n // 2 + 1], charge=q[n // 2:n // 2 + 1], _keep=[]),
+                          pts[box])
+        off = np.abs(got - want).max() / np.abs(want).max()
+        assert off <= 3 * 1.2e-7 + 12 * U, (d / edge, off)
