@@ -845,8 +845,9 @@ __global__ void __launch_bounds__(64) k_an_e(EParams p) {
 // leave 1e-7 of the term on each axis at 4.5 half-edges (2e-7 at 4, 4e-6 at 2.6),
 // 8e-8 at 3.5 in a constant dielectric (8e-7 at 2.6): an FP32 term's own roundings.
 // Bound by the pairs' and nodes' transcendentals (rsq, exp2, rcp), as the all-pairs
-// kernel: 5,000 atoms, 65^3 points 595 -> 368 us (boxes 148, patches 216, sum 4).
+// kernel: 5,000 atoms, 65^3 points 595 -> 395 us (boxes 149, patches 242, sum 4).
 constexpr int kEBoxN = 8, kEBoxNodes = kEBoxN * kEBoxN * kEBoxN, kEPatch = 8, kEWaves = 4;
+constexpr int kEPart = 32;               // terms of an FP32 partial sum (at least; 95 at most)
 __host__ __device__ __forceinline__ constexpr double e_node(int i) {   // Chebyshev nodes, increasing
     constexpr double c[4] = {0.98078528040323044913, 0.83146961230254523708, 0.55557023301960222474,
                              0.19509032201612826785};
@@ -926,7 +927,7 @@ __global__ void __launch_bounds__(64 * kEWaves) k_an_ebox(EParams p) {
                 }
             }
         }
-        if (n_acc >= kEAtoms) {
+        if (n_acc >= kEPart) {
             n_acc = 0;
 #pragma unroll
             for (int j = 0; j < kEBoxN; j++) {
@@ -972,9 +973,14 @@ __global__ void __launch_bounds__(64 * kEWaves) k_an_epatch(EParams p) {
     const int groups = (p.n_atoms + 63) / 64;
     const AN_CONST unsigned long long *mask = (const AN_CONST unsigned long long *)p.box_mask + (size_t)box * groups;
     const AN_CONST EAtom *atoms = (const AN_CONST EAtom *)p.fatoms;   // scalar loads
+    double f[K];
     float sum[K];
 #pragma unroll
-    for (int k = 0; k < K; k++) sum[k] = 0.f;
+    for (int k = 0; k < K; k++) {
+        f[k] = 0.;
+        sum[k] = 0.f;
+    }
+    int n_sum = 0;   // atoms in sum[] since it went to f[]
     for (int a0 = 64 * (part * kEWaves + wave); a0 < p.n_atoms; a0 += 64 * kEWaves * p.split) {
         const int nb = min(64, p.n_atoms - a0);
         unsigned long long set = (nb == 64 ? ~0ull : (1ull << nb) - 1) & ~mask[a0 / 64];
@@ -984,16 +990,24 @@ __global__ void __launch_bounds__(64 * kEWaves) k_an_epatch(EParams p) {
             return EAtom{q.x, q.y, q.z, q.w};
         };
         EAtom nxt = ld(__builtin_ctzll(set));
+        n_sum += __popcll(set);
         while (set) {
             const EAtom at = nxt;
             set &= set - 1;
             if (set) nxt = ld(__builtin_ctzll(set));
             e_pair<K, DD>(at, py, pz, cx, sc, s2, bias, rcap, sum);
         }
-    }
-    double f[K];
+        if (n_sum >= kEPart) {
+            n_sum = 0;
 #pragma unroll
-    for (int k = 0; k < K; k++) f[k] = (double)sum[k];
+            for (int k = 0; k < K; k++) {
+                f[k] += (double)sum[k];
+                sum[k] = 0.f;
+            }
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < K; k++) f[k] += (double)sum[k];
     if (part == 0) {
         constexpr int kOwn = 64 / kEWaves;   // (y, z) nodes of a wave: two rows of eight
         for (int t = lane; t < kOwn * kEBoxN; t += 64) {

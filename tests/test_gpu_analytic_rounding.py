@@ -75,3 +75,28 @@ def test_box_nodes(base, spacing, constant):  # noqa: F811
                           pts[box])
         off = np.abs(got - want).max() / np.abs(want).max()
         assert off <= 3 * 1.2e-7 + 12 * U, (d / edge, off)
+
+
+def test_sums_of_many_pairs(base):  # noqa: F811
+    """Wide boxes, so that each leaves thousands of atoms to its points, a quarter to a
+    wave, and takes thousands at its nodes; places and charges that FP32 holds
+    exactly, a constant dielectric, points 6 A and more from any atom.  Partial sums
+    of up to 95 terms of random signs lose 0.42 u sqrt(95 / 2) = 2.9 u a term, a
+    term itself 1 u (distance, root): 3.1 u T, 3.7 with a fifth for the estimate.
+    (One FP32 sum over n terms loses 0.42 u sqrt(n / 2): 5.5 u for 350.)"""
+    print("[gpu] analytic sums of many pairs", flush=True)
+    st = state(base, 60000, (97, 48, 48), 1.0, 3, 20.0)
+    x = np.round(64.0 * st.coord) / 64.0
+    x[:, 0] -= 62.0                  # the receptor's surface inside the box
+    w = st.weights[2] * st.inv_diel_cal
+    q = (st.charge * w).astype(np.float32).astype(np.float64) / w
+    st = dataclasses.replace(st, coord=x, charge=q, _keep=[])
+    e = forward(st)
+    xyz = place(st, np.arange(st.points))
+    far = np.flatnonzero(np.linalg.norm(xyz - x.mean(0), axis=1) > 59.5 + 6.0)
+    pick = np.random.default_rng(1).choice(far, 2500, replace=False)
+    want, sq, near = sums(st, xyz[pick])
+    m = near >= 6.0
+    ratio = np.sqrt(np.mean((e[pick][m] - want[m]) ** 2) / np.mean(sq[m])) / U
+    print(f"{ratio:.2f} u T", flush=True)
+    assert m.sum() > 1500 and ratio <= 3.7
