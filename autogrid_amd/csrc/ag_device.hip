@@ -90,22 +90,20 @@ enum : int { HC_PLAIN = 1, HC_HRAMP = 2, HC_MINMAX = 4, HC_RACC = 8 };
 // H-bond cases (main.cpp:3286-3390).
 enum : int { HBC_PLAIN = 0, HBC_ACC_PROBE = 1, HBC_MINMAX_RACC = 2, HBC_DON_PROBE = 3 };
 
-struct __align__(16) NearAtom {   // 96 bytes
+struct __align__(16) NearAtom {   // 80 bytes
     double x, y, z;               // grid frame, as the reference holds them
     float qe;                     // charge * coeff_estat
     float vol;
     float solq;                   // solpar + solpar_q * |charge|
     int meta;                     // type | hbond << 8 | rexp << 16 | disorder << 24
     int index;                    // atom index in the receptor
-    float rv2sq;                  // |rv2|^2
+    float rv2rest;                // 1 - |rv2|^2
     float rv[3];
     float pad0;
     float rv2[3];
     float pad1;
-    float rv2xrv[3];              // rv2 x rv
-    float pad2;
 };
-static_assert(sizeof(NearAtom) == 96, "NearAtom layout");
+static_assert(sizeof(NearAtom) == 80, "NearAtom layout");
 
 // One receptor conformation on its own grid, as the kernels see it.  A plan
 // holds one; a batch holds many, their atoms, cells, bricks and far-kernel
@@ -548,10 +546,7 @@ __global__ void k_gather(int ncells, const int *atom_cell, const int *start, con
     a.vol = (float)s.vol[i];
     a.solq = (float)(s.solpar[i] + s.solpar_q * fabs(q));
     const double *u = s.rvec + 3 * (size_t)i, *v = s.rvec2 + 3 * (size_t)i;
-    a.rv2sq = (float)(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
-    a.rv2xrv[0] = (float)(v[1] * u[2] - v[2] * u[1]);
-    a.rv2xrv[1] = (float)(v[2] * u[0] - v[0] * u[2]);
-    a.rv2xrv[2] = (float)(v[0] * u[1] - v[1] * u[0]);
+    a.rv2rest = (float)(1.0 - (v[0] * v[0] + v[1] * v[1] + v[2] * v[2]));
     for (int d = 0; d < 3; d++) {
         a.rv[d] = (float)u[d];
         a.rv2[d] = (float)v[d];
@@ -559,7 +554,7 @@ __global__ void k_gather(int ncells, const int *atom_cell, const int *start, con
     a.meta = (s.type[i] & 0xff) | ((s.hbond[i] & 0xff) << 8) | ((s.rexp[i] & 0xff) << 16) |
              ((s.disorder[i] ? 1 : 0) << 24);
     a.index = i;
-    a.pad0 = a.pad1 = a.pad2 = 0.f;
+    a.pad0 = a.pad1 = 0.f;
     out[k] = a;
 }
 
@@ -1223,16 +1218,18 @@ __global__ void __launch_bounds__(kNearThreads) __attribute__((amdgpu_waves_per_
                             // y = (dn x rv2).rv / |dn x rv2|:
                             //   t0 = pi/2 - acos(x)         -> cos(t0) = sqrt(1 - x^2)
                             //   ti = |acos(y) - pi/2|       -> sin(2 ti) = 2|y| sqrt(1 - y^2)
-                            // and, from the record, (dn x rv2).rv = dn.(rv2 x rv),
-                            // |dn x rv2|^2 = |rv2|^2 - x^2 (dn a unit vector).
-                            const float x = dn0 * unif(a.rv2[0]) + dn1 * unif(a.rv2[1]) + dn2 * unif(a.rv2[2]);
-                            const float cos_t0 = __builtin_amdgcn_sqrtf(max_of(__builtin_fmaf(-x, x, 1.f), 0.f));
+                            // with dn a unit vector, 1 - x^2 = (1 - |rv2|^2) + |dn x rv2|^2: formed
+                            // from x it loses all digits along the axis.
+                            const float rw0 = unif(a.rv2[0]), rw1 = unif(a.rv2[1]), rw2 = unif(a.rv2[2]);
+                            const float cr0 = __builtin_fmaf(dn1, rw2, -(dn2 * rw1)),
+                                        cr1 = __builtin_fmaf(dn2, rw0, -(dn0 * rw2)),
+                                        cr2 = __builtin_fmaf(dn0, rw1, -(dn1 * rw0));
+                            const float cross2 = __builtin_fmaf(cr0, cr0, __builtin_fmaf(cr1, cr1, cr2 * cr2));
+                            const float cos_t0 = __builtin_amdgcn_sqrtf(max_of(unif(a.rv2rest) + cross2, 0.f));
                             rdon = 0.f;
                             if (pos) {
-                                const float rd2 = max_of(__builtin_fmaf(-x, x, unif(a.rv2sq)), 1.0e-6f);
-                                const float yn = dn0 * unif(a.rv2xrv[0]) + dn1 * unif(a.rv2xrv[1]) +
-                                                 dn2 * unif(a.rv2xrv[2]);
-                                const float y = min_of(fabsf(yn) * __builtin_amdgcn_rsqf(rd2), 1.f);
+                                const float yn = __builtin_fmaf(cr0, rv0, __builtin_fmaf(cr1, rv1, cr2 * rv2));
+                                const float y = min_of(fabsf(yn) * __builtin_amdgcn_rsqf(max_of(cross2, 1.0e-6f)), 1.f);
                                 const float s2 = y * __builtin_amdgcn_sqrtf(max_of(__builtin_fmaf(-y, y, 1.f), 0.f));
                                 rdon = __builtin_fmaf(0.2f, s2, 0.9f) * cos_t0;
                             } else if (cos_t >= -0.34202f) {
@@ -3173,7 +3170,7 @@ static ag_plan *plan_build(ag_ctx *c, int n, const ag_receptor *recs, const ag_g
     p.slot_atom.get(sizeof(int) * (size_t)N);
     // the near kernel's candidate lists hold 32-bit byte offsets of records
     if ((unsigned long long)N * sizeof(NearAtom) > UINT32_MAX)
-        ag::fail(AG_ERR_UNSUPPORTED, "too many atoms in one plan for the near kernel (at most 44,739,242)");
+        ag::fail(AG_ERR_UNSUPPORTED, "too many atoms in one plan for the near kernel (at most 53,687,091)");
     p.near_atoms.get(sizeof(NearAtom) * (size_t)N);
     // an arena pool allocates no pinned memory: its plans keep the flag on the device
     if (!p.pool->arena) {
