@@ -218,6 +218,7 @@ struct ag_ctx {
     hipEvent_t chunk_ev[kMaxChunks + 1] = {};   // ordering between the two streams
     std::shared_ptr<DevPool> pool = std::make_shared<DevPool>();   // blocks of destroyed plans
     DevBuf maps;                       // output staging of ag_maps_plain
+    DevBuf far_wide;                   // a far field that runs beside the near one (wide_field)
     HostStage stage;                   // receptor arrays of a plan on their way up
     std::shared_ptr<StatusPage> status_page = std::make_shared<StatusPage>();   // its plans' reports
     double clock_khz = 1.0e5;          // rate of the device's wall clock

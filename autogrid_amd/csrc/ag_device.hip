@@ -2325,7 +2325,7 @@ struct ag_plan {
         rexp{pool}, disorder{pool};
     DevBuf atom_cell{pool}, cell_count{pool}, cell_start{pool}, slot_atom{pool},
         near_atoms{pool}, far_atoms{pool}, fmin_atoms{pool};
-    DevBuf tab{pool}, sol{pool}, reps{pool}, far_part{pool}, far_box{pool}, far_reach{pool}, far_wide{pool}, status{pool};
+    DevBuf tab{pool}, sol{pool}, reps{pool}, far_part{pool}, far_box{pool}, far_reach{pool}, status{pool};
     DevBuf collide{pool};              // tree build: collision mask per point
     bool want_collide = false;
     int e_index = -1;                  // e map slot, -1 if none
@@ -2340,6 +2340,7 @@ struct ag_plan {
     bool run_far = false;
     bool has_boxes = false;            // some conformation's far field has coarse boxes
     bool far_flat = false;             // the electrostatic factor is one value from the far kernel's bins on
+    bool beside = false;               // the far field may run beside the near one, into the context's far_wide
     double coeff_estat = 0.0;
     int far_grid = 0;                  // persistent far-kernel grid
     bool paged = false;                // near kernel in its paged form (a brick overflowed one LDS list)
@@ -2906,6 +2907,27 @@ static float far_band(const ag_grid &g) {
 static long long far_box_count(const ConfDev &cf) { return (long long)cf.box_n[0] * cf.box_n[1] * cf.box_n[2]; }
 static long long far_patch_count(const ConfDev &cf) { return (long long)cf.runs_per_row * cf.far_npy * cf.far_npz; }
 
+// Memory that a plan can do without: null where there is none left.
+static void *room_for(DevBuf &b, size_t bytes) {
+    if (b.pool && b.pool->arena && !b.pool->fits(bytes)) return nullptr;
+    try {
+        return b.get(bytes);
+    } catch (const ag::Error &e) {
+        if (e.status != AG_ERR_OOM) throw;
+        return nullptr;
+    }
+}
+
+// Where a far field beside the near one goes: 8 bytes a point (268 MB at most),
+// one block for all plans of a context, which run one after the other.  A plan that
+// finds no room runs one field after the other.
+static double *wide_field(ag_plan *p) {
+    if (!p->beside) return nullptr;
+    void *const block = room_for(p->ctx->far_wide, sizeof(double) * (size_t)p->confs[0].P);
+    p->beside = block != nullptr;
+    return (double *)block;
+}
+
 // Per-conformation geometry, work prefixes and cell arrays for the plan's
 // cell size.
 static void plan_geometry(ag_plan &p, const ag_grid *grids, const int *natoms, const FarShape *far) {
@@ -3017,22 +3039,19 @@ static void plan_geometry(ag_plan &p, const ag_grid *grids, const int *natoms, c
         p.tile_prefix[n] = p.total_tiles = (int)tile;
     }
     p.far.part = part ? (float *)p.far_part.get(sizeof(float) * (size_t)part) : nullptr;
-    // the far field of a plan in a constant dielectric, up to 268 MB of it
-    if (far && p.far_flat && !p.persistent && n == 1 && !p.pool->arena && !p.want_collide && p.confs[0].far_split == 1 &&
-        p.confs[0].P <= (1ll << 25))
-        p.far_wide.get(sizeof(double) * (size_t)p.confs[0].P);
-    // the coarse boxes' sums, patch values and atom sets, in one block; none
-    // where a fixed arena has no room left
+    p.beside = far && p.far_flat && !p.persistent && n == 1 && !p.pool->arena && !p.want_collide &&
+               p.confs[0].far_split == 1 && p.confs[0].P <= (1ll << 25);
+    // the coarse boxes' sums, patch values and atom sets, in one block; no boxes
+    // where there is no room for it
     p.has_boxes = box_sums > 0;
     if (p.has_boxes) {
-        const size_t bytes = 8 * (size_t)(box_sums + box_patch + box_mask);
-        if (p.pool->arena && !p.pool->fits(bytes)) {
-            p.has_boxes = false;
-            for (ConfDev &cf : p.confs) cf.box_parts = 0;
-        } else {
-            p.far.box_sums = (double *)p.far_box.get(bytes);
+        p.far.box_sums = (double *)room_for(p.far_box, 8 * (size_t)(box_sums + box_patch + box_mask));
+        if (p.far.box_sums) {
             p.far.box_patch = p.far.box_sums + box_sums;
             p.far.box_mask = (unsigned long long *)(p.far.box_patch + box_patch);
+        } else {
+            p.has_boxes = false;
+            for (ConfDev &cf : p.confs) cf.box_parts = 0;
         }
     }
     hipStream_t st = p.ctx->stream;
@@ -3491,7 +3510,8 @@ static void enqueue(ag_plan *p, float *d_maps, float *d_fmap, int32_t *d_cmap, b
     // atoms on 81^3 points with floating and constriction grids 808 -> 700 us; with a
     // table, 5,000 atoms on 127^3 points 1,600 -> 1,563).  Not where copies to the host
     // start behind the near field: it would end later (800 -> 937 us).
-    const bool beside = p->far_wide.ptr && part == kPartAll && !skip_far && !host && !mark_near && nchunks == 1;
+    double *const wide = part == kPartAll && !skip_far && !host && !mark_near && nchunks == 1 ? wide_field(p) : nullptr;
+    const bool beside = wide != nullptr;
     const bool stamps = events && p->report && !p->persistent && !skip_far;
     const auto stamp = [&](int phase) { return stamps ? p->stamp(phase) : nullptr; };
     if (part != kPartFar) {
@@ -3584,7 +3604,7 @@ static void enqueue(ag_plan *p, float *d_maps, float *d_fmap, int32_t *d_cmap, b
             FarParams fp = p->far;
             fp.maps = d_maps;
             fp.stamp = beside ? nullptr : stamp(kStampFar);
-            if (beside) fp.wide = (double *)p->far_wide.ptr;
+            fp.wide = wide;
             fp.item_base = t0;
             fp.item_end = t1;
             fp.queue = p->persistent ? d_queue + queue_base + k : nullptr;
@@ -3665,7 +3685,7 @@ static void enqueue(ag_plan *p, float *d_maps, float *d_fmap, int32_t *d_cmap, b
                 HIP_CHECK(hipStreamWaitEvent(st_main, c->far2_ev, 0));
                 const ConfDev &cf = p->confs[0];
                 k_far_add<<<(unsigned)std::min<long long>((cf.P + 255) / 256, 4096), 256, 0, st_main>>>(
-                    (const double *)p->far_wide.ptr, d_maps + cf.map_off + (long long)p->far.e_slot * cf.P, cf.P);
+                    wide, d_maps + cf.map_off + (long long)p->far.e_slot * cf.P, cf.P);
                 continue;
             }
             if (part != kPartNear) far_pass(k, chunks[k].first, chunks[k].second, st_main);
@@ -3770,7 +3790,9 @@ static Tune autotune(ag_ctx *c, int n, const ag_receptor *recs, const ag_grid *g
 
 ag_plan *plan_create(ag_ctx *c, const ag_receptor *rec, const ag_grid *grid, const ag_mapset *ms,
                      const ag_tables *tab, int potential) {
-    return plan_build(c, 1, rec, grid, ms, tab, potential, false, Tune());
+    std::unique_ptr<ag_plan, void (*)(ag_plan *)> p(plan_build(c, 1, rec, grid, ms, tab, potential, false, Tune()), plan_destroy);
+    (void)wide_field(p.get());   // here rather than in the first map set
+    return p.release();
 }
 
 ag_plan *batch_create(ag_ctx *c, int n, const ag_receptor *recs, const ag_grid *grids, const ag_mapset *ms,
@@ -3989,10 +4011,6 @@ void plan_execute_host(ag_plan *p, float *d_maps, float *d_fmap, int32_t *d_cmap
     read_timing(p);
 }
 
-// One map set, handed to the host map by map: each map is copied into host
-// memory as soon as the kernels are done and on_ready(j) is called for it
-// (j = n_maps for fmap, n_maps + 1 for cmap), so the caller can format and
-// write map j while later maps are still in flight.
 // ag_maps_plain with device outputs, every device buffer drawn from this
 // device's scratch array: a plan on an arena pool over it, built, run and
 // dropped.  Nothing is allocated on the device or pinned on the host.
@@ -4006,6 +4024,10 @@ void maps_plain_noalloc(ag_ctx *c, const ag_receptor *rec, const ag_grid *grid, 
     plan_execute(p.get(), maps, ms->floating_grid ? fmap : nullptr, ms->constriction_grid ? cmap : nullptr);
 }
 
+// One map set, handed to the host map by map: each map is copied into host
+// memory as soon as the kernels are done and on_ready(j) is called for it
+// (j = n_maps for fmap, n_maps + 1 for cmap), so the caller can format and
+// write map j while later maps are still in flight.
 void maps_plain_streamed(ag_ctx *c, const ag_receptor *rec, const ag_grid *grid, const ag_mapset *ms,
                          const ag_tables *tab, float *maps_out, float *fmap, int32_t *cmap,
                          const std::function<void(int)> &on_ready, int potential) {
@@ -4071,7 +4093,10 @@ void maps_plain(ag_ctx *c, const ag_receptor *rec, const ag_grid *grid, const ag
                 float *maps_out, float *fmap, int32_t *cmap, int outputs_on_device, int potential) {
     if ((ms->floating_grid && !fmap) || (ms->constriction_grid && !cmap))
         ag::fail(AG_ERR_BAD_INPUT, "the map set asks for a floating/constriction grid but no output was given");
-    std::unique_ptr<ag_plan, void (*)(ag_plan *)> p(plan_create(c, rec, grid, ms, tab, potential), plan_destroy);
+    std::unique_ptr<ag_plan, void (*)(ag_plan *)> p(
+        outputs_on_device ? plan_create(c, rec, grid, ms, tab, potential)
+                          : plan_build(c, 1, rec, grid, ms, tab, potential, false, Tune()),
+        plan_destroy);
     const long long P = p->P_total;
     const size_t bytes = sizeof(float) * (size_t)p->n_maps * P;
     const size_t pbytes = sizeof(float) * (size_t)P;

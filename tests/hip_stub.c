@@ -18,7 +18,7 @@ static long long done[STREAMS];              /* work the host has waited for */
 static long long events[EVENTS][STREAMS];
 static long long n_streams = 1, n_events = 1;
 static long long mallocs, fail_from = -1, fail_above = -1, bytes_live, bytes_peak, largest, host_mallocs;
-static long long launches, launch_log[LOG];
+static long long launches, launch_log[LOG], size_log[LOG];
 static const char *launch_name[LOG];
 static struct { const void *f; const char *name; } functions[4096];
 static int n_functions;
@@ -34,6 +34,7 @@ long long stub_mallocs(void) { return mallocs; }
 long long stub_largest(void) { const long long v = largest; largest = 0; return v; }
 void stub_fail_from(long long k) { fail_from = k < 0 ? -1 : mallocs + k; }   /* device allocations from the k-th on fail */
 void stub_fail_above(long long bytes) { fail_above = bytes; }                 /* those larger than this fail */
+long long stub_malloc_size(long long i) { return i < mallocs && i < LOG ? size_log[i] : 0; }
 long long stub_launches(void) { return launches; }
 const char *stub_launch_name(long long i) { return i < launches && i < LOG ? launch_name[i] : ""; }
 long long stub_launch_stream(long long i) { return i < launches && i < LOG ? launch_log[i] : -1; }
@@ -48,6 +49,7 @@ int hipMalloc(void **p, size_t n) {
         *p = NULL;
         return 2;
     }
+    if (mallocs < LOG) size_log[mallocs] = (long long)n;
     mallocs++;
     *p = calloc(1, n);
     return *p ? 0 : 2;

@@ -24,10 +24,10 @@ import numpy as np
 import autogrid_amd as ag
 import cases
 stub = C.CDLL("libamdhip64.so.7")
-for f in ("stub_pending", "stub_mallocs", "stub_largest", "stub_launches", "stub_launch_stream"):
+for f in ("stub_pending", "stub_mallocs", "stub_largest", "stub_launches", "stub_launch_stream", "stub_malloc_size"):
     getattr(stub, f).restype = C.c_longlong
 stub.stub_launch_name.restype = C.c_char_p
-for f in ("stub_fail_from", "stub_fail_above", "stub_launch_stream", "stub_launch_name"):
+for f in ("stub_fail_from", "stub_fail_above", "stub_launch_stream", "stub_launch_name", "stub_malloc_size"):
     getattr(stub, f).argtypes = [C.c_longlong]
 
 
