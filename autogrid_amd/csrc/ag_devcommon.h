@@ -178,7 +178,7 @@ __device__ __forceinline__ float hramp_value(float ct) {
 // between its kernels as much again.
 struct MapReport {
     int overflow = 0;                  // a brick of the near kernel overflowed its LDS lists
-    unsigned long long start[4] = {0, 0, 0, 0};   // wall_clock64 at the start of its phases
+    unsigned long long start[7] = {};   // wall_clock64 at the start of its phases, and the ends of overlapping ones
 };
 
 // The reports of a context's plans: one page, allocated with the first and

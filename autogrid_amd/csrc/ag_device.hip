@@ -461,7 +461,7 @@ struct CellParams {
     int *start, *atom_cell, *slot_atom;
     int *status, *queue;
     int nq;
-    unsigned long long *stamp;
+    unsigned long long *stamp, *stamp_end;
 };
 
 // k_zero_cells, k_cell_count, k_scan and k_cell_scatter by one workgroup, the
@@ -506,6 +506,10 @@ __device__ void cell_list(const CellParams &p, int *cnt, int *wave_sum) {
     for (int i = t; i < p.n; i += THREADS) {
         const int cell = p.atom_cell[i];
         if (cell >= 0) p.slot_atom[atomicAdd(&cnt[cell], 1)] = i;
+    }
+    if (p.stamp_end) {
+        __syncthreads();
+        if (t == 0) *p.stamp_end = wall_clock64();
     }
 }
 
@@ -1741,6 +1745,7 @@ template <bool FLAT>
 __global__ void __launch_bounds__(kFarThreads) __attribute__((amdgpu_waves_per_eu(4))) k_far_boxes(FarParams p, int conf) {
     __shared__ float T[FLAT ? kFarStrict + kFarLevels : AG_NDIEL];
     __shared__ double XD[2 * kBoxNodes];   // 40 KiB in all: four workgroups per CU
+    stamp_start(p.stamp);
     const AG_CONST ConfDev &cf = as_const(p.confs)[conf];
     const float flat = FLAT ? as_const(p.tab)[kFarLastBin] : 1.f;
     // the bins below the far kernel's are not read: the distances are there instead
@@ -2269,6 +2274,9 @@ __global__ void __launch_bounds__(kFarThreads) __attribute__((amdgpu_waves_per_e
         __syncthreads();
     }
 }
+
+// When a stream gets here.
+__global__ void k_stamp(unsigned long long *stamp) { stamp_start(stamp); }
 
 // The e map where the far field was summed beside the near one.
 __global__ void __launch_bounds__(256) k_far_add(const double *wide, float *emap, long long P) {
@@ -3463,10 +3471,12 @@ static std::vector<std::pair<int, int>> plan_chunks(const ag_plan &p, int want, 
 }
 
 enum : int { kPartAll = 0, kPartNear = 1, kPartFar = 2 };
-// Phases of MapReport::start: the first kernel (the cell list, or with it the
-// far field), the gather behind a far field that went first, the near field,
-// the far field in its usual place.
-enum : int { kStampFirst = 0, kStampGather = 1, kStampNear = 2, kStampFar = 3 };
+// Stamps of MapReport: the starts of the first kernel (the cell list, or with it
+// the far field), the gather behind a far field that went first, the near field, the
+// far field; the end of a cell list beside the far field, and of a near and a far
+// field beside each other.
+enum : int { kStampFirst = 0, kStampGather = 1, kStampNear = 2, kStampFar = 3, kStampCellsEnd = 4, kStampNearEnd = 5,
+             kStampFarEnd = 6 };
 
 // One conformation whose far field is in parts, with a cell list that one
 // workgroup makes in the far kernel's LDS before the others are done.
@@ -3518,7 +3528,8 @@ static void enqueue(ag_plan *p, float *d_maps, float *d_fmap, int32_t *d_cmap, b
         const int *atom_conf = p->nconf > 1 ? (const int *)p->atom_conf_d.ptr : nullptr;
         const ConfDev *d_confs = (const ConfDev *)p->confs_d.ptr;
         const CellParams cp{d_confs, atom_conf, N, p->total_cells, p->tune.cell_size, (const double *)p->coord.ptr,
-                            d_start, d_atom_cell, d_slot_atom, d_status, d_queue, kMaxChunks, stamp(kStampFirst)};
+                            d_start, d_atom_cell, d_slot_atom, d_status, d_queue, kMaxChunks, stamp(kStampFirst),
+                            far_first ? stamp(kStampCellsEnd) : nullptr};
         if (far_first) {
             FarParams fp = p->far;
             fp.maps = d_maps;
@@ -3603,7 +3614,7 @@ static void enqueue(ag_plan *p, float *d_maps, float *d_fmap, int32_t *d_cmap, b
         if (p->run_far && !skip_far && !far_first && t1 > t0) {
             FarParams fp = p->far;
             fp.maps = d_maps;
-            fp.stamp = beside ? nullptr : stamp(kStampFar);
+            fp.stamp = stamp(kStampFar);
             fp.wide = wide;
             fp.item_base = t0;
             fp.item_end = t1;
@@ -3616,6 +3627,7 @@ static void enqueue(ag_plan *p, float *d_maps, float *d_fmap, int32_t *d_cmap, b
                     const unsigned items = (unsigned)(far_box_count(cf) * cf.box_parts);
                     if (p->far_flat) k_far_boxes<true><<<items, kFarThreads, 0, s>>>(fp, ci);
                     else k_far_boxes<false><<<items, kFarThreads, 0, s>>>(fp, ci);
+                    fp.stamp = nullptr;   // (the far field has begun)
                     k_far_down<<<(unsigned)far_patch_count(cf), 64, 0, s>>>(fp, ci);
                 }
             launch_far(blocks, fp, far_kind(*p, c0, c1), nullptr, s);
@@ -3676,12 +3688,14 @@ static void enqueue(ag_plan *p, float *d_maps, float *d_fmap, int32_t *d_cmap, b
                 HIP_CHECK(hipEventRecord(c->cells_ev, st_main));
                 HIP_CHECK(hipStreamWaitEvent(c->stream2, c->cells_ev, 0));
                 far_pass(k, chunks[k].first, chunks[k].second, c->stream2);
+                if (stamps) k_stamp<<<1, 1, 0, c->stream2>>>(stamp(kStampFarEnd));
                 HIP_CHECK(hipEventRecord(c->far2_ev, c->stream2));
             }
             if (part != kPartFar) near_pass(chunks[k].first, chunks[k].second, st_main);
             if (events && !stamps && k == nchunks - 1) HIP_CHECK(hipEventRecord(c->ev[2], st_main));
             if (mark_near && k == nchunks - 1) HIP_CHECK(hipEventRecord(c->near_ev, st_main));
             if (beside) {
+                if (stamps) k_stamp<<<1, 1, 0, st_main>>>(stamp(kStampNearEnd));
                 HIP_CHECK(hipStreamWaitEvent(st_main, c->far2_ev, 0));
                 const ConfDev &cf = p->confs[0];
                 k_far_add<<<(unsigned)std::min<long long>((cf.P + 255) / 256, 4096), 256, 0, st_main>>>(
@@ -3920,10 +3934,15 @@ static void read_timing(ag_plan *p) {
         const auto span = [&](int from, int to) {
             return t[from] && t[to] > t[from] ? (float)((double)(t[to] - t[from]) / c->clock_khz) : 0.f;
         };
-        if (t[kStampGather]) {   // the far field went first
+        if (t[kStampGather]) {   // the far field went first, the cell list beside it
+            const float gather = span(kStampGather, kStampNear);
             c->last_ms[2] = span(kStampFirst, kStampGather);
-            c->last_ms[0] = span(kStampGather, kStampNear);
-            c->last_ms[1] = std::max(0.f, total - c->last_ms[0] - c->last_ms[2]);
+            c->last_ms[0] = span(kStampFirst, kStampCellsEnd) + gather;
+            c->last_ms[1] = std::max(0.f, total - gather - c->last_ms[2]);
+        } else if (t[kStampFarEnd]) {   // the fields ran beside each other
+            c->last_ms[0] = t[kStampFar] < t[kStampNear] ? span(kStampFirst, kStampFar) : span(kStampFirst, kStampNear);
+            c->last_ms[1] = span(kStampNear, kStampNearEnd);
+            c->last_ms[2] = span(kStampFar, kStampFarEnd);
         } else {
             c->last_ms[0] = span(kStampFirst, kStampNear);
             c->last_ms[1] = t[kStampFar] ? span(kStampNear, kStampFar) : std::max(0.f, total - c->last_ms[0]);

@@ -308,10 +308,10 @@ typedef struct ag_audit {
 ag_status ag_plan_audit(ag_plan *plan, ag_audit *out);
 
 /* Milliseconds of the last execute on ctx: [0] cell list, [1] near-field
- * kernel(s), [2] far-field kernel, by the device's clock (a small plan makes
- * its cell list inside the far-field kernel, and where near and far field run
- * beside each other, in a constant dielectric, [1] is both), [3] total, from
- * HIP events on ctx's stream. */
+ * kernel(s), [2] far-field kernel(s), by the device's clock, [3] total, from
+ * HIP events on ctx's stream.  A small plan makes its cell list beside the far
+ * field, and in a constant dielectric near and far field run beside each other:
+ * there the parts add up to more than the total. */
 ag_status ag_context_timing(ag_ctx *ctx, float ms[4]);
 
 /* ------------------------------------------------------------------------ */
