@@ -1231,7 +1231,7 @@ struct AtomAdjParams {
 // (k_an_gmask) of its word that lie within the sphere's chord.  Each wave packs
 // its lanes' points into its own LDS list in lane order and works through it
 // 64 at a time, every lane busy; no barrier until the waves' sums meet.
-// The chord is a little wide: a point past 8 A has S = 0 and adds nothing.
+// The chord is a little wide: points past 8 A are dropped when they are looked at.
 // Testing the sphere's cube point by point, with the workgroup's barriers,
 // took most of the launch: 865 us (5,000 atoms, 65^3 points, 256 poses), now
 // 450 us.
@@ -1270,6 +1270,7 @@ __global__ void __launch_bounds__(kAT) k_an_atom(AtomAdjParams q) {
         const float c[3] = {(float)(ix - p.ne[0]) * p.h, (float)(iy - p.ne[1]) * p.h, (float)(iz - p.ne[2]) * p.h};
         const float d[3] = {a.x - c[0], a.y - c[1], a.z - c[2]};
         const float r2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
+        if (!(r2 < kCut2)) return;   // (a NaN cotangent there is not this atom's)
         const float r2c = fmaxf(r2, 1.0e-12f);
         const float ir = __builtin_amdgcn_rsqf(r2c);   // hardware rsq and exp2, about 1 ulp
         const float r = r2c * ir;

@@ -100,3 +100,28 @@ def test_sums_of_many_pairs(base):  # noqa: F811
     ratio = np.sqrt(np.mean((e[pick][m] - want[m]) ** 2) / np.mean(sq[m])) / U
     print(f"{ratio:.2f} u T", flush=True)
     assert m.sum() > 1500 and ratio <= 3.7
+
+
+@pytest.mark.parametrize("axis", [0, 1, 2])
+def test_cotangent_past_the_cutoff(base, axis):  # noqa: F811
+    """A cotangent that is not a number, 8.0004 A from the only atom: not that
+    atom's.  At 7.9 A it is."""
+    print(f"[gpu] analytic cutoff {axis}", flush=True)
+    st = state(base, 2, (33, 33, 33), 0.375, 7)
+    for distance, finite in ((8.0004, True), (7.9, False)):
+        x = np.array([[0.0, 0.0, 0.0], [200.0, 0.0, 0.0]])
+        x[0, axis] = 4.0
+        x[0, (axis + 1) % 3] = np.sqrt(distance ** 2 - 16.0)
+        one = dataclasses.replace(st, coord=x, _keep=[])
+        cot = np.zeros((one.n_maps, one.points), np.float32)
+        cot[0, 16 + 33 * (16 + 33 * 16)] = np.nan
+        maps, dmaps = Dev(cot.nbytes), Dev(cot.nbytes)
+        dmaps.put(cot)
+        try:
+            with ag.Context(0) as ctx, ag.Analytic(ctx, one) as an:
+                an.forward(maps.p.value)
+                g = an.adjoint(dmaps.p.value)
+        finally:
+            maps.free()
+            dmaps.free()
+        assert np.isfinite(g["coord"]).all() == finite and np.isfinite(g["eps"]).all() == finite
