@@ -134,3 +134,33 @@ def test_shells_outside_the_receptor(base, n_atoms, spacing, charges):  # noqa: 
     worst = [(lo, err / left) for lo, err, left in shell_error(st, got)]
     print(" ".join(f"{lo:.0f}:{x:.2f}" for lo, x in worst), flush=True)
     assert len(worst) >= 4 and all(x <= 3.0 for _, x in worst), worst
+
+
+@pytest.mark.parametrize("n_atoms, n1, spacing, constant", [
+    (257, (29, 29, 29), 0.375, None),      # a patch's atoms in one workgroup, the last atom in a group of its own
+    (2049, (29, 29, 29), 0.375, None),     # in eight
+    (2049, (29, 29, 29), 0.375, 4.0),
+    (9000, (97, 65, 66), 0.375, None),     # coarse boxes, ragged ones at the ends
+    (9001, (33, 60, 140), 0.375, None),
+    (20000, (97, 65, 66), 0.375, 4.0)])
+def test_every_atom_counts_once(base, n_atoms, n1, spacing, constant):  # noqa: F811
+    """One charge alone, on atoms at the ends of the groups of 64 and of the workgroups'
+    parts: left out or taken twice, by a patch, its box or both, it would be off by
+    all of itself.  A pair's bin is at most one table step off, 1.7e-3 of the term at
+    8 A, and interpolation less."""
+    print(f"[gpu] far every atom {n_atoms} {n1}", flush=True)
+    radius = (n_atoms / 0.068 * 0.75 / np.pi) ** (1 / 3)
+    st = state(base, n_atoms, n1, spacing, radius, 3, constant=constant, offset=0.4 * radius)
+    tab = np.asarray(st.r_eps if st.dddiel else np.full(8192, st.inv_diel_cal), np.float32).astype(np.float64)
+    last = n_atoms - 1
+    pts = grid_points(st)
+    with ag.Context(0) as ctx:
+        for a in sorted({0, 1, 63, 64, 65, 127, 128, 255, 256, n_atoms // 2, last // 64 * 64 - 1, last // 64 * 64, last - 1, last}):
+            q = np.zeros(n_atoms)
+            q[a] = 1.0
+            got = ctx.maps_plain(dataclasses.replace(st, charge=q, _keep=[]))[0].reshape(-1)
+            r = np.linalg.norm(pts - st.coord[a], axis=1)
+            want = st.coeff_estat * tab[np.minimum((128 * r).astype(int), 8191)] / np.maximum(r, 0.5)
+            off = np.abs(got - want) / np.abs(want)
+            assert np.all(off[r > 8.0] <= 2e-3), (a, float(off[r > 8.0].max()))
+            assert np.all(off[r <= 8.0] <= 2e-5), (a, float(off[r <= 8.0].max()))
