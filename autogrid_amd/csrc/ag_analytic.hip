@@ -114,7 +114,6 @@ struct AParams {
     // maps
     int naff;
     int aff_slot[kAMaxAff], des_slot[kAMaxAff];
-    int cases[kAMaxAff][7];           // case per atom H-bond class
     float sp[kAMaxAff], volp[kAMaxAff];  // desolvation parameters of des_slot
     int cov_slot[16], n_cov;
     double cov_pos[3], cov_hw, cov_barrier;
@@ -307,23 +306,6 @@ __device__ __forceinline__ float a2_rdon(const float dn[3], const float rv[3], c
         }
     }
     return rdon;
-}
-
-__device__ __forceinline__ void point_of(const AParams &p, long long pt, int &ix, int &iy, int &iz, float c[3]) {
-    ix = (int)(pt % p.n1[0]);
-    iy = (int)((pt / p.n1[0]) % p.n1[1]);
-    iz = (int)(pt / ((long long)p.n1[0] * p.n1[1]));
-    c[0] = (float)(ix - p.ne[0]) * p.h;
-    c[1] = (float)(iy - p.ne[1]) * p.h;
-    c[2] = (float)(iz - p.ne[2]) * p.h;
-}
-
-// Cell range covering the 8 A sphere around c.
-__device__ __forceinline__ void cell_range(const AParams &p, const float c[3], int lo[3], int hi[3]) {
-    for (int d = 0; d < 3; d++) {
-        lo[d] = max(0, (int)floorf((c[d] - 8.f - p.corg[d]) / kCellA));
-        hi[d] = min(p.nc[d] - 1, (int)floorf((c[d] + 8.f - p.corg[d]) / kCellA));
-    }
 }
 
 // Per-pair directional factors (forward).
@@ -1436,12 +1418,9 @@ __global__ void __launch_bounds__(kAT) k_an_atom(AtomAdjParams q) {
         for (int k = 0; k < kAtomOut; k++) q.out[(long long)blockIdx.x * kAtomOut + k] = acc[k];
 }
 
-// e-map adjoint: lane = atom, workgroup = (atom block, point chunk).
-// The e map's adjoint gathers, per atom, over the points where the
-// cotangent g is nonzero (the poses' trilinear footprint, a fraction of the
-// box).  Those points are packed first, in point order, as (x, y, z, g):
-// k_an_gcount counts them per block of kGPack points, k_an_gscan turns the
-// counts into offsets (one workgroup) and k_an_gpack writes them.
+// The e map's adjoint (k_an_eadj) gathers, per atom, over the points where the
+// cotangent is nonzero (the poses' trilinear footprint, a fraction of the box),
+// packed first.
 constexpr int kGPack = 1024;             // points per packing block (4 per lane)
 constexpr int kEAdjChunk = 1024;         // packed points per e-adjoint chunk
 
@@ -2036,7 +2015,6 @@ static void upload_near(ag_analytic *a, UploadPack up) {
     for (int k = 0; k < a->naff; k++) {
         p.aff_slot[k] = a->aff_slot[k];
         p.des_slot[k] = a->des_slot[k];
-        for (int h = 0; h < 7; h++) p.cases[k][h] = a->cases[k][h];
         const ag_map_desc &md = a->maps[a->des_slot[k]];
         p.sp[k] = (float)md.solpar_probe;
         p.volp[k] = (float)md.vol_probe;

@@ -58,7 +58,6 @@ constexpr int kPlainSlots = 12;                   // of which without H-bond ter
 constexpr int kHbSlots = kMapSlots - kPlainSlots; // of which H-bonding probes
 constexpr int kCandCap = 2048;                    // candidates per brick
 constexpr int kHCap = 256;                        // donor-H candidates per brick
-constexpr int kChunk = 128;                       // candidate records staged per pass
 // The near kernel's bins, as rows of its tables: 0 to 1023, whose rows hold
 // values; 1024 to 1039, past the 8 A cutoff, whose rows are zeros (a distance is
 // clamped to 1039.5 bins), so a lane out of range needs no test; the pair at 8 A
@@ -122,7 +121,7 @@ struct ConfDev {
     long long P;
     long long map_off;            // offset of its [n_maps][P] block in the map output
     long long pt_off;             // offset of its [P] block in the fmap / cmap outputs
-    int runs_per_row, nruns;      // far-kernel runs of kFarK points along x
+    int runs_per_row;             // far-kernel runs of kFarK points along x
     int far_py, far_pz;           // far-kernel patch: rows along y and z, one per lane (far_py * far_pz <= 64)
     int far_npy, far_npz;         // patches along y and z
     int far_split;                // workgroups sharing each patch's atoms
@@ -145,15 +144,10 @@ struct ConfDev {
 // reads become scalar loads the compiler may repeat instead of holding the
 // values in registers across the hot loops.
 #define AG_CONST __attribute__((address_space(4)))
-// float4 layout without HIP_vector_type's constructors, for copies out of
-// the constant address space.
+// float4 layout without HIP_vector_type's constructors.
 struct __align__(16) PlainF4 {
     float x, y, z, w;
 };
-__device__ __forceinline__ PlainF4 ld4(const AG_CONST PlainF4 *p, int i) {
-    const AG_CONST PlainF4 &q = p[i];
-    return PlainF4{q.x, q.y, q.z, q.w};
-}
 template <typename T>
 __device__ __forceinline__ const AG_CONST T *as_const(const T *p) {
     return (const AG_CONST T *)(p);
@@ -187,7 +181,6 @@ struct NearParams {
     const NearAtom *atoms;        // sorted by (cell, index)
     const double *coord64;        // [n][3] by atom index
     const double *rvec64;         // [n][3]
-    const double *rvec2_64;       // [n][3]
     // tables
     const float *tab;             // [T][kNearRows][row slots] for this pass's maps (near_row)
     const float *sol;             // [1025]
@@ -2976,7 +2969,6 @@ static void plan_geometry(ag_plan &p, const ag_grid *grids, const int *natoms, c
         cf.map_off = moff;
         cf.pt_off = poff;
         cf.runs_per_row = (g.n1[0] + kFarK - 1) / kFarK;
-        cf.nruns = cf.runs_per_row * g.n1[1] * g.n1[2];
         const FarShape fs = far ? far[c] : FarShape();
         cf.far_py = fs.py;
         cf.far_pz = fs.pz;
@@ -3288,7 +3280,6 @@ static ag_plan *plan_build(ag_ctx *c, int n, const ag_receptor *recs, const ag_g
     np.atoms = (const NearAtom *)p.near_atoms.ptr;
     np.coord64 = d_coord;
     np.rvec64 = d_rvec;
-    np.rvec2_64 = d_rvec2;
     np.sol = d_sol;
     np.reps = d_reps;
     np.disorder_h = ms->disorder_h;

@@ -409,7 +409,6 @@ struct ag_scorer {
     float outside = 0.f;
     std::vector<int> pose_start;
     std::vector<int> map_index;
-    std::vector<double> charge;
     DevBuf atoms, pose_start_d, xyz, charge_d, map_d, pose_d;
     DevBuf pair[3], count;
     bool counts_clear = false;      // every pass's counts but the last's are clear
@@ -518,7 +517,6 @@ ag_scorer *scorer_create(ag_ctx *c, const ag_grid *grid, int n_maps, int elec_in
     s->outside = (float)outside;
     s->pose_start.assign(pose_start, pose_start + n_poses + 1);
     s->map_index.assign(map_index, map_index + n);
-    s->charge.assign(charge, charge + n);
     std::vector<float> q(std::max(n, 1));
     std::vector<int> pose(std::max(n, 1));
     for (int p = 0; p < n_poses; p++)
