@@ -21,16 +21,19 @@
 //               and d maps, plus the tape the adjoint needs (closest H, the
 //               atoms that gave each point's H-bond min and max);
 //   k_an_e      runs of 13 or 16 points along x per lane over one chunk of
-//               atoms, and k_an_esum the chunks' sums per point: the e map;
-//   k_an_vh     one lane per grid point: the cotangent of the closest H's
-//               bond vector through every Hramp at that point;
+//               atoms, and k_an_esum the chunks' sums per point: the e map; of
+//               larger receptors k_an_ebox sums the atoms beyond boxes of about
+//               16x16x16 points at 512 Chebyshev nodes of each, and k_an_epatch
+//               the rest point by point, with the nodes' values interpolated;
+//   k_an_vh     in the cubes of k_an_near: the cotangent of the closest H's
+//               bond vector through every Hramp at each point;
 //   k_an_hsum   one workgroup per donor H: sums k_an_vh's vectors over the
 //               points whose closest H it is (of the points where they are
 //               nonzero, packed);
 //   k_an_atom   one workgroup per atom: gathers over the grid points within
 //               8 A of it the gradients of the 8 A terms with respect to its
 //               position, bond vectors, charge, pair parameters and the
-//               desolvation weight;
+//               desolvation weight, beside the kernels on the second stream;
 //   k_an_count / k_an_gscan / k_an_pack
 //               points where a cotangent is nonzero, packed in point order
 //               (the e map's for k_an_eadj, the bond-vector one for

@@ -4,7 +4,9 @@
 //   1. cell list   : atoms within 8 A of the box binned into cubic cells by a
 //                    counting sort; each cell's atoms are then ordered by atom
 //                    index so every later traversal is deterministic.
-//   2. near kernel : one workgroup per 8x8x4 brick of grid points.  It stages
+//   2. near kernel : one workgroup per brick of grid points, 8x8x4 on large grids,
+//                    8x4x4 or 4x4x4 on smaller ones, where two or four waves
+//                    share the atoms of a 4x4x4 cube.  It stages
 //                    the atoms within 8.03 A of the brick (cells in fixed
 //                    order, ballot compaction) and evaluates, per point, the
 //                    8 A part of the reference's per-point loop
@@ -13,7 +15,7 @@
 //                    desolvation, the d map, the H-bond min/max fix-up, and
 //                    the electrostatic terms of every atom the far kernel
 //                    leaves out.  Bin indices floor(128 r) are taken from an
-//                    FP32 distance unless 128 r lies within 1e-3 of an
+//                    FP32 distance unless 128 r lies within 4e-4 of an
 //                    integer, where the reference's FP64 distance is
 //                    recomputed, so the table bins match the reference's.
 //   3. far kernel  : the electrostatic sum over all atoms (main.cpp:2940-2982)
@@ -22,7 +24,14 @@
 //                    patch go pair by pair through the dielectric table in
 //                    LDS, with zeros below bin 1025; the others are summed at
 //                    80 Chebyshev nodes of the patch's box and interpolated
-//                    to its points.  The sums join the near kernel's value.
+//                    to its points; in large receptors most of those at the
+//                    512 nodes of a coarse box of patches first.  How far off
+//                    an atom has to be follows its charge, the table's steps
+//                    and the patch's own distance from the receptor.  The sums
+//                    join the near kernel's value.
+// Where kernels do not depend on each other they overlap: a small plan's far field
+// goes first and makes the cell list, and in a constant dielectric the far field
+// runs beside the near one.
 // No atomics touch map values; every sum has a fixed order.
 
 #include <hip/hip_runtime.h>
