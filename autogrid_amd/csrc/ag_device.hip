@@ -2739,14 +2739,16 @@ static void far_distances(F &&error, double r0, double most, double hop, double 
 }
 
 // Share of the pairs that an all-pairs sum in FP32 puts on the wrong side of a
-// table step (5,000 atoms on 127^3 points, 0.375 A; fewer on finer grids), and levels
-// between one such pair and a patch's sum over many, chosen so that the error is
-// the all-pairs sum's or less in the shells around receptors of 600 to 20,000
-// atoms: 16 to 20 A outside 5,000 atoms 0.8 to 1.0 times it (with 3, 0.95 to 1.3;
-// without the stricter levels 13 to 16 times).  20,000 atoms on 257^3 points, two
-// thirds of them outside the receptor: 11.0 ms, with 3 10.2, without 7.9; boxes of
-// which little is outside take the same time.
-constexpr double kFarFlips = 1.6e-4, kFarMargin = 4.0;
+// table step (5,000 atoms on 127^3 points, 0.375 A; fewer on finer grids), what its
+// roundings leave of a term (in wider patches the nodes' error is the same for many
+// atoms, and counts for more), and levels between one such pair and a patch's sum
+// over many.  Chosen so that the error is the all-pairs sum's or less in the shells
+// around receptors of 600 to 20,000 atoms: 0.8 to 0.9 times it at 0.375 A, 1.0 in the
+// shell 16 to 20 A off (1.15 with a margin of 3; without the stricter levels 13 to
+// 16 times).  20,000 atoms on 257^3 points, two thirds of them outside the
+// receptor: 9.1 ms, without 7.9 (10.9 with a rounding of 6e-8, which does not show);
+// boxes of which little is outside take the same time.
+constexpr double kFarFlips = 1.6e-4, kFarRounding = 4.0e-7, kFarMargin = 4.0;
 
 static FarShape far_shape(const ag_grid &g, int n_atoms, const double radius[kFarLevels], const FarError &err,
                           const double *coord, const double *charge, double coeff) {
@@ -2780,9 +2782,10 @@ static FarShape far_shape(const ag_grid &g, int n_atoms, const double radius[kFa
     far_distances([&](double r) { return far_error(err, r, half); }, radius[0], std::max(inside, 17.0 * half[0]),
                   std::max(4.0, half[0] / 2.0), h0, kFarStrict, kFarStrict, strict);
     const double flips = kFarFlips * std::min(1.0, std::pow(g.spacing / 0.375, 4));
+    const double rounding = kFarRounding * std::min(1.0, 0.375 * 0.375 / (g.spacing * g.spacing));
     for (int k = 0; k < kReachTab; k++) {
         const double d = std::max(1.0, 0.5 * k), step = std::sqrt(flips) * err.steps(std::max(d, 8.0)),
-                     round = 6.0e-8 * std::fabs(far_term(err.reps, d));
+                     round = rounding * std::fabs(far_term(err.reps, d));
         f.reach[k] = (float)(2.0 * std::log2(std::max(h0, 1e-300) / std::max(std::hypot(step, round), 1e-300)) + kFarMargin);
     }
     for (int l = 0; l < kFarStrict + kFarLevels; l++) {
