@@ -245,12 +245,16 @@ ag_status ag_maps_plain(ag_ctx *ctx, const ag_receptor *rec,
  * ag_maps_plain with device outputs (outputs_on_device = 1) for callers
  * that cannot allocate device or pinned memory -- serving loops and
  * harnesses that forbid hipMalloc.  Every device buffer of the map set (the
- * receptor arrays, cell list, tables, far-kernel atoms and status flag)
+ * receptor arrays, cell list, tables, far-kernel atoms and sums, status flag)
  * comes from one device array of AG_NOALLOC_SCRATCH_BYTES that each GPU
  * holds from the library's load until the process ends; the call makes no
  * hipMalloc, hipFree or pinned-memory allocation.  A map set that needs
  * more than the array holds returns AG_ERR_UNSUPPORTED with the limit in
- * ag_last_error() and leaves the outputs untouched.  Inputs are host
+ * ag_last_error() and leaves the outputs untouched.  The map set is
+ * ag_maps_plain's bit for bit, but for the e map where the array has no room
+ * for what the far field can do without (the coarse boxes of receptors of
+ * about 8,200 atoms and more, and the parts of few-patch grids): it is summed
+ * without them then, to the same accuracy.  Inputs are host
  * pointers as for ag_maps_plain; maps_dev / fmap_dev / cmap_dev are device
  * pointers.  The call returns after the outputs are written.  All calls on
  * one GPU share its array, so calls that overlap on one GPU (from several
