@@ -1065,7 +1065,8 @@ __global__ void k_an_esum(const float *epart, int nchunk, long long P, float *em
 // Per point: the cotangent of the closest H's bond vector through the Hramp
 // factor of every other D1 atom within 8 A.  Cubes and waves as in k_an_near; a
 // cube without a point to do leaves zeros.  (One lane per point with its own
-// cells: 288 us, now 31 us at the shape above; 235 and 14 us on 41^3 points.)
+// cells: 288 us, now 31 us at the shape above, 184 beside k_an_atom on the other
+// stream; 235 and 14 us on 41^3 points.)
 __global__ void __launch_bounds__(kAT) k_an_vh(AParams p) {
     __shared__ CubeStage st;
     __shared__ int list[2 * kAT];
@@ -1219,7 +1220,7 @@ struct AtomAdjParams {
 // The chord is a little wide: points past 8 A are dropped when they are looked at.
 // Testing the sphere's cube point by point, with the workgroup's barriers,
 // took most of the launch: 865 us (5,000 atoms, 65^3 points, 256 poses), now
-// 450 us.
+// 450 us (490 with the other chain beside it).
 template <int NA>
 __global__ void __launch_bounds__(kAT) k_an_atom(AtomAdjParams q) {
     constexpr int kList = 512;   // a wave's list; one lane appends at most 64

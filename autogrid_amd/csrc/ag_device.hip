@@ -656,8 +656,9 @@ __device__ __forceinline__ int group_lane(int v) {
 // With 32-byte rows bound by its vector operations (49 per pair of a wave and a
 // plain atom, 90 to 140 where the atom is directional), with 64-byte rows by the
 // vector caches: 13 Vina maps make 4.3e8 accesses, 0.70 ms at one per clock and
-// CU.  5,000 atoms, 127^3 points: 13 Vina maps 1,096 -> 746 us, 15 AutoDock maps
-// 1,099 -> 854; 41^3 points and 1,000 atoms 157 -> 61.  CUBE selects the lane layout inside the brick (brick_lane).  FORM:
+// CU.  5,000 atoms, 127^3 points: 13 Vina maps 1,096 -> 731 us, 15 AutoDock maps
+// 1,099 -> 836; 41^3 points and 1,000 atoms 157 -> 61.  CUBE selects the lane
+// layout inside the brick (brick_lane).  FORM:
 //   kNearPlain   neither the tree build's queries, a constriction count
 //                nor disordered hydroxyls (their branches compiled out);
 //   kNearGeneral every map-set option;
@@ -1719,7 +1720,9 @@ __device__ __forceinline__ void far_wy(double t, double w[4]) {
 // about 32 rows each way: 16 patches of 8 x 8), 8 x 8 x 8 nodes for 32,768 points
 // instead of 16 times 80.  The sums go to the patches' own nodes by
 // interpolation, and the far kernel leaves out the atoms in them.  20,000 atoms
-// on 257^3 points: the far field 8.5 -> 4.4 ms (boxes 1.38, transfer 0.02, patches 3.03).
+// on 257^3 points: the far field 8.5 -> 4.4 ms, and with the patches outside the
+// receptor as strict as k_far_reach has them 5.7 (boxes 1.33, transfer 0.02,
+// patches 4.35).
 __host__ __device__ __forceinline__ constexpr double box_node(int i) {   // Chebyshev nodes, increasing
     constexpr double c[4] = {0.98078528040323044913, 0.83146961230254523708, 0.55557023301960222474,
                              0.19509032201612826785};
@@ -2005,11 +2008,12 @@ __global__ void __launch_bounds__(kReachThreads) k_far_reach(FarParams p, int co
 //
 // Measured against every pair through the table (and, in large boxes, the
 // constant beyond 64 A), at protein density: 20,000 atoms on 257^3 points
-// 62.2 -> 8.6 ms, 5,000 on 127^3 2.00 -> 0.81 ms, 1,849 on 61^3 0.42 -> 0.11 ms.
+// 62.2 -> 8.6 ms (5.7 with the coarse boxes), 5,000 on 127^3 2.00 -> 0.81 ms,
+// 1,849 on 61^3 0.42 -> 0.11 ms.
 // Of the 127^3 launch's wave instructions three quarters are direct pairs (28 %
 // of all pairs), a quarter the nodes; it is bound by the vector unit (65 %
 // busy) and the table reads in LDS (60 %, 3.9 conflict cycles each) together.
-// Eight waves per workgroup instead of four: 0.94 ms, 9.7 ms on 257^3.
+// Eight waves per workgroup instead of four: 0.94 ms, 9.7 ms on 257^3 (for 8.6).
 //
 // KIND: kFarTable, kFarClamped or kFarFlat.  Without the table 3,000 atoms on 81^3
 // points take 336 us for 444.
@@ -2595,10 +2599,11 @@ static bool flat_table(const std::vector<float> &reps) {
 // With the Mehler-Solmajer dielectric the steps decide: they leave 2e-7 of
 // the e map (2-norm, 5,000-atom protein) at 20 A, 5e-7 at 18 A and 8e-7 at 16 A,
 // beside the 6e-7 that FP32 bins of the direct pairs leave.  The floor and the
-// reference charge keep the whole error below the all-pairs sum's (whose
+// reference charge keep the map's error below the all-pairs sum's (whose
 // coordinates were rounded in the grid's frame): 6.2e-7 for 6.9e-7 at 0.25 A (2,743
 // atoms), at 0.375 A 9.5e-7 for 1.07e-6 (5,000 atoms) and 1.28e-6 for 1.31e-6 (20,000,
-// 257^3 points).  One distance for every charge: 3 % less error, 830 us instead of 772
+// 257^3 points).  That is a whole map's, which points in and at the receptor make
+// up; outside it k_far_reach takes the distances of stricter levels.  One distance for every charge: 3 % less error, 830 us instead of 772
 // for 5,000 atoms on 127^3 points, 460 instead of 430 for 3,000 on 81^3 in a constant
 // dielectric.
 static void far_radii(const std::vector<float> &reps, double spacing, int nodes, double half_points,

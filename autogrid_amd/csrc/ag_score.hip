@@ -118,8 +118,8 @@ __global__ void k_score_zero(float *out, long long n) {
 // them, from the L2 cache).  10,000 atoms, 80,000 pairs: 39 us for all four
 // passes; as three launches each (count, scan, scatter) 66 us and the gaps
 // between.  (Pairs a workgroup has spread go out one cache line a clock: 40
-// workgroups of 2,048 take 9.5 us a pass, ten of 8,192 15.)  The host's sort of the 250,000 contributions and their upload took
-// 5.4 ms.
+// workgroups of 2,048 take 9.5 us a pass, ten of 8,192 15.)  The host's sort of
+// the 250,000 contributions and their upload took 5.4 ms.
 constexpr int kSortThreads = 512, kSortPer = 4;
 constexpr int kSortTile = kSortThreads * kSortPer;   // pairs of a workgroup
 constexpr int kSortScanned = 64;
